@@ -25,27 +25,40 @@ struct SoftmaxParams {
 
 constexpr float kLog2e = 1.4426950408889634f;
 
-// reductions over aligned groups of kLanes lanes of a wave
-template <int kLanes = 64>
-NT_DEVICE float wave_max(float v) {
-#pragma unroll
-    for (int off = kLanes / 2; off > 0; off >>= 1) v = fmaxf(v, __shfl_xor(v, off, 64));
+template <bool kIsMax>
+NT_DEVICE float combine(float a, float b) {
+    return kIsMax ? fmaxf(a, b) : a + b;
+}
+
+template <bool kIsMax, int kControl>
+NT_DEVICE float combine_dpp(float v) {
+    return combine<kIsMax>(v, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), kControl, 0xf, 0xf, true)));
+}
+
+// Reduction over aligned groups of kLanes lanes of a wave, the result in every lane: lane permutations inside the vector
+// unit (DPP within 16 lanes, then the two half-row swaps), where shuffles would take six dependent trips through LDS.
+template <bool kIsMax, int kLanes = 64>
+NT_DEVICE float wave_reduce(float v) {
+    v = combine_dpp<kIsMax, 0xb1>(v);                            // quad_perm [1, 0, 3, 2]
+    v = combine_dpp<kIsMax, 0x4e>(v);                            // quad_perm [2, 3, 0, 1]
+    v = combine_dpp<kIsMax, 0x141>(v);                           // row_half_mirror: the other quad of 8 lanes
+    if constexpr (kLanes >= 16) v = combine_dpp<kIsMax, 0x140>(v);  // row_mirror: the other 8 of 16 lanes
+    if constexpr (kLanes >= 32) {
+        const auto r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(unsigned, v), __builtin_bit_cast(unsigned, v), false, false);
+        v = combine<kIsMax>(__builtin_bit_cast(float, (unsigned)r[0]), __builtin_bit_cast(float, (unsigned)r[1]));
+    }
+    if constexpr (kLanes >= 64) {
+        const auto r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, v), __builtin_bit_cast(unsigned, v), false, false);
+        v = combine<kIsMax>(__builtin_bit_cast(float, (unsigned)r[0]), __builtin_bit_cast(float, (unsigned)r[1]));
+    }
     return v;
 }
 
-template <int kLanes = 64>
-NT_DEVICE float wave_sum(float v) {
-#pragma unroll
-    for (int off = kLanes / 2; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-    return v;
-}
-
-// Reduction over the kRowThreads threads that share a segment.  Up to 64 it is a
-// pure wave reduction; for more, partial results cross waves through LDS.
+// Reduction over the kRowThreads threads that share a segment: waves, then partial results across waves through LDS.
 template <int kRowThreads, bool kIsMax>
 NT_DEVICE float group_reduce(float v, float *scratch) {
     constexpr int kLanes = kRowThreads < 64 ? kRowThreads : 64;
-    v = kIsMax ? wave_max<kLanes>(v) : wave_sum<kLanes>(v);
+    v = wave_reduce<kIsMax, kLanes>(v);
     if constexpr (kRowThreads > 64) {
         constexpr int kWaves = kRowThreads / 64;
         const int wave = threadIdx.x >> 6;
@@ -54,7 +67,7 @@ NT_DEVICE float group_reduce(float v, float *scratch) {
         __syncthreads();
         v = scratch[0];
 #pragma unroll
-        for (int w = 1; w < kWaves; ++w) v = kIsMax ? fmaxf(v, scratch[w]) : v + scratch[w];
+        for (int w = 1; w < kWaves; ++w) v = combine<kIsMax>(v, scratch[w]);
     }
     return v;
 }
@@ -65,69 +78,151 @@ struct Vec16 {  // 16 bytes of T
     typedef T type __attribute__((ext_vector_type(16 / sizeof(T))));
 };
 
-// Vector path: unit column strides, 16-byte aligned segments whose length is a
-// multiple of the vector width.  Thread t of a segment's group owns vectors
-// t, t + kRowThreads, ...  (coalesced 16-byte accesses).
+// Segments of unit column stride that fit the registers of the kRowThreads threads that share one: read once, written
+// once, in one launch.  A segment is cut into one part per wave; a part has its own maximum and its own sum of
+// exponentials relative to it, and the parts meet in ONE exchange (shared by all: two floats per wave in LDS, one
+// barrier), so a wave computes as soon as its own loads are back.
+//
+// Thread t of a group owns vectors t, t + kRowThreads, ... (coalesced 16-byte accesses).  The segment may start at any
+// element and have any length: vectors are counted from its first 16-byte boundary, and the up to 2 (W - 1) elements
+// before the first and behind the last whole vector belong to the first threads, one each (two in groups of 8).
+//
+// 2-byte elements are kept as they were read where more than 64 fall to a thread (64 registers then hold 128 of them, so 1024
+// threads hold a segment of 131072): the exponential is computed twice, once for the sum and once for the result, which only
+// pays where floats would not fit (fp16 [64, 50257], 49 elements a thread: 6.5 us on floats, 7.4 computed twice).
+//
+// What bounds it: memory where there are segments for every CU (fp32 4096 x 4096 20.3 us = 6.6 TB/s; fp16 8192 x 4099 21.9 us =
+// 6.1 TB/s, 190 us with element-wise loads; fp16 4096 x 50257 145 us = 5.7 TB/s, 230 us in two sweeps over memory), the
+// arithmetic of the CUs that have a segment where there are few (fp16 [64, 50257] 6.5 us, 11.4 over two launches).
 template <typename T, int kRowThreads, int kVecs>
-__global__ __launch_bounds__(kRowThreads > 256 ? kRowThreads : 256) void softmax_vec_kernel(SoftmaxParams p) {
+__global__ __launch_bounds__(kRowThreads > 256 ? kRowThreads : 256) void softmax_split_in_registers_kernel(SoftmaxParams p) {
     typedef typename Vec16<T>::type vec_t;
     constexpr int W = Vec16<T>::kWidth;
+    typedef vec_t access_t __attribute__((aligned(sizeof(T))));
     constexpr int kGroups = kRowThreads > 256 ? 1 : 256 / kRowThreads;  // segments per workgroup
-    __shared__ float scratch[16];
+    constexpr bool kRaw = sizeof(T) == 2 && kVecs * W > 64;
+    constexpr int kHeld = kRaw ? 1 : kVecs;
+    constexpr int kEdgeElems = (2 * (W - 1) + kRowThreads - 1) / kRowThreads;
+    constexpr int kWaves = kRowThreads > 64 ? kRowThreads / 64 : 1;
+    __shared__ float2_t parts[kWaves];
 
     const int group = threadIdx.x / kRowThreads;
     const int t = threadIdx.x % kRowThreads;
     const int64_t seg = (int64_t)blockIdx.x * kGroups + group;
     const int64_t total = p.rows * p.segments;
-    // whole groups leave together, so the barriers below stay uniform (kGroups == 1 when they exist)
-    const bool active = seg < total;
+    const bool active = seg < total;  // (more than one segment per workgroup: no barriers below)
     const int64_t row = active ? seg / p.segments : 0;
     const int64_t start = active ? (seg % p.segments) * p.block : 0;
     const int len = active ? (int)min(p.block, p.cols - start) : 0;
-    const int nvec = len / W;
 
     const T *src = (const T *)p.in + row * p.in_row_stride + start;
     T *dst = (T *)p.out + row * p.out_row_stride + start;
+    const int head = min(len, (int)((0 - (uintptr_t)src) & 15) / (int)sizeof(T));
+    const int nvec = (len - head) / W;
+    const int tail_first = head + nvec * W;
+    const auto edge_index = [&](int j) {  // -> element, len and beyond: none
+        const int e = j * kRowThreads + t;
+        return e < head ? e : tail_first + (e - head);
+    };
 
-    float x[kVecs][W];
+    vec_t raw[kRaw ? kVecs : 1];
+    float x[kHeld][W];
+    float edge[kEdgeElems];
     float m = -INFINITY;
+#pragma unroll
+    for (int j = 0; j < kEdgeElems; ++j) {
+        const int e = edge_index(j);
+        edge[j] = e < len ? (float)src[e] : -INFINITY;
+    }
 #pragma unroll
     for (int j = 0; j < kVecs; ++j) {
         const int v = j * kRowThreads + t;
+        vec_t in;
         if (v < nvec) {
-            vec_t raw = *((const vec_t *)src + v);  // (a non-temporal load here costs 7-20 % of the rate; the non-temporal store below gains)
-#pragma unroll
-            for (int e = 0; e < W; ++e) {
-                x[j][e] = (float)raw[e];
-                m = fmaxf(m, x[j][e]);
-            }
+            in = *(const access_t *)(src + head + (int64_t)v * W);  // (a non-temporal load here costs 7-20 % of the rate; the non-temporal store below gains)
         } else {
 #pragma unroll
-            for (int e = 0; e < W; ++e) x[j][e] = -INFINITY;
+            for (int e = 0; e < W; ++e) in[e] = (T)-INFINITY;
+        }
+        if constexpr (kRaw) {
+            raw[j] = in;
+        } else {
+#pragma unroll
+            for (int e = 0; e < W; ++e) x[j][e] = (float)in[e];
         }
     }
-    m = group_reduce<kRowThreads, true>(m, scratch);
-    const float shift = m * kLog2e;
+#pragma unroll
+    for (int j = 0; j < kEdgeElems; ++j) m = fmaxf(m, edge[j]);
+#pragma unroll
+    for (int j = 0; j < kVecs; ++j)
+#pragma unroll
+        for (int e = 0; e < W; ++e) m = fmaxf(m, kRaw ? (float)raw[kRaw ? j : 0][e] : x[kRaw ? 0 : j][e]);
+    // the compiler must not keep the converted values from one sweep over the registers to the next (two floats per register)
+    const auto forget_conversions = [&] {
+        if constexpr (kRaw) {
+#pragma unroll
+            for (int j = 0; j < kVecs; ++j) {
+                int4_t bits = __builtin_bit_cast(int4_t, raw[j]);
+                asm("" : "+v"(bits));
+                raw[j] = __builtin_bit_cast(vec_t, bits);
+            }
+        }
+    };
+    forget_conversions();
+    m = wave_reduce<true, (kRowThreads < 64 ? kRowThreads : 64)>(m);
+    // (a part without a finite element has nothing to subtract: its exponentials are zeros)
+    const float shift = m == -INFINITY && kWaves > 1 ? 0.0f : m * kLog2e;
     float s = 0.0f;
+    // exp(x - m) as exp2(x * log2e - m * log2e); padding (-inf) gives 0
+    const auto exponential = [&](float value) { return __builtin_amdgcn_exp2f(fmaf(value, kLog2e, -shift)); };
 #pragma unroll
     for (int j = 0; j < kVecs; ++j)
 #pragma unroll
         for (int e = 0; e < W; ++e) {
-            // exp(x - m) as exp2(x * log2e - m * log2e); padding (-inf) gives 0
-            x[j][e] = __builtin_amdgcn_exp2f(fmaf(x[j][e], kLog2e, -shift));
-            s += x[j][e];
+            if constexpr (kRaw) {
+                s += exponential((float)raw[j][e]);
+            } else {
+                x[j][e] = exponential(x[j][e]);
+                s += x[j][e];
+            }
         }
-    s = group_reduce<kRowThreads, false>(s, scratch);
-    const float inv = 1.0f / s;
+#pragma unroll
+    for (int j = 0; j < kEdgeElems; ++j) {
+        edge[j] = exponential(edge[j]);
+        s += edge[j];
+    }
+    forget_conversions();
+    s = wave_reduce<false, (kRowThreads < 64 ? kRowThreads : 64)>(s);
+    float factor;
+    if constexpr (kWaves > 1) {
+        const int wave = threadIdx.x >> 6;
+        if ((threadIdx.x & 63) == 0) parts[wave] = float2_t{m, s};
+        __syncthreads();
+        float total_max = -INFINITY;
+#pragma unroll
+        for (int w = 0; w < kWaves; ++w) total_max = fmaxf(total_max, parts[w][0]);
+        const auto rescale = [&](float part_max) { return part_max == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f((part_max - total_max) * kLog2e); };
+        float sum = 0.0f;
+#pragma unroll
+        for (int w = 0; w < kWaves; ++w) sum += parts[w][1] * rescale(parts[w][0]);
+        factor = rescale(m) / sum;
+    } else {
+        factor = 1.0f / s;
+    }
 #pragma unroll
     for (int j = 0; j < kVecs; ++j) {
         const int v = j * kRowThreads + t;
         if (v < nvec) {
             vec_t o;
 #pragma unroll
-            for (int e = 0; e < W; ++e) o[e] = (T)(x[j][e] * inv);
-            __builtin_nontemporal_store(o, (vec_t *)dst + v);
+            for (int e = 0; e < W; ++e) o[e] = (T)((kRaw ? exponential((float)raw[kRaw ? j : 0][e]) : x[kRaw ? 0 : j][e]) * factor);
+            __builtin_nontemporal_store(o, (access_t *)(dst + head + (int64_t)v * W));
         }
+    }
+#pragma unroll
+    for (int j = 0; j < kEdgeElems; ++j) {
+        const int e = edge_index(j);
+        if (e < len) dst[e] = (T)(edge[j] * factor);
     }
 }
 
@@ -417,15 +512,16 @@ __global__ __launch_bounds__(kSplitThreads) void softmax_split_finish_kernel(Sof
     }
 }
 
-// true when the segments were served by the two launches over parts.  `in_registers`: the segments are short
-// enough for the kernels that read them once (those win unless too few workgroups are left to fetch: measured
-// fp32 [128, 65536] 13 us against 18 us in parts, [16, 65536] 9.1 against 8.1, [16, 262144] fp16 77 against 12).
+// true when the segments were served by the two launches over parts.  `in_registers`: the segments are short enough for
+// the kernel that reads them once in one launch; that one wins unless a few segments of its longest leave most CUs
+// with nothing to compute (fp16 [1, 131072] 12.0 us against 7.8 in parts, [16, 100000] 10.5 against 8.9, [64, 131072] 13.3 against
+// 12.6; but [4, 65536] 6.2 against 7.0, [64, 50257] 6.5 against 11.4, fp32 [16, 50257] 6.4 against 7.4, [128, 50257] 11.0 against 15.7).
 template <typename T>
 bool run_split(const SoftmaxParams &p, int64_t len, bool in_registers, hipStream_t stream, hipError_t *status) {
     const int64_t total = p.rows * p.segments;
     const int64_t bytes = len * (int64_t)sizeof(T);
     if (total > 128) return false;
-    if (in_registers ? (bytes < (1 << 18) || total > 16) : bytes < (1 << 16)) return false;
+    if (in_registers ? (sizeof(T) == 4 || len <= 65536 || total > 64) : bytes < (1 << 16)) return false;
     const int64_t wanted = std::min<int64_t>(kSplitThreads, std::max<int64_t>(2, 1024 / total));  // (the finishing launch reads one part per thread)
     int64_t part_len = std::max<int64_t>(4096, (((len + wanted - 1) / wanted + 2047) / 2048) * 2048);
     const int64_t parts = (len + part_len - 1) / part_len;
@@ -447,22 +543,37 @@ bool run_split(const SoftmaxParams &p, int64_t len, bool in_registers, hipStream
 }
 
 template <typename T, int kRowThreads>
-hipError_t launch_vec(const SoftmaxParams &p, int vecs_needed, hipStream_t stream) {
+hipError_t launch_in_registers(const SoftmaxParams &p, int64_t len, hipStream_t stream) {
     const int64_t total = p.rows * p.segments;
     constexpr int kGroups = kRowThreads > 256 ? 1 : 256 / kRowThreads;
     const dim3 grid((unsigned)((total + kGroups - 1) / kGroups)), block(kRowThreads > 256 ? kRowThreads : 256);
-    note_launch(kLaunchSoftmax, kRowThreads, "softmax_vec_kernel, 16-byte vectors, this many threads per row segment");
-    if (vecs_needed <= 1)
-        softmax_vec_kernel<T, kRowThreads, 1><<<grid, block, 0, stream>>>(p);
-    else if (vecs_needed <= 2)
-        softmax_vec_kernel<T, kRowThreads, 2><<<grid, block, 0, stream>>>(p);
-    else if (vecs_needed <= 4)
-        softmax_vec_kernel<T, kRowThreads, 4><<<grid, block, 0, stream>>>(p);
-    else if (vecs_needed <= 8)
-        softmax_vec_kernel<T, kRowThreads, 8><<<grid, block, 0, stream>>>(p);
-    else
-        softmax_vec_kernel<T, kRowThreads, 16><<<grid, block, 0, stream>>>(p);
-    return hipGetLastError();
+    const int64_t vecs = (len / Vec16<T>::kWidth + kRowThreads - 1) / kRowThreads;  // per thread
+    note_launch(kLaunchSoftmax, kRowThreads, "softmax_split_in_registers_kernel, one launch, this many threads per row segment, one part per wave");
+#define NT_SOFTMAX_VECS(N) \
+    if (vecs <= N) { \
+        softmax_split_in_registers_kernel<T, kRowThreads, N><<<grid, block, 0, stream>>>(p); \
+        return hipGetLastError(); \
+    }
+    // (a thread computes all its vectors, also those behind the end of a segment: steps of one where a step is most of the work)
+    NT_SOFTMAX_VECS(1)
+    NT_SOFTMAX_VECS(2)
+    if constexpr (kRowThreads >= 32) {
+        NT_SOFTMAX_VECS(3)
+    }
+    if constexpr (kRowThreads >= 64) {
+        NT_SOFTMAX_VECS(4)
+        NT_SOFTMAX_VECS(5)
+        NT_SOFTMAX_VECS(6)
+        NT_SOFTMAX_VECS(7)
+        NT_SOFTMAX_VECS(8)
+    }
+    if constexpr (kRowThreads >= 1024) {
+        NT_SOFTMAX_VECS(10)
+        NT_SOFTMAX_VECS(12)
+        NT_SOFTMAX_VECS(16)
+    }
+#undef NT_SOFTMAX_VECS
+    return hipErrorInvalidValue;
 }
 
 template <typename T, int kRowThreads, int kElems>
@@ -483,11 +594,9 @@ int run_softmax(const SoftmaxParams &p, int variant, hipStream_t stream) {
     if (total == 0 || p.cols == 0) return 0;
     if (total > 0x7fffffffll) return NINETOOTHED_NO_KERNEL;
     const int64_t len = p.block < p.cols ? p.block : p.cols;
-    const bool vector_ok = p.in_col_stride == 1 && p.out_col_stride == 1 && p.cols % W == 0 &&
-                           (p.segments == 1 || p.block % W == 0) && p.in_row_stride % W == 0 &&
-                           p.out_row_stride % W == 0 && ((uintptr_t)p.in & 15) == 0 && ((uintptr_t)p.out & 15) == 0;
+    const bool unit_columns = p.in_col_stride == 1 && p.out_col_stride == 1;
     // rows of up to 64 bytes, many of them: a thread per row
-    if (variant == 0 && p.segments == 1 && p.in_col_stride == 1 && p.out_col_stride == 1 && p.cols * (int64_t)sizeof(T) <= 64 && p.rows >= 4096 &&
+    if (variant == 0 && p.segments == 1 && unit_columns && p.cols * (int64_t)sizeof(T) <= 64 && p.rows >= 4096 &&
         (p.rows + 255) / 256 <= 0x7fffffffll) {
         const uint64_t bits = (uint64_t)(p.cols * sizeof(T)) | (uint64_t)(p.in_row_stride * (int64_t)sizeof(T)) | (uint64_t)(p.out_row_stride * (int64_t)sizeof(T)) |
                               (uint64_t)(uintptr_t)p.in | (uint64_t)(uintptr_t)p.out;  // what every piece's address and size is a multiple of
@@ -498,30 +607,30 @@ int run_softmax(const SoftmaxParams &p, int variant, hipStream_t stream) {
             if (p.cols <= 8) return (int)launch_thread_per_row<T, 2>(p, stream);  // (up to 32 pieces of one element would not stay in registers)
         }
     }
-    // (a row of 16 vectors of 2-byte elements per thread -- 128 floats -- does not stay in the registers of 1024 threads)
-    const bool in_registers = vector_ok && len <= (int64_t)1024 * 64;
+    // segments that 1024 threads hold in registers: 64 of them per thread (2-byte elements as they are, two per register)
+    const bool in_registers = unit_columns && len <= (int64_t)1024 * 16 * W;
     if (variant == 0) {
         hipError_t status = hipSuccess;
         if (run_split<T>(p, len, in_registers, stream, &status)) return (int)status;
     }
-    if (in_registers || (vector_ok && variant != 0 && len <= (int64_t)1024 * 16 * W)) {
-        const bool wave_fits = len <= (int64_t)64 * 16 * W;
-        bool use_wave = wave_fits && len <= (int64_t)64 * 8 * W;  // default: keep <= 8 vectors per lane
-        // few segments: a workgroup each, so that more of the chip has something to fetch
-        if (use_wave && len > (int64_t)64 * W && total < 4096) use_wave = false;
-        if (variant == 1 && wave_fits) use_wave = true;
-        if (variant == 2) use_wave = false;
+    if (in_registers) {
         const int64_t nvec = len / W;
-        if (variant == 0 && p.segments == 1) {  // short rows: 8, 16 or 32 lanes each, one vector per lane
-            if (nvec <= 8) return (int)launch_vec<T, 8>(p, 1, stream);
-            if (nvec <= 16) return (int)launch_vec<T, 16>(p, 1, stream);
-            if (nvec <= 32) return (int)launch_vec<T, 32>(p, 1, stream);
+        // Threads per segment.  Few vectors each keep a wave's work short where a launch has many segments; many threads fetch a
+        // segment sooner where it has few.  Measured (us, threads per segment: time): fp16 30000 x 131 16: 4.8, 32: 6.7; 30000 x 515
+        // 32: 10.8, 64: 12.4; 20000 x 1000 32: 13.8, 64: 13.1, 256: 22; 8192 x 4096 64: 20.6, 256: 20.9, 512: 24; 300 x 4099 64: 3.9,
+        // 256: 3.6; fp32 5000 x 3000 256: 19.0, 512: 19.9; 8192 x 4096 64: 47.4, 256: 45.2, 512: 44.0; 4000 x 8195 512: 48.0, 1024: 45.0; fp16
+        // 11832 x 4152 256: 33.5, 512: 44.6; 4000 x 12289 256: 33.4, 512: 32.8, 1024: 39.4; 4000 x 32000 512: 86.6, 1024: 89.5; 4096 x 50257
+        // 512: 149, 1024: 145
+        if (variant == 0 && p.segments == 1) {
+            if (nvec <= 8) return (int)launch_in_registers<T, 8>(p, len, stream);
+            if (nvec <= 32) return (int)launch_in_registers<T, 16>(p, len, stream);
+            if (nvec <= 96) return (int)launch_in_registers<T, 32>(p, len, stream);
         }
-        if (use_wave) return (int)launch_vec<T, 64>(p, (int)((nvec + 63) / 64), stream);
-        // more than 8 vectors per thread of a 256-thread workgroup: 1024 threads (registers per thread, not LDS, hold the row)
-        if (nvec > 256 * 8 && variant != 2) return (int)launch_vec<T, 1024>(p, (int)((nvec + 1023) / 1024), stream);
-        if (nvec > 256 * 16) return (int)launch_vec<T, 1024>(p, (int)((nvec + 1023) / 1024), stream);
-        return (int)launch_vec<T, 256>(p, (int)((nvec + 255) / 256), stream);
+        const bool one_wave = nvec <= 512 && (variant == 1 || (variant == 0 && (total >= 4096 || nvec <= 64)));
+        if (one_wave) return (int)launch_in_registers<T, 64>(p, len, stream);
+        if (nvec <= (sizeof(T) == 4 ? 768 : 2048)) return (int)launch_in_registers<T, 256>(p, len, stream);
+        if (nvec <= (sizeof(T) == 4 ? 2048 : 4096)) return (int)launch_in_registers<T, 512>(p, len, stream);
+        return (int)launch_in_registers<T, 1024>(p, len, stream);
     }
     // element by element (any strides / alignment): as many threads per segment as keep every thread at
     // 4 .. 16 elements, from 8 lanes of a wave to a workgroup of 1024
@@ -536,7 +645,7 @@ int run_softmax(const SoftmaxParams &p, int variant, hipStream_t stream) {
     if (len <= 256 * 32) return (int)launch_elem<T, 256, 64>(p, stream);
     if (len <= 1024 * 16) return (int)launch_elem<T, 1024, 16>(p, stream);
     note_launch(kLaunchSoftmax, kLoopThreads, "softmax_loop_kernel, two sweeps over a long row segment");
-    if (p.in_col_stride == 1 && p.out_col_stride == 1)
+    if (unit_columns)
         softmax_loop_kernel<T, true><<<dim3((unsigned)total), dim3(kLoopThreads), 0, stream>>>(p);
     else
         softmax_loop_kernel<T, false><<<dim3((unsigned)total), dim3(kLoopThreads), 0, stream>>>(p);

@@ -589,6 +589,33 @@ def test_softmax_few_long_rows_are_cut_into_parts(dtype):
         assert torch.allclose(out.float(), expected, **tolerance), replay
 
 
+@pytest.mark.parametrize("dtype", (torch.float32, torch.float16, torch.bfloat16))
+@pytest.mark.parametrize("vectors", (1, 8, 9, 32, 33, 96, 97, 512, 513, 768, 769, 2048, 2049, 4096, 4097, 8192, 8193, 12289, 16384))
+def test_softmax_in_registers_at_the_edges_of_its_thread_counts(vectors, dtype):
+    """Segments held in registers, at the numbers of 16-byte vectors where the threads per segment or the vectors per
+    thread change: a whole number of vectors, and one element less.  Input and output start at different elements of
+    their 16 bytes and lie in poisoned buffers; one row's first half is masked out (waves without a finite element)."""
+    from ninetoothed_amd import runtime
+
+    # fp32 in, a dozen roundings of at most 2^-23 each between input and result; 16-bit results are rounded once more
+    tolerance = {torch.float32: dict(rtol=1e-5, atol=1e-7), torch.float16: dict(rtol=2e-3, atol=1e-6), torch.bfloat16: dict(rtol=1.6e-2, atol=1e-6)}[dtype]
+    width = 16 // torch.empty(0, dtype=dtype).element_size()
+    m = 70 if vectors > 8192 else 5  # (up to 64 of the longest 2-byte segments are cut into parts over two launches)
+    for n, first_in, first_out in ((vectors * width, 0, 0), (vectors * width - 1, 3, 1)):
+        source = torch.full((m, n + 13), float("inf"), dtype=dtype, device="cuda")
+        x = source[:, first_in : first_in + n]
+        x.copy_(torch.randn(m, n, device="cuda").to(dtype))
+        x[1, : n // 2] = float("-inf")
+        buffer = torch.full((m, n + 13), 7.0, dtype=dtype, device="cuda")
+        out = buffer[:, first_out : first_out + n]
+        kernel = ninetoothed.make(programs.softmax.arrangement, programs.softmax.application, programs.softmax.tensors())
+        kernel(x, out, BLOCK_SIZE=1 << (n - 1).bit_length() if n > 1 else 1)
+        _native_only(kernel, "launch_nt_softmax")
+        assert "softmax_split_in_registers_kernel" in runtime.last_launch(), runtime.last_launch()
+        assert torch.allclose(out.float(), torch.softmax(x.float(), dim=-1), **tolerance), n
+        assert bool((buffer[:, :first_out] == 7.0).all()) and bool((buffer[:, first_out + n :] == 7.0).all())
+
+
 def test_softmax_baseline_shape_properties():
     x = torch.randn(4096, 4096, device="cuda")
     out = _softmax(x)
