@@ -14,6 +14,7 @@
 #include "conv2d.h"
 #include "gemm_fast.h"
 #include "gemm_generic.h"
+#include "gemm_skinny.h"
 #include "tune.h"
 #include "workspace.h"
 
@@ -101,6 +102,7 @@ void fill_params(GemmParams &p, const GemmProblem &q, int bm, int bn) {
     p.bias_vector = q.bias != nullptr && q.sin == 1 && q.sim % 8 == 0 && ((uintptr_t)q.bias & 15) == 0 && q.n % 8 == 0 && (q.batch == 1 || q.bias_batch % 8 == 0);
     p.c_vector = ((uintptr_t)q.c & 15) == 0 && q.scm % 8 == 0 && q.n % 8 == 0 && (q.batch == 1 || q.c_batch % 8 == 0);
     p.kt_per_split = 0;
+    p.out_float = q.out_dtype == NINETOOTHED_FLOAT32;
     p.batch = q.batch;
     p.a_batch = q.a_batch;
     p.b_batch = q.b_batch;
@@ -257,6 +259,43 @@ hipError_t split_launch(const GemmProblem &q, hipStream_t stream) {
     return split_launch_typed<bf16_t, BM, BN, BK, WM, WN, kStages, kOcc>(q, stream);
 }
 
+// ---- skinny products: at most 64 rows against a k-contiguous rhs, the k range over the waves of a workgroup ----
+bool skinny_accepts(const GemmProblem &q) { return q.m <= 64 && q.batch == 1 && b_is_transposed(q) && fast_accepts<64, 64, 64, 4, true>(q); }
+
+template <typename T, int MB, int NB, int kWaves, int kStages>
+hipError_t skinny_launch_rows(const GemmProblem &q, hipStream_t stream) {
+    GemmParams p;
+    fill_params(p, q, MB * 16, NB * 16);
+    // a B that the 256 MiB Infinity Cache cannot hold beside a program's other tensors is streamed past the caches (16 x 50256 x
+    // 4096 71 us, 79 otherwise); a smaller one may still lie there from its last use (16 x 4096 x 2048
+    // 5.1 us, 5.6 past the caches; 24 x 8192 x 4096 12.8 against 15.9)
+    if ((int64_t)q.n * q.sbn * 2 > (int64_t)128 << 20) gemm_skinny_kernel<T, MB, NB, kWaves, kStages, 2><<<dim3(p.tiles_n), dim3(kWaves * 64), 0, stream>>>(p);
+    else gemm_skinny_kernel<T, MB, NB, kWaves, kStages, 0><<<dim3(p.tiles_n), dim3(kWaves * 64), 0, stream>>>(p);
+    return hipGetLastError();
+}
+
+template <typename T, int NB>
+hipError_t skinny_launch_typed(const GemmProblem &q, hipStream_t stream) {
+    // (16 columns per workgroup: four waves with rings of four stages, 16-40 KiB each; 32 columns: with more rows than
+    // 16 two waves, so that more than one workgroup fits the LDS of a CU -- 32 x 50256 x 4096 82 us with two, 95 with four)
+    if constexpr (NB == 1) {
+        if (q.m <= 16) return skinny_launch_rows<T, 1, NB, 4, 4>(q, stream);
+        if (q.m <= 32) return skinny_launch_rows<T, 2, NB, 4, 4>(q, stream);
+        if (q.m <= 48) return skinny_launch_rows<T, 3, NB, 4, 4>(q, stream);
+        return skinny_launch_rows<T, 4, NB, 4, 4>(q, stream);
+    } else {
+        if (q.m <= 16) return skinny_launch_rows<T, 1, NB, 4, 3>(q, stream);
+        if (q.m <= 32) return skinny_launch_rows<T, 2, NB, 2, 3>(q, stream);
+        if (q.m <= 48) return skinny_launch_rows<T, 3, NB, 2, 3>(q, stream);
+        return skinny_launch_rows<T, 4, NB, 2, 3>(q, stream);
+    }
+}
+
+template <int NB>
+hipError_t skinny_launch(const GemmProblem &q, hipStream_t stream) {
+    return q.dtype == NINETOOTHED_FLOAT16 ? skinny_launch_typed<half_t, NB>(q, stream) : skinny_launch_typed<bf16_t, NB>(q, stream);
+}
+
 bool generic_accepts(const GemmProblem &q) {
     if (q.batch < 1 || q.batch > 65535) return false;  // (the batch is the grid's y extent)
     if (q.dtype == NINETOOTHED_FLOAT8_E5M2 && q.batch != 1) return false;
@@ -410,7 +449,7 @@ hipError_t generic_launch(const GemmProblem &q, hipStream_t stream) {
 enum InstanceIndex {
     kAnyStride, k256x256x32, k256x256x64, k128x128x64, k64x64x64, k128x256x32,
     kTail256x256x32, kTail128x256x32, kTail128x128x64, kTail64x64x64, kSplit64x64x64, kSplit128x128x64,
-    kSplit128x256x32, kSplit256x256x32,
+    kSplit128x256x32, kSplit256x256x32, kSkinny16, kSkinny32,
 };
 
 const GemmInstance kInstances[] = {
@@ -428,6 +467,8 @@ const GemmInstance kInstances[] = {
     NT_SPLIT_INSTANCE(128, 128, 64, 2, 2, 2, 2),
     NT_SPLIT_INSTANCE(128, 256, 32, 1, 4, 3, 2),  // a few hundred rows against a wide rhs: 64 to 160 large tiles
     NT_SPLIT_INSTANCE(256, 256, 32, 2, 4, 5, 2),
+    {"64x16x64 skinny, split-k over the waves of a workgroup", 64, 16, 64, skinny_accepts, skinny_launch<1>},
+    {"64x32x64 skinny, split-k over the waves of a workgroup", 64, 32, 64, skinny_accepts, skinny_launch<2>},
 #ifdef NT_GEMM_ABLATION
 #define NT_LOAD_INSTANCE(BM, BN, BK, WM, WN, ST, OCC, LD, AUX) \
     {#BM "x" #BN "x" #BK " waves " #WM "x" #WN " stages " #ST " load " #LD " aux " #AUX, BM, BN, BK, fast_accepts<BM, BN, BK, ST>, fast_launch<BM, BN, BK, WM, WN, ST, OCC, 0, LD, AUX>}
@@ -444,7 +485,7 @@ const GemmInstance kInstances[] = {
 #endif
 };
 constexpr int kNumInstances = sizeof(kInstances) / sizeof(kInstances[0]);
-static_assert(kNumInstances > kSplit256x256x32, "InstanceIndex names the first instances of the table");
+static_assert(kNumInstances > kSkinny32, "InstanceIndex names the first instances of the table");
 
 inline bool is_split(int instance) { return instance >= kSplit64x64x64 && instance <= kSplit256x256x32; }
 
@@ -474,6 +515,25 @@ int lookup_tuned(const GemmProblem &q) {
     return choice >= 0 && choice < kNumInstances ? choice : -1;
 }
 
+// The skinny instance that a product runs on whatever has been timed for it, or -1: timing launches find B in the L2 that
+// the launch before has left it in, a program that works through its layers finds it in memory or, at best, in the Infinity
+// Cache, where these kernels stand better (32 x 14336 x 4096: 18.9 us on tiles with B in L2, 29.0 without; 22.9 and 24.9 on
+// 32 columns per workgroup).  The lines lie where the tile instances win with B in the Infinity Cache (us, tiles / 16 columns /
+// 32 columns): m = 16: 4096 x 4096 13.3 / 8.0 / 10.8; 8192 x 4096 15.6 / 12.3 / 11.8; 8192 x 8192 32.5 / 24.1 / 43.5; 16384 x 4096 30.9 /
+// 25.2 / 21.9; 12288 x 2048 10.5 / 11.3 / 11.4; m = 40: 2048 x 2048 6.3 / 5.8 / 8.0; 2048 x 512 3.9 / 4.4 / 4.5; 6144 x 4096 17.0 / 16.5 /
+// 13.8; 12288 x 4096 25.9 / 34.3 / 28.0; m = 64: 4096 x 2048 9.8 / 8.8 / 9.3; 2048 x 1024 4.5 / 5.2 / 5.8; 4096 x 8192 19.4 / 24.0 / 38.1.
+int skinny_choice(const GemmProblem &q) {
+    if (!kInstances[kSkinny16].accepts(q)) return -1;
+    const bool long_k = q.k > 4096;
+    if (q.m <= 32) {
+        if (q.n <= 4096 || long_k) return kSkinny16;
+        return q.n <= 8192 || q.k >= 4096 ? (int)kSkinny32 : -1;
+    }
+    if (q.k < (q.m <= 48 ? 1024 : 2048)) return -1;
+    if (q.n <= 4096) return q.m <= 48 || !long_k || q.n <= 1024 ? (int)kSkinny16 : -1;
+    return q.n <= 8192 && q.k > 2048 && !long_k ? (int)kSkinny32 : -1;
+}
+
 // Untuned choice: the largest direct-to-LDS tile that still gives every CU a
 // tile (256 CUs), falling back to smaller tiles, then to the any-stride kernel.
 int heuristic_choice(const GemmProblem &q, int bm, int bn, int bk) {
@@ -497,6 +557,7 @@ int heuristic_choice(const GemmProblem &q, int bm, int bn, int bk) {
     // (64 x 64 tiles of the product: where they fill the chip, a skinny product runs on them in one pass -- 256 x 4096 x 4096
     // 19 us against 27 with K in parts of 128 x 128 tiles, 128 x 4096 x 14336 33 against 42 -- and tiles that the product
     // fills to less than half along M or N are passed over: 64 x 4096 x 128256 259 us on 256 x 256 tiles, 220 on 64 x 64)
+    if (const int skinny = skinny_choice(q); skinny >= 0) return skinny;
     const int64_t tiles_64 = (int64_t)((q.m + 63) / 64) * ((q.n + 63) / 64);
     const bool small_tiles_fill_the_chip = q.batch == 1 && tiles_64 >= 256 && kInstances[kTail64x64x64].accepts(q);
     const auto few_tiles = [&](int instance) {
@@ -840,7 +901,8 @@ int run_gemm(hipStream_t stream, const GemmProblem &q, int bm, int bn, int bk, b
         if (widened != NINETOOTHED_NO_KERNEL) return widened;
     }
     int choice = -1;
-    if ((bm <= 0 || bn <= 0) && q.batch == 1) choice = lookup_tuned(q);  // (tuned choices are recorded for single products)
+    if (bm <= 0 && bn <= 0 && bk <= 0) choice = skinny_choice(q);
+    if (choice < 0 && (bm <= 0 || bn <= 0) && q.batch == 1) choice = lookup_tuned(q);  // (tuned choices are recorded for single products)
     if (choice < 0 || !kInstances[choice].accepts(q)) choice = heuristic_choice(q, bm, bn, bk);
     if (choice < 0) return NINETOOTHED_NO_KERNEL;
     if (choice == kAnyStride && may_copy) {
@@ -994,6 +1056,11 @@ NineToothedResult nt_tune_gemm(NineToothedStream stream_, NineToothedTensor inpu
     GemmProblem q = output_by_columns(given) ? transposed_problem(given) : given;
     int best = -1;
     float best_time = 0.0f;
+    if (skinny_choice(q) >= 0) {  // (not chosen by timing)
+        if (best_config) *best_config = -2;
+        if (best_ms) *best_ms = 0.0f;
+        return 0;
+    }
     // A problem that a single instance accepts has nothing to time.  Operands that only the any-stride kernel reads
     // in place run on dense copies (launch_nt_matmul / launch_nt_addmm): then the product on the copies is what
     // gets timed and recorded, under its own key, where the launch functions look it up.
@@ -1260,6 +1327,6 @@ NineToothedResult nt_tune_conv2d(NineToothedStream stream, NineToothedTensor inp
 void nt_debug_set_tile_order(int order) { g_tile_order = order; }
 #endif
 
-const char *nt_version(void) { return "nt_hip 0.1 gfx950"; }
+const char *nt_version(void) { return "nt_hip 0.2 gfx950"; }
 
 }  // extern "C"

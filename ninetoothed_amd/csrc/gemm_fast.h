@@ -33,6 +33,7 @@ struct GemmParams {
     int bias_vector;  // addmm input readable with aligned 16-byte loads along N
     int order;  // tile order: 0 = XCD-aware strips of 8 tile rows; other values are measurement aids
     int kt_per_split;  // split-K instances: k tiles per part (the grid holds tiles * parts workgroups)
+    int out_float;     // skinny kernel: C holds fp32 (the tile kernels have it as a template parameter)
     int c_vector;      // rows of C take aligned 16-byte stores (else, in the instances with tails: element stores)
     // batch > 1: the grid holds tiles * batch workgroups; product b uses the operands moved by these element strides
     int batch;

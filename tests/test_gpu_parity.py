@@ -1927,6 +1927,53 @@ def test_gemm_transposed_rhs_any_number_of_columns(m, n, k, dtype):
 
 
 @pytest.mark.parametrize("dtype", (torch.float16, torch.bfloat16))
+@pytest.mark.parametrize("m, n, k", ((1, 1, 8), (15, 16, 64), (16, 17, 56), (17, 33, 72), (32, 31, 248), (33, 48, 256), (48, 64, 264), (49, 100, 1032), (64, 515, 776), (7, 2051, 4104)))
+def test_gemm_skinny_instances_at_the_edges_of_their_tiles(m, n, k, dtype):
+    """At most 64 rows against `w.T`: every number of 16-row blocks, partial blocks of rows and columns, numbers of
+    64-wide pieces of K around the four (two) waves and the depth of their rings, a partial last piece.  Element-type,
+    fp32 and addmm outputs inside sentinels; the operands lie in Inf-filled buffers with row pitches of their own."""
+    from ninetoothed_amd import runtime
+
+    lib = runtime.library()
+    tag = runtime.DATA_TYPE_INDEX["fp16" if dtype == torch.float16 else "bf16"]
+    null = runtime.ArgumentTensor.null()
+    beta, alpha = runtime.ArgumentTensor.from_scalar(0.5), runtime.ArgumentTensor.from_scalar(2.0)
+    # (as in test_gemm_split_k: rtol = atol = 1e-2 against the fp32 product; with a bias one ulp of the product, which is rounded first)
+    biased = dict(rtol=2e-2, atol=2e-2 * max(k / 512, 1) ** 0.5) if dtype == torch.bfloat16 else dict(rtol=1e-2, atol=1e-2 * max(k / 512, 1) ** 0.5)
+    wide_a = torch.full((m + 1, k + 16), float("inf"), dtype=dtype, device="cuda")
+    wide_w = torch.full((n + 1, k + 8), float("inf"), dtype=dtype, device="cuda")
+    a, w = wide_a[:m, :k], wide_w[:n, :k]
+    a.copy_(torch.randn(m, k, device="cuda"))
+    w.copy_(torch.randn(n, k, device="cuda"))
+    bias = torch.randn(m, n, dtype=dtype, device="cuda")
+    product = a.float() @ w.float().t()
+    served = 0
+    for out_dtype, with_bias in ((dtype, False), (torch.float32, False), (dtype, True)):
+        buffer = torch.full((m + 1, n + 5), 7.0, dtype=out_dtype, device="cuda")
+        out = buffer[:m, :n]
+        tensors = [runtime.ArgumentTensor.from_torch_tensor(t) for t in (bias, a, w.t(), out)]
+        if n == 1:  # (a dimension of one element has no stride of its own)
+            tensors[2] = runtime.ArgumentTensor.from_layout(w.data_ptr(), (k, 1), (1, k + 8))
+        expected = 0.5 * bias.float() + 2.0 * product.to(dtype).float() if with_bias else product
+        for instance, name in enumerate(runtime.gemm_config_names()):
+            if "skinny" not in name:
+                continue
+            out.fill_(float("nan"))
+            result = lib.launch_nt_gemm_config(
+                runtime.current_stream(), instance, tensors[0] if with_bias else null, tensors[1], tensors[2], beta if with_bias else null,
+                alpha if with_bias else null, tensors[3], tag, runtime.DATA_TYPE_INDEX["fp32"] if out_dtype == torch.float32 else tag,
+            )
+            assert result == 0, name
+            served += 1
+            assert torch.allclose(out.float(), expected, **(biased if with_bias else HALF_TOL)), (name, out_dtype, with_bias)
+            assert bool((buffer[m:] == 7.0).all()) and bool((buffer[:, n:] == 7.0).all()), name
+    assert served == 6
+    out = torch.full((m, n), float("nan"), dtype=dtype, device="cuda")
+    _matmul_kernel()(a, w.t(), out)
+    assert torch.allclose(out.float(), product, **HALF_TOL)
+
+
+@pytest.mark.parametrize("dtype", (torch.float16, torch.bfloat16))
 @pytest.mark.parametrize("m, n, k", ((1, 2048, 4096), (16, 1024, 8192), (64, 520, 2056), (300, 200, 4104), (512, 512, 16384), (129, 136, 256), (768, 1032, 4096),
                                      (33, 515, 8192), (16, 1001, 4096), (100, 301, 5000), (7, 50, 2048)))
 def test_gemm_split_k(m, n, k, dtype):
