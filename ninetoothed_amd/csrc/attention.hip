@@ -39,8 +39,8 @@ struct AttentionParams {
     // blocks [s * blocks_per_part, ...) and writes a normalised fp32 partial output and the base-2
     // logarithm of its softmax denominator (times 2^max) to scratch memory, which a second kernel merges
     int parts, blocks_per_part;
-    float *part_o;    // [parts][batch * heads][seq_q][D]
-    float *part_lse;  // [parts][batch * heads][seq_q]
+    float *part_o;    // [batch * heads][seq_q][parts][D]
+    float *part_lse;  // [batch * heads][seq_q][parts]
 #ifdef NT_ATTN_STAMPS
     unsigned long long *stamps;  // measurement builds: per wave {entry to loop, loop, epilogue} in 10 ns units and the loop in clocks
 #endif
@@ -749,9 +749,9 @@ __global__ __launch_bounds__(kWaves * 64, kOcc) void attention_fwd_kernel(Attent
 #pragma unroll
         for (int qt = 0; qt < kQTiles; ++qt) {
             const float l_total = l_run[qt] + __shfl_xor(l_run[qt], 32, 64);
-            const float inv = l_total > 0.0f ? 1.0f / l_total : 0.0f;  // a part without keys contributes nothing
+            const float inv = l_total == 0.0f ? 0.0f : 1.0f / l_total;  // a part without keys contributes nothing (a NaN does)
             if (q_row[qt] < p.seq_q) {
-                const int64_t row = ((int64_t)part * p.batch * p.heads + bh) * p.seq_q + q_row[qt];
+                const int64_t row = ((int64_t)bh * p.seq_q + q_row[qt]) * p.parts + part;
                 float *dst = p.part_o + row * D;
 #pragma unroll
                 for (int dt = 0; dt < DT; ++dt)
@@ -763,7 +763,7 @@ __global__ __launch_bounds__(kWaves * 64, kOcc) void attention_fwd_kernel(Attent
                         for (int e = 0; e < 4; ++e) out[e] = o_acc[dt][qt][r4 * 4 + e] * inv;
                         *(float4_t *)(dst + dt * 32 + 8 * r4 + 4 * g) = out;
                     }
-                if (g == 0) p.part_lse[row] = l_total > 0.0f ? m_run[qt] + __builtin_amdgcn_logf(l_total) : -INFINITY;
+                if (g == 0) p.part_lse[row] = l_total == 0.0f ? -INFINITY : m_run[qt] + __builtin_amdgcn_logf(l_total);
             }
         }
         return;
@@ -857,29 +857,58 @@ __global__ __launch_bounds__(kWaves * 64, kOcc) void attention_fwd_kernel(Attent
 #endif
 }
 
-// merges the parts of a split key range: O = sum_s w_s O_s / sum_s w_s with w_s = 2^(lse_s - max lse);
-// one thread per row and four consecutive columns
-template <typename TIO, int D>
+// Merges the parts of a split key range: O = sum_s w_s O_s / sum_s w_s with w_s = 2^(lse_s - max lse).  A thread holds four
+// columns of a row and walks every kLanes-th part; the kLanes threads of a column meet in LDS.  One thread per column
+// (kLanes 1) reads its parts one after another, which a few rows of a decoding step with tens of parts turn into the
+// longest link of the call: 24 rows x 22 parts x 128 16 us in 3 workgroups, 2.4 with eight threads per column.
+template <typename TIO, int D, int kLanes>
 __global__ __launch_bounds__(256) void attention_merge_kernel(AttentionParams p) {
-    typedef float float4_t __attribute__((ext_vector_type(4)));
     constexpr int kGroups = D / 4;
+    constexpr int kRows = 256 / (kGroups * kLanes);  // rows of a workgroup
+    static_assert(kRows >= 1, "threads of a row");
     const int64_t rows = (int64_t)p.batch * p.heads * p.seq_q;
-    const int64_t index = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (index >= rows * kGroups) return;
-    const int64_t row = index / kGroups;
-    const int col = (int)(index - row * kGroups) * 4;
-    if (col >= p.head_dim) return;
-    float top = -INFINITY;
-    for (int s = 0; s < p.parts; ++s) top = fmaxf(top, p.part_lse[s * rows + row]);
+    const int t = threadIdx.x;
+    const int lane = t / kGroups % kLanes;
+    const int64_t row = (int64_t)blockIdx.x * kRows + t / (kGroups * kLanes);
+    const int col = t % kGroups * 4;
+    float top = -INFINITY, weights = 0.0f;
     float4_t sum = {0.0f, 0.0f, 0.0f, 0.0f};
-    float weights = 0.0f;
-    for (int s = 0; s < p.parts; ++s) {
-        const float lse = p.part_lse[s * rows + row];
-        if (lse == -INFINITY) continue;
-        const float w = __builtin_amdgcn_exp2f(lse - top);
-        weights += w;
-        sum += w * *(const float4_t *)(p.part_o + (s * rows + row) * D + col);
+    if (row < rows) {
+        const float *lses = p.part_lse + row * p.parts;
+        const float *values = p.part_o + row * p.parts * D + col;
+        for (int s = lane; s < p.parts; s += kLanes) top = fmaxf(top, lses[s]);
+#pragma unroll 4
+        for (int s = lane; s < p.parts; s += kLanes) {
+            const float lse = lses[s];
+            const float4_t value = *(const float4_t *)(values + (int64_t)s * D);
+            const float w = lse == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(lse - top);  // (an empty part holds zeros)
+            weights += w;
+            sum += w * value;
+        }
     }
+    if constexpr (kLanes > 1) {
+        __shared__ float4_t lds_sum[256];
+        __shared__ float lds_top[256], lds_weights[256];
+        lds_sum[t] = sum;
+        lds_top[t] = top;
+        lds_weights[t] = weights;
+        __syncthreads();
+        if (lane != 0 || row >= rows) return;
+        float whole_top = top;
+#pragma unroll
+        for (int i = 1; i < kLanes; ++i) whole_top = fmaxf(whole_top, lds_top[t + i * kGroups]);
+        sum = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+        weights = 0.0f;
+#pragma unroll
+        for (int i = 0; i < kLanes; ++i) {
+            const float other = lds_top[t + i * kGroups];
+            const float w = other == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(other - whole_top);
+            // (a thread whose parts are all without weight still has their NaN to pass on, if there is one)
+            weights += other == -INFINITY ? lds_weights[t + i * kGroups] : w * lds_weights[t + i * kGroups];
+            sum += w * lds_sum[t + i * kGroups];
+        }
+    }
+    if (row >= rows) return;
     const float inv = 1.0f / weights;
     const int64_t q_in_head = row % p.seq_q;
     const int64_t bh = row / p.seq_q;
@@ -887,11 +916,195 @@ __global__ __launch_bounds__(256) void attention_merge_kernel(AttentionParams p)
     typedef TIO out4_t __attribute__((ext_vector_type(4)));
     out4_t out;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        if constexpr (std::is_same<TIO, float>::value) out[e] = sum[e] * inv;
-        else out[e] = Elem<TIO>::from_float(sum[e] * inv);
-    }
+    for (int e = 0; e < 4; ++e) out[e] = Elem<TIO>::from_float(sum[e] * inv);
     *(out4_t *)dst = out;
+}
+
+// the merge of p.parts parts: several threads per column where one each would leave most of the chip idle
+template <typename T, int D>
+hipError_t launch_merge(const AttentionParams &p, hipStream_t stream) {
+    constexpr int kLanes = 256 / (D / 4);
+    const int64_t rows = (int64_t)p.batch * p.heads * p.seq_q;
+    if (rows <= 2048) attention_merge_kernel<T, D, kLanes><<<dim3((unsigned)rows), dim3(256), 0, stream>>>(p);
+    else attention_merge_kernel<T, D, 1><<<dim3((unsigned)((rows + kLanes - 1) / kLanes)), dim3(256), 0, stream>>>(p);
+    return hipGetLastError();
+}
+
+// ---- one query per (batch, head): a decoding step ----
+//
+// Bound by reading K and V once.  The tile kernels above multiply 128 query rows of which one exists, hold two blocks of K
+// and V per workgroup in LDS behind barriers, and with one workgroup per head keep as few bytes in flight as there are
+// heads.  Here a wave reads whole K rows into registers (D / 8 lanes of 16 bytes per key, 64 / (D / 8) keys per load),
+// multiplies in fp32 on the vector unit -- a quarter of its time at the full memory rate --, and requests its next keys
+// as soon as the last ones are used.  Every group of lanes keeps its own running maximum, so that lanes meet only in the
+// sums over a key's elements (DPP); groups and waves are merged once, at the end.
+// fp16 [8, 32, 1, 128] x 8192 keys 183 -> 181 us (5.9 TB/s), bf16 [15, 12, 1, 128] x 4029 83 -> 63; in parts: fp16
+// [3, 8, 1, 128] x 9606 46 -> 27, [1, 8, 1, 128] x 32768 66 -> 34, [1, 12, 1, 64] x 4936 20 -> 9; [4, 32, 1, 128] x 900 18 -> 11.
+// Four loads per step and operand leave 128 registers, four waves per SIMD; eight: 210 us for the first, 13 for the last.
+constexpr int kDecodeLoads = 4;  // K (and V) loads of a step per lane
+
+template <int D>
+constexpr int kDecodeStepKeys = kDecodeLoads * 64 / (D / 8);  // keys of a wave's step
+
+template <int kControl>
+NT_DEVICE float add_dpp(float v) {
+    return v + __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), kControl, 0xf, 0xf, true));
+}
+
+template <typename T, int D, int kWaves, bool kParts>
+__global__ __launch_bounds__(kWaves * 64) void attention_decode_kernel(AttentionParams p) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    typedef Elem<T> E;
+    typedef typename E::vec8 vec8;
+    constexpr int kLanesPerKey = D / 8, kGroups = 64 / kLanesPerKey, kStepKeys = kDecodeStepKeys<D>;
+    static_assert(kLanesPerKey == 8 || kLanesPerKey == 16, "head dimension");
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int group = lane / kLanesPerKey, col = lane % kLanesPerKey * 8;
+    const int pairs = p.batch * p.heads;
+    const int part = kParts ? blockIdx.x / pairs : 0;
+    const int bh = kParts ? blockIdx.x - part * pairs : blockIdx.x;
+    const int head = bh % p.heads, batch = bh / p.heads;
+    const T *K = (const T *)p.k + batch * p.k_strides[0] + head * p.k_strides[1];
+    const T *V = (const T *)p.v + batch * p.v_strides[0] + head * p.v_strides[1];
+    const int keys = p.causal ? min(p.seq_k, 1) : p.seq_k;  // (a causal mask leaves query 0 its key 0)
+    const int first = kParts ? part * p.blocks_per_part * kWaves * kStepKeys : 0;
+    const int last = kParts ? min(keys, first + p.blocks_per_part * kWaves * kStepKeys) : keys;
+
+    // descriptors that end with the last key's row; lanes without a key get an offset behind them and read zeros
+    const unsigned k_row = (unsigned)p.k_strides[2] * 2u, v_row = (unsigned)p.v_strides[2] * 2u;
+    __amdgpu_buffer_rsrc_t k_rsrc = __builtin_amdgcn_make_buffer_rsrc((void *)K, 0, (unsigned)((keys - 1) * p.k_strides[2] + D) * 2u, 0x00020000);
+    __amdgpu_buffer_rsrc_t v_rsrc = __builtin_amdgcn_make_buffer_rsrc((void *)V, 0, (unsigned)((keys - 1) * p.v_strides[2] + D) * 2u, 0x00020000);
+    constexpr unsigned kBehind = 0xfffffff0u;
+    auto load = [&](__amdgpu_buffer_rsrc_t rsrc, unsigned row_bytes, int key0, vec8(&to)[kDecodeLoads]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < kDecodeLoads; ++j) {
+            const int key = key0 + j * kGroups + group;
+            const unsigned offset = key < last ? (unsigned)key * row_bytes + col * 2 : kBehind;
+            to[j] = __builtin_bit_cast(vec8, __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)offset, 0, 0));
+        }
+    };
+    int key0 = first + wave * kStepKeys;
+    vec8 kf[kDecodeLoads], vf[kDecodeLoads];
+    load(k_rsrc, k_row, key0, kf);
+    load(v_rsrc, v_row, key0, vf);
+    // Q' = round(Q * scale * log2 e)
+    float q[8];
+    {
+        const vec8 raw = *(const vec8 *)((const T *)p.q + batch * p.q_strides[0] + head * p.q_strides[1] + col);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) q[e] = E::to_float(E::from_float(E::to_float(raw[e]) * p.q_scale));
+    }
+    float top = -INFINITY, weights = 0.0f, acc[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) acc[e] = 0.0f;
+    for (; key0 < last; key0 += kWaves * kStepKeys) {
+        float s[kDecodeLoads];
+#pragma unroll
+        for (int j = 0; j < kDecodeLoads; ++j) {
+            float sum = 0.0f;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) sum = fmaf(E::to_float(kf[j][e]), q[e], sum);
+            sum = add_dpp<0xb1>(sum);   // quad_perm [1, 0, 3, 2]
+            sum = add_dpp<0x4e>(sum);   // quad_perm [2, 3, 0, 1]
+            sum = add_dpp<0x141>(sum);  // row_half_mirror: the other quad of 8 lanes
+            if constexpr (kLanesPerKey == 16) sum = add_dpp<0x140>(sum);  // row_mirror: the other 8 of 16 lanes
+            s[j] = key0 + j * kGroups + group < last ? sum : -INFINITY;
+        }
+        load(k_rsrc, k_row, key0 + kWaves * kStepKeys, kf);
+        float new_top = top;
+#pragma unroll
+        for (int j = 0; j < kDecodeLoads; ++j) new_top = fmaxf(new_top, s[j]);
+        const float base = new_top == -INFINITY ? 0.0f : new_top;  // (no key yet, or only scores of -inf: weights of zero)
+        const float scale = __builtin_amdgcn_exp2f(top - base);
+        top = new_top;
+        weights *= scale;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) acc[e] *= scale;
+#pragma unroll
+        for (int j = 0; j < kDecodeLoads; ++j) {
+            const float w = __builtin_amdgcn_exp2f(s[j] - base);
+            weights += w;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) acc[e] = fmaf(w, E::to_float(vf[j][e]), acc[e]);
+        }
+        load(v_rsrc, v_row, key0 + kWaves * kStepKeys, vf);
+    }
+
+    // ---- the groups of a wave, then the waves ----
+#pragma unroll
+    for (int distance = kLanesPerKey; distance < 64; distance *= 2) {
+        const float other_top = __shfl_xor(top, distance, 64);
+        const float new_top = fmaxf(top, other_top);
+        const float base = new_top == -INFINITY ? 0.0f : new_top;
+        const float mine = __builtin_amdgcn_exp2f(top - base), theirs = __builtin_amdgcn_exp2f(other_top - base);
+        weights = weights * mine + __shfl_xor(weights, distance, 64) * theirs;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) acc[e] = acc[e] * mine + __shfl_xor(acc[e], distance, 64) * theirs;
+        top = new_top;
+    }
+    __shared__ float lds_acc[kWaves][D], lds_top[kWaves], lds_weights[kWaves];
+    if (group == 0) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) lds_acc[wave][col + e] = acc[e];
+    }
+    if (lane == 0) {
+        lds_top[wave] = top;
+        lds_weights[wave] = weights;
+    }
+    __syncthreads();
+    if (tid >= D) return;
+    float whole_top = lds_top[0];
+#pragma unroll
+    for (int w = 1; w < kWaves; ++w) whole_top = fmaxf(whole_top, lds_top[w]);
+    const float base = whole_top == -INFINITY ? 0.0f : whole_top;
+    float total = 0.0f, value = 0.0f;
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) {
+        const float factor = __builtin_amdgcn_exp2f(lds_top[w] - base);
+        total += factor * lds_weights[w];
+        value += factor * lds_acc[w][tid];
+    }
+    if constexpr (kParts) {
+        const int64_t row = (int64_t)bh * p.parts + part;
+        p.part_o[row * D + tid] = total == 0.0f ? 0.0f : value / total;
+        if (tid == 0) p.part_lse[row] = total == 0.0f ? -INFINITY : whole_top + __builtin_amdgcn_logf(total);
+    } else {
+        ((T *)p.o)[batch * p.o_strides[0] + head * p.o_strides[1] + tid] = E::from_float(value / total);
+    }
+#endif
+}
+
+// Workgroups of 16 waves that read a head's keys alone, in one launch, where they fill half the chip or have at most
+// four steps; else parts of the keys for four waves each, about 1024 workgroups of at least two steps, and a merge.
+template <typename T, int D>
+int launch_decode(AttentionParams &p, hipStream_t stream) {
+    const int64_t pairs = (int64_t)p.batch * p.heads;
+    const int keys = p.causal ? 1 : p.seq_k;
+    p.q_blocks = 1;
+    if (pairs > 0x7fffffffll) return NINETOOTHED_NO_KERNEL;
+    if (pairs < 128 && keys > 4 * 16 * kDecodeStepKeys<D>) {
+        constexpr int kStep = 4 * kDecodeStepKeys<D>;  // keys of a workgroup's step
+        const int steps = ceil_div(keys, kStep);
+        const int wanted = (int)std::min<int64_t>((1024 + pairs - 1) / pairs, steps / 2);
+        p.blocks_per_part = ceil_div(steps, wanted);
+        p.parts = ceil_div(steps, p.blocks_per_part);
+        WorkspaceLease lease(stream);
+        float *scratch = (float *)lease.get(kWorkspaceAttentionParts, (size_t)p.parts * pairs * (D + 1) * sizeof(float));
+        if (scratch != nullptr) {  // (none under graph capture without a buffer: one launch, as below)
+            p.part_o = scratch;
+            p.part_lse = scratch + (size_t)p.parts * pairs * D;
+            note_launch(kLaunchAttention, p.parts, "one query: split key range (this many parts), then attention_merge_kernel");
+            attention_decode_kernel<T, D, 4, true><<<dim3((unsigned)(pairs * p.parts)), dim3(256), 0, stream>>>(p);
+            const hipError_t err = hipGetLastError();
+            return err != hipSuccess ? (int)err : (int)launch_merge<T, D>(p, stream);
+        }
+        p.parts = 1;
+    }
+    note_launch(kLaunchAttention, 1, "one query: a workgroup per head");
+    if (pairs <= 256) attention_decode_kernel<T, D, 16, false><<<dim3((unsigned)pairs), dim3(1024), 0, stream>>>(p);
+    else attention_decode_kernel<T, D, 8, false><<<dim3((unsigned)pairs), dim3(512), 0, stream>>>(p);
+    return (int)hipGetLastError();
 }
 
 // Few (batch, head, query block) workgroups and a long key sequence (decoding): the key range is split
@@ -928,8 +1141,7 @@ int launch_split_keys(AttentionParams &p, hipStream_t stream) {
     attention_fwd_kernel<T, D, 1, BN, 2, false, T, kAttnWaves, false, true><<<dim3((unsigned)(groups * p.parts)), dim3(kAttnWaves * 64), 0, stream>>>(p);
     hipError_t err = hipGetLastError();
     if (err != hipSuccess) return (int)err;
-    attention_merge_kernel<T, D><<<dim3((unsigned)((rows * (D / 4) + 255) / 256)), dim3(256), 0, stream>>>(p);
-    return (int)hipGetLastError();
+    return (int)launch_merge<T, D>(p, stream);
 }
 
 template <typename T, int D, int kQTiles, int BN, int kOcc, bool kPipelined, typename TIO = T, int kWaves = kAttnWaves, bool kPadded = false, bool kFold = true>
@@ -1252,9 +1464,13 @@ void attention_tune_values(const AttentionParams &p, int dtype, int (&values)[7]
 // whether the variants are alternatives for this problem (they exist for head dimensions 64 and 128)
 bool attention_tunable(const AttentionParams &p, int dtype) { return dtype != NINETOOTHED_FLOAT32 && (p.head_dim == 128 || p.head_dim == 64); }
 
-// the key range is split instead (decoding-like shapes); returns NINETOOTHED_NO_KERNEL when that does not apply
+// one query per head, or a split key range (decoding-like shapes); returns NINETOOTHED_NO_KERNEL when that does not apply
 int attention_split(AttentionParams &p, int dtype, hipStream_t stream) {
     if (p.head_dim != 128 && p.head_dim != 64) return NINETOOTHED_NO_KERNEL;
+    if (p.seq_q == 1) {
+        if (dtype == NINETOOTHED_FLOAT16) return p.head_dim == 128 ? launch_decode<half_t, 128>(p, stream) : launch_decode<half_t, 64>(p, stream);
+        if (dtype == NINETOOTHED_BFLOAT16) return p.head_dim == 128 ? launch_decode<bf16_t, 128>(p, stream) : launch_decode<bf16_t, 64>(p, stream);
+    }
     if (dtype == NINETOOTHED_FLOAT16) return p.head_dim == 128 ? launch_split_keys<half_t, 128>(p, stream) : launch_split_keys<half_t, 64>(p, stream);
     if (dtype == NINETOOTHED_BFLOAT16) return p.head_dim == 128 ? launch_split_keys<bf16_t, 128>(p, stream) : launch_split_keys<bf16_t, 64>(p, stream);
     return NINETOOTHED_NO_KERNEL;
@@ -1266,7 +1482,7 @@ int attention_untuned_variant(const AttentionParams &p) {
     return !p.causal && p.head_dim >= 64 && (int64_t)p.batch * p.heads * ceil_div(p.seq_q, 256) >= 512 ? 4 : 3;
 }
 
-bool attention_would_split(const AttentionParams &p) { return (p.head_dim == 128 || p.head_dim == 64) && split_key_parts(p) > 0; }
+bool attention_would_split(const AttentionParams &p) { return (p.head_dim == 128 || p.head_dim == 64) && (p.seq_q == 1 || split_key_parts(p) > 0); }
 
 }  // namespace
 }  // namespace nt

@@ -744,6 +744,31 @@ def test_attention_split_key_range(batch, heads, seq_q, seq_k, emb_dim, is_causa
     _native_only(kernel, "launch_nt_attention")
 
 
+@pytest.mark.parametrize("dtype", (torch.float16, torch.bfloat16))
+@pytest.mark.parametrize("batch, heads, seq_k, emb_dim", ((1, 1, 1, 64), (2, 3, 15, 128), (3, 1, 257, 128), (1, 5, 513, 64), (2, 8, 1025, 128), (1, 3, 2049, 64), (1, 7, 4999, 128), (128, 1, 1030, 128), (2, 129, 77, 64)))
+def test_attention_of_one_query(batch, heads, seq_k, emb_dim, dtype):
+    """A decoding step: a workgroup per head, or parts of the keys and a merge (few heads, more than four steps of 256 / 512
+    keys); heads innermost in memory, with a causal mask (key 0 alone), and with keys whose scores are -inf."""
+    q, k, v = (_randn(batch, length, heads, emb_dim).cuda().to(dtype).transpose(1, 2) for length in (1, seq_k, seq_k))
+    scale = emb_dim**-0.5
+    kernel = ninetoothed.make(programs.attention.arrangement_with_scale, programs.attention.application_with_scale, programs.attention.tensors(True))
+
+    def run(is_causal):
+        o = torch.full_like(q, float("nan"))
+        kernel(q, k, v, is_causal, scale, o)
+        _native_only(kernel, "launch_nt_attention")
+        return o.float()
+
+    assert torch.allclose(run(False), _attention_reference(q, k, v, False, scale), **HALF_TOL)
+    assert torch.equal(run(True), v[:, :, :1].float())
+    if seq_k > 1:
+        q.fill_(0.5)
+        k[:, :, : seq_k // 2] = -float("inf")
+        assert torch.allclose(run(False), _attention_reference(q, k, v, False, scale), **HALF_TOL)
+    q[:, :, :, 0] = float("nan")
+    assert run(False).isnan().all()
+
+
 def test_attention_closed_forms_and_layouts():
     q, v = _randn(1, 2, 300, 64).cuda(), _randn(1, 2, 300, 64).cuda()
     k = torch.zeros_like(q)
