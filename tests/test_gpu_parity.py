@@ -1143,6 +1143,38 @@ def test_conv2d_channels_last_and_sliced_tensors_on_the_repacked_path(channels, 
         assert bool((wide[untouched] == 7).all())
 
 
+@pytest.mark.parametrize("dtype", (torch.float16, torch.bfloat16))
+@pytest.mark.parametrize(
+    "k, c, r, s_",
+    ((1, 1, 1, 1), (8, 1, 3, 3), (63, 7, 3, 3), (64, 64, 1, 1), (65, 33, 1, 3), (72, 20, 5, 1), (129, 16, 3, 3), (200, 96, 3, 3), (8, 2000, 5, 5)),
+)
+def test_conv2d_filters_are_repacked_the_same_from_tiles_and_element_by_element(k, c, r, s_, dtype):
+    """A filter whose C*R*S elements lie one after another -- at odd elements of a buffer, with rows further apart than they
+    are long -- is transposed in 64 x 64 tiles, one of any other strides element by element: the same products follow."""
+    from ninetoothed_amd import runtime
+
+    tag = runtime.DATA_TYPE_INDEX["fp16" if dtype == torch.float16 else "bf16"]
+    x = _randn(2, c, 13, 9, dtype=dtype, scale=0.3).cuda()
+    weight = _randn(k, c, r, s_, dtype=dtype, scale=(c * r * s_) ** -0.5).cuda()
+    padding = (r // 2, s_ // 2)
+    length = c * r * s_
+    rows = torch.full((k * (length + 5) + 3,), float("inf"), dtype=dtype, device="cuda")
+    apart = torch.as_strided(rows, weight.shape, (length + 5, r * s_, s_, 1), 3)
+    apart.copy_(weight)
+    spread = torch.full((k, c, r, s_, 2), float("inf"), dtype=dtype, device="cuda")[..., 0]
+    spread.copy_(weight)
+    expected = F.conv2d(x.float(), weight.float(), padding=padding)
+    results = []
+    for w_in in (weight, apart, spread, spread.reshape(weight.shape).permute(1, 2, 3, 0).contiguous().permute(3, 0, 1, 2)):
+        y = torch.full(expected.shape, float("nan"), dtype=dtype, device="cuda")
+        tensors = [runtime.ArgumentTensor.from_torch_tensor(t) for t in (x, w_in, y)]
+        assert runtime.library().launch_nt_conv2d(runtime.current_stream(), *tensors, tag, *padding, 2, 0, 0) == 0
+        assert runtime.last_launch().startswith("conv2d path 2"), runtime.last_launch()
+        results.append(y)
+    assert torch.allclose(results[0].float(), expected, **HALF_TOL), float((results[0].float() - expected).abs().max())
+    assert all(torch.equal(results[0], other) for other in results[1:])
+
+
 def test_conv2d_one_launch_path_refuses_what_it_cannot_run():
     from ninetoothed_amd import runtime
 
