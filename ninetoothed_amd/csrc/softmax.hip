@@ -261,7 +261,7 @@ __global__ __launch_bounds__(256) void softmax_thread_per_row_kernel(SoftmaxPara
     for (int j = 0; j < kMaxPieces; ++j)
 #pragma unroll
         for (int e = 0; e < kWidth; ++e) {
-            x[j][e] = __builtin_amdgcn_exp2f(fmaf(x[j][e], kLog2e, -shift));  // (as in softmax_vec_kernel)
+            x[j][e] = __builtin_amdgcn_exp2f(fmaf(x[j][e], kLog2e, -shift));  // (as in softmax_split_in_registers_kernel)
             s += x[j][e];
         }
     const float inv = 1.0f / s;
