@@ -873,6 +873,23 @@ struct MapCodegen {
         return "(" + term + " != " + term + " || " + acc + " != " + acc + ") ? " + acc + " + " + term + " : (" + term + " " + cmp + " " + acc + " ? " + term + " : " + acc + ")";
     }
 
+    // `acc` of the 64 lanes of a wave combined in every lane.  A float goes through lane permutations inside the vector unit
+    // (DPP within 16 lanes, then the two half-row swaps) instead of six dependent trips through LDS (with one barrier per
+    // exchange between waves instead of two: rms norm of 4096 rows of 4096 bf16 values 15.2 -> 13.2 us).
+    void reduce_lanes(int op, int dtype, bool single) {
+        const std::string combined = combine_expr(op, dtype, "acc", "other");
+        const char *pad = "            ";
+        if (!single) {
+            out << pad << "for (int offset = 32; offset > 0; offset >>= 1) { const double other = __shfl_xor(acc, offset, 64); acc = " << combined << "; }\n";
+            return;
+        }
+        for (const char *control : {"0xb1", "0x4e", "0x141", "0x140"})  // the neighbour, the other pair of a quad, the other quad of 8, the other 8 of 16
+            out << pad << "{ const float other = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, acc), " << control << ", 0xf, 0xf, true)); acc = " << combined << "; }\n";
+        for (const char *lanes_apart : {"16", "32"})
+            out << pad << "{ const auto halves = __builtin_amdgcn_permlane" << lanes_apart << "_swap(__builtin_bit_cast(unsigned, acc), __builtin_bit_cast(unsigned, acc), false, false); "
+                << "acc = __builtin_bit_cast(float, (unsigned)halves[0]); const float other = __builtin_bit_cast(float, (unsigned)halves[1]); acc = " << combined << "; }\n";
+    }
+
     void decode_tile_variables() {
         out << indent << "nt_uidx rest = (nt_uidx)element;\n";
         for (int v = p.num_vars - 1; v >= p.num_grid; --v)
@@ -1025,7 +1042,8 @@ struct MapCodegen {
             out << "    const nt_idx member = threadIdx.x & 63;\n"
                 << "    for (nt_idx tile = (nt_idx)blockIdx.x * " << threads / 64 << " + (threadIdx.x >> 6); tile < " << lit(tiles) << "; tile += (nt_idx)gridDim.x * " << threads / 64 << ") {\n";
         else
-            out << "    __shared__ double scratch[" << threads / 64 << "];\n"
+            out << "    __shared__ double scratch[2][" << threads / 64 << "];\n"
+                << "    int turn = 0;\n"
                 << "    const nt_idx member = threadIdx.x;\n"
                 << "    for (nt_idx tile = (nt_idx)blockIdx.x; tile < " << lit(tiles) << "; tile += (nt_idx)gridDim.x) {\n";
         out
@@ -1056,17 +1074,18 @@ struct MapCodegen {
             const std::string term = value_range(begin, p.phase_end[k], "");
             out << indent << "acc = " << combine_expr(op, dtype, "acc", term) << ";\n";
             close_element_loop("            ");
-            out << "            for (int offset = 32; offset > 0; offset >>= 1) { const " << carried << " other = __shfl_xor(acc, offset, 64); acc = "
-                << combine_expr(op, dtype, "acc", "other") << "; }\n";
+            reduce_lanes(op, dtype, single);
             if (wave_tiles) {
                 out << "            r" << k << " = acc;\n        }\n";
                 begin = p.phase_end[k];
                 continue;
             }
-            out << "            __syncthreads();\n            if ((threadIdx.x & 63) == 0) scratch[threadIdx.x >> 6] = acc;\n            __syncthreads();\n"
-                << "            acc = scratch[0];\n"
-                << "            for (int w = 1; w < " << threads / 64 << "; ++w) { const " << carried << " other = scratch[w]; acc = " << combine_expr(op, dtype, "acc", "other")
-                << "; }\n            r" << k << " = acc;\n        }\n";
+            // (two buffers in turn: a wave writes one again only behind the other's barrier, which none reaches before it has read this one)
+            out << "            if ((threadIdx.x & 63) == 0) scratch[turn][threadIdx.x >> 6] = acc;\n            __syncthreads();\n"
+                << "            acc = scratch[turn][0];\n"
+                << "            #pragma unroll\n"
+                << "            for (int w = 1; w < " << threads / 64 << "; ++w) { const " << carried << " other = scratch[turn][w]; acc = " << combine_expr(op, dtype, "acc", "other")
+                << "; }\n            turn ^= 1;\n            r" << k << " = acc;\n        }\n";
             begin = p.phase_end[k];
         }
         const NineToothedMapOperand &target = p.operands[p.output];
