@@ -662,7 +662,18 @@ struct MapCodegen {
     std::vector<bool> kept = std::vector<bool>(NT_MAP_MAX_OPERANDS, false);
     std::map<int, std::string> in_body;
 
-    explicit MapCodegen(const NineToothedMapProgram &program) : p(program), narrow(fits_int32(program)), lanes(cooperative_lanes(program)), threads(workgroup_threads(program)), group(tile_group(program)) {}
+    explicit MapCodegen(const NineToothedMapProgram &program) : p(program), narrow(fits_int32(program)), lanes(cooperative_lanes(program)), threads(workgroup_threads(program)), group(tile_group(program)) {
+        // Tiles of one reduction whose elements come in groups of 8 (16 bytes): two groups per thread.  Two loads in flight per
+        // tensor and half the waves to meet cost less than they hide (bf16 rms norm, a kernel alone: 4096 rows of 4096 on 512 threads
+        // 13.6 us, on 256 10.5, on 128 or 64 with 4 or 8 groups 10.8 and 10.7; 16384 rows of 1024 on 256 threads 12.8 us, on 128
+        // 13.4, on a wave 10.5).  Longer tiles have 16 elements per thread already; element by element 8 per thread stay better.
+        long long tile_elements = 1;
+        for (int v = program.num_grid; v < program.num_vars; ++v) tile_elements *= (long long)program.extents[v];
+        if (program.num_phases == 1 && tile_elements > 512 && tile_elements <= 4096 && tile_vector_width(tile_elements) > 0) {
+            threads = kMapThreads;
+            group = tile_elements <= 1024 ? 64 : kMapThreads;
+        }
+    }
 
     std::string fresh(const char *prefix) { return prefix + std::to_string(counter++); }
 
@@ -1369,15 +1380,20 @@ struct Hiprtc {
 };
 
 std::mutex g_jit_mutex;
-std::unordered_map<std::string, hipFunction_t> g_jit_cache;  // a null function = "do not try again"
+struct SpecialisedKernel {
+    hipFunction_t function = nullptr;  // null: "do not try again"
+    int threads = kMapThreads;         // of a workgroup
+    int group = kMapThreads;           // that share a tile in tile mode
+};
+std::unordered_map<std::string, SpecialisedKernel> g_jit_cache;
 
 // `may_compile` false (the stream is being captured into a graph: compiling and loading code would break
 // the capture): only a kernel specialised earlier is returned, and a miss is not remembered
-hipFunction_t specialised_kernel(const NineToothedMapProgram &p, bool may_compile) {
+SpecialisedKernel specialised_kernel(const NineToothedMapProgram &p, bool may_compile) {
     static Hiprtc rtc;
-    if (!rtc.ok) return nullptr;
+    if (!rtc.ok) return {};
     int device = 0;
-    if (hipGetDevice(&device) != hipSuccess) return nullptr;
+    if (hipGetDevice(&device) != hipSuccess) return {};
     // the key is everything the source depends on: all of the program but pointers,
     // `other` values and value constants (those are kernel arguments)
     NineToothedMapProgram shape = p;
@@ -1397,10 +1413,13 @@ hipFunction_t specialised_kernel(const NineToothedMapProgram &p, bool may_compil
     std::lock_guard<std::mutex> lock(g_jit_mutex);
     auto found = g_jit_cache.find(key);
     if (found != g_jit_cache.end()) return found->second;
-    if (!may_compile) return nullptr;
+    if (!may_compile) return {};
     MapCodegen generator(p);
     const std::string source = generator.generate();
-    hipFunction_t function = nullptr;
+    SpecialisedKernel specialised;
+    specialised.threads = generator.threads;
+    specialised.group = generator.group;
+    hipFunction_t &function = specialised.function;
     hiprtcProgram program = nullptr;
     if (rtc.create(&program, source.c_str(), "nt_map_specialised.hip", 0, nullptr, nullptr) == HIPRTC_SUCCESS) {
         // same code generation switches as the rest of the library: gfx950, packed FP32 off
@@ -1425,8 +1444,8 @@ hipFunction_t specialised_kernel(const NineToothedMapProgram &p, bool may_compil
         }
         rtc.destroy(&program);
     }
-    g_jit_cache.emplace(key, function);
-    return function;
+    g_jit_cache.emplace(key, specialised);
+    return specialised;
 }
 
 }  // namespace
@@ -1456,13 +1475,15 @@ extern "C" NineToothedResult launch_nt_map(NineToothedStream stream, const NineT
     int64_t tiles = 1, tile_elements = 1;
     if (p.num_phases > 0) {  // tile mode: one workgroup per tile
         for (int v = 0; v < p.num_vars; ++v) (v < p.num_grid ? tiles : tile_elements) *= p.extents[v];
-        const int64_t tiles_per_block = tile_group(p) == 64 ? workgroup_threads(p) / 64 : 1;  // (only the generated kernel shares a workgroup)
-        blocks = (tiles + tiles_per_block - 1) / tiles_per_block;
-        if (blocks > 256 * 32) blocks = 256 * 32;
+        blocks = std::min<int64_t>(tiles, 256 * 32);
     }
     const char *interpret = getenv("NT_MAP_INTERPRET");
     if (!(interpret && interpret[0] == '1')) {
-        if (hipFunction_t function = specialised_kernel(p, !stream_is_capturing((hipStream_t)stream))) {
+        if (const SpecialisedKernel kernel = specialised_kernel(p, !stream_is_capturing((hipStream_t)stream)); kernel.function != nullptr) {
+            if (p.num_phases > 0 && kernel.group == 64) {  // (only the generated kernel shares a workgroup)
+                const int64_t tiles_per_block = kernel.threads / 64;
+                blocks = std::min<int64_t>((tiles + tiles_per_block - 1) / tiles_per_block, 256 * 32);
+            }
             MapJitArgs args;
             for (int i = 0; i < NT_MAP_MAX_OPERANDS; ++i) {
                 args.data[i] = i < p.num_operands ? p.operands[i].data : nullptr;
@@ -1473,7 +1494,7 @@ extern "C" NineToothedResult launch_nt_map(NineToothedStream stream, const NineT
             size_t size = sizeof(args);
             void *config[] = {HIP_LAUNCH_PARAM_BUFFER_POINTER, &args, HIP_LAUNCH_PARAM_BUFFER_SIZE, &size, HIP_LAUNCH_PARAM_END};
             nt::note_launch(nt::kLaunchMap, 0, "kernel generated for the program and compiled with hipRTC");
-            return (int)hipModuleLaunchKernel(function, (unsigned)blocks, 1, 1, (unsigned)workgroup_threads(p), 1, 1, 0, (hipStream_t)stream, nullptr, config);
+            return (int)hipModuleLaunchKernel(kernel.function, (unsigned)blocks, 1, 1, (unsigned)kernel.threads, 1, 1, 0, (hipStream_t)stream, nullptr, config);
         }
     }
     nt::note_launch(nt::kLaunchMap, 1, "interpreter kernel");

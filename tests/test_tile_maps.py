@@ -1114,6 +1114,21 @@ def test_grouped_elements_of_16_bit_tensors(dtype):
 
 
 @gpu
+@pytest.mark.parametrize("rows, cols", ((1, 512), (9, 520), (8193, 1016), (5, 1024), (7, 1032), (3, 2048), (8200, 2056), (4, 4088), (6, 4096), (2, 4104)))
+def test_rows_of_one_reduction_in_groups_of_eight_per_wave_and_per_workgroup(rows, cols):
+    """One reduction over rows of 16-bit values: rows of up to 1024 values take a wave each, up to 4096 a workgroup of 256
+    threads, longer ones more; more rows than workgroups are walked by a loop whose exchange between waves uses two
+    buffers in turn.  (The application rounds to the tensors' type after every operation: about six roundings of 2^-11.)"""
+    _, (kernel, inputs, expected), _ = _normalisation_cases("cuda", torch.float16, rows, cols)
+    storage = torch.full((rows, cols + 3), 7.0, dtype=torch.float16, device="cuda")
+    out = storage[:, 2 : 2 + cols]
+    kernel(*inputs, out)
+    _served_by_map(kernel)
+    assert torch.allclose(out.float(), expected, rtol=6 * 2.0**-11, atol=2.0**-20)
+    assert bool((storage[:, :2] == 7).all()) and bool((storage[:, 2 + cols :] == 7).all())
+
+
+@gpu
 @pytest.mark.parametrize("dtype", (torch.float16, torch.bfloat16))
 def test_grouped_elements_in_tile_mode_match_the_interpreter(dtype, monkeypatch):
     """Normalisations over rows of 16-bit tensors whose length is a multiple of 8 keep a thread's elements in groups
