@@ -616,6 +616,44 @@ def test_softmax_in_registers_at_the_edges_of_its_thread_counts(vectors, dtype):
         assert bool((buffer[:, :first_out] == 7.0).all()) and bool((buffer[:, first_out + n :] == 7.0).all())
 
 
+# fp32 rows: the exponents of what counts in a row's sum stay below 32, so that an exponential is off by at most 2^-20 (its exponent's
+# rounding, half of 2^-19, times ln 2), and few are; sums, the division and the product add a few 2^-24: 2^-20 in the 2-norm
+SOFTMAX_REL = {torch.float32: 2.0**-20, torch.float16: 2.0**-10, torch.bfloat16: 2.0**-7}  # (16-bit results: rounded once, 2^-11 and 2^-8)
+
+
+def _softmax_error(out, x):
+    """Distance (2-norm) from the softmax in 64 bits of the same values, relative to it."""
+    expected = torch.softmax(x.double(), dim=-1)
+    return float((out.double() - expected).norm() / expected.norm())
+
+
+@pytest.mark.parametrize("dtype", (torch.float32, torch.float16, torch.bfloat16))
+@pytest.mark.parametrize("rows, cols", ((5, 200), (5, 1600), (5, 3000), (5, 4096), (5, 8190), (7, 16384), (5, 33000), (65, 65536)))
+def test_softmax_of_large_values_is_normalised_against_one_shift(rows, cols, dtype):
+    """Rows that 64, 256, 512 and 1024 threads share, of values far from zero: the parts of a row meet without the
+    rounding of their maxima, and equal values get equal probabilities wherever in the row they stand."""
+    from ninetoothed_amd import runtime
+
+    for offset in (0.0, 1e3, -1e3, 3e4, -3e4, 1e5, -1e5, 1e7, -1e7):
+        if abs(offset) > torch.finfo(dtype).max / 2:
+            continue
+        spread = max(torch.finfo(dtype).eps * abs(offset), 5.0)  # (neighbouring values of the type, where they lie further apart)
+        x = (torch.randn(rows, cols, device="cuda") * spread + offset).to(dtype)
+        out = _softmax(x)
+        assert "softmax_split_in_registers_kernel" in runtime.last_launch(), runtime.last_launch()
+        assert _softmax_error(out, x) <= SOFTMAX_REL[dtype], (offset, _softmax_error(out, x))
+        low = x[0, 0].clone().fill_(offset)
+        high = (low.float() + max(torch.finfo(dtype).eps * abs(offset), 2.0)).to(dtype)
+        level = low.expand(rows, cols).clone()
+        level[:, cols // 3 :] = high  # (waves with other maxima than the row's)
+        level[:, 0] = high
+        level[:, -1] = low
+        probabilities = _softmax(level).float()
+        step = 2.0**-24 if dtype == torch.float16 else 0.0  # (of fp16's smallest values)
+        for value, position in ((high, 0), (low, -1)):
+            assert torch.allclose(probabilities[level == value], probabilities[0, position], rtol=SOFTMAX_REL[dtype], atol=step), (offset, position)
+
+
 def test_softmax_baseline_shape_properties():
     x = torch.randn(4096, 4096, device="cuda")
     out = _softmax(x)
