@@ -369,15 +369,15 @@ NT_DEVICE void wide_store(T *dst, int64_t col_stride, int64_t index, int64_t cou
         if ((index + 1) * W <= count) {
             typename WideAccess<T, kVec>::type v;
 #pragma unroll
-            for (int e = 0; e < W; ++e) v[e] = (T)(__builtin_amdgcn_exp2f(fmaf(x[e], kLog2e, -shift)) * inv);
+            for (int e = 0; e < W; ++e) v[e] = (T)(exponential(x[e], shift) * inv);
             *(typename WideAccess<T, kVec>::type *)(dst + index * W) = v;
         } else {
 #pragma unroll
             for (int e = 0; e < W; ++e)
-                if (index * W + e < count) dst[index * W + e] = (T)(__builtin_amdgcn_exp2f(fmaf(x[e], kLog2e, -shift)) * inv);
+                if (index * W + e < count) dst[index * W + e] = (T)(exponential(x[e], shift) * inv);
         }
     } else {
-        if (index < count) dst[index * col_stride] = (T)(__builtin_amdgcn_exp2f(fmaf(x[0], kLog2e, -shift)) * inv);
+        if (index < count) dst[index * col_stride] = (T)(exponential(x[0], shift) * inv);
     }
 }
 
@@ -409,24 +409,20 @@ __global__ __launch_bounds__(kLoopThreads) void softmax_loop_kernel(SoftmaxParam
 #pragma unroll
             for (int e = 0; e < W; ++e) round_max = fmaxf(round_max, x[u][e]);
         }
-        if (round_max > m) {  // (a first round of -inf only leaves m at -inf and s at 0)
-            s *= __builtin_amdgcn_exp2f((m - round_max) * kLog2e);
+        if (round_max > m) {
+            s *= rescale(m, round_max);
             m = round_max;
         }
-        if (m > -INFINITY) {
-            const float shift = m * kLog2e;
+        const float shift = shift_of(m);
 #pragma unroll
-            for (int u = 0; u < kLoopUnroll; ++u)
+        for (int u = 0; u < kLoopUnroll; ++u)
 #pragma unroll
-                for (int e = 0; e < W; ++e) s += __builtin_amdgcn_exp2f(fmaf(x[u][e], kLog2e, -shift));
-        }
+            for (int e = 0; e < W; ++e) s += exponential(x[u][e], shift);
     }
     const float total_max = group_reduce<kLoopThreads, true>(m, scratch);
-    // every thread's sum is relative to its own maximum
-    s = m > -INFINITY ? s * __builtin_amdgcn_exp2f((m - total_max) * kLog2e) : 0.0f;
-    s = group_reduce<kLoopThreads, false>(s, scratch);
+    s = group_reduce<kLoopThreads, false>(s * rescale(m, total_max), scratch);  // (every thread's sum is relative to its own maximum)
     const float inv = 1.0f / s;
-    const float shift = total_max * kLog2e;
+    const float shift = shift_of(total_max);
     for (int64_t base = threadIdx.x; base < pieces; base += kLoopThreads * kLoopUnroll) {
         float x[kLoopUnroll][W];
 #pragma unroll
@@ -469,20 +465,17 @@ __global__ __launch_bounds__(kSplitThreads) void softmax_split_partial_kernel(So
             for (int e = 0; e < W; ++e) round_max = fmaxf(round_max, x[u][e]);
         }
         if (round_max > m) {
-            s *= __builtin_amdgcn_exp2f((m - round_max) * kLog2e);
+            s *= rescale(m, round_max);
             m = round_max;
         }
-        if (m > -INFINITY) {
-            const float shift = m * kLog2e;
+        const float shift = shift_of(m);
 #pragma unroll
-            for (int u = 0; u < kSplitUnroll; ++u)
+        for (int u = 0; u < kSplitUnroll; ++u)
 #pragma unroll
-                for (int e = 0; e < W; ++e) s += __builtin_amdgcn_exp2f(fmaf(x[u][e], kLog2e, -shift));
-        }
+            for (int e = 0; e < W; ++e) s += exponential(x[u][e], shift);
     }
     const float part_max = group_reduce<kSplitThreads, true>(m, scratch);
-    s = m > -INFINITY ? s * __builtin_amdgcn_exp2f((m - part_max) * kLog2e) : 0.0f;
-    s = group_reduce<kSplitThreads, false>(s, scratch);
+    s = group_reduce<kSplitThreads, false>(s * rescale(m, part_max), scratch);
     if (threadIdx.x == 0) {
         SplitPartial r;
         r.max = part_max;
@@ -506,9 +499,8 @@ __global__ __launch_bounds__(kSplitThreads) void softmax_split_finish_kernel(Sof
     mine.sum = 0.0f;
     if (threadIdx.x < gridDim.x) mine = partials[seg * gridDim.x + threadIdx.x];
     const float total_max = group_reduce<kSplitThreads, true>(mine.max, scratch);
-    const float scaled = mine.max > -INFINITY ? mine.sum * __builtin_amdgcn_exp2f((mine.max - total_max) * kLog2e) : 0.0f;
-    const float inv = 1.0f / group_reduce<kSplitThreads, false>(scaled, scratch);
-    const float shift = total_max * kLog2e;
+    const float inv = 1.0f / group_reduce<kSplitThreads, false>(mine.sum * rescale(mine.max, total_max), scratch);
+    const float shift = shift_of(total_max);
     const T *src = (const T *)p.in + row * p.in_row_stride + start * p.in_col_stride;
     T *dst = (T *)p.out + row * p.out_row_stride + start * p.out_col_stride;
     const int64_t pieces = (count + W - 1) / W;

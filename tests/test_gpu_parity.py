@@ -654,6 +654,28 @@ def test_softmax_of_large_values_is_normalised_against_one_shift(rows, cols, dty
             assert torch.allclose(probabilities[level == value], probabilities[0, position], rtol=SOFTMAX_REL[dtype], atol=step), (offset, position)
 
 
+@pytest.mark.parametrize("dtype", (torch.float32, torch.float16, torch.bfloat16))
+@pytest.mark.parametrize("rows, kernel", ((8, "softmax_split_partial_kernel"), (200, "softmax_loop_kernel")))
+def test_softmax_sums_of_large_values_meet_by_one_shift(rows, kernel, dtype):
+    """Long rows, whose sums are gathered over rounds, threads and parts with maxima of their own.  (fp32: a thread adds up
+    to 200 terms one after another, at most 200 x 2^-24 beside the other roundings.)  A thread that sees nothing but NaN passes it on."""
+    from ninetoothed_amd import runtime
+
+    for offset in (0.0, 1e3, -1e3, 3e4, -3e4, 1e5, -1e5, 1e7, -1e7):
+        if abs(offset) > torch.finfo(dtype).max / 2:
+            continue
+        x = (torch.randn(rows, 200000, device="cuda") * max(torch.finfo(dtype).eps * abs(offset), 5.0) + offset).to(dtype)
+        x[:, 150000:] = x[0, 0].clone().fill_(offset)
+        out = _softmax(x)
+        assert kernel in runtime.last_launch(), runtime.last_launch()
+        assert _softmax_error(out, x) <= max(SOFTMAX_REL[dtype], 2.0**-17), (offset, _softmax_error(out, x))
+    x.fill_(float("-inf"))
+    x[:, 70000] = 1.0
+    x[0, 5] = float("nan")
+    out = _softmax(x)
+    assert bool(out[0].isnan().all()) and bool((out[1:, 70000] == 1.0).all()) and float(out[1:].float().sum()) == rows - 1
+
+
 def test_softmax_baseline_shape_properties():
     x = torch.randn(4096, 4096, device="cuda")
     out = _softmax(x)
