@@ -57,18 +57,29 @@ NT_DEVICE float wave_reduce(float v) {
 
 // exp(x - m) is computed as exp2(x * log2e - shift) with shift = m * log2e, rounded.  That rounding is a factor of up to
 // 1 + |m| 2^-24 on every exponential; where all of a segment's share one shift it cancels against their sum.
-NT_DEVICE float shift_of(float m) {
+//
+// A product that overflows (a mask of fp32's or bf16's lowest value fills a part, or the whole segment) would leave infinity minus
+// infinity: there the factor is 1, since values of that size are equal or at least 2^100 apart.
+struct Base {
+    float scale, shift;
+};
+
+NT_DEVICE bool overflows(float m) { return fabsf(m) > 2.3e38f; }  // m * log2e does
+
+NT_DEVICE Base base_of(float m) {
 #pragma clang fp contract(off)  // (the difference of two shifts is that of the rounded products)
-    return m == -INFINITY ? 0.0f : m * kLog2e;  // (without a finite element there is nothing to subtract: the exponentials are zeros)
+    const float scale = overflows(m) ? 1.0f : kLog2e;
+    return {scale, m == -INFINITY ? 0.0f : m * scale};  // (without a finite element there is nothing to subtract: the exponentials are zeros)
 }
 
-NT_DEVICE float exponential(float x, float shift) { return __builtin_amdgcn_exp2f(fmaf(x, kLog2e, -shift)); }
+NT_DEVICE float exponential(float x, Base base) { return __builtin_amdgcn_exp2f(fmaf(x, base.scale, -base.shift)); }
 
 // The factor that takes exponentials relative to `part_max` to exponentials relative to `total_max`: from the difference of the two
 // SHIFTS, so that the rounding of each cancels.  exp(part_max - total_max) leaves a rounding of its own on every part (fp32
 // rows of 4096 values of spread 5, 2-norm of the error against 64 bits: 1.1e-5 around 1000, 1.2 % around 10^6; so 8e-8 at both).
 NT_DEVICE float rescale(float part_max, float total_max) {
-    return part_max == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(shift_of(part_max) - shift_of(total_max));
+    const float apart = overflows(part_max) || overflows(total_max) ? part_max - total_max : base_of(part_max).shift - base_of(total_max).shift;
+    return part_max == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(apart);
 }
 
 // Reduction over the kRowThreads threads that share a segment: waves, then partial results across waves through LDS.
@@ -187,22 +198,22 @@ __global__ __launch_bounds__(kRowThreads > 256 ? kRowThreads : 256) void softmax
     };
     forget_conversions();
     m = wave_reduce<true, (kRowThreads < 64 ? kRowThreads : 64)>(m);
-    const float shift = shift_of(m);
+    const Base from = base_of(m);
     float s = 0.0f;
 #pragma unroll
     for (int j = 0; j < kVecs; ++j)
 #pragma unroll
         for (int e = 0; e < W; ++e) {
             if constexpr (kRaw) {
-                s += exponential((float)raw[j][e], shift);
+                s += exponential((float)raw[j][e], from);
             } else {
-                x[j][e] = exponential(x[j][e], shift);
+                x[j][e] = exponential(x[j][e], from);
                 s += x[j][e];
             }
         }
 #pragma unroll
     for (int j = 0; j < kEdgeElems; ++j) {
-        edge[j] = exponential(edge[j], shift);
+        edge[j] = exponential(edge[j], from);
         s += edge[j];
     }
     forget_conversions();
@@ -224,7 +235,7 @@ __global__ __launch_bounds__(kRowThreads > 256 ? kRowThreads : 256) void softmax
         if (v < nvec) {
             vec_t o;
 #pragma unroll
-            for (int e = 0; e < W; ++e) o[e] = (T)((kRaw ? exponential((float)raw[kRaw ? j : 0][e], shift) : x[kRaw ? 0 : j][e]) * factor);
+            for (int e = 0; e < W; ++e) o[e] = (T)((kRaw ? exponential((float)raw[kRaw ? j : 0][e], from) : x[kRaw ? 0 : j][e]) * factor);
             __builtin_nontemporal_store(o, (access_t *)(dst + head + (int64_t)v * W));
         }
     }
@@ -264,13 +275,13 @@ __global__ __launch_bounds__(256) void softmax_thread_per_row_kernel(SoftmaxPara
             for (int e = 0; e < kWidth; ++e) x[j][e] = -INFINITY;
         }
     }
-    const float shift = m * kLog2e;
+    const Base from = base_of(m);
     float s = 0.0f;
 #pragma unroll
     for (int j = 0; j < kMaxPieces; ++j)
 #pragma unroll
         for (int e = 0; e < kWidth; ++e) {
-            x[j][e] = __builtin_amdgcn_exp2f(fmaf(x[j][e], kLog2e, -shift));  // (as in softmax_split_in_registers_kernel)
+            x[j][e] = exponential(x[j][e], from);
             s += x[j][e];
         }
     const float inv = 1.0f / s;
@@ -319,11 +330,11 @@ __global__ __launch_bounds__(kRowThreads > 256 ? kRowThreads : 256) void softmax
         m = fmaxf(m, x[j]);
     }
     m = group_reduce<kRowThreads, true>(m, scratch);
-    const float shift = m * kLog2e;
+    const Base from = base_of(m);
     float s = 0.0f;
 #pragma unroll
     for (int j = 0; j < kElems; ++j) {
-        x[j] = __builtin_amdgcn_exp2f(fmaf(x[j], kLog2e, -shift));
+        x[j] = exponential(x[j], from);
         s += x[j];
     }
     s = group_reduce<kRowThreads, false>(s, scratch);
@@ -363,21 +374,21 @@ NT_DEVICE void wide_load(const T *src, int64_t col_stride, int64_t index, int64_
 
 // exp(x - maximum) / sum of one access, stored
 template <typename T, bool kVec>
-NT_DEVICE void wide_store(T *dst, int64_t col_stride, int64_t index, int64_t count, const float (&x)[WideAccess<T, kVec>::kWidth], float shift, float inv) {
+NT_DEVICE void wide_store(T *dst, int64_t col_stride, int64_t index, int64_t count, const float (&x)[WideAccess<T, kVec>::kWidth], Base from, float inv) {
     constexpr int W = WideAccess<T, kVec>::kWidth;
     if constexpr (kVec) {
         if ((index + 1) * W <= count) {
             typename WideAccess<T, kVec>::type v;
 #pragma unroll
-            for (int e = 0; e < W; ++e) v[e] = (T)(exponential(x[e], shift) * inv);
+            for (int e = 0; e < W; ++e) v[e] = (T)(exponential(x[e], from) * inv);
             *(typename WideAccess<T, kVec>::type *)(dst + index * W) = v;
         } else {
 #pragma unroll
             for (int e = 0; e < W; ++e)
-                if (index * W + e < count) dst[index * W + e] = (T)(exponential(x[e], shift) * inv);
+                if (index * W + e < count) dst[index * W + e] = (T)(exponential(x[e], from) * inv);
         }
     } else {
-        if (index < count) dst[index * col_stride] = (T)(exponential(x[0], shift) * inv);
+        if (index < count) dst[index * col_stride] = (T)(exponential(x[0], from) * inv);
     }
 }
 
@@ -413,22 +424,22 @@ __global__ __launch_bounds__(kLoopThreads) void softmax_loop_kernel(SoftmaxParam
             s *= rescale(m, round_max);
             m = round_max;
         }
-        const float shift = shift_of(m);
+        const Base from = base_of(m);
 #pragma unroll
         for (int u = 0; u < kLoopUnroll; ++u)
 #pragma unroll
-            for (int e = 0; e < W; ++e) s += exponential(x[u][e], shift);
+            for (int e = 0; e < W; ++e) s += exponential(x[u][e], from);
     }
     const float total_max = group_reduce<kLoopThreads, true>(m, scratch);
     s = group_reduce<kLoopThreads, false>(s * rescale(m, total_max), scratch);  // (every thread's sum is relative to its own maximum)
     const float inv = 1.0f / s;
-    const float shift = shift_of(total_max);
+    const Base from = base_of(total_max);
     for (int64_t base = threadIdx.x; base < pieces; base += kLoopThreads * kLoopUnroll) {
         float x[kLoopUnroll][W];
 #pragma unroll
         for (int u = 0; u < kLoopUnroll; ++u) wide_load<T, kVec>(src, p.in_col_stride, base + u * kLoopThreads, len, x[u]);
 #pragma unroll
-        for (int u = 0; u < kLoopUnroll; ++u) wide_store<T, kVec>(dst, p.out_col_stride, base + u * kLoopThreads, len, x[u], shift, inv);
+        for (int u = 0; u < kLoopUnroll; ++u) wide_store<T, kVec>(dst, p.out_col_stride, base + u * kLoopThreads, len, x[u], from, inv);
     }
 }
 
@@ -468,11 +479,11 @@ __global__ __launch_bounds__(kSplitThreads) void softmax_split_partial_kernel(So
             s *= rescale(m, round_max);
             m = round_max;
         }
-        const float shift = shift_of(m);
+        const Base from = base_of(m);
 #pragma unroll
         for (int u = 0; u < kSplitUnroll; ++u)
 #pragma unroll
-            for (int e = 0; e < W; ++e) s += exponential(x[u][e], shift);
+            for (int e = 0; e < W; ++e) s += exponential(x[u][e], from);
     }
     const float part_max = group_reduce<kSplitThreads, true>(m, scratch);
     s = group_reduce<kSplitThreads, false>(s * rescale(m, part_max), scratch);
@@ -500,7 +511,7 @@ __global__ __launch_bounds__(kSplitThreads) void softmax_split_finish_kernel(Sof
     if (threadIdx.x < gridDim.x) mine = partials[seg * gridDim.x + threadIdx.x];
     const float total_max = group_reduce<kSplitThreads, true>(mine.max, scratch);
     const float inv = 1.0f / group_reduce<kSplitThreads, false>(mine.sum * rescale(mine.max, total_max), scratch);
-    const float shift = shift_of(total_max);
+    const Base from = base_of(total_max);
     const T *src = (const T *)p.in + row * p.in_row_stride + start * p.in_col_stride;
     T *dst = (T *)p.out + row * p.out_row_stride + start * p.out_col_stride;
     const int64_t pieces = (count + W - 1) / W;
@@ -509,7 +520,7 @@ __global__ __launch_bounds__(kSplitThreads) void softmax_split_finish_kernel(Sof
 #pragma unroll
         for (int u = 0; u < kSplitUnroll; ++u) wide_load<T, kVec>(src, p.in_col_stride, base + u * kSplitThreads, count, x[u]);
 #pragma unroll
-        for (int u = 0; u < kSplitUnroll; ++u) wide_store<T, kVec>(dst, p.out_col_stride, base + u * kSplitThreads, count, x[u], shift, inv);
+        for (int u = 0; u < kSplitUnroll; ++u) wide_store<T, kVec>(dst, p.out_col_stride, base + u * kSplitThreads, count, x[u], from, inv);
     }
 }
 

@@ -676,6 +676,30 @@ def test_softmax_sums_of_large_values_meet_by_one_shift(rows, kernel, dtype):
     assert bool(out[0].isnan().all()) and bool((out[1:, 70000] == 1.0).all()) and float(out[1:].float().sum()) == rows - 1
 
 
+@pytest.mark.parametrize("dtype", (torch.float32, torch.bfloat16, torch.float16))
+@pytest.mark.parametrize("rows, cols, step", ((4096, 8, 1), (5, 8, 1), (6, 100, 1), (5, 700, 1), (4100, 1800, 1), (5, 1800, 1), (5, 8190, 1), (5, 40000, 1), (8, 200000, 1), (200, 200000, 1), (5, 30, 2), (5, 4000, 2), (5, 16000, 2)))
+def test_softmax_of_masks_of_the_lowest_value(rows, cols, step, dtype):
+    """Half a row, most of it, and whole rows at the type's lowest value (times log2 e it overflows), and maxima that large, in
+    every kernel: per thread, per group of lanes, per wave, per workgroup, in parts, in sweeps, element by element."""
+    lowest = torch.finfo(dtype).min
+    x = torch.empty(rows, cols * step, device="cuda", dtype=dtype)[:, ::step]
+    x.copy_(torch.randn(rows, cols, device="cuda"))
+    x[1, : cols // 2] = lowest
+    x[2, 1:] = lowest
+    x[3:] = lowest
+    x[4, cols // 2 :] = lowest * 0.875
+    x[-1, cols // 3] = -lowest
+    out = torch.empty_like(x)
+    kernel = ninetoothed.make(programs.softmax.arrangement, programs.softmax.application, programs.softmax.tensors())
+    kernel(x, out, BLOCK_SIZE=cols)
+    expected = torch.softmax(x.double(), dim=-1)
+    # (as above; fp16's smallest results are multiples of 2^-24: half of one on each)
+    tiny = 2.0**-25 * cols**0.5 if dtype == torch.float16 else 0.0
+    for row in (0, 1, 2, 3, 4, rows - 1):
+        error, size = float((out[row].double() - expected[row]).norm()), float(expected[row].norm())
+        assert error <= max(SOFTMAX_REL[dtype], 2.0**-17) * size + tiny, (row, error, size)
+
+
 def test_softmax_baseline_shape_properties():
     x = torch.randn(4096, 4096, device="cuda")
     out = _softmax(x)
