@@ -324,7 +324,8 @@ NineToothedResult launch_nt_gemm_config(NineToothedStream stream, int config,
  * 3 ms per round, and an instance's figure is the minimum of its rounds -- a
  * clock dip has to hit the same instance in every round to change the choice.
  * The instance of the untuned rule stays the choice unless another one is more
- * than 2 % faster.  This call synchronises.  Returns 0 and the winner in
+ * than 2 % faster (25 % where the rule names a skinny instance: timed launches
+ * find the rhs in the caches, calls of a program do not).  This call synchronises.  Returns 0 and the winner in
  * *best_config, its time per launch in *best_ms.  On a stream that is being
  * captured into a graph nothing is timed or recorded: returns 0 with
  * *best_config = -1.  A problem that a single instance takes (fp32 or fp8 operands; fp16 / bf16 operands that the
@@ -348,7 +349,7 @@ NineToothedResult nt_tune_gemm(NineToothedStream stream,
  * sequence lengths, head dimension, causal flag) without block-size hints; the variant of the untuned rule stays
  * unless another one is more than 2 % faster.  *best_variant = -1 when nothing was timed (a stream that is being
  * captured into a graph), -2 when the problem has no alternatives (FLOAT32 tensors, head dimensions other than 64
- * and 128, shapes whose key range is split). */
+ * and 128, one query per head, shapes whose key range is split). */
 NineToothedResult nt_tune_attention(NineToothedStream stream,
                                     NineToothedTensor q, NineToothedTensor k, NineToothedTensor v,
                                     NineToothedTensor is_causal, NineToothedTensor scale,

@@ -515,10 +515,8 @@ int lookup_tuned(const GemmProblem &q) {
     return choice >= 0 && choice < kNumInstances ? choice : -1;
 }
 
-// The skinny instance that a product runs on whatever has been timed for it, or -1: timing launches find B in the L2 that
-// the launch before has left it in, a program that works through its layers finds it in memory or, at best, in the Infinity
-// Cache, where these kernels stand better (32 x 14336 x 4096: 18.9 us on tiles with B in L2, 29.0 without; 22.9 and 24.9 on
-// 32 columns per workgroup).  The lines lie where the tile instances win with B in the Infinity Cache (us, tiles / 16 columns /
+// The skinny instance that a product runs on if nothing is recorded for it, or -1.  The lines lie where the tile instances win
+// with B in the Infinity Cache (us, tiles / 16 columns /
 // 32 columns): m = 16: 4096 x 4096 13.3 / 8.0 / 10.8; 8192 x 4096 15.6 / 12.3 / 11.8; 8192 x 8192 32.5 / 24.1 / 43.5; 16384 x 4096 30.9 /
 // 25.2 / 21.9; 12288 x 2048 10.5 / 11.3 / 11.4; m = 40: 2048 x 2048 6.3 / 5.8 / 8.0; 2048 x 512 3.9 / 4.4 / 4.5; 6144 x 4096 17.0 / 16.5 /
 // 13.8; 12288 x 4096 25.9 / 34.3 / 28.0; m = 64: 4096 x 2048 9.8 / 8.8 / 9.3; 2048 x 1024 4.5 / 5.2 / 5.8; 4096 x 8192 19.4 / 24.0 / 38.1.
@@ -901,8 +899,7 @@ int run_gemm(hipStream_t stream, const GemmProblem &q, int bm, int bn, int bk, b
         if (widened != NINETOOTHED_NO_KERNEL) return widened;
     }
     int choice = -1;
-    if (bm <= 0 && bn <= 0 && bk <= 0) choice = skinny_choice(q);
-    if (choice < 0 && (bm <= 0 || bn <= 0) && q.batch == 1) choice = lookup_tuned(q);  // (tuned choices are recorded for single products)
+    if ((bm <= 0 || bn <= 0) && q.batch == 1) choice = lookup_tuned(q);  // (tuned choices are recorded for single products)
     if (choice < 0 || !kInstances[choice].accepts(q)) choice = heuristic_choice(q, bm, bn, bk);
     if (choice < 0) return NINETOOTHED_NO_KERNEL;
     if (choice == kAnyStride && may_copy) {
@@ -1056,11 +1053,6 @@ NineToothedResult nt_tune_gemm(NineToothedStream stream_, NineToothedTensor inpu
     GemmProblem q = output_by_columns(given) ? transposed_problem(given) : given;
     int best = -1;
     float best_time = 0.0f;
-    if (skinny_choice(q) >= 0) {  // (not chosen by timing)
-        if (best_config) *best_config = -2;
-        if (best_ms) *best_ms = 0.0f;
-        return 0;
-    }
     // A problem that a single instance accepts has nothing to time.  Operands that only the any-stride kernel reads
     // in place run on dense copies (launch_nt_matmul / launch_nt_addmm): then the product on the copies is what
     // gets timed and recorded, under its own key, where the launch functions look it up.
@@ -1087,14 +1079,19 @@ NineToothedResult nt_tune_gemm(NineToothedStream stream_, NineToothedTensor inpu
     }
     // (inside a graph capture nothing is timed: the problem stays on the fixed preference order and nothing is recorded)
     // the untuned rule's instance is timed first and stays unless another one is more than 2 % faster: timings of a
-    // few launches scatter by about that much, and the choice should not differ from process to process for nothing
+    // few launches scatter by about that much, and the choice should not differ from process to process for nothing.
+    // A skinny instance stays unless another one is more than 25 % faster: timing launches find B in the caches that
+    // the launch before has left it in, a program that works through its layers finds it in memory, where the skinny
+    // kernels lose less (32 x 14336 x 4096: 18.9 us on tiles with B in the caches, 29.0 without; 22.9 and 24.9 on 32
+    // columns per workgroup).
     const int preferred = heuristic_choice(q, 0, 0, 0);
+    const float margin = preferred == kSkinny16 || preferred == kSkinny32 ? 0.25f : 0.02f;
     auto instance_of = [&](int i) { return preferred < 0 ? i : (i == 0 ? preferred : (i - 1 < preferred ? i - 1 : i)); };
     const int result = tune_time(stream, kNumInstances, iters, [&](int i) -> int {
         const int instance = instance_of(i);
         if (!kInstances[instance].accepts(q)) return NINETOOTHED_NO_KERNEL;
         return (int)kInstances[instance].launch(q, stream);
-    }, &best, &best_time, 0.02f);
+    }, &best, &best_time, margin);
     if (best >= 0) best = instance_of(best);
     if (best_config) *best_config = best;
     if (best_ms) *best_ms = best_time;

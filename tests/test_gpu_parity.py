@@ -4,6 +4,7 @@ oracle finishes in seconds, and with the torch ops the reference's own tests
 compare against.  Bars: rtol = atol = 1e-2 for fp16 / bf16 (the reference's
 tests/test_attention.py:102 states the same for fp16), 1e-5 for fp32 softmax."""
 
+import ctypes
 import functools
 
 import numpy as np
@@ -2112,6 +2113,39 @@ def test_gemm_skinny_instances_at_the_edges_of_their_tiles(m, n, k, dtype):
     out = torch.full((m, n), float("nan"), dtype=dtype, device="cuda")
     _matmul_kernel()(a, w.t(), out)
     assert torch.allclose(out.float(), product, **HALF_TOL)
+
+
+@pytest.mark.parametrize("m, n, k", ((16, 1032, 2048), (40, 776, 2056), (16, 1000, 4097)))
+def test_gemm_skinny_products_run_on_the_choice_that_was_timed_or_loaded(m, n, k, tmp_path, monkeypatch):
+    """`x @ w.T` with few rows: without a recorded choice a skinny instance; a timed one is reported and runs from then
+    on, on operands in place and on dense copies (K = 4097) alike; so does one read from a file."""
+    from ninetoothed_amd import auto_tuner, runtime
+
+    monkeypatch.setattr(auto_tuner, "CACHE_DIR", tmp_path)
+    lib = runtime.library()
+    fp16 = runtime.DATA_TYPE_INDEX["fp16"]
+    null = runtime.ArgumentTensor.null()
+    x, w = _randn(m, k).cuda(), _randn(n, k, scale=k**-0.5).cuda()
+    out = torch.empty(m, n, dtype=torch.float16, device="cuda")
+    tensors = [runtime.ArgumentTensor.from_torch_tensor(t) for t in (x, w.t(), out)]
+
+    def launch():
+        out.fill_(float("nan"))
+        assert lib.launch_nt_matmul(runtime.current_stream(), *tensors, fp16, fp16, 0, 0, 0) == 0
+        assert torch.allclose(out.float(), x.float() @ w.float().t(), **HALF_TOL)
+        return runtime.last_launch()
+
+    assert "skinny" in launch()
+    instance, milliseconds = auto_tuner.tune(null, *tensors[:2], null, null, tensors[2], fp16, fp16)
+    assert instance >= 0 and milliseconds > 0.0
+    assert launch().startswith(f"gemm instance {instance}: ")
+    tile = next(i for i, name in enumerate(runtime.gemm_config_names()) if name.startswith("64x64x64") and name.endswith("tails"))
+    dense_k = -(-k // 8) * 8  # (copies have rows of whole 16-byte pieces)
+    path = tmp_path / "tuned.csv"
+    path.write_text(f"\n{lib.nt_tune_file_format()}\n{runtime.TUNE_GEMM},{fp16},{fp16},{m},{n},{dense_k},0,1\n{tile},64,64,64\n")
+    entries = ctypes.c_int(0)
+    assert lib.nt_tune_cache_load(str(path).encode(), ctypes.byref(entries)) == 0 and entries.value == 1
+    assert launch().startswith(f"gemm instance {tile}: ")
 
 
 @pytest.mark.parametrize("dtype", (torch.float16, torch.bfloat16))
