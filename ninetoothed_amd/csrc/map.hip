@@ -585,27 +585,6 @@ long long segment_offset_at(const NineToothedMapProgram &q, int segment, const l
 // per output the lanes of a wave would read a row each.  Returns the lanes per output element: 1, 64, or -- few outputs over long ranges -- the whole workgroup.
 int cooperative_lanes(const NineToothedMapProgram &q);
 
-// Threads of a workgroup.  In tile mode (one workgroup per tile) a tile of up to 16384 elements gets enough
-// threads that each holds at most 16 elements, preferably 8, which the generated code then keeps in registers
-// (layer norm over 4096 rows of fp32, 256 threads -> this choice: 4096 wide 38 -> 27 us, 8192 wide 83 -> 54,
-// 16384 wide 168 -> 119; 1024 threads on 8192 columns: the same for the norms, softmax 64 us against 46).
-int workgroup_threads(const NineToothedMapProgram &q) {
-    if (q.num_phases == 0) return kMapThreads;
-    long long tile_elements = 1;
-    for (int v = q.num_grid; v < q.num_vars; ++v) tile_elements *= (long long)q.extents[v];
-    if (tile_elements > 2048 && tile_elements <= 8192) return 512;
-    if (tile_elements > 8192 && tile_elements <= 16384) return 1024;
-    return kMapThreads;
-}
-
-// Threads that share a tile in tile mode: a wave for tiles of up to 512 elements (a workgroup then holds four
-// tiles and the reductions need no LDS exchange and no barrier), else the whole workgroup.
-int tile_group(const NineToothedMapProgram &q) {
-    long long tile_elements = 1;
-    for (int v = q.num_grid; v < q.num_vars; ++v) tile_elements *= (long long)q.extents[v];
-    return q.num_phases > 0 && tile_elements <= 512 ? 64 : workgroup_threads(q);
-}
-
 int cooperative_lanes(const NineToothedMapProgram &q) {
     const int num_out = q.num_vars - q.num_reduced;
     if (q.num_phases != 0 || q.reduce_op == NT_MAP_REDUCE_NONE || q.num_dynamic != 0 || q.num_reduced == 0 || q.store_op != NT_MAP_STORE_ASSIGN) return 1;
@@ -647,8 +626,8 @@ struct MapCodegen {
 
     bool narrow;  // index arithmetic in 32 bits: every index value provably fits
     int lanes;    // lanes per output element (cooperative_lanes)
-    int threads;  // of a workgroup (workgroup_threads)
-    int group;    // threads that share a tile in tile mode (tile_group)
+    int threads;  // of a workgroup
+    int group;    // threads that share a tile in tile mode
     // Tile mode with small tiles: a thread's elements stay in registers between the phases.
     // `kept` lists the operands whose loaded values an earlier phase left in `ld<slot>[e]`,
     // `in_body` maps operands already loaded in the loop body being emitted to their temporaries.
@@ -662,14 +641,26 @@ struct MapCodegen {
     std::vector<bool> kept = std::vector<bool>(NT_MAP_MAX_OPERANDS, false);
     std::map<int, std::string> in_body;
 
-    explicit MapCodegen(const NineToothedMapProgram &program) : p(program), narrow(fits_int32(program)), lanes(cooperative_lanes(program)), threads(workgroup_threads(program)), group(tile_group(program)) {
+    explicit MapCodegen(const NineToothedMapProgram &program) : p(program), narrow(fits_int32(program)), lanes(cooperative_lanes(program)) { choose_threads(); }
+
+    // Threads of a workgroup and, in tile mode (a workgroup per tile, or a wave), the threads that share a tile.
+    void choose_threads() {
+        threads = group = kMapThreads;
+        if (p.num_phases == 0) return;
+        long long tile_elements = 1;
+        for (int v = p.num_grid; v < p.num_vars; ++v) tile_elements *= (long long)p.extents[v];
+        // A tile of up to 16384 elements gets enough threads that each holds at most 16 elements, preferably 8, which the
+        // generated code then keeps in registers (layer norm over 4096 rows of fp32, 256 threads -> this choice: 4096 wide 38 ->
+        // 27 us, 8192 wide 83 -> 54, 16384 wide 168 -> 119; 1024 threads on 8192 columns: the same for the norms, softmax 64 us against 46).
+        if (tile_elements > 2048 && tile_elements <= 8192) threads = 512;
+        if (tile_elements > 8192 && tile_elements <= 16384) threads = 1024;
+        // a wave for tiles of up to 512 elements: four tiles per workgroup, reductions without LDS and without a barrier
+        group = tile_elements <= 512 ? 64 : threads;
         // Tiles of one reduction whose elements come in groups of 8 (16 bytes): two groups per thread.  Two loads in flight per
         // tensor and half the waves to meet cost less than they hide (bf16 rms norm, a kernel alone: 4096 rows of 4096 on 512 threads
         // 13.6 us, on 256 10.5, on 128 or 64 with 4 or 8 groups 10.8 and 10.7; 16384 rows of 1024 on 256 threads 12.8 us, on 128
         // 13.4, on a wave 10.5).  Longer tiles have 16 elements per thread already; element by element 8 per thread stay better.
-        long long tile_elements = 1;
-        for (int v = program.num_grid; v < program.num_vars; ++v) tile_elements *= (long long)program.extents[v];
-        if (program.num_phases == 1 && tile_elements > 512 && tile_elements <= 4096 && tile_vector_width(tile_elements) > 0) {
+        if (p.num_phases == 1 && tile_elements > 512 && tile_elements <= 4096 && tile_vector_width(tile_elements) > 0) {
             threads = kMapThreads;
             group = tile_elements <= 1024 ? 64 : kMapThreads;
         }
