@@ -967,24 +967,26 @@ __global__ __launch_bounds__(kWaves * 64) void attention_decode_kernel(Attention
     const int head = bh % p.heads, batch = bh / p.heads;
     const T *K = (const T *)p.k + batch * p.k_strides[0] + head * p.k_strides[1];
     const T *V = (const T *)p.v + batch * p.v_strides[0] + head * p.v_strides[1];
-    const int keys = p.causal ? min(p.seq_k, 1) : p.seq_k;  // (a causal mask leaves query 0 its key 0)
-    const int first = kParts ? part * p.blocks_per_part * kWaves * kStepKeys : 0;
-    const int last = kParts ? min(keys, first + p.blocks_per_part * kWaves * kStepKeys) : keys;
+    // (unsigned: one row expanded to as many keys as an int counts is stepped past its end)
+    const unsigned keys = p.causal ? 1u : (unsigned)p.seq_k;  // (a causal mask leaves query 0 its key 0)
+    const unsigned part_keys = (unsigned)p.blocks_per_part * kWaves * kStepKeys;
+    const unsigned first = kParts ? part * part_keys : 0;
+    const unsigned last = kParts ? min(keys, first + part_keys) : keys;
 
     // descriptors that end with the last key's row; lanes without a key get an offset behind them and read zeros
     const unsigned k_row = (unsigned)p.k_strides[2] * 2u, v_row = (unsigned)p.v_strides[2] * 2u;
     __amdgpu_buffer_rsrc_t k_rsrc = __builtin_amdgcn_make_buffer_rsrc((void *)K, 0, (unsigned)((keys - 1) * p.k_strides[2] + D) * 2u, 0x00020000);
     __amdgpu_buffer_rsrc_t v_rsrc = __builtin_amdgcn_make_buffer_rsrc((void *)V, 0, (unsigned)((keys - 1) * p.v_strides[2] + D) * 2u, 0x00020000);
     constexpr unsigned kBehind = 0xfffffff0u;
-    auto load = [&](__amdgpu_buffer_rsrc_t rsrc, unsigned row_bytes, int key0, vec8(&to)[kDecodeLoads]) __attribute__((always_inline)) {
+    auto load = [&](__amdgpu_buffer_rsrc_t rsrc, unsigned row_bytes, unsigned key0, vec8(&to)[kDecodeLoads]) __attribute__((always_inline)) {
 #pragma unroll
         for (int j = 0; j < kDecodeLoads; ++j) {
-            const int key = key0 + j * kGroups + group;
-            const unsigned offset = key < last ? (unsigned)key * row_bytes + col * 2 : kBehind;
+            const unsigned key = key0 + j * kGroups + group;
+            const unsigned offset = key < last ? key * row_bytes + col * 2 : kBehind;
             to[j] = __builtin_bit_cast(vec8, __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)offset, 0, 0));
         }
     };
-    int key0 = first + wave * kStepKeys;
+    unsigned key0 = first + wave * kStepKeys;
     vec8 kf[kDecodeLoads], vf[kDecodeLoads];
     load(k_rsrc, k_row, key0, kf);
     load(v_rsrc, v_row, key0, vf);
@@ -1085,7 +1087,7 @@ int launch_decode(AttentionParams &p, hipStream_t stream) {
     if (pairs > 0x7fffffffll) return NINETOOTHED_NO_KERNEL;
     if (pairs < 128 && keys > 4 * 16 * kDecodeStepKeys<D>) {
         constexpr int kStep = 4 * kDecodeStepKeys<D>;  // keys of a workgroup's step
-        const int steps = ceil_div(keys, kStep);
+        const int steps = (keys - 1) / kStep + 1;
         const int wanted = (int)std::min<int64_t>((1024 + pairs - 1) / pairs, steps / 2);
         p.blocks_per_part = ceil_div(steps, wanted);
         p.parts = ceil_div(steps, p.blocks_per_part);

@@ -854,6 +854,18 @@ def test_attention_of_one_query(batch, heads, seq_k, emb_dim, dtype):
     assert run(False).isnan().all()
 
 
+def test_attention_of_one_query_over_one_row_expanded_to_as_many_keys_as_an_int_counts():
+    # (every key is the same: the result is the row of V.  1024 parts of 32 lane groups: a group adds one number 65536 times
+    # to a running sum, of which every addition may round off 2^-24; then one rounding to fp16)
+    q, k, v = (_randn(1, 1, 1, 64).cuda() for _ in range(3))
+    expanded = (1, 1, 2**31 - 1, 64)
+    o = torch.full_like(q, float("nan"))
+    kernel = ninetoothed.make(programs.attention.arrangement_with_scale, programs.attention.application_with_scale, programs.attention.tensors(True))
+    kernel(q, k.expand(expanded), v.expand(expanded), False, 0.125, o)
+    _native_only(kernel, "launch_nt_attention")
+    assert torch.allclose(o, v, rtol=65536 * 2.0**-24 + 2.0**-11, atol=0)
+
+
 def test_attention_closed_forms_and_layouts():
     q, v = _randn(1, 2, 300, 64).cuda(), _randn(1, 2, 300, 64).cuda()
     k = torch.zeros_like(q)
