@@ -121,7 +121,9 @@ struct Vec16 {  // 16 bytes of T
 //
 // What bounds it: memory where there are segments for every CU (fp32 4096 x 4096 20.3 us = 6.6 TB/s; fp16 8192 x 4099 21.9 us =
 // 6.1 TB/s, 190 us with element-wise loads; fp16 4096 x 50257 145 us = 5.7 TB/s, 230 us in two sweeps over memory), the
-// arithmetic of the CUs that have a segment where there are few (fp16 [64, 50257] 6.5 us, 11.4 over two launches).
+// arithmetic of the CUs that have a segment where there are few (fp16 [64, 50257] 6.2 us, 11.4 over two launches).  Launches of
+// a few microseconds gain or lose a little against loads that were waited for one by one (bf16 9000 x 2000 13.1 -> 12.0 us, fp32
+// 8192 x 2000 20.9 -> 20.1, but bf16 5274 x 1792 6.9 -> 7.3 and fp32 5274 x 1792 11.8 -> 12.0: 64 threads there, 256 are 13 % slower on bf16).
 template <typename T, int kRowThreads, int kVecs>
 __global__ __launch_bounds__(kRowThreads > 256 ? kRowThreads : 256) void softmax_split_in_registers_kernel(SoftmaxParams p) {
     typedef typename Vec16<T>::type vec_t;
@@ -303,7 +305,7 @@ hipError_t launch_thread_per_row(const SoftmaxParams &p, hipStream_t stream) {
     return hipGetLastError();
 }
 
-// Element path: any strides / alignment / length up to kRowThreads * kElems.
+// Element path: any strides, length up to kRowThreads * kElems (what the register kernel does not take: columns that are not one element apart).
 template <typename T, int kRowThreads, int kElems>
 __global__ __launch_bounds__(kRowThreads > 256 ? kRowThreads : 256) void softmax_elem_kernel(SoftmaxParams p) {
     constexpr int kGroups = kRowThreads > 256 ? 1 : 256 / kRowThreads;
@@ -554,36 +556,40 @@ bool run_split(const SoftmaxParams &p, int64_t len, bool in_registers, hipStream
     return true;
 }
 
-template <typename T, int kRowThreads>
+// Whole vectors of the longest segments that 256, 512 and 1024 threads hold (why there: at the choice in run_softmax).
+template <typename T> constexpr int64_t kMostVecs256 = sizeof(T) == 4 ? 768 : 2048;
+template <typename T> constexpr int64_t kMostVecs512 = sizeof(T) == 4 ? 2048 : 4096;
+constexpr int64_t kMostVecs1024 = 1024 * 16;
+
+// Segments of kFewest .. kMost whole vectors.
+template <typename T, int kRowThreads, int64_t kFewest, int64_t kMost>
 hipError_t launch_in_registers(const SoftmaxParams &p, int64_t len, hipStream_t stream) {
     const int64_t total = p.rows * p.segments;
     constexpr int kGroups = kRowThreads > 256 ? 1 : 256 / kRowThreads;
     const dim3 grid((unsigned)((total + kGroups - 1) / kGroups)), block(kRowThreads > 256 ? kRowThreads : 256);
     const int64_t vecs = (len / Vec16<T>::kWidth + kRowThreads - 1) / kRowThreads;  // per thread
     note_launch(kLaunchSoftmax, kRowThreads, "softmax_split_in_registers_kernel, one launch, this many threads per row segment, one part per wave");
-#define NT_SOFTMAX_VECS(N) \
-    if (vecs <= N) { \
-        softmax_split_in_registers_kernel<T, kRowThreads, N><<<grid, block, 0, stream>>>(p); \
-        return hipGetLastError(); \
+    static_assert(kMost <= 16 * kRowThreads, "at most 16 vectors per thread");
+    // kPrevious: the next smaller step
+#define NT_SOFTMAX_VECS(N, kPrevious) \
+    if constexpr (kFewest <= N * kRowThreads && kMost > kPrevious * kRowThreads) { \
+        if (vecs <= N) { \
+            softmax_split_in_registers_kernel<T, kRowThreads, N><<<grid, block, 0, stream>>>(p); \
+            return hipGetLastError(); \
+        } \
     }
     // (a thread computes all its vectors, also those behind the end of a segment: steps of one where a step is most of the work)
-    NT_SOFTMAX_VECS(1)
-    NT_SOFTMAX_VECS(2)
-    if constexpr (kRowThreads >= 32) {
-        NT_SOFTMAX_VECS(3)
-    }
-    if constexpr (kRowThreads >= 64) {
-        NT_SOFTMAX_VECS(4)
-        NT_SOFTMAX_VECS(5)
-        NT_SOFTMAX_VECS(6)
-        NT_SOFTMAX_VECS(7)
-        NT_SOFTMAX_VECS(8)
-    }
-    if constexpr (kRowThreads >= 1024) {
-        NT_SOFTMAX_VECS(10)
-        NT_SOFTMAX_VECS(12)
-        NT_SOFTMAX_VECS(16)
-    }
+    NT_SOFTMAX_VECS(1, 0)
+    NT_SOFTMAX_VECS(2, 1)
+    NT_SOFTMAX_VECS(3, 2)
+    NT_SOFTMAX_VECS(4, 3)
+    NT_SOFTMAX_VECS(5, 4)
+    NT_SOFTMAX_VECS(6, 5)
+    NT_SOFTMAX_VECS(7, 6)
+    NT_SOFTMAX_VECS(8, 7)
+    NT_SOFTMAX_VECS(10, 8)
+    NT_SOFTMAX_VECS(12, 10)
+    NT_SOFTMAX_VECS(16, 12)
 #undef NT_SOFTMAX_VECS
     return hipErrorInvalidValue;
 }
@@ -620,7 +626,7 @@ int run_softmax(const SoftmaxParams &p, int variant, hipStream_t stream) {
         }
     }
     // segments that 1024 threads hold in registers: 64 of them per thread (2-byte elements as they are, two per register)
-    const bool in_registers = unit_columns && len <= (int64_t)1024 * 16 * W;
+    const bool in_registers = unit_columns && len <= kMostVecs1024 * W;
     if (variant == 0) {
         hipError_t status = hipSuccess;
         if (run_split<T>(p, len, in_registers, stream, &status)) return (int)status;
@@ -634,17 +640,17 @@ int run_softmax(const SoftmaxParams &p, int variant, hipStream_t stream) {
         // 11832 x 4152 256: 33.5, 512: 44.6; 4000 x 12289 256: 33.4, 512: 32.8, 1024: 39.4; 4000 x 32000 512: 86.6, 1024: 89.5; 4096 x 50257
         // 512: 149, 1024: 145
         if (variant == 0 && p.segments == 1) {
-            if (nvec <= 8) return (int)launch_in_registers<T, 8>(p, len, stream);
-            if (nvec <= 32) return (int)launch_in_registers<T, 16>(p, len, stream);
-            if (nvec <= 96) return (int)launch_in_registers<T, 32>(p, len, stream);
+            if (nvec <= 8) return (int)launch_in_registers<T, 8, 0, 8>(p, len, stream);
+            if (nvec <= 32) return (int)launch_in_registers<T, 16, 9, 32>(p, len, stream);
+            if (nvec <= 96) return (int)launch_in_registers<T, 32, 33, 96>(p, len, stream);
         }
         const bool one_wave = nvec <= 512 && (variant == 1 || (variant == 0 && (total >= 4096 || nvec <= 64)));
-        if (one_wave) return (int)launch_in_registers<T, 64>(p, len, stream);
-        if (nvec <= (sizeof(T) == 4 ? 768 : 2048)) return (int)launch_in_registers<T, 256>(p, len, stream);
-        if (nvec <= (sizeof(T) == 4 ? 2048 : 4096)) return (int)launch_in_registers<T, 512>(p, len, stream);
-        return (int)launch_in_registers<T, 1024>(p, len, stream);
+        if (one_wave) return (int)launch_in_registers<T, 64, 0, 512>(p, len, stream);
+        if (nvec <= kMostVecs256<T>) return (int)launch_in_registers<T, 256, 0, kMostVecs256<T>>(p, len, stream);
+        if (nvec <= kMostVecs512<T>) return (int)launch_in_registers<T, 512, kMostVecs256<T> + 1, kMostVecs512<T>>(p, len, stream);
+        return (int)launch_in_registers<T, 1024, kMostVecs512<T> + 1, kMostVecs1024>(p, len, stream);
     }
-    // element by element (any strides / alignment): as many threads per segment as keep every thread at
+    // element by element (any strides): as many threads per segment as keep every thread at
     // 4 .. 16 elements, from 8 lanes of a wave to a workgroup of 1024
     if (len <= 8 * 4) return (int)launch_elem<T, 8, 4>(p, stream);
     if (len <= 16 * 4) return (int)launch_elem<T, 16, 4>(p, stream);
@@ -652,8 +658,9 @@ int run_softmax(const SoftmaxParams &p, int variant, hipStream_t stream) {
     if (len <= 64 * 4) return (int)launch_elem<T, 64, 4>(p, stream);
     if (len <= 64 * 16) return (int)launch_elem<T, 64, 16>(p, stream);
     if (len <= 256 * 16) return (int)launch_elem<T, 256, 16>(p, stream);
-    // (measured: 8192 x 4099 fp32 3.0 TB/s with 256 threads, 2.5 with 1024; 4096 x 12289 fp16 1.3 against 1.9;
-    // 2048 x 30001 fp32 2.1 in registers of 1024 threads, 3.9 with the loop kernel)
+    // (us, 256 / 1024 threads / the loop kernel: stored by columns 4096 x 4099 fp32 227 / 233 / 327, fp16 163 / 161 / 221; 4096 x 8192
+    // fp16 305 / 354 / 638; every second column 4096 x 8192 fp32 159 / 153 / 154, but fp16 113 / 65 / 76; 1024 threads / the loop
+    // kernel: every second column 4096 x 12289 fp32 232 / 239, by columns 2048 x 16384 fp32 432 / 620, fp16 393 / 501)
     if (len <= 256 * 32) return (int)launch_elem<T, 256, 64>(p, stream);
     if (len <= 1024 * 16) return (int)launch_elem<T, 1024, 16>(p, stream);
     note_launch(kLaunchSoftmax, kLoopThreads, "softmax_loop_kernel, two sweeps over a long row segment");

@@ -857,7 +857,8 @@ def test_tile_mode_program_layout():
 def test_whole_tile_reductions_on_the_gpu(dtype, tolerance, interpret, monkeypatch):
     monkeypatch.setenv("NT_MAP_INTERPRET", interpret)
     # (rows of up to 512 elements take a wave each, four to a workgroup; rows of 2049 ... 8192 elements run
-    # 512 threads per row, up to 16384 1024 threads, longer ones 256 again)
+    # 512 threads per row, up to 16384 1024 threads, longer ones 256 again -- but for one reduction over rows of 16-bit
+    # values, a multiple of 8 of them: a wave up to 1024, 256 threads up to 4096)
     for rows, cols in ((7, 300), (64, 4096), (3, 1), (1001, 32), (77, 512), (6, 513), (5, 2049), (33, 8192), (9, 8200), (17, 16384), (3, 20000)):
         for kernel, inputs, expected in _normalisation_cases("cuda", dtype, rows, cols):
             out = torch.full_like(inputs[0], float("nan"))
@@ -1114,11 +1115,11 @@ def test_grouped_elements_of_16_bit_tensors(dtype):
 
 
 @gpu
-@pytest.mark.parametrize("rows, cols", ((1, 512), (9, 520), (8193, 1016), (5, 1024), (7, 1032), (3, 2048), (8200, 2056), (4, 4088), (6, 4096), (2, 4104)))
+@pytest.mark.parametrize("rows, cols", ((1, 512), (1, 520), (9, 520), (8193, 1016), (32777, 520), (5, 1024), (7, 1032), (24600, 1032), (3, 2048), (8200, 2056), (4, 4088), (6, 4096), (2, 4104)))
 def test_rows_of_one_reduction_in_groups_of_eight_per_wave_and_per_workgroup(rows, cols):
     """One reduction over rows of 16-bit values: rows of up to 1024 values take a wave each, up to 4096 a workgroup of 256
-    threads, longer ones more; more rows than workgroups are walked by a loop whose exchange between waves uses two
-    buffers in turn.  (The application rounds to the tensors' type after every operation: about six roundings of 2^-11.)"""
+    threads, longer ones more.  At most 8192 workgroups walk all rows: 24600 rows of a workgroup each use both buffers of the
+    exchange between waves and then the first again, 32777 rows of a wave each walk their loop twice.  (The application rounds to the tensors' type after every operation: about six roundings of 2^-11.)"""
     _, (kernel, inputs, expected), _ = _normalisation_cases("cuda", torch.float16, rows, cols)
     storage = torch.full((rows, cols + 3), 7.0, dtype=torch.float16, device="cuda")
     out = storage[:, 2 : 2 + cols]
@@ -1126,6 +1127,19 @@ def test_rows_of_one_reduction_in_groups_of_eight_per_wave_and_per_workgroup(row
     _served_by_map(kernel)
     assert torch.allclose(out.float(), expected, rtol=6 * 2.0**-11, atol=2.0**-20)
     assert bool((storage[:, :2] == 7).all()) and bool((storage[:, 2 + cols :] == 7).all())
+
+
+@gpu
+@pytest.mark.parametrize("rows, cols", ((8200, 600), (16400, 2052)))
+def test_rows_of_two_reductions_take_both_exchange_buffers_and_the_first_again(rows, cols):
+    """A workgroup uses a buffer for each of a row's two reductions, and the same two again for its next row.  (Sums of up to
+    2052 floats in 256 or 512 threads: 2^-23 for each of a dozen roundings on a path, values below 16 in magnitude.)"""
+    softmax, _, layer_norm = _normalisation_cases("cuda", torch.float32, rows, cols)
+    for (kernel, inputs, expected), atol in ((softmax, 1e-9), (layer_norm, 1e-5)):
+        out = torch.full((rows, cols), float("nan"), device="cuda")
+        kernel(*inputs, out)
+        _served_by_map(kernel)
+        assert torch.allclose(out, expected, rtol=1e-5, atol=atol), kernel.kernel_name
 
 
 @gpu
