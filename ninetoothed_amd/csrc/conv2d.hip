@@ -53,6 +53,8 @@ struct ConvParams {
     int M, tiles_m, tiles_n;  // M = N*P*Q rows
     unsigned xt_bytes, wt_bytes;
     int stride_h, stride_w, dil_h, dil_w;  // steps of the window over the input and between its taps
+    int parts, kt_per_part;  // the contraction dealt to parts: this many, k steps of 32 each (1: not dealt)
+    float *scratch;          // ... and their accumulators
 };
 
 // ---- pre-pass: one launch, two jobs ----
@@ -203,55 +205,53 @@ __global__ __launch_bounds__(256) void conv2d_repack_kernel(const T *x, T *xt, i
 }
 
 // ---- main kernel ----
-template <typename T, int BM, int BN, int WM, int WN, int kStages, int kOcc>
+constexpr unsigned kConvBehind = 0x80000000u;  // an offset behind every descriptor: reads zeros
+
+// One LDS object per stage and operand (kKernel keeps those of different kernels apart): distinct objects let the compiler
+// prove that the asynchronous fill of one stage does not alias reads of another.
+template <typename kKernel, int kIndex, int kBytes>
+NT_DEVICE NT_LDS unsigned char *stage_memory() {
+    __shared__ __attribute__((aligned(1024))) unsigned char bytes[kBytes];
+    return (NT_LDS unsigned char *)bytes;
+}
+
+// What bounds it: a CU fetches about 20 bytes a clock into its LDS (45 to 60 GB/s), a quarter of what the MFMAs of a 128 x 64 tile
+// could take; deeper rings (up to 11 steps of 32 channels of a tap in flight) change nothing, tiles that share more do.  So there
+// is a tile of 128 x 128 with eight waves (128 x 64 with four took its place: 32 images of 64 x 56 x 56, 128 filters of 3 x 3, step
+// 2, with the repacking 24.7 -> 20.5 us; 22 of 360 x 28 x 28, 224 of 3 x 3, 69 -> 64), fragments of the next step are read
+// under the MFMAs of this one, and a launch that leaves CUs idle deals the contraction to parts (kParts): part s
+// adds up k steps [s * kt_per_part, ...) and writes its accumulators as they lie in the registers; conv2d_sum_parts_kernel adds the parts.
+template <typename T, int BM, int BN, int WM, int WN, int kStages, int kOcc, bool kParts>
 __global__ __launch_bounds__(WM *WN * 64, kOcc) void conv2d_nhwc_kernel(ConvParams p) {
 #if defined(__HIP_DEVICE_COMPILE__)
     typedef Elem<T> E;
     typedef typename E::vec8 vec8;
+    struct Self;  // (names this instance's LDS)
     constexpr int BK = 32;
     constexpr int kWaves = WM * WN;
     constexpr int kWaveM = BM / WM, kWaveN = BN / WN;
-    constexpr int TM = kWaveM / 32, TN = kWaveN / 32;
+    constexpr int TM = kWaveM / 16, TN = kWaveN / 16;  // 16x16x32 MFMAs of a wave
     constexpr int kStageA = BM * BK * 2, kStageB = BK * BN * 2;
     constexpr int kAChunksPerRow = BK / 8, kARowsPerInstr = 64 / kAChunksPerRow;
     constexpr int kAInstr = kStageA / (kWaves * 1024);
     constexpr int kBChunksPerRow = BN / 8, kBRowsPerInstr = 64 / kBChunksPerRow;
     constexpr int kBInstr = kStageB / (kWaves * 1024);
-    constexpr int kLoadsPerTile = kAInstr + kBInstr;
+    constexpr int kLoadsPerStage = kAInstr + kBInstr;
     static_assert(kStageA % (kWaves * 1024) == 0 && kStageB % (kWaves * 1024) == 0, "every wave issues whole load instructions");
-    static_assert(kWaveM % 32 == 0 && kWaveN % 32 == 0, "wave tile");
-    static_assert(kStages >= 3 && kStages <= 4 && kStages >= WN, "stages (the epilogue slabs of all waves live in the A stages)");
-
-    __shared__ __attribute__((aligned(1024))) unsigned char lds_a0[kStageA];
-    __shared__ __attribute__((aligned(1024))) unsigned char lds_a1[kStageA];
-    __shared__ __attribute__((aligned(1024))) unsigned char lds_a2[kStageA];
-    __shared__ __attribute__((aligned(1024))) unsigned char lds_a3[kStages > 3 ? kStageA : 16];
-    __shared__ __attribute__((aligned(1024))) unsigned char lds_b0[kStageB];
-    __shared__ __attribute__((aligned(1024))) unsigned char lds_b1[kStageB];
-    __shared__ __attribute__((aligned(1024))) unsigned char lds_b2[kStageB];
-    __shared__ __attribute__((aligned(1024))) unsigned char lds_b3[kStages > 3 ? kStageB : 16];
-    auto stage_a = [&](auto tag) -> NT_LDS unsigned char * {
-        constexpr int i = decltype(tag)::value;
-        if constexpr (i == 0) return (NT_LDS unsigned char *)lds_a0;
-        else if constexpr (i == 1) return (NT_LDS unsigned char *)lds_a1;
-        else if constexpr (i == 2) return (NT_LDS unsigned char *)lds_a2;
-        else return (NT_LDS unsigned char *)lds_a3;
-    };
-    auto stage_b = [&](auto tag) -> NT_LDS unsigned char * {
-        constexpr int i = decltype(tag)::value;
-        if constexpr (i == 0) return (NT_LDS unsigned char *)lds_b0;
-        else if constexpr (i == 1) return (NT_LDS unsigned char *)lds_b1;
-        else if constexpr (i == 2) return (NT_LDS unsigned char *)lds_b2;
-        else return (NT_LDS unsigned char *)lds_b3;
-    };
+    static_assert(kStages >= 3 && (kStages - 2) * kLoadsPerStage < 64, "stages");
+    auto stage_a = [&](auto tag) { return stage_memory<Self, 2 * decltype(tag)::value, kStageA>(); };
+    auto stage_b = [&](auto tag) { return stage_memory<Self, 2 * decltype(tag)::value + 1, kStageB>(); };
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wave_m = wave / WN, wave_n = wave % WN;
 
+    // parts: the same part of all tiles goes to as few XCDs as possible, whose L2 then hold that part of the filter only
+    const int tiles = p.tiles_m * p.tiles_n;
+    const int part = kParts ? blockIdx.x % p.parts : 0, tile = kParts ? blockIdx.x / p.parts : blockIdx.x;
     int tile_m, tile_n;
-    map_tile(p.tiles_m, p.tiles_n, 0, tile_m, tile_n);
+    map_tile(p.tiles_m, p.tiles_n, kParts ? 0x100 : 0, tile_m, tile_n, tile, tiles);
     const int m0 = tile_m * BM;
     const int n0 = tile_n * BN;
     const int PQ = p.P * p.Q;
@@ -269,7 +269,7 @@ __global__ __launch_bounds__(WM *WN * 64, kOcc) void conv2d_nhwc_kernel(ConvPara
 #pragma unroll
     for (int j = 0; j < kAInstr; ++j) {
         const int row = (j * kWaves + wave) * kARowsPerInstr + lane / kAChunksPerRow;
-        const int chunk = a_phys_chunk<BK>(row, lane % kAChunksPerRow);
+        const int chunk = a_phys_chunk16<BK>(row, lane % kAChunksPerRow);
         const int m = m0 + row;
         const int image = m / PQ, pq = m - image * PQ;
         const int oy = pq / p.Q, ox = pq - oy * p.Q;
@@ -282,158 +282,197 @@ __global__ __launch_bounds__(WM *WN * 64, kOcc) void conv2d_nhwc_kernel(ConvPara
 #pragma unroll
     for (int j = 0; j < kBInstr; ++j) {
         const int krow = (j * kWaves + wave) * kBRowsPerInstr + lane / kBChunksPerRow;
-        const int chunk = b_phys_chunk<BN>(krow, lane % kBChunksPerRow);
+        const int chunk = b_phys_chunk16<BN>(krow, lane % kBChunksPerRow);
         b_src[j] = (unsigned)(krow * p.Kp + chunk * 8) * 2u;
     }
-    auto issue_loads = [&](auto stage_tag, int kt) {
-        NT_LDS unsigned char *sa = stage_a(stage_tag);
-        NT_LDS unsigned char *sb = stage_b(stage_tag);
-        // k order: channel block outer, filter taps inner -- the R*S taps of a block of 32 channels read the
-        // same pixels shifted by a row or a column, so they hit in L2 while the lines are still there
-        const int taps = p.R * p.S;
+
+    // k order: channel block outer, filter taps inner -- the R*S taps of a block of 32 channels read the
+    // same pixels shifted by a row or a column, so they hit in L2 while the lines are still there
+    const int taps = p.R * p.S;
+    const int all_k = (taps * p.C + BK - 1) / BK;
+    const int k_first = kParts ? part * p.kt_per_part : 0;
+    const int num_k = kParts ? min(p.kt_per_part, all_k - k_first) : all_k;
+    // the k step that is requested next (steps are requested in order): its channel block, tap row and tap column
+    int next_k = 0, next_c = narrow ? 0 : k_first / taps;
+    int next_r = narrow ? 0 : (k_first - next_c * taps) / p.S, next_s = narrow ? 0 : (k_first - next_c * taps) - next_r * p.S;
+    unsigned a_src[kAInstr];
+    int b_k;
+    bool wanted;
+    const auto locate = [&]() {  // where the next k step lies
+        wanted = next_k < num_k;  // past the end zeros are fetched from nowhere, which keeps the count of loads in flight
         if (narrow) {  // (uniform) rows of the repacked filter are (tap, channel) pairs in this order: k step kt is rows 32 kt ...
+            const int kt = k_first + next_k;
             const int taps_per_step = BK / p.C;
 #pragma unroll
             for (int j = 0; j < kAInstr; ++j) {
                 const int tap = kt * taps_per_step + a_tap[j];
                 const int fy = (tap / p.S) * p.dil_h, fx = (tap % p.S) * p.dil_w;
-                const bool inside = tap < taps && (unsigned)(a_y[j] + fy) < (unsigned)p.H && (unsigned)(a_x[j] + fx) < (unsigned)p.W;
-                const unsigned offset = inside ? (unsigned)(a_base[j] + (fy * p.W + fx) * p.C * 2) : 0x80000000u;
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(a_rsrc, sa + (j * kWaves + wave) * 1024, 16, offset, 0, 0, 0);
+                const bool inside = wanted && tap < taps && (unsigned)(a_y[j] + fy) < (unsigned)p.H && (unsigned)(a_x[j] + fx) < (unsigned)p.W;
+                a_src[j] = inside ? (unsigned)(a_base[j] + (fy * p.W + fx) * p.C * 2) : kConvBehind;
             }
-            const int b_k = kt * BK * p.Kp * 2;  // (rows past the last tap lie behind the descriptor: zeros)
+            b_k = wanted ? kt * BK * p.Kp * 2 : 0;  // (rows past the last tap lie behind the descriptor: zeros)
+        } else {
+            const int fy = next_r * p.dil_h, fx = next_s * p.dil_w;  // the tap's distance from the window's corner
+            const int delta = ((fy * p.W + fx) * p.C + next_c * BK) * 2;
+            const unsigned rows = wanted ? (unsigned)p.H : 0u;
 #pragma unroll
-            for (int j = 0; j < kBInstr; ++j)
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(b_rsrc, sb + (j * kWaves + wave) * 1024, 16, b_src[j], b_k, 0, 0);
-            return;
+            for (int j = 0; j < kAInstr; ++j) {
+                const bool inside = (unsigned)(a_y[j] + fy) < rows && (unsigned)(a_x[j] + fx) < (unsigned)p.W;
+                a_src[j] = inside ? (unsigned)(a_base[j] + delta) : kConvBehind;
+            }
+            b_k = wanted ? ((next_r * p.S + next_s) * p.C + next_c * BK) * p.Kp * 2 : 0;
+            ++next_s;
+            const bool row_done = next_s == p.S;
+            next_s = row_done ? 0 : next_s;
+            next_r += row_done;
+            const bool block_done = next_r == p.R;
+            next_r = block_done ? 0 : next_r;
+            next_c += block_done;
         }
-        const int cb = kt / taps;
-        const int tap = kt - cb * taps;
-        const int c0 = cb * BK;
-        const int fy = (tap / p.S) * p.dil_h, fx = (tap % p.S) * p.dil_w;  // the tap's distance from the window's corner
-        const int delta = ((fy * p.W + fx) * p.C + c0) * 2;
+        ++next_k;
+    };
+    const auto issue_loads = [&](auto stage_tag) {
+        NT_LDS unsigned char *sa = stage_a(stage_tag);
+        NT_LDS unsigned char *sb = stage_b(stage_tag);
 #pragma unroll
-        for (int j = 0; j < kAInstr; ++j) {
-            const bool inside = (unsigned)(a_y[j] + fy) < (unsigned)p.H && (unsigned)(a_x[j] + fx) < (unsigned)p.W;
-            const unsigned offset = inside ? (unsigned)(a_base[j] + delta) : 0x80000000u;  // beyond num_records: reads zeros
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(a_rsrc, sa + (j * kWaves + wave) * 1024, 16, offset, 0, 0, 0);
-        }
-        const int b_k = (tap * p.C + c0) * p.Kp * 2;
+        for (int j = 0; j < kAInstr; ++j) __builtin_amdgcn_raw_ptr_buffer_load_lds(a_rsrc, sa + (j * kWaves + wave) * 1024, 16, a_src[j], 0, 0, 0);
 #pragma unroll
         for (int j = 0; j < kBInstr; ++j)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(b_rsrc, sb + (j * kWaves + wave) * 1024, 16, b_src[j], b_k, 0, 0);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(b_rsrc, sb + (j * kWaves + wave) * 1024, 16, wanted ? b_src[j] : kConvBehind, b_k, 0, 0);
     };
 
     // ---- LDS -> registers (as in gemm_fast.h) ----
-    const int g = lane >> 5, l32 = lane & 31;
-    int a_row_off[TM], a_row_sw[TM];
+    const int i16 = lane & 15, kg = lane >> 4;
+    int a_off, b_lo[TN], b_hi[TN];
+    {
+        const int a_row = wave_m * kWaveM + i16;  // + 16 * ti, which leaves the swizzle term as it is
+        a_off = a_row * (BK * 2) + a_phys_chunk16<BK>(a_row, kg) * 16;
 #pragma unroll
-    for (int ti = 0; ti < TM; ++ti) {
-        const int row = wave_m * kWaveM + ti * 32 + l32;
-        a_row_off[ti] = row * (BK * 2);
-        a_row_sw[ti] = a_phys_chunk<BK>(row, 0);
+        for (int tj = 0; tj < TN; ++tj) {
+            const int k_lo = 8 * kg + (i16 >> 2), k_hi = k_lo + 4;
+            const int ncol = wave_n * kWaveN + tj * 16 + 4 * (i16 & 3);
+            b_lo[tj] = k_lo * (BN * 2) + b_phys_chunk16<BN>(k_lo, ncol >> 3) * 16 + (ncol & 7) * 2;
+            b_hi[tj] = k_hi * (BN * 2) + b_phys_chunk16<BN>(k_hi, ncol >> 3) * 16 + (ncol & 7) * 2;
+        }
     }
-    const int i16 = lane & 15, nhalf = (lane >> 4) & 1;
-    const int b_krow = 8 * g + (i16 >> 2);
-    int b_col_chunk[TN], b_col_in[TN];
-#pragma unroll
-    for (int tj = 0; tj < TN; ++tj) {
-        const int ncol = wave_n * kWaveN + tj * 32 + nhalf * 16 + 4 * (i16 & 3);
-        b_col_chunk[tj] = ncol >> 3;
-        b_col_in[tj] = (ncol & 7) * 2;
-    }
+    auto read_a = [&](auto stage_tag, int ti) -> vec8 { return *(const NT_LDS vec8 *)(stage_a(stage_tag) + a_off + ti * 16 * (BK * 2)); };
+    auto read_b = [&](auto stage_tag, int tj) -> vec8 {
+        const NT_LDS unsigned char *sb = stage_b(stage_tag);
+        short4_t lo = lds_read_tr16_b64(sb + b_lo[tj]);
+        short4_t hi = lds_read_tr16_b64(sb + b_hi[tj]);
+        short8_t both = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+        return __builtin_bit_cast(vec8, both);
+    };
 
-    float16_t acc[TM][TN];
+    float4_t acc[TM][TN];
 #pragma unroll
     for (int ti = 0; ti < TM; ++ti)
 #pragma unroll
-        for (int tj = 0; tj < TN; ++tj)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[ti][tj][r] = 0.0f;
+        for (int tj = 0; tj < TN; ++tj) acc[ti][tj] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
 
-    auto multiply_stage = [&](auto stage_tag) {
-        const NT_LDS unsigned char *sa = stage_a(stage_tag);
-        const NT_LDS unsigned char *sb = stage_b(stage_tag);
-#pragma unroll
-        for (int ks = 0; ks < BK / 16; ++ks) {
-            vec8 af[TM], bf[TN];
-#pragma unroll
-            for (int ti = 0; ti < TM; ++ti) {
-                const int chunk = (ks * 2 + g) ^ a_row_sw[ti];
-                af[ti] = *(const NT_LDS vec8 *)(sa + a_row_off[ti] + chunk * 16);
-            }
-#pragma unroll
-            for (int tj = 0; tj < TN; ++tj) {
-                const int k_lo = ks * 16 + b_krow, k_hi = k_lo + 4;
-                const int c_lo = b_phys_chunk<BN>(k_lo, b_col_chunk[tj]);
-                const int c_hi = b_phys_chunk<BN>(k_hi, b_col_chunk[tj]);
-                short4_t lo = lds_read_tr16_b64(sb + k_lo * (BN * 2) + c_lo * 16 + b_col_in[tj]);
-                short4_t hi = lds_read_tr16_b64(sb + k_hi * (BN * 2) + c_hi * 16 + b_col_in[tj]);
-                short8_t both = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
-                bf[tj] = __builtin_bit_cast(vec8, both);
-            }
-#pragma unroll
-            for (int ti = 0; ti < TM; ++ti)
-#pragma unroll
-                for (int tj = 0; tj < TN; ++tj) acc[ti][tj] = E::mfma32(af[ti], bf[tj], acc[ti][tj]);
-        }
-    };
-
-    const int num_k = (p.R * p.S * p.C + BK - 1) / BK;
-    const int last_k = num_k - 1;
-    const int main_k = num_k - num_k % kStages;
-    static_for<0, kStages - 1>([&](auto s) { issue_loads(s, min((int)decltype(s)::value, last_k)); });
-    auto step = [&](auto s, int kt) {
-        constexpr int kS = decltype(s)::value;
-        wait_vmcnt<(kStages - 2) * kLoadsPerTile>();
-        lds_barrier();
-        issue_loads(std::integral_constant<int, (kS + kStages - 1) % kStages>(), min(kt + kS + kStages - 1, last_k));
-        multiply_stage(s);
-    };
-    for (int kt = 0; kt < main_k; kt += kStages) static_for<0, kStages>([&](auto s) { step(s, kt); });
+    // The barrier that opens step t tells that stage t + 1 is complete in LDS and that every wave is done with stage t - 1,
+    // which is refilled right after it.  During a step all fragments of the next one are read, under its MFMAs: a workgroup
+    // that has a SIMD to itself would wait for the LDS before every MFMA otherwise.  Where the loads of the step after lie is
+    // worked out in the same place.
     static_for<0, kStages - 1>([&](auto s) {
-        if (main_k + (int)decltype(s)::value < num_k) step(s, main_k);
+        locate();
+        issue_loads(s);
+    });
+    locate();
+    vec8 as[2][TM];
+    vec8 bs[2][TN];
+    wait_vmcnt<(kStages - 2) * kLoadsPerStage>();
+    lds_barrier();
+#pragma unroll
+    for (int ti = 0; ti < TM; ++ti) as[0][ti] = read_a(std::integral_constant<int, 0>(), ti);
+#pragma unroll
+    for (int tj = 0; tj < TN; ++tj) bs[0][tj] = read_b(std::integral_constant<int, 0>(), tj);
+    auto step = [&](auto position) {
+        constexpr int kI = decltype(position)::value, kS = kI % kStages;  // in the unrolled body: stage and set of fragments follow
+        typedef std::integral_constant<int, (kS + 1) % kStages> NextStage;
+        constexpr int cur = kI & 1, nxt = cur ^ 1;
+        wait_vmcnt<(kStages - 3) * kLoadsPerStage>();
+        lds_barrier_reads_in_flight();
+        issue_loads(std::integral_constant<int, (kS + kStages - 1) % kStages>());
+        locate();
+#pragma unroll
+        for (int ti = 0; ti < TM; ++ti) as[nxt][ti] = read_a(NextStage(), ti);
+#pragma unroll
+        for (int tj = 0; tj < TN; ++tj) bs[nxt][tj] = read_b(NextStage(), tj);
+#pragma unroll
+        for (int ti = 0; ti < TM; ++ti)
+#pragma unroll
+            for (int tj = 0; tj < TN; ++tj) acc[ti][tj] = E::mfma16(as[cur][ti], bs[cur][tj], acc[ti][tj]);
+        // issue order: the loads and the reads spread under the MFMAs
+        constexpr int kMfmas = TM * TN, kReads = TM + 2 * TN, kPer = (kReads + kMfmas - 1) / kMfmas;
+        static_for<0, kMfmas>([&](auto i_tag) {
+            constexpr int i = decltype(i_tag)::value;
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            if constexpr (i * kPer < kReads) __builtin_amdgcn_sched_group_barrier(0x100, kPer, 0);
+            if constexpr (i < kLoadsPerStage) __builtin_amdgcn_sched_group_barrier(0x020, (kLoadsPerStage + kMfmas - 1) / kMfmas, 0);
+        });
+    };
+    constexpr int kBody = kStages % 2 ? 2 * kStages : kStages;
+    const int main_k = num_k - num_k % kBody;
+    for (int kt = 0; kt < main_k; kt += kBody) static_for<0, kBody>([&](auto s) { step(s); });
+    static_for<0, kBody - 1>([&](auto s) {
+        if (main_k + (int)decltype(s)::value < num_k) step(s);
     });
     wait_vmcnt<0>();
     lds_barrier();
 
-    // ---- epilogue: lane holds, per 32x32 tile, output channel l32 and rows 8*(r/4) + 4*g + r%4 ----
-    // slab layout [32 channels][kWaveM rows], 16-byte chunks swizzled by channel; an A stage holds WM slabs
+    if constexpr (kParts) {  // the accumulators as they lie: 16 bytes per lane, a block of 16 x 16 is 1 KiB
+        float4_t *to = (float4_t *)p.scratch + ((((int64_t)part * tiles + tile) * kWaves + wave) * (TM * TN)) * 64 + lane;
+#pragma unroll
+        for (int ti = 0; ti < TM; ++ti)
+#pragma unroll
+            for (int tj = 0; tj < TN; ++tj) to[(ti * TN + tj) * 64] = acc[ti][tj];
+        return;
+    }
+
+    // ---- epilogue: lane holds, per 16x16 block, output channel i16 and rows 4 * kg + 0 .. 3 ----
+    // slab layout [kSlabChannels][kWaveM rows], 16-byte chunks swizzled by channel, in the A stages
+    constexpr int kSlabBlocks = TN < 2 ? 1 : 2;
+    constexpr int kSlabChannels = 16 * kSlabBlocks;
     constexpr int kRowBytes = kWaveM * 2;
-    constexpr int kSlabBytes = 32 * kRowBytes;
+    constexpr int kSlabBytes = kSlabChannels * kRowBytes;
     constexpr int kChunks = kWaveM / 8;
-    static_assert(kStageA == WM * kSlabBytes, "slabs per A stage");
+    constexpr int kSlabsPerStage = kStageA / kSlabBytes;
+    static_assert(kStageA % kSlabBytes == 0 && kWaves <= (kStages < 4 ? kStages : 4) * kSlabsPerStage && TN % kSlabBlocks == 0 && kWaveM % 32 == 0, "slabs in the first four A stages");
     NT_LDS unsigned char *slab;
     {
-        const int which = wave / WM;
-        slab = which == 0 ? (NT_LDS unsigned char *)lds_a0
-               : which == 1 ? (NT_LDS unsigned char *)lds_a1
-               : which == 2 ? (NT_LDS unsigned char *)lds_a2
-                            : (NT_LDS unsigned char *)lds_a3;
-        slab += (wave % WM) * kSlabBytes;
+        const int which = wave / kSlabsPerStage;
+        slab = which == 0   ? stage_a(std::integral_constant<int, 0>())
+               : which == 1 ? stage_a(std::integral_constant<int, 1>())
+               : which == 2 ? stage_a(std::integral_constant<int, 2>())
+                            : stage_a(std::integral_constant<int, kStages < 4 ? 0 : 3>());
+        slab += (wave % kSlabsPerStage) * kSlabBytes;
     }
     T *Y = (T *)p.y;
     const bool whole_chunks = PQ % 8 == 0 && p.dense_out == 1;
 #pragma unroll
-    for (int tj = 0; tj < TN; ++tj) {
+    for (int tg = 0; tg < TN / kSlabBlocks; ++tg) {
 #pragma unroll
-        for (int ti = 0; ti < TM; ++ti)
+        for (int tb = 0; tb < kSlabBlocks; ++tb)
 #pragma unroll
-            for (int r4 = 0; r4 < 4; ++r4) {
+            for (int ti = 0; ti < TM; ++ti) {
                 typedef T vec4 __attribute__((ext_vector_type(4)));
                 vec4 v;
 #pragma unroll
-                for (int e = 0; e < 4; ++e) v[e] = E::from_float(acc[ti][tj][4 * r4 + e]);
-                const int chunk = (ti * 4 + r4) ^ (l32 & (kChunks - 1));
-                *(NT_LDS vec4 *)(slab + l32 * kRowBytes + chunk * 16 + 8 * g) = v;
+                for (int e = 0; e < 4; ++e) v[e] = E::from_float(acc[ti][tg * kSlabBlocks + tb][e]);
+                const int channel = tb * 16 + i16;
+                const int chunk = (ti * 2 + (kg >> 1)) ^ (channel & (kChunks - 1));
+                *(NT_LDS vec4 *)(slab + channel * kRowBytes + chunk * 16 + 8 * (kg & 1)) = v;
             }
+        const int first_channel = n0 + wave_n * kWaveN + tg * kSlabChannels;
         if (p.dense_out == 2) {
             // channels-last output: a lane gathers 8 channels of one row from the slab and stores them with one
-            // instruction (the 32 channels of the slab are 64 consecutive bytes of the tensor)
+            // instruction (the channels of the slab are 32 or 64 consecutive bytes of the tensor)
+            constexpr int kGroups = kSlabChannels / 8;
 #pragma unroll
-            for (int it = 0; it < (32 * kChunks) / 64; ++it) {
+            for (int it = 0; it < kGroups * kWaveM / 64; ++it) {
                 const int idx = it * 64 + lane;
-                const int row = idx >> 2, first = (idx & 3) * 8;
+                const int row = idx / kGroups, first = (idx % kGroups) * 8;
                 vec8 v;
 #pragma unroll
                 for (int e = 0; e < 8; ++e) {
@@ -441,7 +480,7 @@ __global__ __launch_bounds__(WM *WN * 64, kOcc) void conv2d_nhwc_kernel(ConvPara
                     v[e] = *(const NT_LDS T *)(slab + channel * kRowBytes + (((row >> 3) ^ (channel & (kChunks - 1))) * 16) + (row & 7) * 2);
                 }
                 const int m = m0 + wave_m * kWaveM + row;
-                const int out_channel = n0 + wave_n * kWaveN + tj * 32 + first;
+                const int out_channel = first_channel + first;
                 if (m >= p.M || out_channel >= p.K) continue;
                 const int image = m / PQ, pq = m - image * PQ;
                 const int oy = pq / p.Q, ox = pq - oy * p.Q;
@@ -458,7 +497,7 @@ __global__ __launch_bounds__(WM *WN * 64, kOcc) void conv2d_nhwc_kernel(ConvPara
             continue;
         }
 #pragma unroll
-        for (int it = 0; it < (32 * kChunks) / 64; ++it) {
+        for (int it = 0; it < (kSlabChannels * kChunks) / 64; ++it) {
             const int idx = it * 64 + lane;
             const int channel = idx / kChunks;
             const int phys = idx % kChunks;
@@ -466,7 +505,7 @@ __global__ __launch_bounds__(WM *WN * 64, kOcc) void conv2d_nhwc_kernel(ConvPara
             vec8 v = *(const NT_LDS vec8 *)(slab + channel * kRowBytes + phys * 16);
             const int m = m0 + wave_m * kWaveM + chunk * 8;
             if (m >= p.M) continue;
-            const int out_channel = n0 + wave_n * kWaveN + tj * 32 + channel;
+            const int out_channel = first_channel + channel;
             if (out_channel >= p.K) continue;  // a partial last tile of output channels
             int image = m / PQ, pq = m - image * PQ;
             if (whole_chunks) {  // the 8 rows lie in one image and start at a multiple of 8
@@ -494,6 +533,57 @@ __global__ __launch_bounds__(WM *WN * 64, kOcc) void conv2d_nhwc_kernel(ConvPara
         }
     }
 #endif
+}
+
+// The sum over the parts of the contraction: a workgroup takes one block of 16 positions x 16 channels (1 KiB per part, 16
+// bytes per lane), its waves every fourth part, so that a chain of loads is short (a few parts per wave, all in flight) and
+// the blocks of a small output still give the chip enough waves.
+template <typename T, int BM, int BN, int WM, int WN>
+__global__ __launch_bounds__(256) void conv2d_sum_parts_kernel(ConvParams p) {
+    constexpr int kWaveM = BM / WM, kWaveN = BN / WN, TM = kWaveM / 16, TN = kWaveN / 16, kBlocks = BM * BN / 256;
+    __shared__ float4_t sums[3][64];
+    const int lane = threadIdx.x & 63, group = threadIdx.x >> 6;
+    const int tile = blockIdx.x / kBlocks, block = blockIdx.x % kBlocks;
+    const int64_t part_size = (int64_t)p.tiles_m * p.tiles_n * kBlocks * 64;
+    const float4_t *from = (const float4_t *)p.scratch + (int64_t)blockIdx.x * 64 + lane;
+    float4_t sum = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 8
+    for (int part = group; part < p.parts; part += 4) sum += from[part * part_size];
+    if (group > 0) sums[group - 1][lane] = sum;
+    __syncthreads();
+    if (group > 0) return;
+#pragma unroll
+    for (int g = 0; g < 3; ++g) sum += sums[g][lane];
+    int tile_m, tile_n;
+    map_tile(p.tiles_m, p.tiles_n, 0x100, tile_m, tile_n, tile, p.tiles_m * p.tiles_n);
+    const int wave = block / (TM * TN), ti = block / TN % TM, tj = block % TN;
+    const int m = tile_m * BM + wave / WN * kWaveM + ti * 16 + (lane >> 4) * 4;
+    const int channel = tile_n * BN + wave % WN * kWaveN + tj * 16 + (lane & 15);
+    if (m >= p.M || channel >= p.K) return;
+    typedef T vec4 __attribute__((ext_vector_type(4)));
+    vec4 v;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = Elem<T>::from_float(sum[e]);
+    const int PQ = p.P * p.Q;
+    int image = m / PQ, pq = m - image * PQ;
+    T *Y = (T *)p.y;
+    if (p.dense_out == 1 && pq + 4 <= PQ && m + 4 <= p.M) {
+        typedef vec4 unaligned_vec4 __attribute__((aligned(2)));
+        *(unaligned_vec4 *)(Y + ((int64_t)image * p.K + channel) * PQ + pq) = v;
+        return;
+    }
+    int oy = pq / p.Q, ox = pq - oy * p.Q;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        if (m + e < p.M) Y[(int64_t)image * p.ys[0] + (int64_t)channel * p.ys[1] + (int64_t)oy * p.ys[2] + (int64_t)ox * p.ys[3]] = v[e];
+        if (++ox == p.Q) {
+            ox = 0;
+            if (++oy == p.P) {
+                oy = 0;
+                ++image;
+            }
+        }
+    }
 }
 
 // ---- one launch, no scratch: the convolution on the tensors as they lie ----
@@ -1083,6 +1173,50 @@ int run_direct(const Conv2dRequest &q, hipStream_t stream) {
     return (int)hipGetLastError();
 }
 
+// The tiles of the main kernel and what a k step of 32 costs them, in microseconds: `alone` with one workgroup on a CU, where
+// the steps of a workgroup follow one another, `shared` per workgroup with several, where the CU's loads are the bound (about 20
+// bytes a clock whatever the tile).  Fitted to the times of 55 convolutions (1 to 32 images of 7 x 7 to 112 x 112, 64 to 512 channels
+// and filters, windows 1, 3 and 5, steps 1 and 2) on every tile and number of parts: the choice below is 1 % slower than the best of them on average,
+// 8 % at worst.
+struct ConvTile {
+    int m, n;
+    float alone, shared;
+};
+constexpr ConvTile kConvTiles[] = {{128, 128, 0.32f, 0.24f}, {128, 64, 0.33f, 0.16f}, {64, 128, 0.19f, 0.145f}, {64, 64, 0.185f, 0.13f}, {256, 64, 0.51f, 0.31f}};
+constexpr int kConvMaxParts = 32;
+
+struct ConvChoice {
+    int tile, parts;
+};
+
+// The tile and the number of parts of the contraction with the least expected time.  Parts pay where few workgroups would
+// follow a long chain of k steps (before they were there: 3 images of 384 x 56 x 56, 64 filters of 5 x 5, step 2: 104 us, now 25; 1 x 320 x 7 x 7, 192 of
+// 5 x 5, step 2: 90 -> 15; 3 x 448 x 56 x 56, 64 of 3 x 3: 51 -> 28); the second launch and the accumulators in memory cost about 5 us and 6 TB/s.
+ConvChoice conv2d_choose(int64_t rows, int64_t filters, int steps, int max_parts) {
+    const int64_t units = std::max(1, compute_units());
+    ConvChoice best = {0, 1};
+    float best_time = 0.0f;
+    bool found = false;
+    for (int t = 0; t < (int)(sizeof(kConvTiles) / sizeof(kConvTiles[0])); ++t) {
+        const ConvTile &tile = kConvTiles[t];
+        const int64_t tiles = (rows + tile.m - 1) / tile.m * ((filters + tile.n - 1) / tile.n);
+        for (int wanted : {1, 2, 3, 4, 6, 8, 12, 16, 24, kConvMaxParts}) {
+            if (wanted > max_parts || wanted > steps) break;
+            const int per_part = ceil_div(steps, wanted), parts = ceil_div(steps, per_part);
+            const int64_t scratch = parts > 1 ? parts * tiles * tile.m * tile.n * 4 : 0;
+            if (scratch > (int64_t)64 << 20) break;
+            const float rounds = (float)((tiles * parts + units - 1) / units);  // workgroups per CU
+            const float time = (float)per_part * std::max(tile.alone, rounds * tile.shared) + 0.9f * rounds + (parts > 1 ? 5.0f + (float)scratch / 6.4e6f : 0.0f);
+            if (!found || time < best_time) {
+                found = true;
+                best = {t, parts};
+                best_time = time;
+            }
+        }
+    }
+    return best;
+}
+
 // channels of the repacked operands: the k step of 32 holds whole blocks of channels -- or, for up to 16 channels
 // (the first layer of an image network), 4 or 2 filter taps of 8 or 16 channels each; the extra channels are zeros
 inline int conv2d_padded_channels(int channels) { return channels <= 16 ? ceil_div(channels, 8) * 8 : ceil_div(channels, 32) * 32; }
@@ -1130,21 +1264,38 @@ int run_fast(const Conv2dRequest &q, hipStream_t stream) {
     p.M = q.N * q.P * q.Q;
     p.xt_bytes = (unsigned)xt_bytes;
     p.wt_bytes = (unsigned)wt_bytes;
-    // tile by the number of output channels: 256 wide when they fill it and there are enough tiles for the
-    // chip, else 128 (two workgroups per CU), else 128 x 64 tiles of four waves
-    const auto launch = [&](auto kernel, int bm, int bn, int threads) {
-        p.tiles_m = ceil_div(p.M, bm);
-        p.tiles_n = ceil_div(q.K, bn);
-        kernel<<<dim3(p.tiles_m * p.tiles_n), dim3(threads), 0, stream>>>(p);
+    const int steps = ceil_div(Cp * q.R * q.S, 32);
+    ConvChoice choice = conv2d_choose(p.M, q.K, steps, kConvMaxParts);
+    p.scratch = nullptr;
+    if (choice.parts > 1) {
+        const ConvTile &tile = kConvTiles[choice.tile];
+        const int64_t tiles = (int64_t)ceil_div(p.M, tile.m) * ceil_div(q.K, tile.n);
+        p.scratch = (float *)lease.get(kWorkspaceConvParts, (size_t)choice.parts * tiles * tile.m * tile.n * sizeof(float));
+        if (p.scratch == nullptr) choice = conv2d_choose(p.M, q.K, steps, 1);  // no scratch (graph capture, out of memory): in one piece
+    }
+    p.kt_per_part = ceil_div(steps, choice.parts);
+    p.parts = ceil_div(steps, p.kt_per_part);  // every part has at least one k step
+    p.tiles_m = ceil_div(p.M, kConvTiles[choice.tile].m);
+    p.tiles_n = ceil_div(q.K, kConvTiles[choice.tile].n);
+    const unsigned tiles = (unsigned)(p.tiles_m * p.tiles_n);
+    const auto launch = [&](auto kernel, auto in_parts, auto sum, int bm, int bn, int threads) {
+        if (p.parts == 1) {
+            kernel<<<dim3(tiles), dim3(threads), 0, stream>>>(p);
+            return;
+        }
+        in_parts<<<dim3(tiles * p.parts), dim3(threads), 0, stream>>>(p);
+        sum<<<dim3(tiles * (bm * bn / 256)), dim3(256), 0, stream>>>(p);
     };
-    // the widest tile that is at least 4/5 full of output channels and leaves enough tiles for the chip
-    const auto fits = [&](int bm, int bn) {
-        const int64_t tiles = (int64_t)ceil_div(p.M, bm) * ceil_div(q.K, bn);
-        return q.K * 5 >= ceil_div(q.K, bn) * bn * 4 && tiles >= 192;
-    };
-    if (fits(256, 256)) launch(conv2d_nhwc_kernel<T, 256, 256, 2, 4, 4, 2>, 256, 256, 512);
-    else if (fits(256, 128)) launch(conv2d_nhwc_kernel<T, 256, 128, 4, 2, 3, 4>, 256, 128, 512);
-    else launch(conv2d_nhwc_kernel<T, 128, 64, 2, 2, 4, 3>, 128, 64, 256);
+#define NT_CONV_LAUNCH(BM, BN, WM, WN, ST, OCC) \
+    launch(conv2d_nhwc_kernel<T, BM, BN, WM, WN, ST, OCC, false>, conv2d_nhwc_kernel<T, BM, BN, WM, WN, ST, OCC, true>, conv2d_sum_parts_kernel<T, BM, BN, WM, WN>, BM, BN, WM * WN * 64)
+    switch (choice.tile) {
+    case 0: NT_CONV_LAUNCH(128, 128, 2, 4, 4, 4); break;
+    case 1: NT_CONV_LAUNCH(128, 64, 2, 2, 4, 3); break;
+    case 2: NT_CONV_LAUNCH(64, 128, 2, 2, 4, 3); break;
+    case 3: NT_CONV_LAUNCH(64, 64, 2, 2, 6, 3); break;
+    default: NT_CONV_LAUNCH(256, 64, 4, 1, 4, 2); break;
+    }
+#undef NT_CONV_LAUNCH
     return (int)hipGetLastError();
 }
 

@@ -19,7 +19,8 @@ namespace nt {
 enum WorkspacePurpose {
     kWorkspaceConvInput, kWorkspaceConvFilter, kWorkspaceAttentionNarrow, kWorkspaceGemmParts, kWorkspaceAttentionParts,
     kWorkspaceGemmLhsWidened, kWorkspaceGemmRhsWidened, kWorkspaceGemmBiasWidened, kWorkspaceGemmLhsDense, kWorkspaceGemmRhsDense,
-    kWorkspaceAttentionPaddedQ, kWorkspaceAttentionPaddedK, kWorkspaceAttentionPaddedV, kWorkspaceAttentionPaddedO, kWorkspaceSoftmaxParts, kWorkspacePurposes
+    kWorkspaceAttentionPaddedQ, kWorkspaceAttentionPaddedK, kWorkspaceAttentionPaddedV, kWorkspaceAttentionPaddedO, kWorkspaceSoftmaxParts, kWorkspaceConvParts,
+    kWorkspacePurposes
 };
 
 // Holds the registry lock from construction to destruction: create it, take the buffers,
