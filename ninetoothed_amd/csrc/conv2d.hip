@@ -215,13 +215,14 @@ NT_DEVICE NT_LDS unsigned char *stage_memory() {
     return (NT_LDS unsigned char *)bytes;
 }
 
-// What bounds it: a CU fetches about 20 bytes a clock into its LDS (45 to 60 GB/s), a quarter of what the MFMAs of a 128 x 64 tile
-// could take; deeper rings (up to 11 steps of 32 channels of a tap in flight) change nothing, tiles that share more do.  So there
-// is a tile of 128 x 128 with eight waves (128 x 64 with four took its place: 32 images of 64 x 56 x 56, 128 filters of 3 x 3, step
-// 2, with the repacking 24.7 -> 20.5 us; 22 of 360 x 28 x 28, 224 of 3 x 3, 69 -> 64), fragments of the next step are read
-// under the MFMAs of this one, and a launch that leaves CUs idle deals the contraction to parts (kParts): part s
-// adds up k steps [s * kt_per_part, ...) and writes its accumulators as they lie in the registers; conv2d_sum_parts_kernel adds the parts.
-template <typename T, int BM, int BN, int WM, int WN, int kStages, int kOcc, bool kParts>
+// What bounds it: the instructions of a step that are no MFMAs -- where the taps lie, the loads, the reads of fragments -- and with
+// them the number of steps that follow one another.  So the address arithmetic has no branches (kNarrow is an instance of its own)
+// and is dealt out between the MFMAs, fragments of the next step are read under those of this one, and a launch that leaves CUs
+// idle deals the contraction to parts (kParts): part s adds up k steps [s * kt_per_part, ...) and writes its accumulators as
+// they lie in the registers; conv2d_sum_parts_kernel adds the parts.  With branches a step of 128 x 64 took 0.28 us, 0.34 on
+// 32x32x16 MFMAs, however deep the ring (4 to 12 stages); now 0.19: 22 images of 384 x 88 x 88, 256 filters of 3 x 3, 394 -> 350 us, 28
+// of 64 x 56 x 56, 384 of 5 x 5, 141 -> 126.
+template <typename T, int BM, int BN, int WM, int WN, int kStages, int kOcc, bool kParts, bool kNarrow>
 __global__ __launch_bounds__(WM *WN * 64, kOcc) void conv2d_nhwc_kernel(ConvParams p) {
 #if defined(__HIP_DEVICE_COMPILE__)
     typedef Elem<T> E;
@@ -261,10 +262,9 @@ __global__ __launch_bounds__(WM *WN * 64, kOcc) void conv2d_nhwc_kernel(ConvPara
     // the filter descriptor ends with the matrix: a partial last tile of output channels reads the next
     // row's values (they only feed channels that are not stored) and, in the last row, zeros
     __amdgpu_buffer_rsrc_t b_rsrc = __builtin_amdgcn_make_buffer_rsrc((void *)((const T *)p.wt + n0), 0, p.wt_bytes - (unsigned)n0 * 2u, 0x00020000);
-    // Few input channels (p.C = 8 or 16 after padding): a k step of 32 contraction positions then holds 4 or 2
+    // kNarrow, few input channels (p.C = 8 or 16 after padding): a k step of 32 contraction positions then holds 4 or 2
     // filter taps, and which tap a lane fetches follows from its chunk of the step.
-    const bool narrow = p.C < BK;
-    const int chunks_per_tap = narrow ? p.C / 8 : kAChunksPerRow;
+    const int chunks_per_tap = kNarrow ? p.C / 8 : kAChunksPerRow;
     int a_base[kAInstr], a_y[kAInstr], a_x[kAInstr], a_tap[kAInstr];
 #pragma unroll
     for (int j = 0; j < kAInstr; ++j) {
@@ -275,7 +275,7 @@ __global__ __launch_bounds__(WM *WN * 64, kOcc) void conv2d_nhwc_kernel(ConvPara
         const int oy = pq / p.Q, ox = pq - oy * p.Q;
         a_y[j] = m < p.M ? oy * p.stride_h - p.pad_h : -(1 << 20);  // rows past the last image never pass the bounds test
         a_x[j] = ox * p.stride_w - p.pad_w;
-        a_tap[j] = chunk / chunks_per_tap;  // (narrow) the lane's tap within a k step
+        a_tap[j] = chunk / chunks_per_tap;  // (kNarrow) the lane's tap within a k step
         a_base[j] = m < p.M ? (((image * p.H + a_y[j]) * p.W + a_x[j]) * p.C + (chunk % chunks_per_tap) * 8) * 2 : 0;
     }
     unsigned b_src[kBInstr];
@@ -293,34 +293,38 @@ __global__ __launch_bounds__(WM *WN * 64, kOcc) void conv2d_nhwc_kernel(ConvPara
     const int k_first = kParts ? part * p.kt_per_part : 0;
     const int num_k = kParts ? min(p.kt_per_part, all_k - k_first) : all_k;
     // the k step that is requested next (steps are requested in order): its channel block, tap row and tap column
-    int next_k = 0, next_c = narrow ? 0 : k_first / taps;
-    int next_r = narrow ? 0 : (k_first - next_c * taps) / p.S, next_s = narrow ? 0 : (k_first - next_c * taps) - next_r * p.S;
+    int next_k = 0, next_c = kNarrow ? 0 : k_first / taps;
+    int next_r = kNarrow ? 0 : (k_first - next_c * taps) / p.S, next_s = kNarrow ? 0 : (k_first - next_c * taps) - next_r * p.S;
     unsigned a_src[kAInstr];
     int b_k;
-    bool wanted;
-    const auto locate = [&]() {  // where the next k step lies
-        wanted = next_k < num_k;  // past the end zeros are fetched from nowhere, which keeps the count of loads in flight
-        if (narrow) {  // (uniform) rows of the repacked filter are (tap, channel) pairs in this order: k step kt is rows 32 kt ...
+    unsigned b_behind;
+    // where the next k step lies: straight-line code, and scalars but for the lanes' own bounds tests, so that it fills the gaps between
+    // MFMAs (with a branch in it a step took 0.28 us whatever its tile)
+    const auto locate = [&]() {
+        // past the end zeros are fetched from behind the tensors, which keeps the count of loads in flight
+        const int wanted = next_k < num_k ? -1 : 0;
+        b_behind = ~wanted & kConvBehind;
+        if constexpr (kNarrow) {  // rows of the repacked filter are (tap, channel) pairs in this order: k step kt is rows 32 kt ...
             const int kt = k_first + next_k;
             const int taps_per_step = BK / p.C;
 #pragma unroll
             for (int j = 0; j < kAInstr; ++j) {
                 const int tap = kt * taps_per_step + a_tap[j];
                 const int fy = (tap / p.S) * p.dil_h, fx = (tap % p.S) * p.dil_w;
-                const bool inside = wanted && tap < taps && (unsigned)(a_y[j] + fy) < (unsigned)p.H && (unsigned)(a_x[j] + fx) < (unsigned)p.W;
+                const bool inside = wanted != 0 && tap < taps && (unsigned)(a_y[j] + fy) < (unsigned)p.H && (unsigned)(a_x[j] + fx) < (unsigned)p.W;
                 a_src[j] = inside ? (unsigned)(a_base[j] + (fy * p.W + fx) * p.C * 2) : kConvBehind;
             }
-            b_k = wanted ? kt * BK * p.Kp * 2 : 0;  // (rows past the last tap lie behind the descriptor: zeros)
+            b_k = kt * BK * p.Kp * 2 & wanted;  // (rows past the last tap lie behind the descriptor: zeros)
         } else {
             const int fy = next_r * p.dil_h, fx = next_s * p.dil_w;  // the tap's distance from the window's corner
             const int delta = ((fy * p.W + fx) * p.C + next_c * BK) * 2;
-            const unsigned rows = wanted ? (unsigned)p.H : 0u;
+            const unsigned rows = (unsigned)(p.H & wanted);
 #pragma unroll
             for (int j = 0; j < kAInstr; ++j) {
                 const bool inside = (unsigned)(a_y[j] + fy) < rows && (unsigned)(a_x[j] + fx) < (unsigned)p.W;
                 a_src[j] = inside ? (unsigned)(a_base[j] + delta) : kConvBehind;
             }
-            b_k = wanted ? ((next_r * p.S + next_s) * p.C + next_c * BK) * p.Kp * 2 : 0;
+            b_k = ((next_r * p.S + next_s) * p.C + next_c * BK) * p.Kp * 2 & wanted;
             ++next_s;
             const bool row_done = next_s == p.S;
             next_s = row_done ? 0 : next_s;
@@ -338,7 +342,7 @@ __global__ __launch_bounds__(WM *WN * 64, kOcc) void conv2d_nhwc_kernel(ConvPara
         for (int j = 0; j < kAInstr; ++j) __builtin_amdgcn_raw_ptr_buffer_load_lds(a_rsrc, sa + (j * kWaves + wave) * 1024, 16, a_src[j], 0, 0, 0);
 #pragma unroll
         for (int j = 0; j < kBInstr; ++j)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(b_rsrc, sb + (j * kWaves + wave) * 1024, 16, wanted ? b_src[j] : kConvBehind, b_k, 0, 0);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(b_rsrc, sb + (j * kWaves + wave) * 1024, 16, b_src[j] | b_behind, b_k, 0, 0);
     };
 
     // ---- LDS -> registers (as in gemm_fast.h) ----
@@ -396,9 +400,9 @@ __global__ __launch_bounds__(WM *WN * 64, kOcc) void conv2d_nhwc_kernel(ConvPara
         issue_loads(std::integral_constant<int, (kS + kStages - 1) % kStages>());
         locate();
 #pragma unroll
-        for (int ti = 0; ti < TM; ++ti) as[nxt][ti] = read_a(NextStage(), ti);
-#pragma unroll
         for (int tj = 0; tj < TN; ++tj) bs[nxt][tj] = read_b(NextStage(), tj);
+#pragma unroll
+        for (int ti = 0; ti < TM; ++ti) as[nxt][ti] = read_a(NextStage(), ti);
 #pragma unroll
         for (int ti = 0; ti < TM; ++ti)
 #pragma unroll
@@ -410,6 +414,7 @@ __global__ __launch_bounds__(WM *WN * 64, kOcc) void conv2d_nhwc_kernel(ConvPara
             __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
             if constexpr (i * kPer < kReads) __builtin_amdgcn_sched_group_barrier(0x100, kPer, 0);
             if constexpr (i < kLoadsPerStage) __builtin_amdgcn_sched_group_barrier(0x020, (kLoadsPerStage + kMfmas - 1) / kMfmas, 0);
+            __builtin_amdgcn_sched_group_barrier(0x006, 8, 0);
         });
     };
     constexpr int kBody = kStages % 2 ? 2 * kStages : kStages;
@@ -1174,16 +1179,16 @@ int run_direct(const Conv2dRequest &q, hipStream_t stream) {
 }
 
 // The tiles of the main kernel and what a k step of 32 costs them, in microseconds: `alone` with one workgroup on a CU, where
-// the steps of a workgroup follow one another, `shared` per workgroup with several, where the CU's loads are the bound (about 20
-// bytes a clock whatever the tile).  Fitted to the times of 55 convolutions (1 to 32 images of 7 x 7 to 112 x 112, 64 to 512 channels
-// and filters, windows 1, 3 and 5, steps 1 and 2) on every tile and number of parts: the choice below is 1 % slower than the best of them on average,
-// 8 % at worst.
+// the steps of a workgroup follow one another, `shared` per workgroup with several.  Fitted to the times of 75 convolutions (1 to 32
+// images of 7 x 7 to 112 x 112, 64 to 512 channels and filters, windows 1, 3 and 5, steps 1 and 2) on every tile and number of
+// parts: the choice below is 2 % slower than the best of them on average, 9 % at worst.
 struct ConvTile {
     int m, n;
     float alone, shared;
 };
-constexpr ConvTile kConvTiles[] = {{128, 128, 0.32f, 0.24f}, {128, 64, 0.33f, 0.16f}, {64, 128, 0.19f, 0.145f}, {64, 64, 0.185f, 0.13f}, {256, 64, 0.51f, 0.31f}};
+constexpr ConvTile kConvTiles[] = {{128, 128, 0.28f, 0.21f}, {128, 64, 0.19f, 0.19f}, {64, 128, 0.205f, 0.14f}, {64, 64, 0.145f, 0.107f}, {256, 64, 0.39f, 0.235f}};
 constexpr int kConvMaxParts = 32;
+constexpr int kConvNarrowTile = 1;  // of up to 16 channels
 
 struct ConvChoice {
     int tile, parts;
@@ -1191,7 +1196,7 @@ struct ConvChoice {
 
 // The tile and the number of parts of the contraction with the least expected time.  Parts pay where few workgroups would
 // follow a long chain of k steps (before they were there: 3 images of 384 x 56 x 56, 64 filters of 5 x 5, step 2: 104 us, now 25; 1 x 320 x 7 x 7, 192 of
-// 5 x 5, step 2: 90 -> 15; 3 x 448 x 56 x 56, 64 of 3 x 3: 51 -> 28); the second launch and the accumulators in memory cost about 5 us and 6 TB/s.
+// 5 x 5, step 2: 90 -> 15; 3 x 448 x 56 x 56, 64 of 3 x 3: 51 -> 28); the second launch and the accumulators in memory cost about 5 us and 5.9 TB/s.
 ConvChoice conv2d_choose(int64_t rows, int64_t filters, int steps, int max_parts) {
     const int64_t units = std::max(1, compute_units());
     ConvChoice best = {0, 1};
@@ -1206,7 +1211,8 @@ ConvChoice conv2d_choose(int64_t rows, int64_t filters, int steps, int max_parts
             const int64_t scratch = parts > 1 ? parts * tiles * tile.m * tile.n * 4 : 0;
             if (scratch > (int64_t)64 << 20) break;
             const float rounds = (float)((tiles * parts + units - 1) / units);  // workgroups per CU
-            const float time = (float)per_part * std::max(tile.alone, rounds * tile.shared) + 0.9f * rounds + (parts > 1 ? 5.0f + (float)scratch / 6.4e6f : 0.0f);
+            const float time = (float)per_part * std::max(tile.alone, rounds * tile.shared) + 0.48f * rounds * (float)(tile.m * tile.n) / 8192.0f +
+                               (parts > 1 ? 5.0f + (float)scratch / 5.85e6f : 0.0f);
             if (!found || time < best_time) {
                 found = true;
                 best = {t, parts};
@@ -1265,7 +1271,7 @@ int run_fast(const Conv2dRequest &q, hipStream_t stream) {
     p.xt_bytes = (unsigned)xt_bytes;
     p.wt_bytes = (unsigned)wt_bytes;
     const int steps = ceil_div(Cp * q.R * q.S, 32);
-    ConvChoice choice = conv2d_choose(p.M, q.K, steps, kConvMaxParts);
+    ConvChoice choice = Cp < 32 ? ConvChoice{kConvNarrowTile, 1} : conv2d_choose(p.M, q.K, steps, kConvMaxParts);
     p.scratch = nullptr;
     if (choice.parts > 1) {
         const ConvTile &tile = kConvTiles[choice.tile];
@@ -1287,10 +1293,11 @@ int run_fast(const Conv2dRequest &q, hipStream_t stream) {
         sum<<<dim3(tiles * (bm * bn / 256)), dim3(256), 0, stream>>>(p);
     };
 #define NT_CONV_LAUNCH(BM, BN, WM, WN, ST, OCC) \
-    launch(conv2d_nhwc_kernel<T, BM, BN, WM, WN, ST, OCC, false>, conv2d_nhwc_kernel<T, BM, BN, WM, WN, ST, OCC, true>, conv2d_sum_parts_kernel<T, BM, BN, WM, WN>, BM, BN, WM * WN * 64)
-    switch (choice.tile) {
-    case 0: NT_CONV_LAUNCH(128, 128, 2, 4, 4, 4); break;
-    case 1: NT_CONV_LAUNCH(128, 64, 2, 2, 4, 3); break;
+    launch(conv2d_nhwc_kernel<T, BM, BN, WM, WN, ST, OCC, false, false>, conv2d_nhwc_kernel<T, BM, BN, WM, WN, ST, OCC, true, false>, conv2d_sum_parts_kernel<T, BM, BN, WM, WN>, BM, BN, WM * WN * 64)
+    if (Cp < 32) conv2d_nhwc_kernel<T, 128, 64, 2, 2, 6, 2, false, true><<<dim3(tiles), dim3(256), 0, stream>>>(p);
+    else switch (choice.tile) {
+    case 0: NT_CONV_LAUNCH(128, 128, 2, 2, 4, 2); break;
+    case 1: NT_CONV_LAUNCH(128, 64, 2, 2, 6, 2); break;
     case 2: NT_CONV_LAUNCH(64, 128, 2, 2, 4, 3); break;
     case 3: NT_CONV_LAUNCH(64, 64, 2, 2, 6, 3); break;
     default: NT_CONV_LAUNCH(256, 64, 4, 1, 4, 2); break;
