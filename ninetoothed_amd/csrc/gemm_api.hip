@@ -138,19 +138,37 @@ hipError_t fast_launch(const GemmProblem &q, hipStream_t stream) {
 // The k range is cut into parts, each (tile, part) is a workgroup that writes an fp32 tile to scratch
 // memory of the stream, and a second kernel sums the parts and applies the epilogue.
 
-// number of parts for tiles of bm x bn x bk, 1 = do not split
-// (`scratch_limit`: bytes the partial products may take)
+// Number of parts for tiles of bm x bn x bk, 1 = do not split (`scratch_limit`: bytes the partial products may take).
+// Of the numbers whose workgroups are all on the chip at once, the one of least expected time: `alone` is what a k tile takes a
+// workgroup with a CU to itself, `shared` what it takes the CU per workgroup (us), the partial products are written and read at `rate`.
+// Fitted to 59 products of 1 to 3000 rows, 2 to 48 parts: 3 % (64 x 64), 1 % (others) slower than the best number on average; 512
+// workgroups whatever the shape were 11, 9 and 10 % slower (509 x 2752 x 6800 on 128 x 128: six parts, 528 workgroups, 54 us, five 37.5).
 int split_parts(const GemmProblem &q, int bm, int bn, int bk, int *kt_per_part, int64_t scratch_limit = int64_t(64) << 20) {
+    struct Cost {
+        int area, resident;  // workgroups per CU
+        float alone, shared, rate;
+    };
+    constexpr Cost costs[] = {{64 * 64, 2, 0.234f, 0.214f, 0.8e6f}, {128 * 128, 2, 0.7f, 0.35f, 4.0e6f}, {128 * 256, 2, 0.39f, 0.28f, 5.1e6f}, {256 * 256, 1, 0.29f, 0.29f, 5.8e6f}};
     const int64_t tiles = (int64_t)((q.m + bm - 1) / bm) * ((q.n + bn - 1) / bn);
     const int num_kt = (q.k + bk - 1) / bk;
     if (tiles >= 320) return 1;  // (the untuned choice only splits below 192 tiles; between, the tuner decides)
-    // about two workgroups per CU; of 256 x 256 tiles a CU holds one, so there all of them should run at once
-    int64_t parts = bm * bn >= 256 * 256 ? 256 / tiles : (512 + tiles - 1) / tiles;
-    parts = std::min<int64_t>(parts, num_kt / 2);                  // at least two k tiles each
-    parts = std::min<int64_t>(parts, 256);
-    while (parts >= 2 && parts * q.m * ((q.n + 7) / 8 * 8) * 4 > scratch_limit) --parts;  // scratch of at most 64 MiB, or what the caller's fixed array holds
-    if (parts < 2) return 1;
-    const int per_part = (int)((num_kt + parts - 1) / parts);
+    const Cost *cost = costs;
+    while (cost->area != bm * bn) ++cost;
+    const int64_t part_bytes = (int64_t)q.m * ((q.n + 7) / 8 * 8) * 4;
+    int best = 1;
+    float best_time = 0.0f;
+    for (int parts = 2; parts <= std::min(256, num_kt / 2); parts += std::max(1, parts / 8)) {  // at least two k tiles each
+        const int64_t workgroups = tiles * parts;
+        if (parts * part_bytes > scratch_limit || (parts > 2 && workgroups > 256 * cost->resident) || (cost->resident == 1 && workgroups > 256)) break;
+        const int per_part = (num_kt + parts - 1) / parts;
+        const float time = (float)per_part * std::max(cost->alone, (float)((workgroups + 255) / 256) * cost->shared) + (float)(parts * part_bytes) / cost->rate;
+        if (best == 1 || time < best_time) {
+            best = parts;
+            best_time = time;
+        }
+    }
+    if (best == 1) return 1;
+    const int per_part = (num_kt + best - 1) / best;
     if (kt_per_part) *kt_per_part = per_part;
     return (num_kt + per_part - 1) / per_part;                      // every part has at least one k tile
 }
@@ -165,43 +183,57 @@ bool split_accepts(const GemmProblem &q) {
 
 // out[m][n] = epilogue(sum over parts): four consecutive columns per thread.  The parts are [m][pitch] tiles, pitch = N
 // rounded up to 8; kVector: N is a multiple of 4 and the rows of C start on 16-byte (fp32) / 8-byte boundaries -- else
-// the four values are stored one by one, those inside N
-template <typename T, typename TOut, bool kAddmm, bool kVector = true>
+// the four values are stored one by one, those inside N.  Bound by the latency of a chain of loads where C is small and the parts are
+// many: kGroups threads share the parts of a value (every kGroups-th each, met in LDS) and a thread keeps eight loads in flight.
+template <typename T, typename TOut, bool kAddmm, bool kVector, int kGroups>
 __global__ __launch_bounds__(256) void gemm_split_reduce_kernel(const float *parts, int num_parts, int m, int n, TOut *c, int64_t ldc, const T *bias,
                                                                int64_t bias_stride_m, int64_t bias_stride_n, float alpha, float beta) {
     typedef float float4_t __attribute__((ext_vector_type(4)));
     typedef TOut out4_t __attribute__((ext_vector_type(4)));
+    constexpr int kColumns = 256 / kGroups;  // values (of four columns) per workgroup
+    __shared__ float4_t sums[kGroups > 1 ? kGroups - 1 : 1][kColumns];
     const int pitch = (n + 7) / 8 * 8;
-    const int groups = pitch / 4;
-    const int64_t total = (int64_t)m * groups;
-    for (int64_t index = (int64_t)blockIdx.x * 256 + threadIdx.x; index < total; index += (int64_t)gridDim.x * 256) {
-        const int row = (int)(index / groups);
-        const int col = (int)(index - (int64_t)row * groups) * 4;
-        if (col >= n) continue;
+    const int columns = pitch / 4;
+    const int64_t total = (int64_t)m * columns;
+    const int slot = threadIdx.x % kColumns, group = threadIdx.x / kColumns;
+    const int64_t index = (int64_t)blockIdx.x * kColumns + slot;
+    const int row = (int)(index / columns);
+    const int col = (int)(index - (int64_t)row * columns) * 4;
+    const bool inside = index < total && col < n;
+    float4_t sum = {0.0f, 0.0f, 0.0f, 0.0f};
+    if (inside) {
         const float *src = parts + (int64_t)row * pitch + col;
-        float4_t sum = *(const float4_t *)src;
-        for (int part = 1; part < num_parts; ++part) sum += *(const float4_t *)(src + (int64_t)part * m * pitch);
-        out4_t out;
+#pragma unroll 8
+        for (int part = group; part < num_parts; part += kGroups) sum += *(const float4_t *)(src + (int64_t)part * m * pitch);
+    }
+    if constexpr (kGroups > 1) {
+        if (group > 0) sums[group - 1][slot] = sum;
+        __syncthreads();
+        if (group > 0) return;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            if constexpr (kAddmm) {
-                // as in the one-pass kernels: the product is rounded to the element type, then combined in fp32
-                const float product = Elem<T>::to_float(Elem<T>::from_float(sum[e]));
-                const float input = kVector || col + e < n ? Elem<T>::to_float(bias[(int64_t)row * bias_stride_m + (int64_t)(col + e) * bias_stride_n]) : 0.0f;
-                out[e] = Elem<T>::from_float(beta * input + alpha * product);
-            } else if constexpr (std::is_same<TOut, float>::value) {
-                out[e] = sum[e];
-            } else {
-                out[e] = Elem<T>::from_float(sum[e]);
-            }
-        }
-        if constexpr (kVector) {
-            __builtin_nontemporal_store(out, (out4_t *)(c + (int64_t)row * ldc + col));
+        for (int g = 0; g < kGroups - 1; ++g) sum += sums[g][slot];
+    }
+    if (!inside) return;
+    out4_t out;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        if constexpr (kAddmm) {
+            // as in the one-pass kernels: the product is rounded to the element type, then combined in fp32
+            const float product = Elem<T>::to_float(Elem<T>::from_float(sum[e]));
+            const float input = kVector || col + e < n ? Elem<T>::to_float(bias[(int64_t)row * bias_stride_m + (int64_t)(col + e) * bias_stride_n]) : 0.0f;
+            out[e] = Elem<T>::from_float(beta * input + alpha * product);
+        } else if constexpr (std::is_same<TOut, float>::value) {
+            out[e] = sum[e];
         } else {
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-                if (col + e < n) c[(int64_t)row * ldc + col + e] = out[e];
+            out[e] = Elem<T>::from_float(sum[e]);
         }
+    }
+    if constexpr (kVector) {
+        __builtin_nontemporal_store(out, (out4_t *)(c + (int64_t)row * ldc + col));
+    } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            if (col + e < n) c[(int64_t)row * ldc + col + e] = out[e];
     }
 }
 
@@ -235,21 +267,28 @@ hipError_t split_launch_typed(const GemmProblem &q, hipStream_t stream) {
     else gemm_nn_fast_kernel<T, BM, BN, BK, WM, WN, kStages, kOcc, false, 0, 1, 0, true, false, true, true><<<grid, block, 0, stream>>>(p);
     hipError_t err = hipGetLastError();
     if (err != hipSuccess) return err;
-    const int64_t groups = (int64_t)q.m * (pitch / 4);
-    const dim3 reduce_grid((unsigned)std::min<int64_t>((groups + 255) / 256, 256 * 8));
+    const int64_t values = (int64_t)q.m * (pitch / 4);
     const int64_t out_size = q.out_dtype == NINETOOTHED_FLOAT32 ? 4 : 2;
     const bool vector = q.n % 4 == 0 && (q.scm * out_size) % (4 * out_size) == 0 && ((uintptr_t)q.c & (4 * out_size - 1)) == 0;
-    const auto reduce = [&](auto vector_tag) {
+    const auto reduce = [&](auto vector_tag, auto groups_tag) {
         constexpr bool kVector = decltype(vector_tag)::value;
+        constexpr int kGroups = decltype(groups_tag)::value;
+        const dim3 reduce_grid((unsigned)((values + 256 / kGroups - 1) / (256 / kGroups)));
         if (q.addmm())
-            gemm_split_reduce_kernel<T, T, true, kVector><<<reduce_grid, dim3(256), 0, stream>>>(scratch, parts, q.m, q.n, (T *)q.c, q.scm, (const T *)q.bias, q.sim, q.sin, q.alpha, q.beta);
+            gemm_split_reduce_kernel<T, T, true, kVector, kGroups><<<reduce_grid, dim3(256), 0, stream>>>(scratch, parts, q.m, q.n, (T *)q.c, q.scm, (const T *)q.bias, q.sim, q.sin, q.alpha, q.beta);
         else if (q.out_dtype == NINETOOTHED_FLOAT32)
-            gemm_split_reduce_kernel<T, float, false, kVector><<<reduce_grid, dim3(256), 0, stream>>>(scratch, parts, q.m, q.n, (float *)q.c, q.scm, nullptr, 0, 0, 1.0f, 0.0f);
+            gemm_split_reduce_kernel<T, float, false, kVector, kGroups><<<reduce_grid, dim3(256), 0, stream>>>(scratch, parts, q.m, q.n, (float *)q.c, q.scm, nullptr, 0, 0, 1.0f, 0.0f);
         else
-            gemm_split_reduce_kernel<T, T, false, kVector><<<reduce_grid, dim3(256), 0, stream>>>(scratch, parts, q.m, q.n, (T *)q.c, q.scm, nullptr, 0, 0, 1.0f, 0.0f);
+            gemm_split_reduce_kernel<T, T, false, kVector, kGroups><<<reduce_grid, dim3(256), 0, stream>>>(scratch, parts, q.m, q.n, (T *)q.c, q.scm, nullptr, 0, 0, 1.0f, 0.0f);
     };
-    if (vector) reduce(std::true_type());
-    else reduce(std::false_type());
+    const auto reduce_in_groups = [&](auto vector_tag) {
+        // one thread per value where that fills the chip, or the parts are few; else a value's parts over four or sixteen threads
+        if (parts < 8 || values >= 256 * 1024) reduce(vector_tag, std::integral_constant<int, 1>());
+        else if (parts < 32 || values >= 64 * 1024) reduce(vector_tag, std::integral_constant<int, 4>());
+        else reduce(vector_tag, std::integral_constant<int, 16>());
+    };
+    if (vector) reduce_in_groups(std::true_type());
+    else reduce_in_groups(std::false_type());
     return hipGetLastError();
 }
 
@@ -560,8 +599,8 @@ int heuristic_choice(const GemmProblem &q, int bm, int bn, int bk) {
     const bool small_tiles_fill_the_chip = q.batch == 1 && tiles_64 >= 256 && kInstances[kTail64x64x64].accepts(q);
     const auto few_tiles = [&](int instance) {
         const GemmInstance &inst = kInstances[instance];
-        // (with a short K the second kernel costs more than the idle CUs: 512^3 8 us split, 5 in one pass)
-        return q.batch == 1 && !small_tiles_fill_the_chip && q.k >= 2048 && (int64_t)((q.m + inst.bm - 1) / inst.bm) * ((q.n + inst.bn - 1) / inst.bn) < 192 &&
+        // (with a short K the second kernel costs more than the idle CUs: 512^3 8 us split, 5 in one pass; 23 x 384 x 2112 10.8 and 7.7)
+        return q.batch == 1 && !small_tiles_fill_the_chip && q.k >= (q.m <= 64 ? 3072 : 2048) && (int64_t)((q.m + inst.bm - 1) / inst.bm) * ((q.n + inst.bn - 1) / inst.bn) < 192 &&
                inst.accepts(q);
     };
     if (q.m <= 64 && few_tiles(kSplit64x64x64)) return kSplit64x64x64;
@@ -1087,11 +1126,15 @@ NineToothedResult nt_tune_gemm(NineToothedStream stream_, NineToothedTensor inpu
     const int preferred = heuristic_choice(q, 0, 0, 0);
     const float margin = preferred == kSkinny16 || preferred == kSkinny32 ? 0.25f : 0.02f;
     auto instance_of = [&](int i) { return preferred < 0 ? i : (i == 0 ? preferred : (i - 1 < preferred ? i - 1 : i)); };
+    // short products follow one another no faster than the host calls them, from Python about 6.2 us apart with one launch,
+    // 9.2 with the two of a split product (23 x 384 x 2112: 6.0 us split and 7.0 in one pass on the GPU, 10.8 and 7.7 in a program)
+    float least_ms[kNumInstances];
+    for (int i = 0; i < kNumInstances; ++i) least_ms[i] = is_split(instance_of(i)) ? 0.0092f : 0.0062f;
     const int result = tune_time(stream, kNumInstances, iters, [&](int i) -> int {
         const int instance = instance_of(i);
         if (!kInstances[instance].accepts(q)) return NINETOOTHED_NO_KERNEL;
         return (int)kInstances[instance].launch(q, stream);
-    }, &best, &best_time, margin);
+    }, &best, &best_time, margin, least_ms);
     if (best >= 0) best = instance_of(best);
     if (best_config) *best_config = best;
     if (best_ms) *best_ms = best_time;

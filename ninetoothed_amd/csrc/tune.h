@@ -46,12 +46,13 @@ void note_launch(int program, int choice, const char *name);
 // every candidate over a region of about 3 ms (at least one launch, at most 256) -- and a candidate's figure is the
 // minimum of its rounds, so that a slow spell has to hit the same candidate in every round to mislead.
 // Candidates are in order of preference: with a `margin`, a later candidate replaces an earlier one only when it
-// is faster by more than that fraction.  *best = -1 when none ran.
+// is faster by more than that fraction; `least_ms` (per candidate) is what a call costs its program whatever the GPU does.
+// *best = -1 when none ran.
 // Synchronises; returns without timing anything (*best = -1, result 0) when the stream is being captured into a graph.
 constexpr int kTuneMaxCandidates = 64;
 
 template <typename Launch>
-int tune_time(hipStream_t stream, int candidates, int iters, Launch launch, int *best, float *best_ms, float margin = 0.0f) {
+int tune_time(hipStream_t stream, int candidates, int iters, Launch launch, int *best, float *best_ms, float margin = 0.0f, const float *least_ms = nullptr) {
     *best = -1;
     *best_ms = 0.0f;
     hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
@@ -116,6 +117,7 @@ int tune_time(hipStream_t stream, int candidates, int iters, Launch launch, int 
             }
         }
         for (int c = 0; c < alive && result == 0; ++c) {
+            if (least_ms != nullptr && fastest[c] < least_ms[live[c]]) fastest[c] = least_ms[live[c]];
             if (*best < 0 || fastest[c] < *best_ms * (1.0f - margin)) {
                 *best = live[c];
                 *best_ms = fastest[c];
