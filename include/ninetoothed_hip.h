@@ -141,6 +141,24 @@ NineToothedResult launch_nt_addmm(NineToothedStream stream,
                                   int block_size_m, int block_size_n,
                                   int block_size_k);
 
+/* output = max(scale * (lhs @ rhs) + bias[column], lower), the sums, the scaling, the bias and the comparison in fp32, one
+ * rounding on store, NaN passes: the kernel the reference generates (src/ninetoothed/generation.py:46-133) for the
+ * matmul application of tests/test_matmul.py:41-45 with that work on its accumulator.  `bias` is one-dimensional, N
+ * values of `bias_dtype` (the operands' type or FLOAT32); bias.data == NULL: none.  `lower` of -INFINITY: no bound.
+ * dtype FLOAT16 or BFLOAT16, of lhs, rhs and output.  Returns NINETOOTHED_NO_KERNEL, with nothing launched, for operands that
+ * only launch_nt_matmul takes (strides, K no multiple of 8, an output by columns) and where the output shares memory
+ * with an operand: the caller then runs the product and the rest as two launches. */
+NineToothedResult launch_nt_linear(NineToothedStream stream,
+                                   NineToothedTensor lhs,
+                                   NineToothedTensor rhs,
+                                   NineToothedTensor bias,
+                                   int bias_dtype,
+                                   double scale, double lower,
+                                   NineToothedTensor output,
+                                   int dtype,
+                                   int block_size_m, int block_size_n,
+                                   int block_size_k);
+
 /* output[r, :] = softmax(input[r, :]) over the last of two dims, in fp32
  * arithmetic.  Replaces the kernel generated for tests/test_softmax.py:10-27
  * (one program per row, BLOCK_SIZE >= row length).  Up to 128 row segments of

@@ -24,11 +24,14 @@ struct GemmParams {
     const void *a;
     const void *b;
     void *c;
-    const void *bias;  // addmm `input`; nullptr for plain matmul
+    const void *bias;  // addmm `input`, or the bias of a linear epilogue (a value per column); nullptr for plain matmul
     int m, n, k;
     int64_t lda, ldb, ldc;            // row pitches in elements
     int64_t bias_stride_m, bias_stride_n;
     float alpha, beta;
+    int linear;      // skinny kernel: a linear epilogue (the tile kernels have it as a template parameter)
+    int bias_float;  // linear epilogue: the bias holds fp32
+    float lower;     // ... and its results are at least this
     int tiles_m, tiles_n;
     int bias_vector;  // addmm input readable with aligned 16-byte loads along N
     int order;  // tile order: 0 = XCD-aware strips of 8 tile rows; other values are measurement aids
@@ -126,6 +129,28 @@ NT_DEVICE void lds_barrier_reads_in_flight() {
     __builtin_amdgcn_sched_barrier(0);
 }
 
+// What happens to the sums of products.  kAddmm: rounded to the element type, then beta * input + alpha * product in fp32.
+// kLinear: max(sum * alpha + bias[column], lower) in fp32, rounded once on the store -- on the accumulators, before they pass through
+// LDS as 16-bit values: a lane's columns stay the same over all rows, so their bias costs TN16 loads per tile.
+enum Epilogue { kPlain, kAddmm, kLinear };
+
+// one value of a linear epilogue, with the rounding points of a program that multiplies, adds and compares fp32 tiles one
+// after another (no contraction) and lets NaN pass
+NT_DEVICE float linear_value(const GemmParams &p, float sum, float bias) {
+#pragma clang fp contract(off)
+    const float scaled = sum * p.alpha;
+    const float value = p.bias != nullptr ? scaled + bias : scaled;
+    return value <= p.lower ? p.lower : value;
+}
+
+// the bias of a column inside the output (zero without one)
+template <typename T>
+NT_DEVICE float linear_bias(const GemmParams &p, int col) {
+    if (p.bias == nullptr) return 0.0f;
+    const int64_t at = (int64_t)col * p.bias_stride_n;
+    return p.bias_float ? ((const float *)p.bias)[at] : Elem<T>::to_float(((const T *)p.bias)[at]);
+}
+
 #ifndef NT_GEMM_SCHEDULE
 #define NT_GEMM_SCHEDULE 1
 #endif
@@ -138,7 +163,7 @@ NT_DEVICE void lds_barrier_reads_in_flight() {
 
 // kAblate is a measurement aid (bit 0: no global loads inside the K loop,
 // bit 1: operand fragments read from LDS only once); 0 in every shipped instance.
-template <typename T, int BM, int BN, int BK, int WM, int WN, int kStages, int kWavesPerSimd, bool kAddmm, int kAblate = 0, int kLoad = 0, int kAux = 0,
+template <typename T, int BM, int BN, int BK, int WM, int WN, int kStages, int kWavesPerSimd, int kEpilogue, int kAblate = 0, int kLoad = 0, int kAux = 0,
           bool kFloatOut = false, bool kBT = false, bool kTail = false, bool kSplit = false>
 __global__ __launch_bounds__(WM *WN * 64, kWavesPerSimd) void gemm_nn_fast_kernel(GemmParams p) {
 #if defined(__HIP_DEVICE_COMPILE__)  // the body uses device-only builtins; the host pass only needs the stub
@@ -177,7 +202,7 @@ __global__ __launch_bounds__(WM *WN * 64, kWavesPerSimd) void gemm_nn_fast_kerne
     // kSplit: the grid holds tiles x parts workgroups; part s multiplies k tiles [s * kt_per_split, ...) and
     // writes its fp32 accumulators to slice s of a [parts][M][N] scratch tensor (p.c, pitch p.ldc), which a
     // second kernel sums -- for problems with too few output tiles to occupy the chip
-    static_assert(!kSplit || (kFloatOut && kTail && !kAddmm), "split-K parts are fp32 tiles with tails");
+    static_assert(!kSplit || (kFloatOut && kTail && kEpilogue == kPlain), "split-K parts are fp32 tiles with tails");
     static_assert(kStageA % (kWaves * 1024) == 0 && kStageB % (kWaves * 1024) == 0, "tile/wave mismatch");
     static_assert(kBChunksPerRow <= 64, "BN too large for one-instruction rows");
     static_assert(kWaveM % 32 == 0 && kWaveN % 32 == 0 && BK % 16 == 0, "wave tile");
@@ -779,7 +804,8 @@ __global__ __launch_bounds__(WM *WN * 64, kWavesPerSimd) void gemm_nn_fast_kerne
     // whole 128-byte lines.  (All fills have landed and all waves are done with
     // the stages before the slabs overwrite them.)
     // (fp32 output, matmul and split-K parts only, takes the same route with rows twice as long.)
-    static_assert(!(kFloatOut && kAddmm), "the fp32 output path has no addmm epilogue");
+    static_assert(!kFloatOut || kEpilogue == kPlain, "the fp32 output path has no epilogue");
+    static_assert(kEpilogue != kLinear || kM16, "the linear epilogue reads 16x16 blocks of accumulators");
     using TOut = std::conditional_t<kFloatOut, float, T>;
     constexpr int kChunkElems = 16 / (int)sizeof(TOut);
     constexpr int kRowBytes = kWaveN * (int)sizeof(TOut);
@@ -811,6 +837,17 @@ __global__ __launch_bounds__(WM *WN * 64, kWavesPerSimd) void gemm_nn_fast_kerne
     const T *bias = (const T *)p.bias + batch * p.bias_batch;
     typedef TOut vec_out __attribute__((ext_vector_type(kChunkElems)));
     const int slab_sw = (l32 >> kCShift) & (kCChunks - 1);
+    // (a lane's columns are the same in every block of rows: their bias stays in registers)
+    float4_t column_bias[kEpilogue == kLinear ? TN16 : 1];
+    if constexpr (kEpilogue == kLinear) {
+#pragma unroll
+        for (int tj = 0; tj < TN16; ++tj)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int col = n0 + wave_n * kWaveN + tj * 16 + kg * 4 + e;
+                column_bias[tj][e] = !kTail || col < p.n ? linear_bias<T>(p, col) : 0.0f;
+            }
+    }
 #pragma unroll
     for (int ti = 0; ti < TM; ++ti) {
         if constexpr (kM16) {
@@ -830,7 +867,7 @@ __global__ __launch_bounds__(WM *WN * 64, kWavesPerSimd) void gemm_nn_fast_kerne
                         *(NT_LDS vec4 *)(slab + row * kRowBytes + ((tj * 4 + kg) ^ sw) * 16) = v;
                     } else {
 #pragma unroll
-                        for (int e = 0; e < 4; ++e) v[e] = E::from_float(a4[e]);
+                        for (int e = 0; e < 4; ++e) v[e] = E::from_float(kEpilogue == kLinear ? linear_value(p, a4[e], column_bias[kEpilogue == kLinear ? tj : 0][e]) : a4[e]);
                         *(NT_LDS vec4 *)(slab + row * kRowBytes + ((tj * 2 + (kg >> 1)) ^ sw) * 16 + 8 * (kg & 1)) = v;
                     }
                 }
@@ -866,7 +903,7 @@ __global__ __launch_bounds__(WM *WN * 64, kWavesPerSimd) void gemm_nn_fast_kerne
             const int gcol = n0 + wave_n * kWaveN + chunk * kChunkElems;
             if (grow >= p.m) continue;  // a partial last tile of rows
             if (kTail && gcol >= p.n) continue;  // ... of columns (with vector stores N is a multiple of 8: whole chunks)
-            if constexpr (kAddmm) {
+            if constexpr (kEpilogue == kAddmm) {
                 // the matmul result was rounded to the element type; beta, alpha
                 // are fp32 scalars, so the combination happens in fp32
                 const T *src = bias + (int64_t)grow * p.bias_stride_m + (int64_t)gcol * p.bias_stride_n;

@@ -172,6 +172,10 @@ __global__ __launch_bounds__(kWaves * 64) void gemm_skinny_kernel(GemmParams p) 
             out_t v;
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
+                if (p.linear) {
+                    v[e] = E::from_float(linear_value(p, sum[e], col + e < p.n ? linear_bias<T>(p, col + e) : 0.0f));
+                    continue;
+                }
                 v[e] = E::from_float(sum[e]);
                 if (p.bias != nullptr && col + e < p.n) {  // the product is rounded to the element type, then combined in fp32
                     const T input = ((const T *)p.bias)[(int64_t)row * p.bias_stride_m + (int64_t)(col + e) * p.bias_stride_n];

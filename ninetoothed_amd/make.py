@@ -25,6 +25,7 @@ from ninetoothed_amd import recognition, runtime
 from ninetoothed_amd.recognition import UnsupportedProgram
 from ninetoothed_amd.symbol import Symbol
 from ninetoothed_amd.tensor import Tensor
+from ninetoothed_amd.tracing import ScalarParam
 
 CACHE_DIR = pathlib.Path(os.environ.get("NINETOOTHED_AMD_CACHE_DIR") or pathlib.Path.home() / ".ninetoothed_amd")
 
@@ -320,7 +321,9 @@ class Kernel:
             raise UnsupportedProgram(f"The application rounds the product to `{self.details.get('cast')}` but the tensors hold `{tag}`.")
         return self._gemm_plan(info, tag, tag, positions=(0, 1, 2, 3, 4, 5))
 
-    def _gemm_plan(self, info, tag, out_tag, positions):
+    def _gemm_plan(self, info, tag, out_tag, positions, epilogue=None):
+        """``epilogue(call_args, lhs, rhs, output, blocks)`` launches the product instead and returns the library's result; the
+        plan's ``launch`` then says whether the library took the operands."""
         lib = runtime.library()
         itemsize = {"fp8e5m2": 1, "fp32": 4}.get(tag, 2)
         out_itemsize = 4 if out_tag == "fp32" else 2
@@ -381,6 +384,16 @@ class Kernel:
             a_arg.data = call_args[a_pos].data_ptr() + a.base * itemsize
             b_arg.data = call_args[b_pos].data_ptr() + b.base * itemsize
             c_arg.data = call_args[c_pos].data_ptr() + c.base * out_itemsize
+            if epilogue is not None:
+                result = epilogue(call_args, a_arg, b_arg, c_arg, blocks)
+                if result == runtime.NO_KERNEL:
+                    return False
+                if result == 0 and state["tune"]:
+                    null = runtime.ArgumentTensor.null()
+                    maybe_tune(call_args, null, null, null)  # (the product's instance is the one that its epilogue rides on)
+                    result = epilogue(call_args, a_arg, b_arg, c_arg, blocks)
+                runtime.check(result)
+                return True
             if state["tune"]:
                 null = runtime.ArgumentTensor.null()
                 maybe_tune(call_args, null, null, null)
@@ -477,8 +490,9 @@ class Kernel:
         return _Plan("launch_nt_map " + "; ".join(description for _, description, _, _ in launches), launch)
 
     def _prepare_gemm_epilogue(self, args, env):
-        """A matmul accumulator followed by element-wise work (bias, activation, scaling, residual):
-        the product goes to an fp32 scratch tensor laid out like the output (what the reference
+        """A matmul accumulator followed by element-wise work (bias, activation, scaling, residual).  A scale, a bias
+        per column and a lower bound ride on the product (`_linear_launch`); in general, and where that entry point does not
+        take the operands, the product goes to an fp32 scratch tensor laid out like the output (what the reference
         holds in the accumulator tile), then the rest runs as a tile map over it."""
         import ctypes
 
@@ -514,8 +528,11 @@ class Kernel:
         if built is None:
             return _Plan("empty launch", lambda call_args: None)
         program, description, scalar_slots, operand_params = built
+        linear = self._linear_launch(info, args, env, tag)
 
         def launch(call_args):
+            if linear is not None and linear(call_args):
+                return
             extended = with_scratch(call_args)  # from torch's stream-ordered allocator: free again once both launches are queued
             gemm(extended)
             for slot, param in enumerate(operand_params):
@@ -525,7 +542,39 @@ class Kernel:
             runtime.check(lib.launch_nt_map(runtime.current_stream(), ctypes.addressof(program)))
 
         self._map_programs = [program]
-        return _Plan(f"{gemm.description}; launch_nt_map {description}", launch)
+        two_passes = f"{gemm.description}; launch_nt_map {description}"
+        return _Plan(two_passes if linear is None else f"launch_nt_linear, or {two_passes}", launch)
+
+    def _linear_launch(self, info, args, env, tag):
+        """``max(product * scale + bias[None, :], lower)`` in one launch: a function of the call's arguments that says whether
+        the library took them; None for other epilogues, element types and arrangements."""
+        linear, details = self.details["linear"], self.details
+        lhs_pos, rhs_pos, out_pos = details["lhs"], details["rhs"], details["output"]
+        m, n, k = info["m"], info["n"], info["k"]
+        if linear is None or tag not in ("fp16", "bf16") or _dtype_tag(args[out_pos].dtype) != tag or min(m, n, k) == 0:
+            return None
+        a, b, c = info["a"], info["b"], info["c"]
+        bias_pos, bias_tag, bias_arg = linear["bias"], tag, runtime.ArgumentTensor.null()
+        if bias_pos is not None:
+            bias_tag = _dtype_tag(args[bias_pos].dtype)
+            layout = recognition.analyze_column_vector(self.types[bias_pos], env, info["blocks"], n)
+            if bias_tag not in (tag, "fp32") or layout is None:
+                return None
+            bias_base, bias_stride = layout
+            bias_arg = runtime.ArgumentTensor.from_layout(0, (n,), (bias_stride,))
+        lib = runtime.library()
+        dtype, bias_dtype, bias_size = runtime.DATA_TYPE_INDEX[tag], runtime.DATA_TYPE_INDEX[bias_tag], 4 if bias_tag == "fp32" else 2
+        scale = 1.0 if linear["scale"] is None else linear["scale"]
+        scale_pos = scale.param if isinstance(scale, ScalarParam) else None
+        lower = float("-inf") if linear["lower"] is None else float(linear["lower"])
+
+        def epilogue(call_args, lhs, rhs, output, blocks):
+            if bias_pos is not None:
+                bias_arg.data = call_args[bias_pos].data_ptr() + bias_base * bias_size
+            factor = float(scale if scale_pos is None else call_args[scale_pos])
+            return lib.launch_nt_linear(runtime.current_stream(), lhs, rhs, bias_arg, bias_dtype, factor, lower, output, dtype, *blocks)
+
+        return self._gemm_plan(info, tag, tag, positions=(bias_pos, lhs_pos, rhs_pos, None, None, out_pos), epilogue=epilogue).launch
 
     def _prepare_attention(self, args, env):
         scaled = self.details["scale"]

@@ -23,7 +23,7 @@ from ninetoothed_amd.affine import Affine, NotAffine, Ranges
 from ninetoothed_amd.symbol import Symbol, evaluate
 from ninetoothed_amd.symbolic_int import constant_difference, integer, is_symbolic, same_structure
 from ninetoothed_amd.tensor import Tensor
-from ninetoothed_amd.tracing import Carried, Dim, LoopVar, Node, Program, TensorRef, TracingError, trace
+from ninetoothed_amd.tracing import Carried, Dim, LoopVar, Node, Program, ScalarParam, TensorRef, TracingError, trace
 
 
 class UnsupportedProgram(NotImplementedError):
@@ -151,7 +151,58 @@ def match_gemm_with_epilogue(program, types):
         mapping.check_application(candidate)
     except UnsupportedProgram:
         return None
-    return {"lhs": lhs, "rhs": rhs, "output": ref.param, "epilogue": candidate}
+    return {"lhs": lhs, "rhs": rhs, "output": ref.param, "epilogue": candidate, "linear": _match_linear(epilogue, len(types))}
+
+
+def _match_linear(value, accumulator):
+    """``max(accumulator * scale + bias[None, :], lower)``, each part optional except for the accumulator (parameter position
+    ``accumulator``): ``{"scale": ScalarParam / number / None, "bias": parameter position / None, "lower": number / None}``;
+    None for any other expression."""
+
+    def number(item):
+        return isinstance(item, (int, float)) and not isinstance(item, bool)
+
+    def parts(node, op, accepts):
+        """(the rest, the operand that ``accepts`` says yes to) of a commutative node, or (node, None)."""
+        if isinstance(node, Node) and node.op == op and len(node.args) == 2:
+            for rest, operand in (node.args, node.args[::-1]):
+                if isinstance(rest, Node) and accepts(operand):
+                    return rest, operand
+        return node, None
+
+    def is_row(item):  # bias[None, :] of a one-dimensional tile
+        if not (isinstance(item, Node) and item.op == "index" and len(item.args) == 2 and item.args[1] == (None, slice(None))):
+            return False
+        load = item.args[0]
+        if not (isinstance(load, Node) and load.op == "load" and len(load.args) == 1 and isinstance(load.args[0], TensorRef)):
+            return False
+        ref = load.args[0]
+        return ref.param != accumulator and ref.level == 1 and ref.is_tile and not ref.indices and ref.tensor.ndim == 1
+
+    value, lower = parts(value, "maximum", number)
+    value, row = parts(value, "add", is_row)
+    value, scale = parts(value, "mul", lambda item: number(item) or isinstance(item, ScalarParam))
+    if not (isinstance(value, Node) and value.op == "load" and isinstance(value.args[0], TensorRef) and value.args[0].param == accumulator):
+        return None
+    return {"scale": scale, "bias": None if row is None else row.args[0].args[0].param, "lower": lower}
+
+
+def analyze_column_vector(bias_type, env, blocks, n):
+    """The layout of a one-dimensional tensor whose element j belongs to column j of an output of ``n`` columns, for every
+    block of rows: ``(first element, stride)``; None when the arrangement says something else."""
+    try:
+        bias = Operand(bias_type, env)
+        _level_shape(bias, [2, 1])
+        if bias.empty or bias.fuse(bias.names[0][1], bias.names[1][0], "n") != blocks["n"]:
+            return None
+        bias.settle()
+        bias.require_absent(bias.names[0][0])
+    except UnsupportedProgram:
+        return None
+    offset = bias.offset()
+    if bias.constraints or not offset.is_linear() or (offset.variables() - {"n"}) or bias.extent("n") != n:
+        return None
+    return offset.const, offset.coef("n")
 
 
 def substitute(value, digest, replacement):

@@ -91,6 +91,7 @@ _SIGNATURES = {
     "launch_nt_matmul_static_scratch": (_S, _T, _T, _T, _I, _I, _I, _I, _I),
     "launch_nt_batched_matmul": (_S, _T, _T, _T, _I, _I, _I, _I, _I),
     "launch_nt_addmm": (_S, _T, _T, _T, _T, _T, _T, _I, _I, _I, _I),
+    "launch_nt_linear": (_S, _T, _T, _T, _I, ctypes.c_double, ctypes.c_double, _T, _I, _I, _I, _I),
     "launch_nt_softmax": (_S, _T, _T, _I, _I),
     "launch_nt_softmax_config": (_S, _I, _T, _T, _I, _I),
     "launch_nt_attention": (_S, _T, _T, _T, _T, _T, _T, _I, _I, _I),
