@@ -298,7 +298,17 @@ __global__ __launch_bounds__(kWaves * 64, kOcc) void attention_fwd_kernel(Attent
     // (or when the row sees its first key), which after the first blocks is rare, so the steady state has
     // no subtraction, no rescale factor and no rescaling of the output.  Probabilities are then at most
     // 2^kFoldSlack instead of at most 1; the final division by the row sum cancels the reference.
-    constexpr float kFoldSlack = 8.0f;
+    // kLazyMax: nothing looks for the row maximum in the steady state either.  The probabilities are computed
+    // relative to the reference as it stands, and only where a lane's add up to more than kLazySum (they may then be too
+    // large for the element type) or the row sees its first key, the maximum is found, the reference moved to it and the
+    // probabilities computed again; a block as high as the one that set the reference adds up to at most 32 per lane.  A
+    // sixth of the loop's vector arithmetic, and no chain of maxima between the scores and the exponentials.  For head
+    // dimension 64, where that arithmetic takes as long as the MFMAs: bf16 [8, 16, 1000, 64] 42.0 -> 39.1 us, [2, 8, 1500, 64] 21.3 ->
+    // 16.6, causal fp16 [1, 16, 4096, 64] 54.3 -> 45.7.  At 128 the scores have to outlive the exponentials in registers
+    // that are not there: [4, 32, 4096, 128] 920 -> 955, so that one keeps looking.
+    constexpr bool kLazyMax = kFold && kPipelined && D == 64;
+    constexpr float kFoldSlack = kLazyMax ? 0.0f : 8.0f;
+    constexpr float kLazySum = 256.0f;
     float16_t c_init[kQTiles];     // -m_run in all 16 registers
     float fold_limit[kQTiles];     // -inf until the row has seen a key, kFoldSlack afterwards
 #pragma unroll
@@ -385,8 +395,9 @@ __global__ __launch_bounds__(kWaves * 64, kOcc) void attention_fwd_kernel(Attent
     };
     // ... the move of the reference when some row of the wave needs it (wave-uniform branch, rare after
     // the first blocks): the block's scores, the row sums and the accumulator start values follow the
-    // new reference; alpha is the factor for the output accumulators ...
-    auto rebase = [&](float16_t (&s_acc)[KT][kQTiles], const float (&mx)[kQTiles], float (&alpha)[kQTiles]) __attribute__((always_inline)) {
+    // new reference; alpha is the factor for the output accumulators
+    // (s_next: the scores of the block behind it where they have been computed already, else null) ...
+    auto rebase = [&](float16_t (&s_acc)[KT][kQTiles], float16_t (*s_next)[kQTiles], const float (&mx)[kQTiles], float (&alpha)[kQTiles]) __attribute__((always_inline)) {
 #pragma unroll
         for (int qt = 0; qt < kQTiles; ++qt) {
             alpha[qt] = 1.0f;
@@ -400,7 +411,10 @@ __global__ __launch_bounds__(kWaves * 64, kOcc) void attention_fwd_kernel(Attent
 #pragma unroll
                 for (int kt = 0; kt < KT; ++kt)
 #pragma unroll
-                    for (int r = 0; r < 16; ++r) s_acc[kt][qt][r] -= delta;
+                    for (int r = 0; r < 16; ++r) {
+                        s_acc[kt][qt][r] -= delta;
+                        if (s_next != nullptr) s_next[kt][qt][r] -= delta;
+                    }
 #pragma unroll
                 for (int r = 0; r < 16; ++r) c_init[qt][r] = -m_run[qt];
             }
@@ -432,11 +446,47 @@ __global__ __launch_bounds__(kWaves * 64, kOcc) void attention_fwd_kernel(Attent
                 for (int e = 0; e < 8; ++e) pf[ps][qt][e] = E::from_float(s_acc[ps / 2][qt][8 * (ps & 1) + e]);
     };
 
+    // kLazyMax: the probabilities and this lane's part of their sums (the scores stay as they are, for a second time)
+    auto probabilities = [&](const float16_t (&s_acc)[KT][kQTiles], vec8 (&pf)[PS][kQTiles], float (&sums)[kQTiles]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int qt = 0; qt < kQTiles; ++qt) {
+            float sum[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int ps = 0; ps < PS; ++ps)
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    const float pv = __builtin_amdgcn_exp2f(s_acc[ps / 2][qt][8 * (ps & 1) + e]);
+                    pf[ps][qt][e] = E::from_float(pv);
+                    sum[e & 3] += pv;
+                }
+            sums[qt] = (sum[0] + sum[1]) + (sum[2] + sum[3]);
+        }
+    };
+    // ... and, behind them, the sums' way into the row sums: straight, or (wave-uniform branch, rare; also where a sum is no
+    // number) after the reference has moved and the probabilities have been computed again
+    auto finish_probabilities = [&](float16_t (&s_acc)[KT][kQTiles], float16_t (*s_next)[kQTiles], vec8 (&pf)[PS][kQTiles], float (&sums)[kQTiles],
+                                    float (&alpha)[kQTiles]) __attribute__((always_inline)) {
+        bool above = false;
+#pragma unroll
+        for (int qt = 0; qt < kQTiles; ++qt) {
+            alpha[qt] = 1.0f;
+            above = above || !(sums[qt] <= kLazySum + fold_limit[qt]);
+        }
+        if (__builtin_amdgcn_ballot_w64(above) != 0) {
+            float mx[kQTiles];
+            row_max(s_acc, mx);
+            rebase(s_acc, s_next, mx, alpha);
+            probabilities(s_acc, pf, sums);
+        }
+#pragma unroll
+        for (int qt = 0; qt < kQTiles; ++qt) l_run[qt] += sums[qt];
+    };
+
     auto softmax = [&](float16_t (&s_acc)[KT][kQTiles], vec8 (&pf)[PS][kQTiles], float (&alpha)[kQTiles]) __attribute__((always_inline)) {
         if constexpr (kFold) {
             float mx[kQTiles];
             row_max(s_acc, mx);
-            rebase(s_acc, mx, alpha);
+            rebase(s_acc, nullptr, mx, alpha);
             exponentials(s_acc, pf);
             return;
         }
@@ -585,7 +635,30 @@ __global__ __launch_bounds__(kWaves * 64, kOcc) void attention_fwd_kernel(Attent
                 issue_k(Own(), min(j + 2, last_block));
                 issue_v(Own(), j);
                 if constexpr (decltype(masked_tag)::value) apply_masks(s_buf[kParity], j);
-                if constexpr (kFold) {
+                if constexpr (kLazyMax) {
+                    // One scheduling region: the exponentials, sums and conversions of block j under the MFMAs of
+                    // P(j-1) . V(j-1) and K(j+1) . Q, whose accumulators start from the reference before a move in this step.
+                    float sums[kQTiles];
+                    probabilities(s_buf[kParity], p_buf[kParity], sums);
+                    accumulate(Other(), p_buf[1 - kParity], PsBegin(), PsEnd());
+                    if constexpr (kScores) scores(Other(), s_buf[1 - kParity]);
+                    {
+                        constexpr int kMfma = (PS * DT + (kScores ? KS * KT : 0)) * kQTiles;
+                        constexpr int kReads = PS * DT * 2 + (kScores ? KS * KT : 0);
+                        constexpr int kExps = (PS * 8 * kQTiles + kMfma - 1) / kMfma;  // exponentials under an MFMA
+                        __builtin_amdgcn_sched_group_barrier(0x100, 6, 0);
+                        __builtin_amdgcn_sched_group_barrier(0x020, 2 * kInstr, 0);
+                        __builtin_amdgcn_sched_group_barrier(0x400, 2, 0);
+                        static_for<0, kMfma>([&](auto i_tag) __attribute__((always_inline)) {
+                            constexpr int i = decltype(i_tag)::value;
+                            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                            if constexpr (6 + 2 * i < kReads) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+                            __builtin_amdgcn_sched_group_barrier(0x400, kExps, 0);
+                            __builtin_amdgcn_sched_group_barrier(0x002, kExps * 2, 0);
+                        });
+                    }
+                    finish_probabilities(s_buf[kParity], kScores ? s_buf[1 - kParity] : nullptr, p_buf[kParity], sums, alpha);
+                } else if constexpr (kFold) {
                     // Two scheduling regions with the (rare) move of the reference between them: the row
                     // maxima run under the first MFMAs of P(j-1) . V(j-1); the exponentials, row sums and
                     // conversions under the rest of them and under K(j+1) . Q, whose accumulators start
@@ -610,7 +683,7 @@ __global__ __launch_bounds__(kWaves * 64, kOcc) void attention_fwd_kernel(Attent
                             __builtin_amdgcn_sched_group_barrier(0x002, 3, 0);
                         });
                     }
-                    rebase(s_buf[kParity], mx, alpha);
+                    rebase(s_buf[kParity], nullptr, mx, alpha);
                     exponentials(s_buf[kParity], p_buf[kParity]);
                     accumulate(Other(), p_buf[1 - kParity], PsSplit(), PsEnd());
                     if constexpr (kScores) scores(Other(), s_buf[1 - kParity]);
@@ -1347,13 +1420,15 @@ int attention_float32(AttentionParams p, int head_dim, const NineToothedTensor &
 // variant: 0 = 128 query rows per workgroup, 64-key blocks, two workgroups per CU
 //          1 = 256 query rows per workgroup, 64-key blocks, one workgroup per CU
 //          2 = 128 query rows per workgroup, 32-key blocks, three workgroups per CU
+//              (head dimension 64: its loop is software-pipelined too -- 162 registers, so that the beginnings and ends of three workgroups
+//              overlap: bf16 [8, 16, 1000, 64] against 256 keys 16.9 us in variant 3, here 15.7, against 4000 132 and 134; the plain loop 40.4 against 1000, here 39.3)
 //          3 = variant 0 with the software-pipelined main loop
 //          4 = variant 3 with eight waves (256 query rows) per workgroup, one workgroup per CU
 constexpr int kAttentionVariants = 5;
 const char *const kAttentionVariantNames[kAttentionVariants] = {
     "plain loop, 64-key blocks, four waves (128 query rows), two workgroups per CU",
     "plain loop, 64-key blocks, 256 query rows per four-wave workgroup, one workgroup per CU",
-    "plain loop, 32-key blocks, four waves, three workgroups per CU",
+    "32-key blocks, four waves, three workgroups per CU (plain loop; pipelined for head dimension 64)",
     "software-pipelined loop, 64-key blocks, four waves (128 query rows), two workgroups per CU",
     "software-pipelined loop, 64-key blocks, eight waves (256 query rows), one workgroup per CU",
 };
@@ -1385,7 +1460,7 @@ int dispatch_attention(AttentionParams &p, int head_dim, int variant, hipStream_
         if (variant == 4) return (int)launch_attention<T, 64, 1, 64, 2, true, T, 8>(p, stream);
         if (variant == 3) return (int)launch_attention<T, 64, 1, 64, 2, true>(p, stream);
         if (variant == 1) return (int)launch_attention<T, 64, 2, 64, 1, false>(p, stream);
-        if (variant == 2) return (int)launch_attention<T, 64, 1, 32, 3, false>(p, stream);
+        if (variant == 2) return (int)launch_attention<T, 64, 1, 32, 3, true>(p, stream);
         return (int)launch_attention<T, 64, 1, 64, 2, false>(p, stream);
     }
     if (head_dim == 32) return (int)launch_attention<T, 32, 1, 64, 2, false>(p, stream);
