@@ -153,13 +153,14 @@ hipError_t fast_launch(const GemmProblem &q, hipStream_t stream) {
 // Of the numbers whose workgroups are all on the chip at once, the one of least expected time: `alone` is what a k tile takes a
 // workgroup with a CU to itself, `shared` what it takes the CU per workgroup (us), the partial products are written and read at `rate`.
 // Fitted to 59 products of 1 to 3000 rows, 2 to 48 parts: 3 % (64 x 64), 1 % (others) slower than the best number on average; 512
-// workgroups whatever the shape were 11, 9 and 10 % slower (509 x 2752 x 6800 on 128 x 128: six parts, 528 workgroups, 54 us, five 37.5).
+// workgroups whatever the shape were 11 and 10 % slower.  (128 x 128: five products of 100 to 1024 rows, a step 0.22 to 0.46 us with
+// the rhs in the caches and in memory; 222 x 2752 x 15040 34.5 us in five parts, 39 in four, 43 in eight, without the summing.)
 int split_parts(const GemmProblem &q, int bm, int bn, int bk, int *kt_per_part, int64_t scratch_limit = int64_t(64) << 20) {
     struct Cost {
         int area, resident;  // workgroups per CU
         float alone, shared, rate;
     };
-    constexpr Cost costs[] = {{64 * 64, 2, 0.234f, 0.214f, 0.8e6f}, {128 * 128, 2, 0.7f, 0.35f, 4.0e6f}, {128 * 256, 2, 0.39f, 0.28f, 5.1e6f}, {256 * 256, 1, 0.29f, 0.29f, 5.8e6f}};
+    constexpr Cost costs[] = {{64 * 64, 2, 0.234f, 0.214f, 0.8e6f}, {128 * 128, 1, 0.3f, 0.3f, 4.0e6f}, {128 * 256, 2, 0.39f, 0.28f, 5.1e6f}, {256 * 256, 1, 0.29f, 0.29f, 5.8e6f}};
     const int64_t tiles = (int64_t)((q.m + bm - 1) / bm) * ((q.n + bn - 1) / bn);
     const int num_kt = (q.k + bk - 1) / bk;
     if (tiles >= 320) return 1;  // (the untuned choice only splits below 192 tiles; between, the tuner decides)
@@ -502,7 +503,7 @@ hipError_t generic_launch(const GemmProblem &q, hipStream_t stream) {
 enum InstanceIndex {
     kAnyStride, k256x256x32, k256x256x64, k128x128x64, k64x64x64, k128x256x32,
     kTail256x256x32, kTail128x256x32, kTail128x128x64, kTail64x64x64, kSplit64x64x64, kSplit128x128x64,
-    kSplit128x256x32, kSplit256x256x32, kSkinny16, kSkinny32,
+    kSplit128x256x32, kSplit256x256x32, kSkinny16, kSkinny32, kDeep128x128x64, kDeep64x64x128, kDeep64x128x64,
 };
 
 const GemmInstance kInstances[] = {
@@ -517,11 +518,16 @@ const GemmInstance kInstances[] = {
     NT_TAIL_INSTANCE(128, 128, 64, 2, 2, 2, 2),
     NT_TAIL_INSTANCE(64, 64, 64, 2, 2, 4, 2),
     NT_SPLIT_INSTANCE(64, 64, 64, 2, 2, 4, 2),
-    NT_SPLIT_INSTANCE(128, 128, 64, 2, 2, 2, 2),
+    NT_SPLIT_INSTANCE(128, 128, 64, 2, 4, 4, 2),  // (two stages, two workgroups per CU: 222 x 2752 x 15040 43.3 us, here 39.4; 283 x 1016 x 12224 26.8, 23.3; 256 x 8192 x 8192 59.9, 52.2)
     NT_SPLIT_INSTANCE(128, 256, 32, 1, 4, 3, 2),  // a few hundred rows against a wide rhs: 64 to 160 large tiles
     NT_SPLIT_INSTANCE(256, 256, 32, 2, 4, 5, 2),
     {"64x16x64 skinny, split-k over the waves of a workgroup", 64, 16, 64, skinny_accepts, skinny_launch<1>},
     {"64x32x64 skinny, split-k over the waves of a workgroup", 64, 32, 64, skinny_accepts, skinny_launch<2>},
+    // One workgroup per CU with most of its LDS: three or four fills of 16 to 32 KiB in flight instead of one, for products whose
+    // tiles the chip holds all at once, so that nothing else covers the latency of a fill.
+    NT_TAIL_INSTANCE(128, 128, 64, 2, 4, 4, 2),
+    NT_TAIL_INSTANCE(64, 64, 128, 2, 2, 4, 1),
+    NT_TAIL_INSTANCE(64, 128, 64, 2, 4, 5, 2),
 #ifdef NT_GEMM_ABLATION
 #define NT_LOAD_INSTANCE(BM, BN, BK, WM, WN, ST, OCC, LD, AUX) \
     {#BM "x" #BN "x" #BK " waves " #WM "x" #WN " stages " #ST " load " #LD " aux " #AUX, BM, BN, BK, fast_accepts<BM, BN, BK, ST>, fast_launch<BM, BN, BK, WM, WN, ST, OCC, 0, LD, AUX>}
@@ -538,7 +544,7 @@ const GemmInstance kInstances[] = {
 #endif
 };
 constexpr int kNumInstances = sizeof(kInstances) / sizeof(kInstances[0]);
-static_assert(kNumInstances > kSkinny32, "InstanceIndex names the first instances of the table");
+static_assert(kNumInstances > kDeep64x128x64, "InstanceIndex names the first instances of the table");
 
 inline bool is_split(int instance) { return instance >= kSplit64x64x64 && instance <= kSplit256x256x32; }
 
@@ -620,6 +626,17 @@ int heuristic_choice(const GemmProblem &q, int bm, int bn, int bk) {
     if (q.m <= 64 && few_tiles(kSplit64x64x64)) return kSplit64x64x64;
     if (few_tiles(kSplit128x128x64)) return kSplit128x128x64;
     if (few_tiles(kSplit64x64x64)) return kSplit64x64x64;
+    // All tiles on the chip at once, one per CU: the largest deep ring of which that holds (bf16, us, the best of the other
+    // instances / this): 64 x 64 x 128 512 x 512 x 2048 10.4 / 9.2, 130 x 4096 x 4096 19.2 / 15.8, 1000 x 1000 x 16384 80.5 / 58.2 (with a K
+    // of four steps nothing is left in flight: 1024 x 1024 x 128 3.8 / 4.1); 64 x 128 x 64 1024 x 2048 x 2048 15.2 / 12.9, 70 x 14336 x
+    // 2048 16.6 / 15.3; 128 x 128 x 64 2048 x 2048 x 4096 47.2 / 32.1, 1500 x 2048 x 512 10.1 / 7.3.  More tiles: 384 of 128 x 128, 700 x 8192 x
+    // 2048 35.7 / 34.4, but 1024 of them with a K of 256 17.3 / 18.0, so that the rules below keep those.
+    struct DeepRule { int instance, min_k; };
+    for (const DeepRule &rule : {DeepRule{kDeep64x64x128, 1024}, DeepRule{kDeep64x128x64, 512}, DeepRule{kDeep128x128x64, 256}}) {
+        const GemmInstance &inst = kInstances[rule.instance];
+        const int64_t per_matrix = (int64_t)((q.m + inst.bm - 1) / inst.bm) * ((q.n + inst.bn - 1) / inst.bn);
+        if (q.k >= rule.min_k && per_matrix * q.batch <= 256 && inst.accepts(q)) return rule.instance;
+    }
     // (an instance with tails accepts what its plain form accepts, so it comes right after it: a partial
     // last tile costs less than a smaller tile everywhere)
     const Rule rules[] = {{k256x256x32, 256}, {k256x256x64, 256}, {kTail256x256x32, 256}, {k128x256x32, 128}, {kTail128x256x32, 128},

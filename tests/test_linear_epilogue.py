@@ -108,7 +108,7 @@ def test_bias_and_bound_in_one_launch(m, n, k, transposed, tuned, dtype, monkeyp
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("block", ((64, 64, 64), (128, 128, 64), (128, 256, 32), (256, 256, 32), (256, 256, 64)))
+@pytest.mark.parametrize("block", ((64, 64, 64), (64, 64, 128), (64, 128, 64), (128, 128, 64), (128, 256, 32), (256, 256, 32), (256, 256, 64)))
 @pytest.mark.parametrize("m, n, k, transposed", ((512, 512, 512, False), (512, 512, 512, True), (300, 1000, 520, False), (300, 1001, 520, True)))
 def test_every_tile(m, n, k, transposed, block):
     lhs, rhs, bias = _operands(m, n, k, torch.bfloat16, transposed, torch.float32)
