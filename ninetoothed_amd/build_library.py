@@ -1,5 +1,5 @@
 """Builds ``libnt_hip.so`` (the gfx950 kernels behind the C ABI) and ``libnt_probe.so`` (measurement kernels
-that only bench.py loads) in-tree with hipcc.
+that only bench.py loads) in-tree with hipcc, and ``nt_call.so`` (the way from Python into the former) with g++.
 
 Usage: ``python -m ninetoothed_amd.build_library`` or ``build_library()``.  The library
 is written to ``ninetoothed_amd/lib/libnt_hip.so``; object files go to
@@ -22,6 +22,10 @@ SOURCES = ("gemm_api.hip", "conv2d.hip", "softmax.hip", "attention.hip", "map.hi
 # they are built into a library of their own that only bench.py loads.
 PROBE_LIBRARY_PATH = PACKAGE_DIR / "lib" / "libnt_probe.so"
 PROBE_SOURCES = ("probe.hip",)
+
+# The way of a repeated call from Python into the library: host code against torch's and Python's headers.
+CALL_LIBRARY_PATH = PACKAGE_DIR / "lib" / "nt_call.so"
+CALL_SOURCE = "call.cpp"
 
 OFFLOAD_ARCH = "gfx950"
 
@@ -79,8 +83,27 @@ def build_library(verbose=False, extra_flags=()):
         _run(command)
         temporary.replace(path)
 
+    def compile_call():
+        import sysconfig
+
+        import torch
+
+        torch_dir = pathlib.Path(torch.__file__).resolve().parent
+        temporary = CALL_LIBRARY_PATH.with_suffix(".so.tmp")
+        command = [
+            shutil.which("g++") or "c++", "-O2", "-std=c++17", "-fPIC", "-shared", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}",
+            f"-I{torch_dir / 'include'}", f"-I{sysconfig.get_paths()['include']}", str(CSRC_DIR / CALL_SOURCE), "-o", str(temporary),
+            f"-L{torch_dir / 'lib'}", "-lc10", "-ltorch_cpu", "-ltorch_python",
+        ]  # fmt: skip
+        if verbose:
+            print(" ".join(command), flush=True)
+        _run(command)
+        temporary.replace(CALL_LIBRARY_PATH)
+
     with concurrent.futures.ThreadPoolExecutor(max_workers=4) as pool:
+        call = pool.submit(compile_call)
         objects = list(pool.map(compile_one, SOURCES + PROBE_SOURCES))
+        call.result()
 
     link(objects[: len(SOURCES)], LIBRARY_PATH)
     link(objects[len(SOURCES) :], PROBE_LIBRARY_PATH)

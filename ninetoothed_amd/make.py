@@ -129,7 +129,9 @@ class Kernel:
         self.parameters = list(inspect.signature(application).parameters)
         self.meta_symbols = recognition.unbound_meta_symbols(self.types)
         self._plans = {}
+        self._prepared = {}  # what `runtime.run` launches without coming back here: {signature as bytes: (recipe, plan)}
         self._scalar_flags = tuple((t.ndim == 0 and not isinstance(t.dtype, Tensor), bool(t.constexpr)) for t in self.types)
+        self._flags = b"".join(b"t" if not is_scalar else b"c" if constexpr else b"s" for is_scalar, constexpr in self._scalar_flags)
         self._source_path = None
         self.last_plan = None  # description of the launch used by the latest call
 
@@ -166,6 +168,13 @@ class Kernel:
         return self(*args, **kwargs)
 
     def __call__(self, *args, **kwargs):
+        plan = runtime.run(self._prepared, args, kwargs, self._flags)
+        if plan is None:
+            self._call(args, kwargs)
+        else:
+            self.last_plan = plan.description
+
+    def _call(self, args, kwargs):
         if len(args) != len(self.types):
             raise TypeError(f"`{self.kernel_name}` takes {len(self.types)} positional arguments but {len(args)} were given.")
         key = self._signature(args, kwargs)
@@ -174,6 +183,10 @@ class Kernel:
             plan = self._plans[key] = self._prepare(args, kwargs)
         self.last_plan = plan.description
         plan(args)
+        if plan.recipe is not None and plan.settled():
+            text = runtime.call_library().signature(args, kwargs, self._flags)
+            if text is not None and text not in self._prepared:
+                self._prepared[text] = (plan.recipe(), plan)
 
     # ---- plan construction ----------------------------------------------
     def _signature(self, args, kwargs):
@@ -378,7 +391,17 @@ class Kernel:
                     maybe_tune(call_args, i_arg, beta, alpha)
                 runtime.check(lib.launch_nt_addmm(runtime.current_stream(), i_arg, a_arg, b_arg, beta, alpha, c_arg, dtype, *blocks))
 
-            return _Plan(f"launch_nt_addmm {m}x{n}x{k} {tag} blocks {blocks}", launch)
+            def recipe():
+                slots = (
+                    runtime.slot(in_pos, i_arg, i.base * itemsize), runtime.slot(a_pos, a_arg, a.base * itemsize), runtime.slot(b_pos, b_arg, b.base * itemsize),
+                    ("f", beta_pos), ("f", alpha_pos), runtime.slot(c_pos, c_arg, c.base * out_itemsize),
+                )  # fmt: skip
+                return runtime.recipe("addmm", slots, (dtype, *blocks))
+
+            return _Plan(f"launch_nt_addmm {m}x{n}x{k} {tag} blocks {blocks}", launch, recipe, lambda: not state["tune"])
+
+        def product_slots():
+            return runtime.slot(a_pos, a_arg, a.base * itemsize), runtime.slot(b_pos, b_arg, b.base * itemsize), runtime.slot(c_pos, c_arg, c.base * out_itemsize)
 
         def launch(call_args):
             a_arg.data = call_args[a_pos].data_ptr() + a.base * itemsize
@@ -399,7 +422,11 @@ class Kernel:
                 maybe_tune(call_args, null, null, null)
             runtime.check(lib.launch_nt_matmul(runtime.current_stream(), a_arg, b_arg, c_arg, dtype, out_dtype, *blocks))
 
-        return _Plan(f"launch_nt_matmul {m}x{n}x{k} {tag}->{out_tag} blocks {blocks}", launch)
+        plan = _Plan(
+            f"launch_nt_matmul {m}x{n}x{k} {tag}->{out_tag} blocks {blocks}", launch, lambda: runtime.recipe("matmul", product_slots(), (dtype, out_dtype, *blocks)), lambda: not state["tune"]
+        )
+        plan.product_slots = product_slots
+        return plan
 
     def _conv2d_plan(self, info, tag, args):
         lib = runtime.library()
@@ -417,7 +444,9 @@ class Kernel:
                 runtime.check(lib.launch_nt_conv2d_strided(runtime.current_stream(), x, w, y, dtype, pad_h, pad_w, *steps, *blocks))
 
             return _Plan(
-                f"launch_nt_conv2d_strided gemm {info['m']}x{info['n']}x{info['k']} {tag} padding ({pad_h}, {pad_w}) stride {steps[:2]} dilation {steps[2:]}", launch_strided
+                f"launch_nt_conv2d_strided gemm {info['m']}x{info['n']}x{info['k']} {tag} padding ({pad_h}, {pad_w}) stride {steps[:2]} dilation {steps[2:]}",
+                launch_strided,
+                lambda: runtime.recipe("conv2d_strided", (runtime.slot(0, x), runtime.slot(1, w), runtime.slot(2, y)), (dtype, pad_h, pad_w, *steps, *blocks)),
             )
 
         from ninetoothed_amd import auto_tuner
@@ -439,7 +468,12 @@ class Kernel:
                     state["tune"] = auto_tuner.tune_conv2d(x, w, y, dtype, pad_h, pad_w) == -1
             runtime.check(lib.launch_nt_conv2d(runtime.current_stream(), x, w, y, dtype, pad_h, pad_w, *blocks))
 
-        return _Plan(f"launch_nt_conv2d gemm {info['m']}x{info['n']}x{info['k']} {tag} padding ({pad_h}, {pad_w})", launch)
+        return _Plan(
+            f"launch_nt_conv2d gemm {info['m']}x{info['n']}x{info['k']} {tag} padding ({pad_h}, {pad_w})",
+            launch,
+            lambda: runtime.recipe("conv2d", (runtime.slot(0, x), runtime.slot(1, w), runtime.slot(2, y)), (dtype, pad_h, pad_w, *blocks)),
+            lambda: not state["tune"],
+        )
 
     def _prepare_softmax(self, args, env):
         kind, info = recognition.analyze_softmax(self.types[0], self.types[1], env)
@@ -456,7 +490,11 @@ class Kernel:
             input.data, output.data = call_args[0].data_ptr(), call_args[1].data_ptr()
             runtime.check(lib.launch_nt_softmax(runtime.current_stream(), input, output, dtype, block))
 
-        return _Plan(f"launch_nt_softmax {info['input']['rows']}x{info['input']['cols']} {tag} block {block}", launch)
+        return _Plan(
+            f"launch_nt_softmax {info['input']['rows']}x{info['input']['cols']} {tag} block {block}",
+            launch,
+            lambda: runtime.recipe("softmax", (runtime.slot(0, input), runtime.slot(1, output)), (dtype, block)),
+        )
 
     def _prepare_map(self, args, env):
         """Element-wise / reducing programs: one interpreter launch per store."""
@@ -487,7 +525,14 @@ class Kernel:
                 runtime.check(lib.launch_nt_map(stream, ctypes.addressof(program)))
 
         self._map_programs = [program for program, _, _, _ in launches]
-        return _Plan("launch_nt_map " + "; ".join(description for _, description, _, _ in launches), launch)
+        recipe = None
+        if not any(isinstance(param, tuple) for _, _, _, operand_params in launches for param in operand_params):  # (jagged arguments: Python reads their offsets)
+
+            def recipe():
+                programs = ((ctypes.addressof(program), tuple(operand_params), tuple(scalar_slots)) for program, _, scalar_slots, operand_params in launches)
+                return runtime.recipe("map", (), (), launches=programs)
+
+        return _Plan("launch_nt_map " + "; ".join(description for _, description, _, _ in launches), launch, recipe)
 
     def _prepare_gemm_epilogue(self, args, env):
         """A matmul accumulator followed by element-wise work (bias, activation, scaling, residual).  A scale, a bias
@@ -530,8 +575,11 @@ class Kernel:
         program, description, scalar_slots, operand_params = built
         linear = self._linear_launch(info, args, env, tag)
 
+        taken = {"linear": False}
+
         def launch(call_args):
-            if linear is not None and linear(call_args):
+            taken["linear"] = linear is not None and linear.launch(call_args)
+            if taken["linear"]:
                 return
             extended = with_scratch(call_args)  # from torch's stream-ordered allocator: free again once both launches are queued
             gemm(extended)
@@ -543,11 +591,13 @@ class Kernel:
 
         self._map_programs = [program]
         two_passes = f"{gemm.description}; launch_nt_map {description}"
-        return _Plan(two_passes if linear is None else f"launch_nt_linear, or {two_passes}", launch)
+        if linear is None:
+            return _Plan(two_passes, launch)
+        return _Plan(f"launch_nt_linear, or {two_passes}", launch, linear.recipe, lambda: taken["linear"] and linear.settled())
 
     def _linear_launch(self, info, args, env, tag):
-        """``max(product * scale + bias[None, :], lower)`` in one launch: a function of the call's arguments that says whether
-        the library took them; None for other epilogues, element types and arrangements."""
+        """``max(product * scale + bias[None, :], lower)`` in one launch: a plan whose `launch` says whether
+        the library took the call's arguments; None for other epilogues, element types and arrangements."""
         linear, details = self.details["linear"], self.details
         lhs_pos, rhs_pos, out_pos = details["lhs"], details["rhs"], details["output"]
         m, n, k = info["m"], info["n"], info["k"]
@@ -574,7 +624,17 @@ class Kernel:
             factor = float(scale if scale_pos is None else call_args[scale_pos])
             return lib.launch_nt_linear(runtime.current_stream(), lhs, rhs, bias_arg, bias_dtype, factor, lower, output, dtype, *blocks)
 
-        return self._gemm_plan(info, tag, tag, positions=(bias_pos, lhs_pos, rhs_pos, None, None, out_pos), epilogue=epilogue).launch
+        plan = self._gemm_plan(info, tag, tag, positions=(bias_pos, lhs_pos, rhs_pos, None, None, out_pos), epilogue=epilogue)
+        slots, blocks = plan.product_slots, [info["blocks"][axis] if info["blocks"][axis] > 1 else 0 for axis in ("m", "n", "k")]
+
+        def recipe():
+            lhs, rhs, output = slots()
+            bias = None if bias_pos is None else runtime.slot(bias_pos, bias_arg, bias_base * bias_size)
+            doubles = (1.0 if scale_pos is not None else float(scale), lower)
+            return runtime.recipe("linear", (lhs, rhs, bias, output), (bias_dtype, dtype, *blocks), doubles, -1 if scale_pos is None else scale_pos)
+
+        plan.recipe = recipe
+        return plan
 
     def _prepare_attention(self, args, env):
         scaled = self.details["scale"]
@@ -618,7 +678,11 @@ class Kernel:
                     state["tune"] = auto_tuner.tune_attention(tensors[0], tensors[1], tensors[2], causal, scale_arg, tensors[3], dtype) == -1
             runtime.check(lib.launch_nt_attention(runtime.current_stream(), tensors[0], tensors[1], tensors[2], causal, scale_arg, tensors[3], dtype, 0, 0))
 
-        return _Plan(f"launch_nt_attention q{info['q']['shape']} k{info['k']['shape']} {tag}", launch)
+        def recipe():
+            slot_q, slot_k, slot_v, slot_o = (runtime.slot(p, tensor) for p, tensor in zip(positions, tensors))
+            return runtime.recipe("attention", (slot_q, slot_k, slot_v, ("b", 3), ("f", 4) if scaled else None, slot_o), (dtype, 0, 0))
+
+        return _Plan(f"launch_nt_attention q{info['q']['shape']} k{info['k']['shape']} {tag}", launch, recipe, lambda: not state["tune"])
 
 
 def _storage(args, param):
@@ -646,13 +710,15 @@ class _Plan:
     """A prepared launch.  Its argument structs are filled in per call, so calls from several
     host threads take turns (the launches themselves are asynchronous)."""
 
-    __slots__ = ("description", "launch", "_lock")
+    __slots__ = ("description", "launch", "recipe", "settled", "product_slots", "_lock")
 
-    def __init__(self, description, launch):
+    def __init__(self, description, launch, recipe=None, settled=lambda: True):
         import threading
 
         self.description = description
         self.launch = launch
+        self.recipe = recipe  # makes what `runtime.run` launches; None for plans that need Python at every call
+        self.settled = settled  # whether nothing is left to be timed, or asked of the library, by later calls
         self._lock = threading.Lock()
 
     def __call__(self, args):

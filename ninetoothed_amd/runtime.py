@@ -46,6 +46,7 @@ class ArgumentTensor(ctypes.Structure):
         strides_array = (ctypes.c_int64 * max(len(strides), 1))(*strides)
         tensor = ArgumentTensor(data_ptr, shape_array, strides_array)
         tensor._keepalive = (shape_array, strides_array)
+        tensor.layout = (tuple(int(size) for size in shape), tuple(int(stride) for stride in strides))
         return tensor
 
     @staticmethod
@@ -140,6 +141,53 @@ def library():
             lib.nt_release_workspaces.argtypes = []
             _library = lib
     return _library
+
+
+# ---- the way of a repeated call (csrc/call.cpp) ----
+
+CALL_LIBRARY_PATH = LIBRARY_PATH.with_name("nt_call.so")
+
+
+def run(prepared, args, kwargs, flags):
+    """Launches what ``prepared`` (``{signature: (recipe, plan)}``) holds for these arguments and returns the plan; None where it
+    holds nothing, or the library did not take the call.  (The first call puts the native function in this one's place.)"""
+    return call_library().run(prepared, args, kwargs, flags)
+
+
+_call_library = None
+
+
+def call_library():
+    """Loads ``nt_call.so`` once; raises if it has not been built."""
+    global _call_library, run
+    with _lock:
+        if _call_library is None:
+            import importlib.machinery
+            import importlib.util
+
+            import torch
+
+            if not CALL_LIBRARY_PATH.exists():
+                raise RuntimeError(f"{CALL_LIBRARY_PATH} is missing: build it with `python -m ninetoothed_amd.build_library`.")
+            loader = importlib.machinery.ExtensionFileLoader("nt_call", str(CALL_LIBRARY_PATH))
+            module = importlib.util.module_from_spec(importlib.util.spec_from_loader("nt_call", loader))
+            loader.exec_module(module)
+            module.use(torch._C._cuda_getDevice, torch._C._cuda_getCurrentRawStream)
+            run = module.run
+            _call_library = module
+    return _call_library
+
+
+def recipe(kind, slots, ints, doubles=(), scale_position=-1, launches=()):
+    """What ``run`` needs for entry point ``launch_nt_<kind>``: its tensors (`slot`, ``("f", position)`` a float, ``("b", position)`` a
+    truth value, None), then its numbers."""
+    address = ctypes.cast(getattr(library(), "launch_nt_" + kind), ctypes.c_void_p).value
+    return call_library().recipe(kind, address, tuple(slots), tuple(int(value) for value in ints), tuple(doubles), scale_position, tuple(launches))
+
+
+def slot(position, argument, offset=0):
+    """A call's tensor in ``argument``'s layout, ``offset`` bytes into its memory."""
+    return ("t", position, int(offset), *argument.layout)
 
 
 def exported_symbols():

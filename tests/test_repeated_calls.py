@@ -1,0 +1,152 @@
+"""Repeated calls take the way of csrc/call.cpp: the signature that it reads tells apart what the one in Python does, and calls
+that it does not know are left to Python."""
+
+import gc
+import threading
+
+import pytest
+import torch
+
+import ninetoothed_amd as ninetoothed
+import ninetoothed_amd.language as ntl
+from ninetoothed_amd import Tensor, programs, runtime
+
+
+def _signature(*args, flags=b"ttt", **kwargs):
+    return runtime.call_library().signature(args, kwargs, flags)
+
+
+def test_signature_tells_layouts_apart():
+    a, b, c = torch.empty(4, 6), torch.empty(6, 4), torch.empty(4, 4)
+    base = _signature(a, b, c)
+    assert base is not None and base == _signature(torch.empty(4, 6), b, c)
+    others = [
+        (a.half(), b, c), (a, b.t().contiguous().t(), c), (torch.empty(4, 8)[:, :6], b, c), (torch.empty(1, 4, 6), b, c), (a, b, torch.empty(4, 5)), (a.to("meta"), b, c),
+        (torch.empty(6, 4).t(), b, c),
+    ]  # fmt: skip
+    signatures = [_signature(*args) for args in others]
+    assert None not in signatures and len({base, *signatures}) == len(others) + 1
+    # (4, 6) beside (6, 4) is not (4, 6, 6) beside (4)
+    assert _signature(torch.empty(4), torch.empty(6, 6, 4), c) != base
+
+
+def test_signature_scalars_and_keywords():
+    a = torch.empty(3)
+    assert _signature(a, 1.0, 2, flags=b"tss") == _signature(a, 3.0, 5, flags=b"tss")
+    assert len({_signature(a, x, 2, flags=b"tss") for x in (1.0, 1, True)}) == 3
+    assert _signature(a, 1.0, 2, flags=b"tcs") != _signature(a, 3.0, 2, flags=b"tcs")
+    assert _signature(a, 1, 2, flags=b"tcs") != _signature(a, 1.0, 2, flags=b"tcs")
+    assert _signature(a, flags=b"t", BLOCK=1) != _signature(a, flags=b"t", BLOCK=2) != _signature(a, flags=b"t", BLOCKS=2)
+
+
+def test_what_is_left_to_python():
+    a, b, c = torch.empty(4, 6), torch.empty(6, 4), torch.empty(4, 4)
+
+    class Sub(torch.Tensor):
+        pass
+
+    nested = torch.nested.nested_tensor([torch.empty(2, 6), torch.empty(3, 6)], layout=torch.jagged)
+    for other in (a.as_subclass(Sub), nested, a.to_sparse(), [1.0], None, a.numpy()):
+        assert _signature(other, b, c) is None
+    assert _signature(a, b) is None  # a missing argument
+    assert _signature(a, b, c, d=1.5) is None and _signature(a, b, c, d=True) is None
+    assert _signature(a, b, 2**80, flags=b"ttc") is None
+    assert torch.vmap(lambda x: x if _signature(x, b, c) is None else x + float("nan"))(torch.zeros(2, 4, 6)).isnan().sum() == 0
+    assert _signature(*(torch.empty((1,) * 20) for _ in range(6)), flags=b"tttttt") is None  # longer than the buffer
+    assert runtime.run({}, (a, b, c), {}, b"ttt") is None
+
+
+def test_recipes_that_do_not_fit_are_refused():
+    layout = runtime.ArgumentTensor.from_layout(0, (1, 1), (1, 1))
+    with pytest.raises(ValueError):
+        runtime.call_library().recipe("matmul", 1, (runtime.slot(0, layout),), (1, 2, 3, 4, 5), (), -1, ())
+    with pytest.raises(ValueError):
+        runtime.call_library().recipe("nothing", 1, (), (), (), -1, ())
+
+
+def _add():
+    def arrangement(lhs, scale, output, block=ninetoothed.block_size()):
+        return lhs.tile((block,)), scale, output.tile((block,))
+
+    def application(lhs, scale, output):
+        output = lhs * scale + 1  # noqa: F841
+
+    return ninetoothed.make(arrangement, application, (Tensor(1), Tensor(0), Tensor(1)))
+
+
+@pytest.mark.gpu
+def test_each_entry_point_repeats_what_its_first_call_does():
+    def normal(*shape):
+        return torch.randn(shape, device="cuda", dtype=torch.float16)
+
+    def linear_application(lhs, rhs, bias, output):
+        accumulator = ntl.zeros(output.shape, dtype=ntl.float32)
+        for k in range(lhs.shape[0]):
+            accumulator += ntl.dot(lhs[k], rhs[k])
+        output = ntl.maximum(accumulator + bias[None, :], 0)  # noqa: F841
+
+    def linear_arrangement(lhs, rhs, bias, output, BM=ninetoothed.block_size(), BN=ninetoothed.block_size(), BK=ninetoothed.block_size()):
+        lhs_arranged, rhs_arranged, output_arranged = programs.matmul.arrangement(lhs, rhs, output, BM, BN, BK)
+        return lhs_arranged, rhs_arranged, bias.tile((BN,)).unsqueeze(0).expand((output_arranged.shape[0], -1)), output_arranged
+
+    attention = ninetoothed.make(programs.attention.arrangement_with_scale, programs.attention.application_with_scale, programs.attention.tensors(True))
+    conv2d = ninetoothed.make(programs.conv2d.arrangement, programs.conv2d.application, programs.conv2d.tensors())
+    softmax = ninetoothed.make(programs.softmax.arrangement, programs.softmax.application, programs.softmax.tensors())
+    cases = [
+        (ninetoothed.make(programs.matmul.arrangement, programs.matmul.application, programs.matmul.tensors()), lambda: (normal(96, 64), normal(64, 80)), (96, 80), {}),
+        (ninetoothed.make(programs.addmm.arrangement, programs.addmm.application, programs.addmm.tensors()), lambda: (normal(96, 80), normal(96, 64), normal(64, 80), 0.5, 2), (96, 80), {}),
+        (ninetoothed.make(linear_arrangement, linear_application, (Tensor(2), Tensor(2), Tensor(1), Tensor(2))), lambda: (normal(96, 64), normal(80, 64).t(), normal(80)), (96, 80), {}),
+        (softmax, lambda: (normal(50, 333),), (50, 333), {"BLOCK_SIZE": 333}),
+        (attention, lambda: (normal(1, 2, 70, 64), normal(1, 2, 70, 64), normal(1, 2, 70, 64), True, 0.125), (1, 2, 70, 64), {}),
+        (conv2d, lambda: (normal(2, 32, 9, 9), normal(64, 32, 3, 3)), (2, 64, 9, 9), {"padding_h": 1, "padding_w": 1}),
+        (_add(), lambda: (normal(1000), 3.0), (1000,), {}),
+    ]
+    for kernel, make_inputs, shape, options in cases:
+        first_inputs, outputs = make_inputs(), []
+        for inputs in (first_inputs, make_inputs(), first_inputs):  # new buffers in between, then the first ones again
+            output = torch.full(shape, float("nan"), device="cuda", dtype=torch.float16)
+            kernel(*inputs, output, **options)
+            outputs.append(output)
+        assert len(kernel._prepared) == 1, kernel.kind
+        assert torch.equal(outputs[0], outputs[2]) and not torch.equal(outputs[0], outputs[1]) and not outputs[1].isnan().any(), kernel.kind
+        # a scalar of this call, and a stream of its own
+        stream = torch.cuda.Stream()
+        stream.wait_stream(torch.cuda.current_stream())
+        output = torch.full(shape, float("nan"), device="cuda", dtype=torch.float16)
+        stream.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(stream):
+            kernel(*first_inputs, output, **options)
+        stream.synchronize()
+        assert torch.equal(output, outputs[0]), kernel.kind
+    kernel = cases[-1][0]
+    values, output = normal(1000), normal(1000)
+    for scale in (2.0, -1.5, 0.75):
+        kernel(values, scale, output)
+        assert torch.equal(output, (values.float() * scale + 1).half())
+
+
+@pytest.mark.gpu
+def test_threads_share_a_kernel():
+    kernel = _add()
+    inputs = [torch.randn(5000, device="cuda") for _ in range(8)]
+    kernel(inputs[0], 1.0, torch.empty_like(inputs[0]))
+    failures = []
+
+    def work(index):
+        stream = torch.cuda.Stream()
+        with torch.cuda.stream(stream):
+            for round in range(50):
+                output = torch.empty_like(inputs[index])
+                kernel(inputs[index], float(index + round), output)
+                if not torch.equal(output, inputs[index] * float(index + round) + 1):
+                    failures.append((index, round))
+
+    torch.cuda.synchronize()
+    threads = [threading.Thread(target=work, args=(index,)) for index in range(8)]
+    for thread in threads:
+        thread.start()
+    for thread in threads:
+        thread.join()
+    assert not failures
+    del kernel
+    gc.collect()
