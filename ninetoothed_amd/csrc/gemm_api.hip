@@ -1189,10 +1189,11 @@ NineToothedResult nt_tune_gemm(NineToothedStream stream_, NineToothedTensor inpu
     const int preferred = heuristic_choice(q, 0, 0, 0);
     const float margin = preferred == kSkinny16 || preferred == kSkinny32 ? 0.25f : 0.02f;
     auto instance_of = [&](int i) { return preferred < 0 ? i : (i == 0 ? preferred : (i - 1 < preferred ? i - 1 : i)); };
-    // short products follow one another no faster than the host calls them, from Python about 6.2 us apart with one launch,
-    // 9.2 with the two of a split product (23 x 384 x 2112: 6.0 us split and 7.0 in one pass on the GPU, 10.8 and 7.7 in a program)
+    // short products follow one another no faster than the host calls them, from Python 3.5 us apart with one launch, 6.2 with the two of a
+    // split product.  (With 6.2 and 9.2, the host's part before repeated calls went past Python, instances between 3.6 and 6.2 us were
+    // alike: bf16 512^3 5.3 us a call on 32 tiles of 64 x 128, 3.7 on 64 of 64 x 64; 512 x 1024 x 512 5.2 and 3.8, 100 x 640 x 768 5.8 and 4.2.)
     float least_ms[kNumInstances];
-    for (int i = 0; i < kNumInstances; ++i) least_ms[i] = is_split(instance_of(i)) ? 0.0092f : 0.0062f;
+    for (int i = 0; i < kNumInstances; ++i) least_ms[i] = is_split(instance_of(i)) ? 0.0064f : 0.0036f;
     const int result = tune_time(stream, kNumInstances, iters, [&](int i) -> int {
         const int instance = instance_of(i);
         if (!kInstances[instance].accepts(q)) return NINETOOTHED_NO_KERNEL;
