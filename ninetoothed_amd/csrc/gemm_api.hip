@@ -970,7 +970,8 @@ int run_gemm(hipStream_t stream, const GemmProblem &q, int bm, int bn, int bk, b
     }
     int choice = -1;
     if ((bm <= 0 || bn <= 0) && q.batch == 1) choice = lookup_tuned(q);  // (tuned choices are recorded for single products)
-    if (choice < 0 || !kInstances[choice].accepts(q)) choice = heuristic_choice(q, bm, bn, bk);
+    // (choices are timed and recorded for the plain product, which the any-stride kernel may win; it has no linear epilogue)
+    if (choice < 0 || !kInstances[choice].accepts(q) || (choice == kAnyStride && q.linear)) choice = heuristic_choice(q, bm, bn, bk);
     if (choice < 0 || (choice == kAnyStride && q.linear)) return NINETOOTHED_NO_KERNEL;
     if (choice == kAnyStride && may_copy) {
         const int copied = run_gemm_on_repacked_copies(stream, q, bm, bn, bk);

@@ -152,3 +152,23 @@ def test_calls_that_stay_two_launches():
     output = lhs.clone()
     kernel(output, rhs, bias, output)
     _check(output, lhs, rhs, bias, lower=0)
+
+
+@pytest.mark.gpu
+def test_recorded_any_stride_choice(tmp_path, monkeypatch):
+    # the any-stride kernel, recorded as the fastest for the plain product, has no linear epilogue: the call stays one launch on
+    # the instance of the untuned rule
+    monkeypatch.setenv("NINETOOTHED_AMD_AUTOTUNE", "0")
+    lhs, rhs, bias = _operands(152, 344, 200, torch.bfloat16, False)
+    names, tag = runtime.gemm_config_names(), runtime.DATA_TYPE_INDEX["bf16"]
+    assert names[0].startswith("128x128x32 ") and "any-stride" in names[0]
+    path = tmp_path / "choices.csv"
+    path.write_text(f"\n{runtime.library().nt_tune_file_format()}\n0,{tag},{tag},152,344,200,0,0\n0,128,128,32\n")
+    runtime.check(runtime.library().nt_tune_cache_load(str(path).encode(), None))
+    assert runtime.library().nt_tune_cache_lookup(tag, tag, 152, 344, 200, 0) == 0
+    kernel = _linear()
+    for _ in range(2):
+        output = torch.full((152, 344), float("nan"), dtype=torch.bfloat16, device="cuda")
+        kernel(lhs, rhs, bias, output)
+        assert "gemm" in runtime.last_launch() and "any-stride" not in runtime.last_launch()
+        _check(output, lhs, rhs, bias, lower=0)
