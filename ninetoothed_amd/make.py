@@ -367,15 +367,17 @@ class Kernel:
             state["tune"] = auto_tuner.lookup(dtype, out_dtype, m, n, k, i is not None, rhs_layout) < 0
 
         def maybe_tune(call_args, input_arg, beta, alpha):
+            """Returns whether timing launches have written over the output."""
             state["tune"] = False
             out = call_args[c_pos]
             sources = [call_args[p] for p in (in_pos, a_pos, b_pos) if p is not None]
             # timing launches rewrite the output; skip when it overlaps an operand
             if any(t.untyped_storage().data_ptr() == out.untyped_storage().data_ptr() for t in sources):
-                return
+                return False
             instance, _ = auto_tuner.tune(input_arg, a_arg, b_arg, beta, alpha, c_arg, dtype, out_dtype)
             # inside a graph capture nothing is timed (-1): the next call outside one tunes; -2: nothing to choose from
             state["tune"] = instance == -1
+            return instance >= 0
 
         if i is not None:
             i_arg = runtime.ArgumentTensor.from_layout(0, (m, n), (i.row_stride, i.col_stride))  # (a stride of 0 is a broadcast here)
@@ -409,12 +411,12 @@ class Kernel:
             c_arg.data = call_args[c_pos].data_ptr() + c.base * out_itemsize
             if epilogue is not None:
                 result = epilogue(call_args, a_arg, b_arg, c_arg, blocks)
-                if result == runtime.NO_KERNEL:
-                    return False
                 if result == 0 and state["tune"]:
                     null = runtime.ArgumentTensor.null()
-                    maybe_tune(call_args, null, null, null)  # (the product's instance is the one that its epilogue rides on)
-                    result = epilogue(call_args, a_arg, b_arg, c_arg, blocks)
+                    if maybe_tune(call_args, null, null, null):  # (the product's instance is the one that its epilogue rides on)
+                        result = epilogue(call_args, a_arg, b_arg, c_arg, blocks)
+                if result == runtime.NO_KERNEL:
+                    return False
                 runtime.check(result)
                 return True
             if state["tune"]:

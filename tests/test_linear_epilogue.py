@@ -172,3 +172,44 @@ def test_recorded_any_stride_choice(tmp_path, monkeypatch):
         kernel(lhs, rhs, bias, output)
         assert "gemm" in runtime.last_launch() and "any-stride" not in runtime.last_launch()
         _check(output, lhs, rhs, bias, lower=0)
+
+
+# What a call of an untuned linear program asks of the library (a stand-in here, which only notes the entry points): `tuned` is
+# what the tuner answers -- an instance it has timed, -1 during a graph capture, -2 with nothing to choose from -- and `results`
+# what the linear entry point returns, call after call.
+@pytest.mark.parametrize(
+    "tuned, results, shared, expected",
+    (
+        (3, (0, 0), False, ["linear", "tune", "linear"]),  # timing wrote over the output
+        (-1, (0, 0), False, ["linear", "tune"]),  # a capture records one product
+        (-2, (0, 0), False, ["linear", "tune"]),
+        (3, (0, 0), True, ["linear"]),  # the output lies in an operand's storage: nothing is timed
+        (3, (runtime.NO_KERNEL,), False, ["linear", "tune", "matmul", "map"]),  # (the product of the two launches is tuned as well)
+        (3, (0, runtime.NO_KERNEL), False, ["linear", "tune", "linear", "tune", "matmul", "map"]),
+    ),
+)
+def test_launches_of_an_untuned_call(tuned, results, shared, expected, monkeypatch):
+    import types
+
+    from ninetoothed_amd import auto_tuner
+
+    asked, answers = [], list(results)
+
+    def note(name, answer=lambda: 0):
+        return lambda *args: (asked.append(name), answer())[1]
+
+    library = types.SimpleNamespace(launch_nt_linear=note("linear", lambda: answers.pop(0)), launch_nt_matmul=note("matmul"), launch_nt_map=note("map"))
+    monkeypatch.setattr(runtime, "library", lambda: library)
+    monkeypatch.setattr(runtime, "current_stream", lambda: None)
+    monkeypatch.setattr(auto_tuner, "enabled", lambda: True)
+    monkeypatch.setattr(auto_tuner, "load_once", lambda: None)
+    monkeypatch.setattr(auto_tuner, "lookup", lambda *args: -1)
+    monkeypatch.setattr(auto_tuner, "tune", note("tune", lambda: (tuned, 0.0)))
+    storage = torch.zeros(64 * 32 + 64 * 48, dtype=torch.float16)
+    output = storage[64 * 32 :].view(64, 48) if shared else torch.zeros(64, 48, dtype=torch.float16)
+    args = (storage[: 64 * 32].view(64, 32), torch.zeros(32, 48, dtype=torch.float16), torch.zeros(48, dtype=torch.float16), output)
+    kernel = _linear()
+    plan = kernel._prepare_gemm_epilogue(args, kernel._environment(args, {}, check_device=False))
+    plan(args)
+    assert asked == expected
+    assert plan.settled() == (tuned != -1 and "map" not in expected)
