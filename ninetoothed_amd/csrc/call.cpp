@@ -158,10 +158,33 @@ bool current_stream(void *&stream) {
 // (throws for a tensor whose memory may not be seen)
 char *address(PyObject *args, Py_ssize_t position) { return (char *)THPVariable_Unpack(PyTuple_GET_ITEM(args, position)).data_ptr(); }
 
-// The library's result; everything that is read from Python objects is read before the lock of the interpreter is let go
-// (a launch may wait for room in the stream's queue, and what makes room may be a Python callback).
-int launch(const Recipe &recipe, PyObject *args, void *stream) {
-    int result = 0;
+// The interpreter's lock is let go while this lives.
+struct Unlocked {
+    PyThreadState *state = PyEval_SaveThread();
+    ~Unlocked() { PyEval_RestoreThread(state); }
+};
+
+// Whether the library answered: `result` is its result.  (Where it ended with an exception a Python exception is set: whether
+// something has been launched is not known.)
+template <typename Call>
+bool in_library(Call call, int &result) {
+    bool answered = false;
+    {
+        Unlocked unlocked;
+        try {
+            result = call();
+            answered = true;
+        } catch (...) {
+        }
+    }
+    if (!answered) PyErr_SetString(PyExc_RuntimeError, "The launch ended with a C++ exception (out of host memory?).");
+    return answered;
+}
+
+// Whether the library answered; everything that is read from Python objects is read before the lock of the interpreter is let go
+// (a launch may wait for room in the stream's queue, and what makes room may be a Python callback).  Throws, with nothing
+// launched, what the tensors throw.
+bool launch(const Recipe &recipe, PyObject *args, void *stream, int &result) {
     if (recipe.kind == kMap) {
         std::vector<NineToothedMapProgram> programs;  // copies: other threads launch the same plan
         programs.reserve(recipe.launches.size());
@@ -171,13 +194,16 @@ int launch(const Recipe &recipe, PyObject *args, void *stream) {
             for (size_t slot = 0; slot < each.operands.size(); ++slot) program.operands[slot].data = address(args, each.operands[slot]);
             for (const auto &scalar : each.scalars) program.value_constants[scalar.first] = PyFloat_AsDouble(PyTuple_GET_ITEM(args, scalar.second));
         }
-        if (PyErr_Occurred()) return -1;
+        if (PyErr_Occurred()) return false;
         const auto function = (decltype(&launch_nt_map))recipe.function;
-        Py_BEGIN_ALLOW_THREADS
-        for (const NineToothedMapProgram &program : programs)
-            if (result == 0) result = function(stream, &program);
-        Py_END_ALLOW_THREADS
-        return result;
+        return in_library(
+            [&] {
+                int answer = 0;
+                for (const NineToothedMapProgram &program : programs)
+                    if (answer == 0) answer = function(stream, &program);
+                return answer;
+            },
+            result);
     }
     constexpr size_t kMaxSlots = 6;
     NineToothedTensor t[kMaxSlots];
@@ -200,24 +226,25 @@ int launch(const Recipe &recipe, PyObject *args, void *stream) {
     }
     double scale = recipe.doubles.empty() ? 1.0 : recipe.doubles[0];
     if (recipe.scale_position >= 0) scale = PyFloat_AsDouble(PyTuple_GET_ITEM(args, recipe.scale_position));
-    if (PyErr_Occurred()) return -1;
+    if (PyErr_Occurred()) return false;
     const int *n = recipe.ints.data();
     void *f = recipe.function;
-    Py_BEGIN_ALLOW_THREADS
-    switch (recipe.kind) {
-        case kMatmul: result = ((decltype(&launch_nt_matmul))f)(stream, t[0], t[1], t[2], n[0], n[1], n[2], n[3], n[4]); break;
-        case kAddmm: result = ((decltype(&launch_nt_addmm))f)(stream, t[0], t[1], t[2], t[3], t[4], t[5], n[0], n[1], n[2], n[3]); break;
-        case kLinear: result = ((decltype(&launch_nt_linear))f)(stream, t[0], t[1], t[2], n[0], scale, recipe.doubles[1], t[3], n[1], n[2], n[3], n[4]); break;
-        case kSoftmax: result = ((decltype(&launch_nt_softmax))f)(stream, t[0], t[1], n[0], n[1]); break;
-        case kAttention: result = ((decltype(&launch_nt_attention))f)(stream, t[0], t[1], t[2], t[3], t[4], t[5], n[0], n[1], n[2]); break;
-        case kConv2d: result = ((decltype(&launch_nt_conv2d))f)(stream, t[0], t[1], t[2], n[0], n[1], n[2], n[3], n[4], n[5]); break;
-        case kConv2dStrided:
-            result = ((decltype(&launch_nt_conv2d_strided))f)(stream, t[0], t[1], t[2], n[0], n[1], n[2], n[3], n[4], n[5], n[6], n[7], n[8], n[9]);
-            break;
-        case kMap: break;
-    }
-    Py_END_ALLOW_THREADS
-    return result;
+    return in_library(
+        [&]() -> int {
+            switch (recipe.kind) {
+                case kMatmul: return ((decltype(&launch_nt_matmul))f)(stream, t[0], t[1], t[2], n[0], n[1], n[2], n[3], n[4]);
+                case kAddmm: return ((decltype(&launch_nt_addmm))f)(stream, t[0], t[1], t[2], t[3], t[4], t[5], n[0], n[1], n[2], n[3]);
+                case kLinear: return ((decltype(&launch_nt_linear))f)(stream, t[0], t[1], t[2], n[0], scale, recipe.doubles[1], t[3], n[1], n[2], n[3], n[4]);
+                case kSoftmax: return ((decltype(&launch_nt_softmax))f)(stream, t[0], t[1], n[0], n[1]);
+                case kAttention: return ((decltype(&launch_nt_attention))f)(stream, t[0], t[1], t[2], t[3], t[4], t[5], n[0], n[1], n[2]);
+                case kConv2d: return ((decltype(&launch_nt_conv2d))f)(stream, t[0], t[1], t[2], n[0], n[1], n[2], n[3], n[4], n[5]);
+                case kConv2dStrided:
+                    return ((decltype(&launch_nt_conv2d_strided))f)(stream, t[0], t[1], t[2], n[0], n[1], n[2], n[3], n[4], n[5], n[6], n[7], n[8], n[9]);
+                case kMap: break;  // (above)
+            }
+            return NINETOOTHED_NO_KERNEL;
+        },
+        result);
 }
 
 // ---- module ----------------------------------------------------------------------------------------
@@ -258,8 +285,9 @@ PyObject *run(PyObject *, PyObject *const *arguments, Py_ssize_t given) {
     if (const Recipe *recipe = (const Recipe *)PyCapsule_GetPointer(PyTuple_GET_ITEM(entry, 0), kCapsule); recipe != nullptr && current_stream(stream)) {
         int result = -1;
         try {
-            result = launch(*recipe, args, stream);
+            (void)launch(*recipe, args, stream, result);
         } catch (...) {  // (nothing has been launched: the way through Python reports it)
+            PyErr_Clear();
         }
         if (!PyErr_Occurred()) {
             outcome = result == 0 ? PyTuple_GET_ITEM(entry, 1) : Py_None;

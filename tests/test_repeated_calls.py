@@ -1,6 +1,7 @@
 """Repeated calls take the way of csrc/call.cpp: the signature that it reads tells apart what the one in Python does, and calls
 that it does not know are left to Python."""
 
+import ctypes
 import gc
 import threading
 
@@ -62,6 +63,32 @@ def test_recipes_that_do_not_fit_are_refused():
         runtime.call_library().recipe("matmul", 1, (runtime.slot(0, layout),), (1, 2, 3, 4, 5), (), -1, ())
     with pytest.raises(ValueError):
         runtime.call_library().recipe("nothing", 1, (), (), (), -1, ())
+
+
+@pytest.fixture
+def no_gpu():
+    """The native module with stand-ins for torch's current device and stream."""
+    module = runtime.call_library()
+    module.use(lambda: 0, lambda device: 0)
+    yield module
+    module.use(torch._C._cuda_getDevice, torch._C._cuda_getCurrentRawStream)
+
+
+def _prepared(module, address):
+    """What a softmax kernel keeps of its first call, with a function of this test as the entry point."""
+    tensors = (torch.zeros(4, 6), torch.zeros(4, 6))
+    slots = tuple(runtime.slot(position, runtime.ArgumentTensor.like(tensor)) for position, tensor in enumerate(tensors))
+    recipe = module.recipe("softmax", address, slots, (runtime.DATA_TYPE_INDEX["fp32"], 6), (), -1, ())
+    return {module.signature(tensors, {}, b"tt"): (recipe, "the plan")}, tensors
+
+
+def test_an_exception_of_the_library_is_raised(no_gpu):
+    # (libstdc++'s own function that throws std::bad_alloc stands in for the library)
+    throws = ctypes.cast(ctypes.CDLL("libstdc++.so.6")._ZSt17__throw_bad_allocv, ctypes.c_void_p).value
+    prepared, tensors = _prepared(no_gpu, throws)
+    for _ in range(2):
+        with pytest.raises(RuntimeError, match="C\\+\\+ exception"):
+            no_gpu.run(prepared, tensors, {}, b"tt")
 
 
 def _add():
