@@ -5,7 +5,8 @@
 // point, layouts, constants -- and only the addresses and scalars of this call are filled in.
 //
 // Every call whose arguments are not ordinary strided tensors, numbers of the built-in types and integer keywords takes
-// the way through Python (None is returned), and so does the first call of a signature and a call that the library does not accept.
+// the way through Python (None is returned), and so does the first call of a signature and a linear program's whose operands that
+// entry point does not take.  Any other result of the library is raised here: what it may have launched is not launched again.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
@@ -142,6 +143,7 @@ bool read_signature(PyObject *args, PyObject *kwargs, const char *flags, Py_ssiz
 // ---- launches --------------------------------------------------------------------------------------
 
 PyObject *g_current_device = nullptr, *g_current_stream = nullptr;  // torch's own functions
+PyObject *g_check = nullptr;                                        // raises for a result that is not 0
 
 // the current stream of the current device, as torch has it for this thread
 bool current_stream(void *&stream) {
@@ -261,7 +263,7 @@ PyObject *signature(PyObject *, PyObject *arguments) {
 }
 
 // run(prepared, args, kwargs, flags) -> the plan that `prepared` ({signature: (recipe, plan)}) holds for these arguments, launched; None
-// when there is none, or the library did not take the call
+// when there is none, or nothing was launched because the linear entry point does not take the operands
 PyObject *run(PyObject *, PyObject *const *arguments, Py_ssize_t given) {
     if (given != 4 || !PyDict_CheckExact(arguments[0]) || !PyBytes_CheckExact(arguments[3])) {
         PyErr_SetString(PyExc_TypeError, "run(prepared, args, kwargs, flags)");
@@ -283,15 +285,24 @@ PyObject *run(PyObject *, PyObject *const *arguments, Py_ssize_t given) {
     PyObject *outcome = nullptr;
     void *stream = nullptr;
     if (const Recipe *recipe = (const Recipe *)PyCapsule_GetPointer(PyTuple_GET_ITEM(entry, 0), kCapsule); recipe != nullptr && current_stream(stream)) {
-        int result = -1;
+        int result = 0;
+        bool answered = false, thrown = false;
         try {
-            (void)launch(*recipe, args, stream, result);
+            answered = launch(*recipe, args, stream, result);
         } catch (...) {  // (nothing has been launched: the way through Python reports it)
+            thrown = true;
             PyErr_Clear();
         }
-        if (!PyErr_Occurred()) {
-            outcome = result == 0 ? PyTuple_GET_ITEM(entry, 1) : Py_None;
+        if (thrown || (answered && recipe->kind == kLinear && result == NINETOOTHED_NO_KERNEL)) {
+            outcome = Py_None;
             Py_INCREF(outcome);
+        } else if (answered && result == 0) {
+            outcome = PyTuple_GET_ITEM(entry, 1);
+            Py_INCREF(outcome);
+        } else if (answered) {
+            PyObject *raised = PyObject_CallFunction(g_check, "i", result);
+            if (raised != nullptr) PyErr_SetString(PyExc_SystemError, "a failed launch was not reported");
+            Py_XDECREF(raised);
         }
     }
     Py_DECREF(entry);
@@ -355,14 +366,16 @@ PyObject *make_recipe(PyObject *, PyObject *arguments) {
     return capsule;
 }
 
-// use(current_device, current_stream): the functions that say where a launch goes
+// use(current_device, current_stream, check): the functions that say where a launch goes, and the one that raises for a result
 PyObject *use(PyObject *, PyObject *arguments) {
-    PyObject *device, *stream;
-    if (!PyArg_ParseTuple(arguments, "OO", &device, &stream)) return nullptr;
+    PyObject *device, *stream, *check;
+    if (!PyArg_ParseTuple(arguments, "OOO", &device, &stream, &check)) return nullptr;
     Py_INCREF(device);
     Py_INCREF(stream);
+    Py_INCREF(check);
     Py_XSETREF(g_current_device, device);
     Py_XSETREF(g_current_stream, stream);
+    Py_XSETREF(g_check, check);
     Py_RETURN_NONE;
 }
 

@@ -150,7 +150,7 @@ CALL_LIBRARY_PATH = LIBRARY_PATH.with_name("nt_call.so")
 
 def run(prepared, args, kwargs, flags):
     """Launches what ``prepared`` (``{signature: (recipe, plan)}``) holds for these arguments and returns the plan; None where it
-    holds nothing, or the library did not take the call.  (The first call puts the native function in this one's place.)"""
+    holds nothing, or the linear entry point does not take the operands.  (The first call puts the native function in this one's place.)"""
     return call_library().run(prepared, args, kwargs, flags)
 
 
@@ -172,7 +172,7 @@ def call_library():
             loader = importlib.machinery.ExtensionFileLoader("nt_call", str(CALL_LIBRARY_PATH))
             module = importlib.util.module_from_spec(importlib.util.spec_from_loader("nt_call", loader))
             loader.exec_module(module)
-            module.use(torch._C._cuda_getDevice, torch._C._cuda_getCurrentRawStream)
+            module.use(torch._C._cuda_getDevice, torch._C._cuda_getCurrentRawStream, check)
             run = module.run
             _call_library = module
     return _call_library

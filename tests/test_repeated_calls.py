@@ -69,9 +69,9 @@ def test_recipes_that_do_not_fit_are_refused():
 def no_gpu():
     """The native module with stand-ins for torch's current device and stream."""
     module = runtime.call_library()
-    module.use(lambda: 0, lambda device: 0)
+    module.use(lambda: 0, lambda device: 0, runtime.check)
     yield module
-    module.use(torch._C._cuda_getDevice, torch._C._cuda_getCurrentRawStream)
+    module.use(torch._C._cuda_getDevice, torch._C._cuda_getCurrentRawStream, runtime.check)
 
 
 def _prepared(module, address):
@@ -80,6 +80,47 @@ def _prepared(module, address):
     slots = tuple(runtime.slot(position, runtime.ArgumentTensor.like(tensor)) for position, tensor in enumerate(tensors))
     recipe = module.recipe("softmax", address, slots, (runtime.DATA_TYPE_INDEX["fp32"], 6), (), -1, ())
     return {module.signature(tensors, {}, b"tt"): (recipe, "the plan")}, tensors
+
+
+_SOFTMAX = ctypes.CFUNCTYPE(ctypes.c_int, ctypes.c_void_p, runtime.ArgumentTensor, runtime.ArgumentTensor, ctypes.c_int, ctypes.c_int)
+
+
+@pytest.mark.parametrize("result", (0, 1, 2, 700))
+def test_a_launch_that_fails_is_not_repeated(no_gpu, result):
+    calls = []
+
+    def entry_point(stream, input, output, dtype, block):
+        calls.append((input.data, output.data, input.shape[1], output.strides[0], block))
+        return result
+
+    function = _SOFTMAX(entry_point)
+    prepared, tensors = _prepared(no_gpu, ctypes.cast(function, ctypes.c_void_p).value)
+    if result == 0:
+        assert no_gpu.run(prepared, tensors, {}, b"tt") == "the plan"
+    else:  # (a part of it may have run, or all of it with an error of an earlier launch reported here)
+        with pytest.raises(runtime.KernelLaunchError) as raised:
+            no_gpu.run(prepared, tensors, {}, b"tt")
+        assert raised.value.error_code == result
+    assert calls == [(tensors[0].data_ptr(), tensors[1].data_ptr(), 6, 6, 6)]
+
+
+_LINEAR = ctypes.CFUNCTYPE(
+    ctypes.c_int, ctypes.c_void_p, *(runtime.ArgumentTensor,) * 3, ctypes.c_int, ctypes.c_double, ctypes.c_double, runtime.ArgumentTensor, *(ctypes.c_int,) * 4
+)
+
+
+def test_linear_operands_that_are_not_taken_go_through_python(no_gpu):
+    results = [0, runtime.NO_KERNEL, 700]
+    function = _LINEAR(lambda *args: results.pop(0))
+    tensors = tuple(torch.zeros(8, 8) for _ in range(3))
+    lhs, rhs, output = (runtime.slot(position, runtime.ArgumentTensor.like(tensor)) for position, tensor in enumerate(tensors))
+    recipe = no_gpu.recipe("linear", ctypes.cast(function, ctypes.c_void_p).value, (lhs, rhs, None, output), (10, 8, 0, 0, 0), (1.0, 0.0), -1, ())
+    prepared = {no_gpu.signature(tensors, {}, b"ttt"): (recipe, "the plan")}
+    assert no_gpu.run(prepared, tensors, {}, b"ttt") == "the plan"
+    assert no_gpu.run(prepared, tensors, {}, b"ttt") is None
+    with pytest.raises(runtime.KernelLaunchError):
+        no_gpu.run(prepared, tensors, {}, b"ttt")
+    assert not results
 
 
 def test_an_exception_of_the_library_is_raised(no_gpu):
