@@ -1,5 +1,6 @@
 """Builds ``libnt_hip.so`` (the gfx950 kernels behind the C ABI) and ``libnt_probe.so`` (measurement kernels
-that only bench.py loads) in-tree with hipcc, and ``nt_call.so`` (the way from Python into the former) with g++.
+that only bench.py loads) in-tree with hipcc, and ``nt_call`` (the way from Python into the former, for the Python and the torch that
+build it) with the host's C++ compiler.
 
 Usage: ``python -m ninetoothed_amd.build_library`` or ``build_library()``.  The library
 is written to ``ninetoothed_amd/lib/libnt_hip.so``; object files go to
@@ -11,6 +12,7 @@ import pathlib
 import shutil
 import subprocess
 import sys
+import sysconfig
 
 PACKAGE_DIR = pathlib.Path(__file__).resolve().parent
 CSRC_DIR = PACKAGE_DIR / "csrc"
@@ -24,7 +26,7 @@ PROBE_LIBRARY_PATH = PACKAGE_DIR / "lib" / "libnt_probe.so"
 PROBE_SOURCES = ("probe.hip",)
 
 # The way of a repeated call from Python into the library: host code against torch's and Python's headers.
-CALL_LIBRARY_PATH = PACKAGE_DIR / "lib" / "nt_call.so"
+CALL_LIBRARY_PATH = PACKAGE_DIR / "lib" / ("nt_call" + sysconfig.get_config_var("EXT_SUFFIX"))
 CALL_SOURCE = "call.cpp"
 
 OFFLOAD_ARCH = "gfx950"
@@ -84,14 +86,13 @@ def build_library(verbose=False, extra_flags=()):
         temporary.replace(path)
 
     def compile_call():
-        import sysconfig
-
         import torch
 
         torch_dir = pathlib.Path(torch.__file__).resolve().parent
         temporary = CALL_LIBRARY_PATH.with_suffix(".so.tmp")
         command = [
-            shutil.which("g++") or "c++", "-O2", "-std=c++17", "-fPIC", "-shared", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}",
+            shutil.which("g++") or shutil.which("c++") or str(pathlib.Path(hipcc).with_name("amdclang++")), "-O2", "-std=c++17", "-fPIC", "-shared",
+            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}", f'-DNT_TORCH_VERSION="{torch.__version__}"',
             f"-I{torch_dir / 'include'}", f"-I{sysconfig.get_paths()['include']}", str(CSRC_DIR / CALL_SOURCE), "-o", str(temporary),
             f"-L{torch_dir / 'lib'}", "-lc10", "-ltorch_cpu", "-ltorch_python",
         ]  # fmt: skip

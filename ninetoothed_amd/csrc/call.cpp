@@ -391,4 +391,9 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "nt_call", nullptr, -1, methods, nu
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit_nt_call() { return PyModule_Create(&module); }
+PyMODINIT_FUNC PyInit_nt_call() {
+    PyObject *self = PyModule_Create(&module);
+    // (tensors are read through torch's own headers: their layout belongs to this version)
+    if (self != nullptr && PyModule_AddStringConstant(self, "torch_version", NT_TORCH_VERSION) != 0) Py_CLEAR(self);
+    return self;
+}

@@ -184,7 +184,8 @@ class Kernel:
         self.last_plan = plan.description
         plan(args)
         if plan.recipe is not None and plan.settled():
-            text = runtime.call_library().signature(args, kwargs, self._flags)
+            native = runtime.native_calls()
+            text = None if native is None else native.signature(args, kwargs, self._flags)
             if text is not None and text not in self._prepared:
                 self._prepared[text] = (plan.recipe(), plan)
 

@@ -12,7 +12,9 @@ library is missing, loading fails.
 
 import ctypes
 import pathlib
+import sysconfig
 import threading
+import warnings
 
 LIBRARY_PATH = pathlib.Path(__file__).resolve().parent / "lib" / "libnt_hip.so"
 
@@ -145,21 +147,31 @@ def library():
 
 # ---- the way of a repeated call (csrc/call.cpp) ----
 
-CALL_LIBRARY_PATH = LIBRARY_PATH.with_name("nt_call.so")
+# (Python's own suffix: a module that was built for another version of Python is not found)
+CALL_LIBRARY_PATH = LIBRARY_PATH.with_name("nt_call" + sysconfig.get_config_var("EXT_SUFFIX"))
 
 
 def run(prepared, args, kwargs, flags):
     """Launches what ``prepared`` (``{signature: (recipe, plan)}``) holds for these arguments and returns the plan; None where it
-    holds nothing, or the linear entry point does not take the operands.  (The first call puts the native function in this one's place.)"""
-    return call_library().run(prepared, args, kwargs, flags)
+    holds nothing, or the linear entry point does not take the operands.  (The first call puts the native function in this one's
+    place, or, where that cannot be loaded, one that leaves every call to Python.)"""
+    global run
+    module = native_calls()
+    run = _left_to_python if module is None else module.run
+    return run(prepared, args, kwargs, flags)
+
+
+def _left_to_python(prepared, args, kwargs, flags):
+    return None
 
 
 _call_library = None
+_call_library_failed = False
 
 
 def call_library():
-    """Loads ``nt_call.so`` once; raises if it has not been built."""
-    global _call_library, run
+    """Loads the module of repeated calls once; raises if it has not been built for this Python and this torch."""
+    global _call_library
     with _lock:
         if _call_library is None:
             import importlib.machinery
@@ -168,14 +180,29 @@ def call_library():
             import torch
 
             if not CALL_LIBRARY_PATH.exists():
-                raise RuntimeError(f"{CALL_LIBRARY_PATH} is missing: build it with `python -m ninetoothed_amd.build_library`.")
+                raise ImportError(f"{CALL_LIBRARY_PATH} is missing: build it with `python -m ninetoothed_amd.build_library`.")
             loader = importlib.machinery.ExtensionFileLoader("nt_call", str(CALL_LIBRARY_PATH))
             module = importlib.util.module_from_spec(importlib.util.spec_from_loader("nt_call", loader))
             loader.exec_module(module)
+            if module.torch_version != torch.__version__:
+                raise ImportError(f"{CALL_LIBRARY_PATH} was built against torch {module.torch_version}, this is {torch.__version__}: build it again.")
             module.use(torch._C._cuda_getDevice, torch._C._cuda_getCurrentRawStream, check)
-            run = module.run
             _call_library = module
     return _call_library
+
+
+def native_calls():
+    """The module of repeated calls, or None, with one warning, where it cannot be loaded: calls then go through Python, each as the
+    first one does (about 2 us more)."""
+    global _call_library_failed
+    if _call_library_failed:
+        return None
+    try:
+        return call_library()
+    except (ImportError, AttributeError) as error:  # (AttributeError: a torch without these accessors)
+        _call_library_failed = True
+        warnings.warn(f"Repeated calls go through Python: {error}", RuntimeWarning, stacklevel=4)
+        return None
 
 
 def recipe(kind, slots, ints, doubles=(), scale_position=-1, launches=()):

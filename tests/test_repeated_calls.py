@@ -4,6 +4,7 @@ that it does not know are left to Python."""
 import ctypes
 import gc
 import threading
+import types
 
 import pytest
 import torch
@@ -11,6 +12,9 @@ import torch
 import ninetoothed_amd as ninetoothed
 import ninetoothed_amd.language as ntl
 from ninetoothed_amd import Tensor, programs, runtime
+
+
+_FIRST_RUN = runtime.run  # (as it is before the first call)
 
 
 def _signature(*args, flags=b"ttt", **kwargs):
@@ -130,6 +134,31 @@ def test_an_exception_of_the_library_is_raised(no_gpu):
     for _ in range(2):
         with pytest.raises(RuntimeError, match="C\\+\\+ exception"):
             no_gpu.run(prepared, tensors, {}, b"tt")
+
+
+@pytest.mark.parametrize("reason", ("missing", "no library", "another torch", "no accessors"))
+def test_calls_go_through_python_without_the_module(reason, tmp_path, monkeypatch):
+    monkeypatch.setattr(runtime, "_call_library", None)
+    monkeypatch.setattr(runtime, "_call_library_failed", False)
+    monkeypatch.setattr(runtime, "run", runtime.run)  # (put back afterwards)
+    monkeypatch.setattr(runtime, "run", _FIRST_RUN)
+    if reason in ("missing", "no library"):
+        path = tmp_path / runtime.CALL_LIBRARY_PATH.name
+        if reason == "no library":
+            path.write_bytes(b"text")
+        monkeypatch.setattr(runtime, "CALL_LIBRARY_PATH", path)
+    elif reason == "another torch":
+        monkeypatch.setattr(torch, "__version__", "1.0")
+    else:
+        monkeypatch.delattr(torch._C, "_cuda_getDevice")
+    kernel = _add()
+    ran = []
+    plan = types.SimpleNamespace(description="the plan", recipe=lambda: ran.append("recipe"), settled=lambda: True)
+    monkeypatch.setattr(kernel, "_prepare", lambda args, kwargs: type("Plan", (types.SimpleNamespace,), {"__call__": lambda self, args: ran.append("launch")})(**vars(plan)))
+    with pytest.warns(RuntimeWarning, match="through Python") as warned:
+        for _ in range(3):
+            kernel(torch.zeros(4), 1.0, torch.zeros(4))
+    assert ran == ["launch"] * 3 and kernel.last_plan == "the plan" and len(warned) == 1
 
 
 def _add():
