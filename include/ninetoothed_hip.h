@@ -361,6 +361,22 @@ NineToothedResult nt_tune_gemm(NineToothedStream stream,
                                int dtype, int output_dtype, int iters,
                                int *best_config, float *best_ms);
 
+/* As nt_tune_gemm for a program whose calls follow one another no faster than every `call_ms`, or `split_call_ms` where an instance
+ * takes two launches (K in parts): an instance counts for at least that in the comparison, and among those that count for the same the
+ * one the GPU runs faster is taken.  (So such a program is not given two launches that its own pace would show; a program that
+ * replays captured launches, or calls faster, wants nt_tune_gemm, which is this with 0 and 0.)  *best_ms is the time
+ * measured all the same.  There is one record per problem: the latest call's. */
+NineToothedResult nt_tune_gemm_for_caller(NineToothedStream stream,
+                                          NineToothedTensor input,
+                                          NineToothedTensor mat1,
+                                          NineToothedTensor mat2,
+                                          NineToothedTensor beta,
+                                          NineToothedTensor alpha,
+                                          NineToothedTensor output,
+                                          int dtype, int output_dtype, int iters,
+                                          float call_ms, float split_call_ms,
+                                          int *best_config, float *best_ms);
+
 /* As nt_tune_gemm for launch_nt_attention: times its loop variants (0 plain 64-key blocks; 1 256 query rows per
  * workgroup; 2 32-key blocks; 3 software-pipelined; 4 software-pipelined with eight waves) on the given tensors the
  * same way and records the fastest for later launches of the same problem (element type, batch, heads, both

@@ -29,6 +29,10 @@ from ninetoothed_amd import runtime
 # descriptions) away from the home directory
 CACHE_DIR = pathlib.Path(os.environ.get("NINETOOTHED_AMD_CACHE_DIR") or pathlib.Path.home() / ".ninetoothed_amd") / "auto_tuning"
 
+# What a call through `make` costs the host, with one launch and with the two of a product whose K is in parts: calls of one program follow
+# one another no faster.  (An instance of 4 us in two launches against one of 5 us in one: 6.2 and 5 us a call.)
+CALL_MS, SPLIT_CALL_MS = 0.0035, 0.0062
+
 _lock = threading.Lock()
 _loaded = False
 
@@ -98,13 +102,15 @@ def tune_conv2d(x, w, y, dtype, padding_h, padding_w, iters=5):
 
 def tune(input, mat1, mat2, beta, alpha, output, dtype, out_dtype, iters=5):
     """Times the instances on these arguments (:class:`runtime.ArgumentTensor`), records the
-    winner in the library and on disk.  Returns ``(instance, milliseconds)``; the instance is -1
+    winner at the pace of calls from Python in the library and on disk.  Returns ``(instance, milliseconds)``; the instance is -1
     when the stream is being captured into a graph (nothing is timed or recorded then) and -2
     when a single instance takes the problem (nothing to time)."""
     lib = runtime.library()
     best, best_ms = ctypes.c_int(-1), ctypes.c_float(0.0)
     runtime.check(
-        lib.nt_tune_gemm(runtime.current_stream(), input, mat1, mat2, beta, alpha, output, dtype, out_dtype, iters, ctypes.byref(best), ctypes.byref(best_ms))
+        lib.nt_tune_gemm_for_caller(
+            runtime.current_stream(), input, mat1, mat2, beta, alpha, output, dtype, out_dtype, iters, CALL_MS, SPLIT_CALL_MS, ctypes.byref(best), ctypes.byref(best_ms)
+        )
     )
     if best.value < 0:  # nothing was timed: the stream is being captured into a graph
         return best.value, best_ms.value

@@ -1145,10 +1145,10 @@ NineToothedResult launch_nt_gemm_config(NineToothedStream stream, int config, Ni
     return (int)kInstances[config].launch(q, (hipStream_t)stream);
 }
 
-NineToothedResult nt_tune_gemm(NineToothedStream stream_, NineToothedTensor input, NineToothedTensor mat1,
-                               NineToothedTensor mat2, NineToothedTensor beta, NineToothedTensor alpha,
-                               NineToothedTensor output, int dtype, int output_dtype, int iters, int *best_config,
-                               float *best_ms) {
+NineToothedResult nt_tune_gemm_for_caller(NineToothedStream stream_, NineToothedTensor input, NineToothedTensor mat1,
+                                          NineToothedTensor mat2, NineToothedTensor beta, NineToothedTensor alpha,
+                                          NineToothedTensor output, int dtype, int output_dtype, int iters, float call_ms,
+                                          float split_call_ms, int *best_config, float *best_ms) {
     hipStream_t stream = (hipStream_t)stream_;
     GemmProblem given;
     if (int err = build_problem(given, &input, mat1, mat2, &beta, &alpha, output, dtype, output_dtype)) return err;
@@ -1190,16 +1190,11 @@ NineToothedResult nt_tune_gemm(NineToothedStream stream_, NineToothedTensor inpu
     const int preferred = heuristic_choice(q, 0, 0, 0);
     const float margin = preferred == kSkinny16 || preferred == kSkinny32 ? 0.25f : 0.02f;
     auto instance_of = [&](int i) { return preferred < 0 ? i : (i == 0 ? preferred : (i - 1 < preferred ? i - 1 : i)); };
-    // short products follow one another no faster than the host calls them, from Python 3.5 us apart with one launch, 6.2 with the two of a
-    // split product.  (With 6.2 and 9.2, the host's part before repeated calls went past Python, instances between 3.6 and 6.2 us were
-    // alike: bf16 512^3 5.3 us a call on 32 tiles of 64 x 128, 3.7 on 64 of 64 x 64; 512 x 1024 x 512 5.2 and 3.8, 100 x 640 x 768 5.8 and 4.2.)
-    float least_ms[kNumInstances];
-    for (int i = 0; i < kNumInstances; ++i) least_ms[i] = is_split(instance_of(i)) ? 0.0064f : 0.0036f;
     const int result = tune_time(stream, kNumInstances, iters, [&](int i) -> int {
         const int instance = instance_of(i);
         if (!kInstances[instance].accepts(q)) return NINETOOTHED_NO_KERNEL;
         return (int)kInstances[instance].launch(q, stream);
-    }, &best, &best_time, margin, least_ms);
+    }, &best, &best_time, margin, [&](int i, float measured) { return std::max(measured, is_split(instance_of(i)) ? split_call_ms : call_ms); });
     if (best >= 0) best = instance_of(best);
     if (best_config) *best_config = best;
     if (best_ms) *best_ms = best_time;
@@ -1210,6 +1205,13 @@ NineToothedResult nt_tune_gemm(NineToothedStream stream_, NineToothedTensor inpu
     const int blocks[3] = {kInstances[best].bm, kInstances[best].bn, kInstances[best].bk};
     tune_record(kTuneGemm, values, 7, best, blocks, 3);
     return 0;
+}
+
+NineToothedResult nt_tune_gemm(NineToothedStream stream, NineToothedTensor input, NineToothedTensor mat1,
+                               NineToothedTensor mat2, NineToothedTensor beta, NineToothedTensor alpha,
+                               NineToothedTensor output, int dtype, int output_dtype, int iters, int *best_config,
+                               float *best_ms) {
+    return nt_tune_gemm_for_caller(stream, input, mat1, mat2, beta, alpha, output, dtype, output_dtype, iters, 0.0f, 0.0f, best_config, best_ms);
 }
 
 // The cached instance for a problem given by its sizes (row-major rhs), or -1.

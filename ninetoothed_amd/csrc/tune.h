@@ -9,6 +9,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include "choose.h"
+
 namespace nt {
 
 enum TuneKind { kTuneGemm = 0, kTuneAttention = 1, kTuneConv2d = 2, kTuneKinds };
@@ -46,13 +48,17 @@ void note_launch(int program, int choice, const char *name);
 // every candidate over a region of about 3 ms (at least one launch, at most 256) -- and a candidate's figure is the
 // minimum of its rounds, so that a slow spell has to hit the same candidate in every round to mislead.
 // Candidates are in order of preference: with a `margin`, a later candidate replaces an earlier one only when it
-// is faster by more than that fraction; `least_ms` (per candidate) is what a call costs its program whatever the GPU does.
-// *best = -1 when none ran.
+// is faster by more than that fraction; `counted(i, ms)` is what candidate i counts for in this comparison (choose.h), and
+// *best_ms what was measured.  *best = -1 when none ran.
 // Synchronises; returns without timing anything (*best = -1, result 0) when the stream is being captured into a graph.
 constexpr int kTuneMaxCandidates = 64;
 
-template <typename Launch>
-int tune_time(hipStream_t stream, int candidates, int iters, Launch launch, int *best, float *best_ms, float margin = 0.0f, const float *least_ms = nullptr) {
+struct CountedAsMeasured {
+    float operator()(int, float measured) const { return measured; }
+};
+
+template <typename Launch, typename Counted = CountedAsMeasured>
+int tune_time(hipStream_t stream, int candidates, int iters, Launch launch, int *best, float *best_ms, float margin = 0.0f, Counted counted = Counted()) {
     *best = -1;
     *best_ms = 0.0f;
     hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
@@ -116,16 +122,12 @@ int tune_time(hipStream_t stream, int candidates, int iters, Launch launch, int 
                 if (result == 0 && (round == 0 || one < fastest[c])) fastest[c] = one;
             }
         }
-        for (int c = 0; c < alive && result == 0; ++c) {
-            if (least_ms != nullptr && fastest[c] < least_ms[live[c]]) fastest[c] = least_ms[live[c]];
-            if (*best < 0 || fastest[c] < *best_ms * (1.0f - margin)) {
-                *best = live[c];
-                *best_ms = fastest[c];
-            }
-        }
-        if (result != 0) {
-            *best = -1;
-            *best_ms = 0.0f;
+        if (result == 0) {
+            float figures[kTuneMaxCandidates];
+            for (int c = 0; c < alive; ++c) figures[c] = counted(live[c], fastest[c]);
+            const int chosen = choose(fastest, figures, alive, margin);
+            *best = live[chosen];
+            *best_ms = fastest[chosen];
         }
     }
     (void)hipEventDestroy(start);

@@ -102,6 +102,7 @@ _SIGNATURES = {
     "launch_nt_conv2d_strided": (_S, _T, _T, _T, _I, _I, _I, _I, _I, _I, _I, _I, _I, _I),
     "launch_nt_gemm_config": (_S, _I, _T, _T, _T, _T, _T, _T, _I, _I),
     "nt_tune_gemm": (_S, _T, _T, _T, _T, _T, _T, _I, _I, _I, ctypes.POINTER(ctypes.c_int), ctypes.POINTER(ctypes.c_float)),
+    "nt_tune_gemm_for_caller": (_S, _T, _T, _T, _T, _T, _T, _I, _I, _I, ctypes.c_float, ctypes.c_float, ctypes.POINTER(ctypes.c_int), ctypes.POINTER(ctypes.c_float)),
     "nt_tune_attention": (_S, _T, _T, _T, _T, _T, _T, _I, _I, ctypes.POINTER(ctypes.c_int), ctypes.POINTER(ctypes.c_float)),
     "nt_tune_conv2d": (_S, _T, _T, _T, _I, _I, _I, _I, ctypes.POINTER(ctypes.c_int), ctypes.POINTER(ctypes.c_float)),
     "nt_tune_lookup": (_I, ctypes.POINTER(ctypes.c_int), _I),

@@ -1,0 +1,70 @@
+"""Which candidate the tuner takes, from figures of this test, and what nt_tune_gemm answers."""
+
+import ctypes
+import pathlib
+import shutil
+import struct
+import subprocess
+
+import pytest
+import torch
+
+from ninetoothed_amd import runtime
+
+CSRC = pathlib.Path(__file__).resolve().parent.parent / "ninetoothed_amd" / "csrc"
+
+
+@pytest.fixture(scope="module")
+def choose(tmp_path_factory):
+    compiler = shutil.which("g++") or shutil.which("c++")
+    if compiler is None:
+        pytest.skip("no C++ compiler on this host")
+    folder = tmp_path_factory.mktemp("choose")
+    (folder / "choose.cpp").write_text(
+        '#include "choose.h"\nextern "C" int choose(const float *measured, const float *counted, int count, float margin) { return nt::choose(measured, counted, count, margin); }\n'
+    )
+    subprocess.run([compiler, "-std=c++17", "-shared", "-fPIC", f"-I{CSRC}", str(folder / "choose.cpp"), "-o", str(folder / "choose.so")], check=True)
+    function = ctypes.CDLL(str(folder / "choose.so")).choose
+
+    def call(measured, counted=None, margin=0.02):
+        array = ctypes.c_float * len(measured)
+        return function(array(*measured), array(*(counted or measured)), len(measured), ctypes.c_float(margin))
+
+    return call
+
+
+def test_a_later_candidate_needs_the_margin(choose):
+    assert choose([]) == -1
+    assert choose([5.0, 4.95, 6.0]) == 0
+    assert choose([5.0, 4.85, 4.8]) == 1  # (2 % of the one that stands)
+    assert choose([5.0, 4.0], margin=0.25) == 0
+
+
+def test_candidates_at_the_callers_pace(choose):
+    # one launch counts for 3.5 at least, two for 6.2: positions 0 and 1 take one launch, 2 two
+    def paced(*measured):
+        return choose(measured, [max(ms, 6.2 if position == 2 else 3.5) for position, ms in enumerate(measured)])
+
+    assert paced(3.4, 2.0, 9.0) == 1  # alike for the caller: the GPU's time decides
+    assert paced(2.0, 3.4, 9.0) == 0
+    assert paced(5.0, 8.0, 4.0) == 0  # two launches would show
+    assert paced(8.0, 9.0, 4.0) == 2
+    assert paced(7.0, 9.0, 6.9) == 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m, n, k", ((64, 64, 64), (64, 256, 4096)))
+def test_measured_times_come_back(m, n, k):
+    # short products, timed for a caller of any pace: what comes back is a launch's time, not the pace
+    tag, library = runtime.DATA_TYPE_INDEX["bf16"], runtime.library()
+    lhs, rhs, out = (torch.randn(shape, device="cuda", dtype=torch.bfloat16) for shape in ((m, k), (k, n), (m, n)))
+    arguments = [runtime.ArgumentTensor.null()] + [runtime.ArgumentTensor.from_torch_tensor(t) for t in (lhs, rhs)] + [runtime.ArgumentTensor.null()] * 2
+    best, milliseconds = ctypes.c_int(-1), ctypes.c_float(0.0)
+    answer = (ctypes.byref(best), ctypes.byref(milliseconds))
+    output = runtime.ArgumentTensor.from_torch_tensor(out)
+    runtime.check(library.nt_tune_gemm(runtime.current_stream(), *arguments, output, tag, tag, 5, *answer))
+    for pace in (0.0036, 0.0064):  # (as 32-bit floats: no measured time is one of them but by chance)
+        assert best.value >= 0 and 0 < milliseconds.value < 1 and milliseconds.value != struct.unpack("f", struct.pack("f", pace))[0]
+    runtime.check(library.nt_tune_gemm_for_caller(runtime.current_stream(), *arguments, output, tag, tag, 5, 10.0, 20.0, *answer))
+    assert best.value >= 0 and 0 < milliseconds.value < 1
+    assert "tails split-k" not in runtime.gemm_config_names()[best.value]  # (its two launches count for twice as much there)
