@@ -182,7 +182,7 @@ class Kernel:
         if plan is None:
             plan = self._plans[key] = self._prepare(args, kwargs)
         self.last_plan = plan.description
-        plan(args)
+        self.last_plan = plan(args) or plan.description
         if plan.recipe is not None and plan.settled():
             native = runtime.native_calls()
             text = None if native is None else native.signature(args, kwargs, self._flags)
@@ -583,7 +583,7 @@ class Kernel:
         def launch(call_args):
             taken["linear"] = linear is not None and linear.launch(call_args)
             if taken["linear"]:
-                return
+                return None
             extended = with_scratch(call_args)  # from torch's stream-ordered allocator: free again once both launches are queued
             gemm(extended)
             for slot, param in enumerate(operand_params):
@@ -591,12 +591,13 @@ class Kernel:
             for index, param in scalar_slots:
                 program.value_constants[index] = float(extended[param])
             runtime.check(lib.launch_nt_map(runtime.current_stream(), ctypes.addressof(program)))
+            return two_passes
 
         self._map_programs = [program]
         two_passes = f"{gemm.description}; launch_nt_map {description}"
         if linear is None:
             return _Plan(two_passes, launch)
-        return _Plan(f"launch_nt_linear, or {two_passes}", launch, linear.recipe, lambda: taken["linear"] and linear.settled())
+        return _Plan(linear.description, launch, linear.recipe, lambda: taken["linear"] and linear.settled())
 
     def _linear_launch(self, info, args, env, tag):
         """``max(product * scale + bias[None, :], lower)`` in one launch: a plan whose `launch` says whether
@@ -637,6 +638,7 @@ class Kernel:
             return runtime.recipe("linear", (lhs, rhs, bias, output), (bias_dtype, dtype, *blocks), doubles, -1 if scale_pos is None else scale_pos)
 
         plan.recipe = recipe
+        plan.description = f"launch_nt_linear {m}x{n}x{k} {tag} blocks {blocks}"
         return plan
 
     def _prepare_attention(self, args, env):
@@ -725,5 +727,6 @@ class _Plan:
         self._lock = threading.Lock()
 
     def __call__(self, args):
+        """Returns a description of what ran where that is not the plan's own."""
         with self._lock:
-            self.launch(args)
+            return self.launch(args)

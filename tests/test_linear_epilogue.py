@@ -103,7 +103,7 @@ def test_bias_and_bound_in_one_launch(m, n, k, transposed, tuned, dtype, monkeyp
     for _ in range(2):  # (the first call is the one that times the instances)
         output = torch.full((m, n), float("nan"), dtype=dtype, device="cuda")
         kernel(lhs, rhs, bias, output)
-        assert "gemm" in runtime.last_launch()
+        assert "gemm" in runtime.last_launch() and kernel.last_plan.startswith("launch_nt_linear")
         _check(output, lhs, rhs, bias, lower=0)
 
 
@@ -146,7 +146,7 @@ def test_calls_that_stay_two_launches():
         lhs, rhs, bias = _operands(m, n, k, torch.bfloat16, False)
         output = torch.empty(n, m, dtype=torch.bfloat16, device="cuda").t() if columns else torch.empty(m, n, dtype=torch.bfloat16, device="cuda")
         kernel(lhs, rhs, bias, output)
-        assert "gemm" not in runtime.last_launch()
+        assert "gemm" not in runtime.last_launch() and kernel.last_plan.startswith("launch_nt_matmul") and "launch_nt_map" in kernel.last_plan
         _check(output, lhs, rhs, bias, lower=0)
     lhs, rhs, bias = _operands(256, 256, 256, torch.bfloat16, False)  # an operand that is the output
     output = lhs.clone()
@@ -210,6 +210,7 @@ def test_launches_of_an_untuned_call(tuned, results, shared, expected, monkeypat
     args = (storage[: 64 * 32].view(64, 32), torch.zeros(32, 48, dtype=torch.float16), torch.zeros(48, dtype=torch.float16), output)
     kernel = _linear()
     plan = kernel._prepare_gemm_epilogue(args, kernel._environment(args, {}, check_device=False))
-    plan(args)
+    ran = plan(args) or plan.description
     assert asked == expected
+    assert ("launch_nt_linear" in ran, "launch_nt_matmul" in ran, "launch_nt_map" in ran) == ((False, True, True) if "map" in expected else (True, False, False))
     assert plan.settled() == (tuned != -1 and "map" not in expected)
