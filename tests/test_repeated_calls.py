@@ -2,6 +2,7 @@
 that it does not know are left to Python."""
 
 import ctypes
+import functools
 import gc
 import threading
 import types
@@ -182,42 +183,71 @@ def test_each_entry_point_repeats_what_its_first_call_does():
             accumulator += ntl.dot(lhs[k], rhs[k])
         output = ntl.maximum(accumulator + bias[None, :], 0)  # noqa: F841
 
+    def scaled_application(lhs, rhs, bias, scale, output):
+        accumulator = ntl.zeros(output.shape, dtype=ntl.float32)
+        for k in range(lhs.shape[0]):
+            accumulator += ntl.dot(lhs[k], rhs[k])
+        output = scale * accumulator + bias[None, :]  # noqa: F841
+
     def linear_arrangement(lhs, rhs, bias, output, BM=ninetoothed.block_size(), BN=ninetoothed.block_size(), BK=ninetoothed.block_size()):
         lhs_arranged, rhs_arranged, output_arranged = programs.matmul.arrangement(lhs, rhs, output, BM, BN, BK)
         return lhs_arranged, rhs_arranged, bias.tile((BN,)).unsqueeze(0).expand((output_arranged.shape[0], -1)), output_arranged
 
-    attention = ninetoothed.make(programs.attention.arrangement_with_scale, programs.attention.application_with_scale, programs.attention.tensors(True))
+    def scaled_arrangement(lhs, rhs, bias, scale, output, BM=ninetoothed.block_size(), BN=ninetoothed.block_size(), BK=ninetoothed.block_size()):
+        *inputs, output_arranged = linear_arrangement(lhs, rhs, bias, output, BM, BN, BK)
+        return *inputs, scale, output_arranged
+
+    scaled_attention = ninetoothed.make(programs.attention.arrangement_with_scale, programs.attention.application_with_scale, programs.attention.tensors(True))
+    attention = ninetoothed.make(programs.attention.arrangement, programs.attention.application, programs.attention.tensors())
     conv2d = ninetoothed.make(programs.conv2d.arrangement, programs.conv2d.application, programs.conv2d.tensors())
+    strided = ninetoothed.make(functools.partial(programs.conv2d.arrangement, stride=(2, 2), floor_mode=True), programs.conv2d.application, programs.conv2d.tensors())
     softmax = ninetoothed.make(programs.softmax.arrangement, programs.softmax.application, programs.softmax.tensors())
+    qkv = lambda: tuple(normal(1, 2, 70, 64) for _ in range(3))  # noqa: E731
     cases = [
         (ninetoothed.make(programs.matmul.arrangement, programs.matmul.application, programs.matmul.tensors()), lambda: (normal(96, 64), normal(64, 80)), (96, 80), {}),
         (ninetoothed.make(programs.addmm.arrangement, programs.addmm.application, programs.addmm.tensors()), lambda: (normal(96, 80), normal(96, 64), normal(64, 80), 0.5, 2), (96, 80), {}),
         (ninetoothed.make(linear_arrangement, linear_application, (Tensor(2), Tensor(2), Tensor(1), Tensor(2))), lambda: (normal(96, 64), normal(80, 64).t(), normal(80)), (96, 80), {}),
+        (
+            ninetoothed.make(scaled_arrangement, scaled_application, (Tensor(2), Tensor(2), Tensor(1), Tensor(0), Tensor(2))),
+            lambda: (normal(96, 64), normal(80, 64).t(), normal(80), float(torch.rand(())) + 0.5), (96, 80), {},
+        ),
         (softmax, lambda: (normal(50, 333),), (50, 333), {"BLOCK_SIZE": 333}),
-        (attention, lambda: (normal(1, 2, 70, 64), normal(1, 2, 70, 64), normal(1, 2, 70, 64), True, 0.125), (1, 2, 70, 64), {}),
+        (scaled_attention, lambda: (*qkv(), True, 0.125), (1, 2, 70, 64), {}),
+        (attention, lambda: (*qkv(), True), (1, 2, 70, 64), {}),
         (conv2d, lambda: (normal(2, 32, 9, 9), normal(64, 32, 3, 3)), (2, 64, 9, 9), {"padding_h": 1, "padding_w": 1}),
+        (strided, lambda: (normal(2, 32, 9, 9), normal(64, 32, 3, 3)), (2, 64, 5, 5), {"padding_h": 1, "padding_w": 1}),
         (_add(), lambda: (normal(1000), 3.0), (1000,), {}),
-    ]
+    ]  # fmt: skip
+
+    def fresh(shape):
+        return torch.full(shape, float("nan"), device="cuda", dtype=torch.float16)
+
     for kernel, make_inputs, shape, options in cases:
-        first_inputs, outputs = make_inputs(), []
-        for inputs in (first_inputs, make_inputs(), first_inputs):  # new buffers in between, then the first ones again
-            output = torch.full(shape, float("nan"), device="cuda", dtype=torch.float16)
-            kernel(*inputs, output, **options)
-            outputs.append(output)
+        # each call's result through Python, then the same calls without a way back to Python
+        all_inputs = [make_inputs(), make_inputs()]
+        expected = []
+        for inputs in all_inputs:
+            expected.append(fresh(shape))
+            kernel._call((*inputs, expected[-1]), options)
         assert len(kernel._prepared) == 1, kernel.kind
-        assert torch.equal(outputs[0], outputs[2]) and not torch.equal(outputs[0], outputs[1]) and not outputs[1].isnan().any(), kernel.kind
-        # a scalar of this call, and a stream of its own
-        stream = torch.cuda.Stream()
-        stream.wait_stream(torch.cuda.current_stream())
-        output = torch.full(shape, float("nan"), device="cuda", dtype=torch.float16)
+        assert not torch.equal(*expected) and not any(output.isnan().any() for output in expected), kernel.kind
+        ((_, plan),) = kernel._prepared.values()
+        for round in range(2):  # new buffers each time
+            for inputs, result in zip(all_inputs, expected):
+                output = fresh(shape)
+                assert runtime.run(kernel._prepared, (*inputs, output), options, kernel._flags) is plan, kernel.kind
+                assert torch.equal(output, result), kernel.kind
+        kernel._call = None  # (a call that went through Python would raise)
+        output = fresh(shape)
+        stream = torch.cuda.Stream()  # a stream of its own
         stream.wait_stream(torch.cuda.current_stream())
         with torch.cuda.stream(stream):
-            kernel(*first_inputs, output, **options)
+            kernel(*all_inputs[0], output, **options)
         stream.synchronize()
-        assert torch.equal(output, outputs[0]), kernel.kind
+        assert torch.equal(output, expected[0]) and kernel.last_plan == plan.description, kernel.kind
     kernel = cases[-1][0]
     values, output = normal(1000), normal(1000)
-    for scale in (2.0, -1.5, 0.75):
+    for scale in (2.0, -1.5, 0.75):  # a scalar of this call
         kernel(values, scale, output)
         assert torch.equal(output, (values.float() * scale + 1).half())
 
