@@ -6,6 +6,10 @@
 
 namespace nt {
 
+// the ways to run a convolution; kConvAuto tries them from the top (a 1 x 1 filter without padding first runs
+// as a batch of plain products when it can)
+enum ConvPath { kConvAuto = 0, kConvGather = 1, kConvRepack = 2, kConvDirect = 3, kConvPointwise = 4 };
+
 struct Conv2dRequest {
     int dtype;
     const void *x;

@@ -36,6 +36,7 @@
 
 #include "conv2d.h"
 #include "gemm_fast.h"
+#include "tune.h"
 #include "workspace.h"
 
 namespace nt {
@@ -1185,8 +1186,14 @@ int run_direct(const Conv2dRequest &q, hipStream_t stream) {
 struct ConvTile {
     int m, n;
     float alone, shared;
+    const char *name;  // of a launch
 };
-constexpr ConvTile kConvTiles[] = {{128, 128, 0.28f, 0.21f}, {128, 64, 0.19f, 0.19f}, {64, 128, 0.205f, 0.14f}, {64, 64, 0.145f, 0.107f}, {256, 64, 0.39f, 0.235f}};
+#define NT_CONV_NAME(TILE) "conv2d_repack_kernel, then conv2d_nhwc_kernel on channels-last copies, tiles of " TILE
+constexpr ConvTile kConvTiles[] = {
+    {128, 128, 0.28f, 0.21f, NT_CONV_NAME("128x128")}, {128, 64, 0.19f, 0.19f, NT_CONV_NAME("128x64")}, {64, 128, 0.205f, 0.14f, NT_CONV_NAME("64x128")},
+    {64, 64, 0.145f, 0.107f, NT_CONV_NAME("64x64")}, {256, 64, 0.39f, 0.235f, NT_CONV_NAME("256x64")},
+};
+#undef NT_CONV_NAME
 constexpr int kConvMaxParts = 32;
 constexpr int kConvNarrowTile = 1;  // of up to 16 channels
 
@@ -1284,6 +1291,7 @@ int run_fast(const Conv2dRequest &q, hipStream_t stream) {
     p.tiles_m = ceil_div(p.M, kConvTiles[choice.tile].m);
     p.tiles_n = ceil_div(q.K, kConvTiles[choice.tile].n);
     const unsigned tiles = (unsigned)(p.tiles_m * p.tiles_n);
+    note_launch(kLaunchConv2d, kConvRepack, kConvTiles[choice.tile].name, p.parts);
     const auto launch = [&](auto kernel, auto in_parts, auto sum, int bm, int bn, int threads) {
         if (p.parts == 1) {
             kernel<<<dim3(tiles), dim3(threads), 0, stream>>>(p);

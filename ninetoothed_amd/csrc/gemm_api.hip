@@ -1226,9 +1226,6 @@ int nt_tune_cache_lookup(int dtype, int output_dtype, int m, int n, int k, int a
 namespace nt {
 namespace {
 
-// the ways to run a convolution; kConvAuto tries them from the top (a 1 x 1 filter without padding first runs
-// as a batch of plain products when it can)
-enum ConvPath { kConvAuto = 0, kConvGather = 1, kConvRepack = 2, kConvDirect = 3, kConvPointwise = 4 };
 bool conv2d_choice_known(int index, const int *, int) { return index >= kConvGather && index <= kConvPointwise; }
 const bool g_conv2d_check_registered = tune_register_check(kTuneConv2d, conv2d_choice_known);
 
@@ -1343,7 +1340,6 @@ int conv2d_run(const Conv2dRequest &r, int path, hipStream_t stream) {
         if (direct != NINETOOTHED_NO_KERNEL || path == kConvDirect) return direct;
     }
     if (path == kConvAuto || path == kConvRepack) {
-        note_launch(kLaunchConv2d, kConvRepack, "conv2d_repack_kernel, then conv2d_nhwc_kernel on channels-last copies");
         const int fast = conv2d_fast(r, stream);
         if (fast != NINETOOTHED_NO_KERNEL || path == kConvRepack) return fast;
     }

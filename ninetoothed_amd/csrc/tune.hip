@@ -81,12 +81,14 @@ namespace {
 thread_local int t_launch_program = kLaunchNone;
 thread_local int t_launch_choice = -1;
 thread_local const char *t_launch_name = nullptr;
+thread_local int t_launch_parts = 1;
 }  // namespace
 
-void note_launch(int program, int choice, const char *name) {
+void note_launch(int program, int choice, const char *name, int parts) {
     t_launch_program = program;
     t_launch_choice = choice;
     t_launch_name = name;
+    t_launch_parts = parts;
 }
 
 }  // namespace nt
@@ -101,8 +103,10 @@ NineToothedResult nt_last_launch(char *buffer, int size) {
     if (buffer == nullptr || size <= 0) return hipErrorInvalidValue;
     static const char *const programs[] = {"none", "gemm instance", "attention variant", "conv2d path", "softmax kernel", "tile map"};
     const int program = t_launch_program >= kLaunchNone && t_launch_program <= kLaunchMap ? t_launch_program : kLaunchNone;
+    const char *name = t_launch_name ? t_launch_name : "";
     if (program == kLaunchNone) snprintf(buffer, (size_t)size, "none");
-    else snprintf(buffer, (size_t)size, "%s %d: %s", programs[program], t_launch_choice, t_launch_name ? t_launch_name : "");
+    else if (t_launch_parts > 1) snprintf(buffer, (size_t)size, "%s %d: %s, %d parts", programs[program], t_launch_choice, name, t_launch_parts);
+    else snprintf(buffer, (size_t)size, "%s %d: %s", programs[program], t_launch_choice, name);
     return 0;
 }
 

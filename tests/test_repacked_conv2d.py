@@ -29,22 +29,27 @@ def _outputs(shape, dtype, layout):
 @pytest.mark.parametrize("layout", ("nchw", "channels_last", "sliced"))
 @pytest.mark.parametrize("dtype", (torch.float16, torch.bfloat16))
 @pytest.mark.parametrize(
-    "n, c, size, k, window, stride",
+    "n, c, size, k, window, stride, tile, parts",
     (
-        (1, 320, 7, 192, 5, 2),    # 16 positions, 250 k steps: many parts
-        (2, 104, 9, 60, 3, 1),     # channels padded to the k step, filters no multiple of 8
-        (3, 448, 20, 64, 3, 1),
-        (4, 344, 7, 152, 3, 1),    # 49 positions an image: blocks of positions span images
-        (14, 200, 14, 384, 3, 1),  # 64 x 128 tiles in parts
-        (3, 192, 56, 120, 3, 2),
-        (12, 128, 38, 128, 5, 1),  # 128 x 128 tiles
-        (6, 64, 57, 320, 3, 1),    # 256 x 64 tiles
-        (21, 192, 29, 64, 3, 1),   # 128 x 64 tiles
-        (5, 3, 31, 24, 3, 1),      # a k step of several taps
-        (1, 40, 7, 8, 1, 1),       # one k step and a bit
+        (1, 320, 7, 192, 5, 2, "64x64", 32),     # 16 positions, 250 k steps: many parts
+        (2, 104, 9, 60, 3, 1, "64x64", 1),       # channels padded to the k step, filters no multiple of 8
+        (3, 448, 20, 64, 3, 1, "64x64", 12),
+        (4, 344, 7, 152, 3, 1, "64x64", 20),     # 49 positions an image: blocks of positions span images
+        (14, 200, 14, 384, 3, 1, "128x64", 1),
+        (3, 192, 56, 120, 3, 2, "64x64", 1),
+        (12, 128, 38, 128, 5, 1, "128x128", 3),
+        (6, 64, 57, 320, 3, 1, "128x128", 1),
+        (21, 192, 29, 64, 3, 1, "128x64", 1),
+        (27, 72, 10, 24, 5, 1, "128x64", 11),
+        (24, 32, 15, 384, 3, 1, "64x128", 1),
+        (2, 192, 18, 72, 5, 1, "64x128", 22),
+        (39, 32, 46, 24, 3, 1, "256x64", 1),
+        (12, 104, 37, 24, 5, 1, "256x64", 6),
+        (5, 3, 31, 24, 3, 1, "128x64", 1),       # a k step of several taps
+        (1, 40, 7, 8, 1, 1, "64x64", 1),         # one k step and a bit
     ),
 )
-def test_tiles_and_parts_against_fp32(n, c, size, k, window, stride, dtype, layout):
+def test_tiles_and_parts_against_fp32(n, c, size, k, window, stride, tile, parts, dtype, layout):
     from ninetoothed_amd import runtime
 
     padding = window // 2
@@ -57,7 +62,8 @@ def test_tiles_and_parts_against_fp32(n, c, size, k, window, stride, dtype, layo
         buffer, out = _outputs(expected.shape, dtype, layout)
         tensors = [runtime.ArgumentTensor.from_torch_tensor(t) for t in (x, weight, out)]
         assert runtime.library().launch_nt_conv2d_strided(runtime.current_stream(), *tensors, tag, padding, padding, stride, stride, 1, 1, REPACK, 0, 0) == 0
-        assert "conv2d_repack_kernel" in runtime.last_launch()
+        # the tile and the parts follow from times expected on 256 compute units
+        assert "conv2d_repack_kernel" in runtime.last_launch() and runtime.last_launch().endswith(f"tiles of {tile}" + (f", {parts} parts" if parts > 1 else "")), runtime.last_launch()
         results.append(out.clone())
         if layout == "sliced":
             assert bool((buffer[..., 1::2] == 7.0).all())
