@@ -218,12 +218,14 @@ NT_DEVICE NT_LDS unsigned char *stage_memory() {
 
 // What bounds it: the instructions of a step that are no MFMAs -- where the taps lie, the loads, the reads of fragments -- and with
 // them the number of steps that follow one another.  So the address arithmetic has no branches (kNarrow is an instance of its own)
-// and is dealt out between the MFMAs, fragments of the next step are read under those of this one, and a launch that leaves CUs
+// and is dealt out between the MFMAs, fragments of the next step are read under those of this one (kAhead), and a launch that leaves CUs
 // idle deals the contraction to parts (kParts): part s adds up k steps [s * kt_per_part, ...) and writes its accumulators as
 // they lie in the registers; conv2d_sum_parts_kernel adds the parts.  With branches a step of 128 x 64 took 0.28 us, 0.34 on
 // 32x32x16 MFMAs, however deep the ring (4 to 12 stages); now 0.19: 22 images of 384 x 88 x 88, 256 filters of 3 x 3, 394 -> 350 us, 28
 // of 64 x 56 x 56, 384 of 5 x 5, 141 -> 126.
-template <typename T, int BM, int BN, int WM, int WN, int kStages, int kOcc, bool kParts, bool kNarrow>
+// Without kAhead a step reads its own fragments: half the registers for them, which is what three workgroups of 128 x 128 on a CU
+// need, and a stage more in flight; the other waves of the SIMD cover the reads.
+template <typename T, int BM, int BN, int WM, int WN, int kStages, int kOcc, bool kParts, bool kNarrow, bool kAhead>
 __global__ __launch_bounds__(WM *WN * 64, kOcc) void conv2d_nhwc_kernel(ConvParams p) {
 #if defined(__HIP_DEVICE_COMPILE__)
     typedef Elem<T> E;
@@ -312,8 +314,10 @@ __global__ __launch_bounds__(WM *WN * 64, kOcc) void conv2d_nhwc_kernel(ConvPara
             for (int j = 0; j < kAInstr; ++j) {
                 const int tap = kt * taps_per_step + a_tap[j];
                 const int fy = (tap / p.S) * p.dil_h, fx = (tap % p.S) * p.dil_w;
-                const bool inside = wanted != 0 && tap < taps && (unsigned)(a_y[j] + fy) < (unsigned)p.H && (unsigned)(a_x[j] + fx) < (unsigned)p.W;
-                a_src[j] = inside ? (unsigned)(a_base[j] + (fy * p.W + fx) * p.C * 2) : kConvBehind;
+                const unsigned rows = tap < taps ? (unsigned)(p.H & wanted) : 0u;
+                const bool inside = ((unsigned)(a_y[j] + fy) < rows) & ((unsigned)(a_x[j] + fx) < (unsigned)p.W);  // (both compared: no branch)
+                const unsigned offset = (unsigned)(a_base[j] + (fy * p.W + fx) * p.C * 2);
+                a_src[j] = inside ? offset : kConvBehind;
             }
             b_k = kt * BK * p.Kp * 2 & wanted;  // (rows past the last tap lie behind the descriptor: zeros)
         } else {
@@ -375,50 +379,55 @@ __global__ __launch_bounds__(WM *WN * 64, kOcc) void conv2d_nhwc_kernel(ConvPara
 #pragma unroll
         for (int tj = 0; tj < TN; ++tj) acc[ti][tj] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
 
-    // The barrier that opens step t tells that stage t + 1 is complete in LDS and that every wave is done with stage t - 1,
+    // kAhead: the barrier that opens step t tells that stage t + 1 is complete in LDS and that every wave is done with stage t - 1,
     // which is refilled right after it.  During a step all fragments of the next one are read, under its MFMAs: a workgroup
     // that has a SIMD to itself would wait for the LDS before every MFMA otherwise.  Where the loads of the step after lie is
-    // worked out in the same place.
+    // worked out in the same place.  Else it tells that stage t is complete, whose fragments the step reads itself, before its MFMAs;
+    // both forms have consumed what they read of a stage before the barrier after which it is refilled.
     static_for<0, kStages - 1>([&](auto s) {
         locate();
         issue_loads(s);
     });
     locate();
-    vec8 as[2][TM];
-    vec8 bs[2][TN];
-    wait_vmcnt<(kStages - 2) * kLoadsPerStage>();
-    lds_barrier();
+    vec8 as[kAhead ? 2 : 1][TM];
+    vec8 bs[kAhead ? 2 : 1][TN];
+    const auto read_fragments = [&](auto set, auto stage_tag) {
 #pragma unroll
-    for (int ti = 0; ti < TM; ++ti) as[0][ti] = read_a(std::integral_constant<int, 0>(), ti);
+        for (int tj = 0; tj < TN; ++tj) bs[decltype(set)::value][tj] = read_b(stage_tag, tj);
 #pragma unroll
-    for (int tj = 0; tj < TN; ++tj) bs[0][tj] = read_b(std::integral_constant<int, 0>(), tj);
+        for (int ti = 0; ti < TM; ++ti) as[decltype(set)::value][ti] = read_a(stage_tag, ti);
+    };
+    if constexpr (kAhead) {
+        wait_vmcnt<(kStages - 2) * kLoadsPerStage>();
+        lds_barrier();
+        read_fragments(std::integral_constant<int, 0>(), std::integral_constant<int, 0>());
+    }
     auto step = [&](auto position) {
         constexpr int kI = decltype(position)::value, kS = kI % kStages;  // in the unrolled body: stage and set of fragments follow
-        typedef std::integral_constant<int, (kS + 1) % kStages> NextStage;
-        constexpr int cur = kI & 1, nxt = cur ^ 1;
-        wait_vmcnt<(kStages - 3) * kLoadsPerStage>();
+        constexpr int kReadStage = kAhead ? (kS + 1) % kStages : kS;
+        constexpr int cur = kAhead ? kI & 1 : 0, nxt = kAhead ? cur ^ 1 : 0;
+        wait_vmcnt<(kStages - (kAhead ? 3 : 2)) * kLoadsPerStage>();
         lds_barrier_reads_in_flight();
         issue_loads(std::integral_constant<int, (kS + kStages - 1) % kStages>());
         locate();
-#pragma unroll
-        for (int tj = 0; tj < TN; ++tj) bs[nxt][tj] = read_b(NextStage(), tj);
-#pragma unroll
-        for (int ti = 0; ti < TM; ++ti) as[nxt][ti] = read_a(NextStage(), ti);
+        read_fragments(std::integral_constant<int, nxt>(), std::integral_constant<int, kReadStage>());
 #pragma unroll
         for (int ti = 0; ti < TM; ++ti)
 #pragma unroll
             for (int tj = 0; tj < TN; ++tj) acc[ti][tj] = E::mfma16(as[cur][ti], bs[cur][tj], acc[ti][tj]);
-        // issue order: the loads and the reads spread under the MFMAs
-        constexpr int kMfmas = TM * TN, kReads = TM + 2 * TN, kPer = (kReads + kMfmas - 1) / kMfmas;
-        static_for<0, kMfmas>([&](auto i_tag) {
-            constexpr int i = decltype(i_tag)::value;
-            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-            if constexpr (i * kPer < kReads) __builtin_amdgcn_sched_group_barrier(0x100, kPer, 0);
-            if constexpr (i < kLoadsPerStage) __builtin_amdgcn_sched_group_barrier(0x020, (kLoadsPerStage + kMfmas - 1) / kMfmas, 0);
-            __builtin_amdgcn_sched_group_barrier(0x006, 8, 0);
-        });
+        if constexpr (kAhead) {
+            // issue order: the loads and the reads spread under the MFMAs
+            constexpr int kMfmas = TM * TN, kReads = TM + 2 * TN, kPer = (kReads + kMfmas - 1) / kMfmas;
+            static_for<0, kMfmas>([&](auto i_tag) {
+                constexpr int i = decltype(i_tag)::value;
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                if constexpr (i * kPer < kReads) __builtin_amdgcn_sched_group_barrier(0x100, kPer, 0);
+                if constexpr (i < kLoadsPerStage) __builtin_amdgcn_sched_group_barrier(0x020, (kLoadsPerStage + kMfmas - 1) / kMfmas, 0);
+                __builtin_amdgcn_sched_group_barrier(0x006, 8, 0);
+            });
+        }
     };
-    constexpr int kBody = kStages % 2 ? 2 * kStages : kStages;
+    constexpr int kBody = kAhead && kStages % 2 ? 2 * kStages : kStages;
     const int main_k = num_k - num_k % kBody;
     for (int kt = 0; kt < main_k; kt += kBody) static_for<0, kBody>([&](auto s) { step(s); });
     static_for<0, kBody - 1>([&](auto s) {
@@ -1195,7 +1204,7 @@ constexpr ConvTile kConvTiles[] = {
 };
 #undef NT_CONV_NAME
 constexpr int kConvMaxParts = 32;
-constexpr int kConvNarrowTile = 1;  // of up to 16 channels
+constexpr int kConv128x128 = 0, kConv128x64 = 1;  // the tiles for up to 16 channels
 
 struct ConvChoice {
     int tile, parts;
@@ -1228,6 +1237,17 @@ ConvChoice conv2d_choose(int64_t rows, int64_t filters, int steps, int max_parts
         }
     }
     return best;
+}
+
+// The tile for up to 16 channels, whose few k steps are bound by the output that they store.  As many workgroups on a CU as fit (three of
+// 128 x 128, four of 128 x 64, three stages each), and 128 filters a tile where that leaves no more than 15 % of the columns' time to
+// empty ones and gives every CU a tile: fp16, us, both tiles / before (one of 128 x 64, 256 x 128 and 256 x 256): 32 images of 3 x 224 x 224, 3 x 3, 96 filters 120 and
+// 139 / 180, 192 filters 207 and 202 / 255, 256 filters 219 and 258 / 244; 7 x 7 step 2, 64 filters 76 and 62 / 72, 512 filters 205 and 248 / 233; one such
+// image, 256 filters 12.6 and 12.5 / 13.2.  (784 tiles, 16 over three on every CU, remain behind the 392 of 256 x 128 they replace: 8 of those
+// images, 128 filters 28.5 / 26.9.)
+int conv2d_narrow_tile(int64_t rows, int64_t filters) {
+    const int64_t wide = (filters + 127) / 128, narrow = (filters + 63) / 64;
+    return wide * 128 * 17 < narrow * 64 * 20 && (rows + 127) / 128 * wide >= compute_units() ? kConv128x128 : kConv128x64;
 }
 
 // channels of the repacked operands: the k step of 32 holds whole blocks of channels -- or, for up to 16 channels
@@ -1278,7 +1298,7 @@ int run_fast(const Conv2dRequest &q, hipStream_t stream) {
     p.xt_bytes = (unsigned)xt_bytes;
     p.wt_bytes = (unsigned)wt_bytes;
     const int steps = ceil_div(Cp * q.R * q.S, 32);
-    ConvChoice choice = Cp < 32 ? ConvChoice{kConvNarrowTile, 1} : conv2d_choose(p.M, q.K, steps, kConvMaxParts);
+    ConvChoice choice = Cp < 32 ? ConvChoice{conv2d_narrow_tile(p.M, q.K), 1} : conv2d_choose(p.M, q.K, steps, kConvMaxParts);
     p.scratch = nullptr;
     if (choice.parts > 1) {
         const ConvTile &tile = kConvTiles[choice.tile];
@@ -1301,11 +1321,12 @@ int run_fast(const Conv2dRequest &q, hipStream_t stream) {
         sum<<<dim3(tiles * (bm * bn / 256)), dim3(256), 0, stream>>>(p);
     };
 #define NT_CONV_LAUNCH(BM, BN, WM, WN, ST, OCC) \
-    launch(conv2d_nhwc_kernel<T, BM, BN, WM, WN, ST, OCC, false, false>, conv2d_nhwc_kernel<T, BM, BN, WM, WN, ST, OCC, true, false>, conv2d_sum_parts_kernel<T, BM, BN, WM, WN>, BM, BN, WM * WN * 64)
-    if (Cp < 32) conv2d_nhwc_kernel<T, 128, 64, 2, 2, 6, 2, false, true><<<dim3(tiles), dim3(256), 0, stream>>>(p);
+    launch(conv2d_nhwc_kernel<T, BM, BN, WM, WN, ST, OCC, false, false, true>, conv2d_nhwc_kernel<T, BM, BN, WM, WN, ST, OCC, true, false, true>, conv2d_sum_parts_kernel<T, BM, BN, WM, WN>, BM, BN, WM * WN * 64)
+    if (Cp < 32 && choice.tile == kConv128x128) conv2d_nhwc_kernel<T, 128, 128, 2, 2, 3, 3, false, true, false><<<dim3(tiles), dim3(256), 0, stream>>>(p);
+    else if (Cp < 32) conv2d_nhwc_kernel<T, 128, 64, 2, 2, 3, 4, false, true, false><<<dim3(tiles), dim3(256), 0, stream>>>(p);
     else switch (choice.tile) {
-    case 0: NT_CONV_LAUNCH(128, 128, 2, 2, 4, 2); break;
-    case 1: NT_CONV_LAUNCH(128, 64, 2, 2, 6, 2); break;
+    case kConv128x128: NT_CONV_LAUNCH(128, 128, 2, 2, 4, 2); break;
+    case kConv128x64: NT_CONV_LAUNCH(128, 64, 2, 2, 6, 2); break;
     case 2: NT_CONV_LAUNCH(64, 128, 2, 2, 4, 3); break;
     case 3: NT_CONV_LAUNCH(64, 64, 2, 2, 6, 3); break;
     default: NT_CONV_LAUNCH(256, 64, 4, 1, 4, 2); break;

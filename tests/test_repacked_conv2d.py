@@ -45,7 +45,9 @@ def _outputs(shape, dtype, layout):
         (2, 192, 18, 72, 5, 1, "64x128", 22),
         (39, 32, 46, 24, 3, 1, "256x64", 1),
         (12, 104, 37, 24, 5, 1, "256x64", 6),
-        (5, 3, 31, 24, 3, 1, "128x64", 1),       # a k step of several taps
+        (5, 3, 31, 24, 3, 1, "128x64", 1),       # k steps of several taps
+        (9, 5, 61, 120, 3, 1, "128x128", 1),
+        (40, 3, 45, 250, 5, 2, "128x128", 1),
         (1, 40, 7, 8, 1, 1, "64x64", 1),         # one k step and a bit
     ),
 )
