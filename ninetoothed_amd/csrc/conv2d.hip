@@ -1,4 +1,4 @@
-// conv2d (stride 1, dilation 1, zero padding) as implicit GEMM on the MFMA main loop of gemm_fast.h.  Two paths:
+// conv2d (zero padding; (1) steps and dilation of 1, (2) any) as implicit GEMM on the MFMA main loop of gemm_fast.h.  Two paths:
 //
 // (1) conv2d_direct: one launch on the tensors as they lie, no scratch memory (described with its kernel
 //     below); needs an output width that is a multiple of 8, padding_w <= 1, C*R*S a multiple of 32, a contiguous
@@ -17,8 +17,8 @@
 // asynchronous, and allocates only when a call needs more than any before it):
 //   x[N,C,H,W]  -> xt[N,H,W,C]              (tiled transpose through LDS, 16-byte accesses)
 //   w[K,C,R,S]  -> wt[(r*S+s)*C + c, K]     (row-major K x N operand of the GEMM)
-// The main kernel then is the direct-to-LDS GEMM loop (256x256x32 tiles for wide layers,
-// 256x128 and 128x64 for layers with fewer output channels): a K step is 32 channels of
+// The main kernel then is the direct-to-LDS GEMM loop (tiles of 64x64 to 256x256, the contraction
+// in parts where few tiles would leave CUs idle: conv2d_choose): a K step is 32 channels of
 // one filter tap (r, s); the A rows of a step are 64-byte runs of xt whose
 // addresses differ from step to step by a uniform offset; taps that fall into
 // the padding are fetched with an out-of-range buffer offset, which the
@@ -28,10 +28,11 @@
 // laid out [channel][row] and leave as 16-byte stores when P*Q is a multiple of 8
 // (8 consecutive rows then lie in one image, aligned), element by element otherwise.
 //
-// Requirements of path (2) (anything else uses the any-stride gather kernel):
-// fp16/bf16, K_out % 8 == 0, contiguous output.  The repacked operands hold C rounded up to a
-// multiple of 32 channels, the extra ones zero (a 3-channel stem layer multiplies ten times the
-// useful work and is still twice as fast as the gather kernel).
+// Requirements of path (2) (anything else uses the any-stride gather kernel): fp16/bf16, repacked operands below 2 GiB each.
+// Tensors of any strides and any number of output channels: rows of the repacked filter are rounded up to 8 of them, and an output
+// that is neither a contiguous NCHW tensor nor channels last is stored element by element.  The repacked operands hold C
+// rounded up to a multiple of 32 channels, the extra ones zero -- up to 16 channels to 8 or 16: a K step then is
+// 4 or 2 filter taps (kNarrow).
 #include <algorithm>
 
 #include "conv2d.h"
@@ -223,8 +224,8 @@ NT_DEVICE NT_LDS unsigned char *stage_memory() {
 // they lie in the registers; conv2d_sum_parts_kernel adds the parts.  With branches a step of 128 x 64 took 0.28 us, 0.34 on
 // 32x32x16 MFMAs, however deep the ring (4 to 12 stages); now 0.19: 22 images of 384 x 88 x 88, 256 filters of 3 x 3, 394 -> 350 us, 28
 // of 64 x 56 x 56, 384 of 5 x 5, 141 -> 126.
-// Without kAhead a step reads its own fragments: half the registers for them, which is what three workgroups of 128 x 128 on a CU
-// need, and a stage more in flight; the other waves of the SIMD cover the reads.
+// Without kAhead a step reads its own fragments: half the registers for them, which is what 256 x 256 tiles and three workgroups of 128 x 128
+// on a CU need, and a stage more in flight; the other waves of the SIMD cover the reads.
 template <typename T, int BM, int BN, int WM, int WN, int kStages, int kOcc, bool kParts, bool kNarrow, bool kAhead>
 __global__ __launch_bounds__(WM *WN * 64, kOcc) void conv2d_nhwc_kernel(ConvParams p) {
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -1189,21 +1190,24 @@ int run_direct(const Conv2dRequest &q, hipStream_t stream) {
 }
 
 // The tiles of the main kernel and what a k step of 32 costs them, in microseconds: `alone` with one workgroup on a CU, where
-// the steps of a workgroup follow one another, `shared` per workgroup with several.  Fitted to the times of 75 convolutions (1 to 32
+// the steps of a workgroup follow one another, `shared` per workgroup with several.  Fitted to the times of 220 convolutions (1 to 32
 // images of 7 x 7 to 112 x 112, 64 to 512 channels and filters, windows 1, 3 and 5, steps 1 and 2) on every tile and number of
-// parts: the choice below is 2 % slower than the best of them on average, 9 % at worst.
+// parts: the choice below is 1.2 % slower than the best of them on average, 20 % at worst.  256 x 256 is for whole contractions of many
+// filters, where a byte of LDS feeds more MFMAs (fp16, us, the best other tile / this): 4 images of 256 x 112 x 112, 256 filters of 5 x 5, 190 / 150; 32 of
+// 512 x 28 x 28, 512 of 3 x 3, 147 / 119; 2 of 168 x 112 x 112, 480 of 5 x 5, 144 / 113; 9 of 128 x 56 x 56, 440 of 3 x 3, 47.5 / 40.
 struct ConvTile {
-    int m, n;
+    int m, n, max_parts;
     float alone, shared;
     const char *name;  // of a launch
 };
 #define NT_CONV_NAME(TILE) "conv2d_repack_kernel, then conv2d_nhwc_kernel on channels-last copies, tiles of " TILE
+constexpr int kConvMaxParts = 32;
 constexpr ConvTile kConvTiles[] = {
-    {128, 128, 0.28f, 0.21f, NT_CONV_NAME("128x128")}, {128, 64, 0.19f, 0.19f, NT_CONV_NAME("128x64")}, {64, 128, 0.205f, 0.14f, NT_CONV_NAME("64x128")},
-    {64, 64, 0.145f, 0.107f, NT_CONV_NAME("64x64")}, {256, 64, 0.39f, 0.235f, NT_CONV_NAME("256x64")},
+    {128, 128, kConvMaxParts, 0.28f, 0.203f, NT_CONV_NAME("128x128")}, {128, 64, kConvMaxParts, 0.20f, 0.172f, NT_CONV_NAME("128x64")},
+    {64, 128, kConvMaxParts, 0.19f, 0.14f, NT_CONV_NAME("64x128")}, {64, 64, kConvMaxParts, 0.125f, 0.10f, NT_CONV_NAME("64x64")},
+    {256, 64, 1, 0.39f, 0.32f, NT_CONV_NAME("256x64")}, {256, 256, 1, 0.52f, 0.52f, NT_CONV_NAME("256x256")},
 };
 #undef NT_CONV_NAME
-constexpr int kConvMaxParts = 32;
 constexpr int kConv128x128 = 0, kConv128x64 = 1;  // the tiles for up to 16 channels
 
 struct ConvChoice {
@@ -1212,8 +1216,10 @@ struct ConvChoice {
 
 // The tile and the number of parts of the contraction with the least expected time.  Parts pay where few workgroups would
 // follow a long chain of k steps (before they were there: 3 images of 384 x 56 x 56, 64 filters of 5 x 5, step 2: 104 us, now 25; 1 x 320 x 7 x 7, 192 of
-// 5 x 5, step 2: 90 -> 15; 3 x 448 x 56 x 56, 64 of 3 x 3: 51 -> 28); the second launch and the accumulators in memory cost about 5 us and 5.9 TB/s.
-ConvChoice conv2d_choose(int64_t rows, int64_t filters, int steps, int max_parts) {
+// 5 x 5, step 2: 90 -> 15; 3 x 448 x 56 x 56, 64 of 3 x 3: 51 -> 28); the second launch and the accumulators in memory cost about 2.4 us and 2.7 TB/s.
+// `scattered`: an output that is stored element by element, 3.9 us a tile of 8192 values at the end of the launch (32 images of 128 x 28 x 28, 512
+// filters of 1 x 1, step 2: 18.0 us on 128 x 128 tiles, 13.8 on 64 x 64).
+ConvChoice conv2d_choose(int64_t rows, int64_t filters, int steps, bool scattered, int max_parts) {
     const int64_t units = std::max(1, compute_units());
     ConvChoice best = {0, 1};
     float best_time = 0.0f;
@@ -1222,13 +1228,14 @@ ConvChoice conv2d_choose(int64_t rows, int64_t filters, int steps, int max_parts
         const ConvTile &tile = kConvTiles[t];
         const int64_t tiles = (rows + tile.m - 1) / tile.m * ((filters + tile.n - 1) / tile.n);
         for (int wanted : {1, 2, 3, 4, 6, 8, 12, 16, 24, kConvMaxParts}) {
-            if (wanted > max_parts || wanted > steps) break;
+            if (wanted > std::min(max_parts, tile.max_parts) || wanted > steps) break;
             const int per_part = ceil_div(steps, wanted), parts = ceil_div(steps, per_part);
             const int64_t scratch = parts > 1 ? parts * tiles * tile.m * tile.n * 4 : 0;
             if (scratch > (int64_t)64 << 20) break;
             const float rounds = (float)((tiles * parts + units - 1) / units);  // workgroups per CU
-            const float time = (float)per_part * std::max(tile.alone, rounds * tile.shared) + 0.48f * rounds * (float)(tile.m * tile.n) / 8192.0f +
-                               (parts > 1 ? 5.0f + (float)scratch / 5.85e6f : 0.0f);
+            const float values = (float)(tile.m * tile.n) / 8192.0f;
+            const float time = (float)per_part * std::max(tile.alone, rounds * tile.shared) + 0.66f * rounds * values +
+                               (parts > 1 ? 2.4f + (float)scratch / 2.7e6f : scattered ? 3.9f * values : 0.0f);
             if (!found || time < best_time) {
                 found = true;
                 best = {t, parts};
@@ -1298,13 +1305,14 @@ int run_fast(const Conv2dRequest &q, hipStream_t stream) {
     p.xt_bytes = (unsigned)xt_bytes;
     p.wt_bytes = (unsigned)wt_bytes;
     const int steps = ceil_div(Cp * q.R * q.S, 32);
-    ConvChoice choice = Cp < 32 ? ConvChoice{conv2d_narrow_tile(p.M, q.K), 1} : conv2d_choose(p.M, q.K, steps, kConvMaxParts);
+    const bool scattered = p.dense_out == 0 || (p.dense_out == 1 && q.P * q.Q % 8 != 0);
+    ConvChoice choice = Cp < 32 ? ConvChoice{conv2d_narrow_tile(p.M, q.K), 1} : conv2d_choose(p.M, q.K, steps, scattered, kConvMaxParts);
     p.scratch = nullptr;
     if (choice.parts > 1) {
         const ConvTile &tile = kConvTiles[choice.tile];
         const int64_t tiles = (int64_t)ceil_div(p.M, tile.m) * ceil_div(q.K, tile.n);
         p.scratch = (float *)lease.get(kWorkspaceConvParts, (size_t)choice.parts * tiles * tile.m * tile.n * sizeof(float));
-        if (p.scratch == nullptr) choice = conv2d_choose(p.M, q.K, steps, 1);  // no scratch (graph capture, out of memory): in one piece
+        if (p.scratch == nullptr) choice = conv2d_choose(p.M, q.K, steps, scattered, 1);  // no scratch (graph capture, out of memory): in one piece
     }
     p.kt_per_part = ceil_div(steps, choice.parts);
     p.parts = ceil_div(steps, p.kt_per_part);  // every part has at least one k step
@@ -1329,7 +1337,8 @@ int run_fast(const Conv2dRequest &q, hipStream_t stream) {
     case kConv128x64: NT_CONV_LAUNCH(128, 64, 2, 2, 6, 2); break;
     case 2: NT_CONV_LAUNCH(64, 128, 2, 2, 4, 3); break;
     case 3: NT_CONV_LAUNCH(64, 64, 2, 2, 6, 3); break;
-    default: NT_CONV_LAUNCH(256, 64, 4, 1, 4, 2); break;
+    case 4: conv2d_nhwc_kernel<T, 256, 64, 4, 1, 4, 2, false, false, true><<<dim3(tiles), dim3(256), 0, stream>>>(p); break;
+    default: conv2d_nhwc_kernel<T, 256, 256, 2, 4, 4, 2, false, false, false><<<dim3(tiles), dim3(512), 0, stream>>>(p);
     }
 #undef NT_CONV_LAUNCH
     return (int)hipGetLastError();
