@@ -149,29 +149,38 @@ hipError_t fast_launch(const GemmProblem &q, hipStream_t stream) {
 // The k range is cut into parts, each (tile, part) is a workgroup that writes an fp32 tile to scratch
 // memory of the stream, and a second kernel sums the parts and applies the epilogue.
 
+// What a k tile costs a workgroup with a CU to itself (`alone`) and the CU per workgroup (`shared`), in microseconds, and the rate at which
+// the partial products are written and read (bytes per microsecond), by the tile of the instance.
+struct SplitCost {
+    int area, resident;  // workgroups per CU
+    float alone, shared, rate;
+};
+constexpr SplitCost kSplitCosts[] = {{64 * 64, 2, 0.234f, 0.214f, 0.8e6f}, {128 * 128, 1, 0.3f, 0.3f, 4.0e6f}, {128 * 256, 2, 0.39f, 0.28f, 5.1e6f}, {256 * 256, 1, 0.29f, 0.29f, 5.8e6f}};
+
+constexpr const SplitCost *split_cost(int bm, int bn) {
+    for (const SplitCost &cost : kSplitCosts)
+        if (cost.area == bm * bn) return &cost;
+    return nullptr;
+}
+
 // Number of parts for tiles of bm x bn x bk, 1 = do not split (`scratch_limit`: bytes the partial products may take).
-// Of the numbers whose workgroups are all on the chip at once, the one of least expected time: `alone` is what a k tile takes a
-// workgroup with a CU to itself, `shared` what it takes the CU per workgroup (us), the partial products are written and read at `rate`.
+// Of the numbers whose workgroups are all on the chip at once, the one of least expected time -- and two parts of any number of tiles below
+// 320 (of 256 x 256 ones, whose parts are the largest, up to 128): more of them than the chip holds run in rounds, which the untuned choice
+// leaves alone; the tuner, or a call by the instance's index, takes them.
 // Fitted to 59 products of 1 to 3000 rows, 2 to 48 parts: 3 % (64 x 64), 1 % (others) slower than the best number on average; 512
 // workgroups whatever the shape were 11 and 10 % slower.  (128 x 128: five products of 100 to 1024 rows, a step 0.22 to 0.46 us with
 // the rhs in the caches and in memory; 222 x 2752 x 15040 34.5 us in five parts, 39 in four, 43 in eight, without the summing.)
 int split_parts(const GemmProblem &q, int bm, int bn, int bk, int *kt_per_part, int64_t scratch_limit = int64_t(64) << 20) {
-    struct Cost {
-        int area, resident;  // workgroups per CU
-        float alone, shared, rate;
-    };
-    constexpr Cost costs[] = {{64 * 64, 2, 0.234f, 0.214f, 0.8e6f}, {128 * 128, 1, 0.3f, 0.3f, 4.0e6f}, {128 * 256, 2, 0.39f, 0.28f, 5.1e6f}, {256 * 256, 1, 0.29f, 0.29f, 5.8e6f}};
     const int64_t tiles = (int64_t)((q.m + bm - 1) / bm) * ((q.n + bn - 1) / bn);
     const int num_kt = (q.k + bk - 1) / bk;
-    if (tiles >= 320) return 1;  // (the untuned choice only splits below 192 tiles; between, the tuner decides)
-    const Cost *cost = costs;
-    while (cost->area != bm * bn) ++cost;
+    if (tiles >= 320) return 1;
+    const SplitCost *cost = split_cost(bm, bn);
     const int64_t part_bytes = (int64_t)q.m * ((q.n + 7) / 8 * 8) * 4;
     int best = 1;
     float best_time = 0.0f;
     for (int parts = 2; parts <= std::min(256, num_kt / 2); parts += std::max(1, parts / 8)) {  // at least two k tiles each
         const int64_t workgroups = tiles * parts;
-        if (parts * part_bytes > scratch_limit || (parts > 2 && workgroups > 256 * cost->resident) || (cost->resident == 1 && workgroups > 256)) break;
+        if (parts * part_bytes > scratch_limit || ((parts > 2 || cost->area == 256 * 256) && workgroups > 256 * cost->resident)) break;
         const int per_part = (num_kt + parts - 1) / parts;
         const float time = (float)per_part * std::max(cost->alone, (float)((workgroups + 255) / 256) * cost->shared) + (float)(parts * part_bytes) / cost->rate;
         if (best == 1 || time < best_time) {
@@ -255,6 +264,7 @@ __global__ __launch_bounds__(256) void gemm_split_reduce_kernel(const float *par
 
 template <typename T, int BM, int BN, int BK, int WM, int WN, int kStages, int kOcc>
 hipError_t split_launch_typed(const GemmProblem &q, hipStream_t stream) {
+    static_assert(split_cost(BM, BN) != nullptr, "a cost for the tile");
     int kt_per_part = 0;
     // with a fixed array the part count shrinks until the partial products fit; the call is refused when not even two parts do
     const int parts = q.fixed_scratch != nullptr ? split_parts(q, BM, BN, BK, &kt_per_part, (int64_t)q.fixed_scratch_bytes) : split_parts(q, BM, BN, BK, &kt_per_part);
@@ -620,7 +630,8 @@ int heuristic_choice(const GemmProblem &q, int bm, int bn, int bk) {
     const auto few_tiles = [&](int instance) {
         const GemmInstance &inst = kInstances[instance];
         // (with a short K the second kernel costs more than the idle CUs: 512^3 8 us split, 5 in one pass; 23 x 384 x 2112 10.8 and 7.7)
-        return q.batch == 1 && !small_tiles_fill_the_chip && q.k >= (q.m <= 64 ? 3072 : 2048) && (int64_t)((q.m + inst.bm - 1) / inst.bm) * ((q.n + inst.bn - 1) / inst.bn) < 192 &&
+        const int64_t tiles = (int64_t)((q.m + inst.bm - 1) / inst.bm) * ((q.n + inst.bn - 1) / inst.bn);
+        return q.batch == 1 && !small_tiles_fill_the_chip && q.k >= (q.m <= 64 ? 3072 : 2048) && tiles < 192 && 2 * tiles <= 256 * split_cost(inst.bm, inst.bn)->resident &&
                inst.accepts(q);
     };
     if (q.m <= 64 && few_tiles(kSplit64x64x64)) return kSplit64x64x64;

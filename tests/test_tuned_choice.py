@@ -53,6 +53,22 @@ def test_candidates_at_the_callers_pace(choose):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("m, n, k", ((1024, 2560, 264), (2001, 2432, 520)))  # 160 and 304 tiles of 128 x 128
+@pytest.mark.parametrize("bk", (64, 32))
+def test_two_parts_of_more_tiles_than_the_chip_holds(m, n, k, bk):
+    tag, library = runtime.DATA_TYPE_INDEX["bf16"], runtime.library()
+    lhs, rhs = torch.randn(m, k, device="cuda", dtype=torch.bfloat16), torch.randn(k, n, device="cuda", dtype=torch.bfloat16)
+    out = torch.full((m, n), float("nan"), device="cuda", dtype=torch.bfloat16)
+    (index,) = (index for index, name in enumerate(runtime.gemm_config_names()) if name.startswith("128x128x64" if bk == 64 else "128x256x32") and name.endswith("split-k"))
+    null, arguments = runtime.ArgumentTensor.null(), [runtime.ArgumentTensor.from_torch_tensor(t) for t in (lhs, rhs, out)]
+    assert library.launch_nt_gemm_config(runtime.current_stream(), index, null, *arguments[:2], null, null, arguments[2], tag, tag) == 0
+    expected = lhs.double() @ rhs.double()
+    # one rounding to the element type over fp32 sums of k products
+    bound = 2.0**-8 * expected.abs() + (k + 4) * 2.0**-24 * (lhs.double().abs() @ rhs.double().abs())
+    assert ((out.double() - expected).abs() <= bound).all()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("m, n, k", ((64, 64, 64), (64, 256, 4096)))
 def test_measured_times_come_back(m, n, k):
     # short products, timed for a caller of any pace: what comes back is a launch's time, not the pace
