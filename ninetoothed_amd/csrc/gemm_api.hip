@@ -629,24 +629,29 @@ int heuristic_choice(const GemmProblem &q, int bm, int bn, int bk) {
     const bool small_tiles_fill_the_chip = q.batch == 1 && tiles_64 >= 256 && kInstances[kTail64x64x64].accepts(q);
     const auto few_tiles = [&](int instance) {
         const GemmInstance &inst = kInstances[instance];
-        // (with a short K the second kernel costs more than the idle CUs: 512^3 8 us split, 5 in one pass; 23 x 384 x 2112 10.8 and 7.7)
+        // (with a short K the second kernel costs more than the idle CUs: 512^3 8 us split, 5 in one pass; of up to 64 rows 33 x 832 x 2088 9.1 and
+        // 7.4, but 14 x 1688 x 2528 7.3 and 11.4, 9 x 136 x 2640 7.3 and 8.7)
         const int64_t tiles = (int64_t)((q.m + inst.bm - 1) / inst.bm) * ((q.n + inst.bn - 1) / inst.bn);
-        return q.batch == 1 && !small_tiles_fill_the_chip && q.k >= (q.m <= 64 ? 3072 : 2048) && tiles < 192 && 2 * tiles <= 256 * split_cost(inst.bm, inst.bn)->resident &&
+        return q.batch == 1 && !small_tiles_fill_the_chip && q.k >= (q.m <= 64 ? 2304 : 2048) && tiles < 192 && 2 * tiles <= 256 * split_cost(inst.bm, inst.bn)->resident &&
                inst.accepts(q);
     };
     if (q.m <= 64 && few_tiles(kSplit64x64x64)) return kSplit64x64x64;
     if (few_tiles(kSplit128x128x64)) return kSplit128x128x64;
     if (few_tiles(kSplit64x64x64)) return kSplit64x64x64;
-    // All tiles on the chip at once, one per CU: the largest deep ring of which that holds (bf16, us, the best of the other
-    // instances / this): 64 x 64 x 128 512 x 512 x 2048 10.4 / 9.2, 130 x 4096 x 4096 19.2 / 15.8, 1000 x 1000 x 16384 80.5 / 58.2 (with a K
-    // of four steps nothing is left in flight: 1024 x 1024 x 128 3.8 / 4.1); 64 x 128 x 64 1024 x 2048 x 2048 15.2 / 12.9, 70 x 14336 x
-    // 2048 16.6 / 15.3; 128 x 128 x 64 2048 x 2048 x 4096 47.2 / 32.1, 1500 x 2048 x 512 10.1 / 7.3.  More tiles: 384 of 128 x 128, 700 x 8192 x
-    // 2048 35.7 / 34.4, but 1024 of them with a K of 256 17.3 / 18.0, so that the rules below keep those.
-    struct DeepRule { int instance, min_k; };
-    for (const DeepRule &rule : {DeepRule{kDeep64x64x128, 1024}, DeepRule{kDeep64x128x64, 512}, DeepRule{kDeep128x128x64, 256}}) {
+    // All tiles on the chip at once, one per CU: the deep ring of the smallest tiles of which that holds (bf16, us on the GPU, the best of the other
+    // instances / this): 64 x 64 x 128 512 x 512 x 2048 10.4 / 9.2, 130 x 4096 x 4096 19.2 / 15.8, 1000 x 1000 x 16384 80.5 / 58.2; 64 x 128 x 64
+    // 1024 x 2048 x 2048 15.2 / 12.9, 70 x 14336 x 2048 16.6 / 15.3; 128 x 128 x 64 2048 x 2048 x 4096 47.2 / 32.1, 1500 x 2048 x 512 10.1 / 7.3.
+    // Where the next smaller tiles fit too, or a ring of them would be filled but a few times, the larger ones only leave more CUs idle: 276 x 128
+    // x 384 3.9 on 64 x 64 x 64, 4.7 on 64 x 128, 5.7 on 128 x 128; 720 x 448 x 832 4.8, 5.4 on 64 x 64 x 128, 6.1 on 64 x 128; 34 x 2944 x 1792 6.2,
+    // 6.9; 361 x 776 x 1920 9.8, 8.6.  (660 products: where the limits are, 0.99 of the time of 64 x 64 x 64 below 257 tiles of that size.)
+    // More tiles: 384 of 128 x 128, 700 x 8192 x 2048 35.7 / 34.4, but 1024 of them with a K of 256 17.3 / 18.0, so that the rules below keep those.
+    struct DeepRule { int instance, min_k, min_tiles; };
+    for (const DeepRule &rule : {DeepRule{kDeep64x64x128, 1920, 48}, DeepRule{kDeep64x128x64, 320, 1}, DeepRule{kDeep128x128x64, 256, 1}}) {
         const GemmInstance &inst = kInstances[rule.instance];
-        const int64_t per_matrix = (int64_t)((q.m + inst.bm - 1) / inst.bm) * ((q.n + inst.bn - 1) / inst.bn);
-        if (q.k >= rule.min_k && per_matrix * q.batch <= 256 && inst.accepts(q)) return rule.instance;
+        const int64_t tiles = (int64_t)((q.m + inst.bm - 1) / inst.bm) * ((q.n + inst.bn - 1) / inst.bn) * q.batch;
+        if (tiles > 256) continue;
+        if (q.k >= rule.min_k && tiles >= rule.min_tiles && inst.accepts(q)) return rule.instance;
+        break;
     }
     // (an instance with tails accepts what its plain form accepts, so it comes right after it: a partial
     // last tile costs less than a smaller tile everywhere)

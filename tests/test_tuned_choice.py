@@ -53,6 +53,28 @@ def test_candidates_at_the_callers_pace(choose):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize(
+    "m, n, k, tile",
+    (
+        (276, 128, 384, "64x64x64"), (1024, 1024, 1856, "64x64x64"), (1024, 1024, 1920, "64x64x128"), (384, 448, 1920, "64x64x64"),  # 10, 256 and 42 tiles of 64 x 64
+        (1088, 1024, 256, "64x64x64"), (1088, 1024, 320, "64x128x64"), (1024, 2048, 2048, "64x128x64"),  # 272 of them, 136 and 256 of 64 x 128
+        (1500, 2048, 512, "128x128x64"), (2048, 2048, 256, "128x128x64"),
+    ),
+)  # fmt: skip
+def test_untuned_choice_of_tiles_that_the_chip_holds(m, n, k, tile):
+    tag = runtime.DATA_TYPE_INDEX["bf16"]
+    lhs, rhs = torch.randn(m, k, device="cuda", dtype=torch.bfloat16), torch.randn(k, n, device="cuda", dtype=torch.bfloat16)
+    out = torch.full((m, n), float("nan"), device="cuda", dtype=torch.bfloat16)
+    arguments = [runtime.ArgumentTensor.from_torch_tensor(t) for t in (lhs, rhs, out)]
+    assert runtime.library().nt_tune_cache_lookup(tag, tag, m, n, k, 0) < 0
+    runtime.check(runtime.library().launch_nt_matmul(runtime.current_stream(), *arguments, tag, tag, 0, 0, 0))
+    assert f": {tile} " in runtime.last_launch() and "split-k" not in runtime.last_launch(), runtime.last_launch()
+    expected = lhs.double() @ rhs.double()
+    bound = 2.0**-8 * expected.abs() + (k + 4) * 2.0**-24 * (lhs.double().abs() @ rhs.double().abs())
+    assert ((out.double() - expected).abs() <= bound).all()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("m, n, k", ((1024, 2560, 264), (2001, 2432, 520)))  # 160 and 304 tiles of 128 x 128
 @pytest.mark.parametrize("bk", (64, 32))
 def test_two_parts_of_more_tiles_than_the_chip_holds(m, n, k, bk):
