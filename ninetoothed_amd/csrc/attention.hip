@@ -303,8 +303,9 @@ __global__ __launch_bounds__(kWaves * 64, kOcc) void attention_fwd_kernel(Attent
     // large for the element type) or the row sees its first key, the maximum is found, the reference moved to it and the
     // probabilities computed again; a block as high as the one that set the reference adds up to at most 32 per lane.  A
     // sixth of the loop's vector arithmetic, and no chain of maxima between the scores and the exponentials.  For head
-    // dimension 64, where that arithmetic takes as long as the MFMAs: bf16 [8, 16, 1000, 64] 42.0 -> 39.1 us, [2, 8, 1500, 64] 21.3 ->
-    // 16.6, causal fp16 [1, 16, 4096, 64] 54.3 -> 45.7.  At 128 the scores have to outlive the exponentials in registers
+    // dimension 64, where that arithmetic takes longer than the MFMAs: bf16 [8, 16, 1000, 64] 42.0 -> 39.1 us, [2, 8, 1500, 64] 21.3 ->
+    // 16.6, causal fp16 [1, 16, 4096, 64] 54.3 -> 45.7.  Scores that rise by more than eight powers of two from block to block (a query along the
+    // keys' drift) are computed twice in every block: causal bf16 [4, 16, 2048, 64], 200 powers of two over the keys, 64 -> 82, ordinary ones 50 -> 45.  At 128 the scores have to outlive the exponentials in registers
     // that are not there: [4, 32, 4096, 128] 920 -> 955, so that one keeps looking.
     constexpr bool kLazyMax = kFold && kPipelined && D == 64;
     constexpr float kFoldSlack = kLazyMax ? 0.0f : 8.0f;
