@@ -225,7 +225,7 @@ NineToothedResult launch_nt_attention(NineToothedStream stream,
  * dilation 1 (launch_nt_conv2d_strided takes others) and zero padding (padding_h, padding_w), computed as the implicit
  * GEMM [N*P*Q, C*R*S] x [C*R*S, K] the arrangement of
  * tests/test_conv2d.py:13-48 describes.
- * Ways to run it, tried in this order unless block_size_m names one (4, 3, 2, 1)
+ * Ways to run it, tried in this order unless block_size_m names one (4, 3, 5, 2, 1)
  * or nt_tune_conv2d has recorded one for the problem:
  * 4 -- 1 x 1 filters without padding (P*Q and C multiples of 8): one batched
  *   launch of the GEMM kernels on the tensors as they lie, without scratch;
@@ -234,6 +234,9 @@ NineToothedResult launch_nt_attention(NineToothedStream stream,
  *   tap)-shifted pixel runs of the NCHW input; needs an output width that is a
  *   multiple of 8, padding_w <= 1, C*R*S a multiple of 32, R*S / gcd(32, R*S) <= 25, pixels of an input row
  *   contiguous, contiguous filter and output, K filling 256-wide tiles to 4/5;
+ * 5 -- 3 x 3 filters, C >= 32 a multiple of 8, positions of a channel and each filter's values contiguous, input windows of 224 output
+ *   positions that fit LDS: one launch, no scratch memory, a workgroup reads its input rows once for all taps.  Without
+ *   block_size_m = 5 taken only where way 2 is expected to be slower;
  * 2 -- fp16 / bf16 tensors of any strides (a contiguous NCHW output is stored in
  *   16-byte pieces of 8 positions, a channels-last one in pieces of 8 channels,
  *   any other element by element): the
@@ -263,8 +266,8 @@ NineToothedResult launch_nt_conv2d(NineToothedStream stream,
  * dilation_w))` (src/ninetoothed/tensor.py:199-286).  The output holds, per dimension, either the windows that fit
  * (`floor_mode=True`: (H + 2 padding - dilation (R - 1) - 1) / stride + 1, rounded down) or one more that hangs over
  * the edge (`Tensor.tile`'s default rounds up; what hangs over reads as padding); other sizes are rejected.
- * Steps of 1 with the fitting output are launch_nt_conv2d.  Otherwise way 2 (repacking pass plus GEMM loop, same
- * conditions and scratch buffers) or way 1 (gather kernel) runs; block_size_m = 2 or 1 names one. */
+ * Steps of 1 with the fitting output are launch_nt_conv2d.  Otherwise way 5, way 2 (repacking pass plus GEMM loop) --
+ * same conditions and scratch buffers -- or way 1 (gather kernel) runs; block_size_m = 5, 2 or 1 names one. */
 NineToothedResult launch_nt_conv2d_strided(NineToothedStream stream,
                                            NineToothedTensor input,
                                            NineToothedTensor filter,
@@ -391,7 +394,7 @@ NineToothedResult nt_tune_attention(NineToothedStream stream,
                                     int dtype, int iters, int *best_variant, float *best_ms);
 
 /* As nt_tune_gemm for launch_nt_conv2d: times the ways to run the convolution -- 4 = a 1 x 1 filter as a batch of
- * plain products, 3 = one launch on the tensors as they lie, 2 = repacking pass plus GEMM loop, 1 = gather kernel; a
+ * plain products, 3 = one launch on the tensors as they lie, 5 = one launch with input windows in LDS, 2 = repacking pass plus GEMM loop, 1 = gather kernel; a
  * way that does not take the problem is skipped -- and records the fastest (the block_size_m value that selects
  * it) for later launches of the same problem with block_size_m = 0; a way that needs scratch memory or more
  * launches replaces one before it in that order only when it is more than 3 % faster.  *best_path = -1 when

@@ -18,7 +18,7 @@ PACKAGE_DIR = pathlib.Path(__file__).resolve().parent
 CSRC_DIR = PACKAGE_DIR / "csrc"
 LIBRARY_PATH = PACKAGE_DIR / "lib" / "libnt_hip.so"
 
-SOURCES = ("gemm_api.hip", "conv2d.hip", "softmax.hip", "attention.hip", "map.hip", "workspace.hip", "tune.hip")
+SOURCES = ("gemm_api.hip", "conv2d.hip", "conv2d_window.hip", "softmax.hip", "attention.hip", "map.hip", "workspace.hip", "tune.hip")
 
 # Measurement aids (MFMA issue-rate kernels that bench.py times next to the programs) are no part of the C ABI:
 # they are built into a library of their own that only bench.py loads.

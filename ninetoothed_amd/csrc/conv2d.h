@@ -6,9 +6,8 @@
 
 namespace nt {
 
-// the ways to run a convolution; kConvAuto tries them from the top (a 1 x 1 filter without padding first runs
-// as a batch of plain products when it can)
-enum ConvPath { kConvAuto = 0, kConvGather = 1, kConvRepack = 2, kConvDirect = 3, kConvPointwise = 4 };
+// the ways to run a convolution; kConvAuto tries kConvPointwise, kConvDirect, kConvWindow (where it pays), kConvRepack and kConvGather, in this order
+enum ConvPath { kConvAuto = 0, kConvGather = 1, kConvRepack = 2, kConvDirect = 3, kConvPointwise = 4, kConvWindow = 5 };
 
 struct Conv2dRequest {
     int dtype;
@@ -31,5 +30,18 @@ int conv2d_fast(const Conv2dRequest &request, hipStream_t stream);
 // C*R*S a multiple of 32, contiguous filter and output, output channels filling 256-wide tiles --; returns
 // NINETOOTHED_NO_KERNEL when it does not.
 int conv2d_direct(const Conv2dRequest &request, hipStream_t stream);
+
+// Runs the convolution in one launch with input windows in LDS, no scratch memory, when the request qualifies; returns
+// NINETOOTHED_NO_KERNEL when it does not, or (if_it_pays) when the repacking path is expected to be as fast.
+int conv2d_window(const Conv2dRequest &request, hipStream_t stream, bool if_it_pays = false);
+
+// The expected time of the repacking path, in microseconds.
+float conv2d_repacked_time(const Conv2dRequest &request);
+
+// 1: the output is a contiguous NCHW tensor on a 16-byte boundary; 2: its channels are its innermost dimension; 0: any strides.
+inline int conv2d_dense_output(const Conv2dRequest &q) {
+    if (q.ys[3] == 1 && q.ys[2] == q.Q && q.ys[1] == (int64_t)q.P * q.Q && q.ys[0] == (int64_t)q.K * q.P * q.Q && ((uintptr_t)q.y & 15) == 0) return 1;
+    return q.ys[1] == 1 && q.K > 1 ? 2 : 0;
+}
 
 }  // namespace nt

@@ -1,4 +1,5 @@
-// conv2d (zero padding; (1) steps and dilation of 1, (2) any) as implicit GEMM on the MFMA main loop of gemm_fast.h.  Two paths:
+// conv2d (zero padding; (1) steps and dilation of 1, (2) any) as implicit GEMM on the MFMA main loop of gemm_fast.h.  Two paths (a third, one
+// launch for small and strided layers, is in conv2d_window.hip):
 //
 // (1) conv2d_direct: one launch on the tensors as they lie, no scratch memory (described with its kernel
 //     below); needs an output width that is a multiple of 8, padding_w <= 1, C*R*S a multiple of 32, a contiguous
@@ -36,6 +37,7 @@
 #include <algorithm>
 
 #include "conv2d.h"
+#include "conv2d_store.h"
 #include "gemm_fast.h"
 #include "tune.h"
 #include "workspace.h"
@@ -53,6 +55,7 @@ struct ConvParams {
                               // innermost dimension (channels last); 0: any strides, stored element by element
     int64_t ys[4];            // element strides of the output
     int M, tiles_m, tiles_n;  // M = N*P*Q rows
+    float one_by_pq;          // 1.0f / (P*Q)
     unsigned xt_bytes, wt_bytes;
     int stride_h, stride_w, dil_h, dil_w;  // steps of the window over the input and between its taps
     int parts, kt_per_part;  // the contraction dealt to parts: this many, k steps of 32 each (1: not dealt)
@@ -446,15 +449,13 @@ __global__ __launch_bounds__(WM *WN * 64, kOcc) void conv2d_nhwc_kernel(ConvPara
         return;
     }
 
-    // ---- epilogue: lane holds, per 16x16 block, output channel i16 and rows 4 * kg + 0 .. 3 ----
-    // slab layout [kSlabChannels][kWaveM rows], 16-byte chunks swizzled by channel, in the A stages
+    // ---- epilogue: through slabs of LDS in the A stages ----
     constexpr int kSlabBlocks = TN < 2 ? 1 : 2;
     constexpr int kSlabChannels = 16 * kSlabBlocks;
     constexpr int kRowBytes = kWaveM * 2;
     constexpr int kSlabBytes = kSlabChannels * kRowBytes;
-    constexpr int kChunks = kWaveM / 8;
     constexpr int kSlabsPerStage = kStageA / kSlabBytes;
-    static_assert(kStageA % kSlabBytes == 0 && kWaves <= (kStages < 4 ? kStages : 4) * kSlabsPerStage && TN % kSlabBlocks == 0 && kWaveM % 32 == 0, "slabs in the first four A stages");
+    static_assert(kStageA % kSlabBytes == 0 && kWaves <= (kStages < 4 ? kStages : 4) * kSlabsPerStage, "slabs in the first four A stages");
     NT_LDS unsigned char *slab;
     {
         const int which = wave / kSlabsPerStage;
@@ -464,90 +465,7 @@ __global__ __launch_bounds__(WM *WN * 64, kOcc) void conv2d_nhwc_kernel(ConvPara
                             : stage_a(std::integral_constant<int, kStages < 4 ? 0 : 3>());
         slab += (wave % kSlabsPerStage) * kSlabBytes;
     }
-    T *Y = (T *)p.y;
-    const bool whole_chunks = PQ % 8 == 0 && p.dense_out == 1;
-#pragma unroll
-    for (int tg = 0; tg < TN / kSlabBlocks; ++tg) {
-#pragma unroll
-        for (int tb = 0; tb < kSlabBlocks; ++tb)
-#pragma unroll
-            for (int ti = 0; ti < TM; ++ti) {
-                typedef T vec4 __attribute__((ext_vector_type(4)));
-                vec4 v;
-#pragma unroll
-                for (int e = 0; e < 4; ++e) v[e] = E::from_float(acc[ti][tg * kSlabBlocks + tb][e]);
-                const int channel = tb * 16 + i16;
-                const int chunk = (ti * 2 + (kg >> 1)) ^ (channel & (kChunks - 1));
-                *(NT_LDS vec4 *)(slab + channel * kRowBytes + chunk * 16 + 8 * (kg & 1)) = v;
-            }
-        const int first_channel = n0 + wave_n * kWaveN + tg * kSlabChannels;
-        if (p.dense_out == 2) {
-            // channels-last output: a lane gathers 8 channels of one row from the slab and stores them with one
-            // instruction (the channels of the slab are 32 or 64 consecutive bytes of the tensor)
-            constexpr int kGroups = kSlabChannels / 8;
-#pragma unroll
-            for (int it = 0; it < kGroups * kWaveM / 64; ++it) {
-                const int idx = it * 64 + lane;
-                const int row = idx / kGroups, first = (idx % kGroups) * 8;
-                vec8 v;
-#pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    const int channel = first + e;
-                    v[e] = *(const NT_LDS T *)(slab + channel * kRowBytes + (((row >> 3) ^ (channel & (kChunks - 1))) * 16) + (row & 7) * 2);
-                }
-                const int m = m0 + wave_m * kWaveM + row;
-                const int out_channel = first_channel + first;
-                if (m >= p.M || out_channel >= p.K) continue;
-                const int image = m / PQ, pq = m - image * PQ;
-                const int oy = pq / p.Q, ox = pq - oy * p.Q;
-                T *to = Y + (int64_t)image * p.ys[0] + (int64_t)oy * p.ys[2] + (int64_t)ox * p.ys[3] + out_channel;
-                if (out_channel + 8 <= p.K) {
-                    typedef vec8 unaligned_vec8 __attribute__((aligned(2)));
-                    *(unaligned_vec8 *)to = v;
-                } else {
-#pragma unroll
-                    for (int e = 0; e < 8; ++e)
-                        if (out_channel + e < p.K) to[e] = v[e];
-                }
-            }
-            continue;
-        }
-#pragma unroll
-        for (int it = 0; it < (kSlabChannels * kChunks) / 64; ++it) {
-            const int idx = it * 64 + lane;
-            const int channel = idx / kChunks;
-            const int phys = idx % kChunks;
-            const int chunk = phys ^ (channel & (kChunks - 1));
-            vec8 v = *(const NT_LDS vec8 *)(slab + channel * kRowBytes + phys * 16);
-            const int m = m0 + wave_m * kWaveM + chunk * 8;
-            if (m >= p.M) continue;
-            const int out_channel = first_channel + channel;
-            if (out_channel >= p.K) continue;  // a partial last tile of output channels
-            int image = m / PQ, pq = m - image * PQ;
-            if (whole_chunks) {  // the 8 rows lie in one image and start at a multiple of 8
-                __builtin_nontemporal_store(v, (vec8 *)(Y + ((int64_t)image * p.K + out_channel) * PQ + pq));  // +2 % over a plain store
-            } else if (p.dense_out == 1 && pq + 8 <= PQ && m + 8 <= p.M) {
-                // the 8 rows lie in one image, only not on a 16-byte boundary (a 7 x 7 map): one store all the same
-                // (global accesses need the element's alignment only)
-                typedef vec8 unaligned_vec8 __attribute__((aligned(2)));
-                *(unaligned_vec8 *)(Y + ((int64_t)image * p.K + out_channel) * PQ + pq) = v;
-            } else {
-                // (any output strides: a channels-last tensor, a slice of a wider one)
-                int oy = pq / p.Q, ox = pq - oy * p.Q;
-#pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    if (m + e < p.M) Y[(int64_t)image * p.ys[0] + (int64_t)out_channel * p.ys[1] + (int64_t)oy * p.ys[2] + (int64_t)ox * p.ys[3]] = v[e];
-                    if (++ox == p.Q) {
-                        ox = 0;
-                        if (++oy == p.P) {
-                            oy = 0;
-                            ++image;
-                        }
-                    }
-                }
-            }
-        }
-    }
+    store_conv_tile<T, TM, TN, kSlabBlocks>(p, acc, slab, m0 + wave_m * kWaveM, n0 + wave_n * kWaveN, lane);
 #endif
 }
 
@@ -1212,6 +1130,7 @@ constexpr int kConv128x128 = 0, kConv128x64 = 1;  // the tiles for up to 16 chan
 
 struct ConvChoice {
     int tile, parts;
+    float time;
 };
 
 // The tile and the number of parts of the contraction with the least expected time.  Parts pay where few workgroups would
@@ -1221,8 +1140,7 @@ struct ConvChoice {
 // filters of 1 x 1, step 2: 18.0 us on 128 x 128 tiles, 13.8 on 64 x 64).
 ConvChoice conv2d_choose(int64_t rows, int64_t filters, int steps, bool scattered, int max_parts) {
     const int64_t units = std::max(1, compute_units());
-    ConvChoice best = {0, 1};
-    float best_time = 0.0f;
+    ConvChoice best = {0, 1, 0.0f};
     bool found = false;
     for (int t = 0; t < (int)(sizeof(kConvTiles) / sizeof(kConvTiles[0])); ++t) {
         const ConvTile &tile = kConvTiles[t];
@@ -1236,10 +1154,9 @@ ConvChoice conv2d_choose(int64_t rows, int64_t filters, int steps, bool scattere
             const float values = (float)(tile.m * tile.n) / 8192.0f;
             const float time = (float)per_part * std::max(tile.alone, rounds * tile.shared) + 0.66f * rounds * values +
                                (parts > 1 ? 2.4f + (float)scratch / 2.7e6f : scattered ? 3.9f * values : 0.0f);
-            if (!found || time < best_time) {
+            if (!found || time < best.time) {
                 found = true;
-                best = {t, parts};
-                best_time = time;
+                best = {t, parts, time};
             }
         }
     }
@@ -1296,17 +1213,17 @@ int run_fast(const Conv2dRequest &q, hipStream_t stream) {
     p.y = q.y;
     p.N = q.N; p.C = Cp; p.H = q.H; p.W = q.W; p.K = q.K; p.R = q.R; p.S = q.S; p.P = q.P; p.Q = q.Q;
     p.Kp = Kp;
-    p.dense_out = q.ys[3] == 1 && q.ys[2] == q.Q && q.ys[1] == (int64_t)q.P * q.Q && q.ys[0] == (int64_t)q.K * q.P * q.Q && ((uintptr_t)q.y & 15) == 0;
-    if (!p.dense_out && q.ys[1] == 1 && q.K > 1) p.dense_out = 2;
+    p.dense_out = conv2d_dense_output(q);
     for (int d = 0; d < 4; ++d) p.ys[d] = q.ys[d];
     p.stride_h = q.stride_h; p.stride_w = q.stride_w; p.dil_h = q.dil_h; p.dil_w = q.dil_w;
     p.pad_h = q.pad_h; p.pad_w = q.pad_w;
     p.M = q.N * q.P * q.Q;
+    p.one_by_pq = 1.0f / (float)(q.P * q.Q);
     p.xt_bytes = (unsigned)xt_bytes;
     p.wt_bytes = (unsigned)wt_bytes;
     const int steps = ceil_div(Cp * q.R * q.S, 32);
     const bool scattered = p.dense_out == 0 || (p.dense_out == 1 && q.P * q.Q % 8 != 0);
-    ConvChoice choice = Cp < 32 ? ConvChoice{conv2d_narrow_tile(p.M, q.K), 1} : conv2d_choose(p.M, q.K, steps, scattered, kConvMaxParts);
+    ConvChoice choice = Cp < 32 ? ConvChoice{conv2d_narrow_tile(p.M, q.K), 1, 0.0f} : conv2d_choose(p.M, q.K, steps, scattered, kConvMaxParts);
     p.scratch = nullptr;
     if (choice.parts > 1) {
         const ConvTile &tile = kConvTiles[choice.tile];
@@ -1360,6 +1277,14 @@ int conv2d_fast(const Conv2dRequest &q, hipStream_t stream) {
     // fetch their 16 values of a k step one after another: [2, 32, 9, 9] * [16, 32, 3, 3] 48 against 13 us)
     if ((int64_t)q.N * q.P * q.Q < 1) return NINETOOTHED_NO_KERNEL;
     return q.dtype == NINETOOTHED_FLOAT16 ? run_fast<half_t>(q, stream) : run_fast<bf16_t>(q, stream);
+}
+
+float conv2d_repacked_time(const Conv2dRequest &q) {
+    const int Cp = conv2d_padded_channels(q.C);
+    const int dense = conv2d_dense_output(q);
+    const ConvChoice choice = conv2d_choose((int64_t)q.N * q.P * q.Q, q.K, ceil_div(Cp * q.R * q.S, 32), dense == 0 || (dense == 1 && q.P * q.Q % 8 != 0), kConvMaxParts);
+    const float moved = (float)(q.C + Cp) * ((float)q.N * q.H * q.W + (float)q.K * q.R * q.S) * 2e-6f;  // by the repacking pass, in megabytes
+    return 6.3f + 1.18f * choice.time + 0.2f * moved;
 }
 
 int conv2d_direct(const Conv2dRequest &q, hipStream_t stream) {

@@ -1242,7 +1242,7 @@ int nt_tune_cache_lookup(int dtype, int output_dtype, int m, int n, int k, int a
 namespace nt {
 namespace {
 
-bool conv2d_choice_known(int index, const int *, int) { return index >= kConvGather && index <= kConvPointwise; }
+bool conv2d_choice_known(int index, const int *, int) { return index >= kConvGather && index <= kConvWindow; }
 const bool g_conv2d_check_registered = tune_register_check(kTuneConv2d, conv2d_choice_known);
 
 // validates the call and fills the request; returns 0, an error, or -1 when there is nothing to compute
@@ -1355,6 +1355,10 @@ int conv2d_run(const Conv2dRequest &r, int path, hipStream_t stream) {
         const int direct = conv2d_direct(r, stream);
         if (direct != NINETOOTHED_NO_KERNEL || path == kConvDirect) return direct;
     }
+    if (path == kConvAuto || path == kConvWindow) {
+        const int window = conv2d_window(r, stream, path == kConvAuto);
+        if (window != NINETOOTHED_NO_KERNEL || path == kConvWindow) return window;
+    }
     if (path == kConvAuto || path == kConvRepack) {
         const int fast = conv2d_fast(r, stream);
         if (fast != NINETOOTHED_NO_KERNEL || path == kConvRepack) return fast;
@@ -1383,13 +1387,13 @@ NineToothedResult launch_nt_conv2d(NineToothedStream stream, NineToothedTensor i
     const int status = conv2d_request(request, input, filter, output, dtype, padding_h, padding_w);
     if (status != 0) return status < 0 ? 0 : status;
     // block_size_m: 1 = the gather kernel, 2 = the repacking path, 3 = the one-launch path, 4 = a 1 x 1 filter as a
-    // batch of plain products; otherwise the tuned choice for this problem, else the library's order
-    int path = block_size_m >= kConvGather && block_size_m <= kConvPointwise ? block_size_m : kConvAuto;
+    // batch of plain products, 5 = input windows in LDS; otherwise the tuned choice for this problem, else the library's order
+    int path = block_size_m >= kConvGather && block_size_m <= kConvWindow ? block_size_m : kConvAuto;
     if (block_size_m == 0) {
         int values[11];
         conv2d_tune_values(request, values);
         const int tuned = tune_lookup(kTuneConv2d, values, 11);
-        if (tuned >= kConvGather && tuned <= kConvPointwise) path = tuned;
+        if (tuned >= kConvGather && tuned <= kConvWindow) path = tuned;
     }
     int result = conv2d_run(request, path, (hipStream_t)stream);
     // (a tuned path that needs scratch memory it cannot get, e.g. under graph capture: the library's order)
@@ -1413,8 +1417,8 @@ NineToothedResult launch_nt_conv2d_strided(NineToothedStream stream, NineToothed
     Conv2dRequest request;
     const int status = conv2d_request(request, input, filter, output, dtype, padding_h, padding_w, stride_h, stride_w, dilation_h, dilation_w);
     if (status != 0) return status < 0 ? 0 : status;
-    // the ways that take windows with steps: 2 = repacking pass plus GEMM loop, 1 = gather kernel (nothing is tuned here)
-    const int path = block_size_m == kConvGather || block_size_m == kConvRepack ? block_size_m : kConvAuto;
+    // the ways that take windows with steps: 5 = input windows in LDS, 2 = repacking pass plus GEMM loop, 1 = gather kernel (nothing is tuned here)
+    const int path = block_size_m == kConvGather || block_size_m == kConvRepack || block_size_m == kConvWindow ? block_size_m : kConvAuto;
     int result = conv2d_run(request, path, (hipStream_t)stream);
     if (result == NINETOOTHED_NO_KERNEL && path == kConvRepack) result = conv2d_run(request, kConvGather, (hipStream_t)stream);
     return result;
@@ -1429,11 +1433,11 @@ NineToothedResult nt_tune_conv2d(NineToothedStream stream, NineToothedTensor inp
     if (status != 0) return status < 0 ? 0 : status;
     int values[11];
     conv2d_tune_values(request, values);
-    const int paths[4] = {kConvPointwise, kConvDirect, kConvRepack, kConvGather};
+    const int paths[5] = {kConvPointwise, kConvDirect, kConvWindow, kConvRepack, kConvGather};
     int best = -1;
     float best_time = 0.0f;
-    // an earlier way stays unless a later one is more than 3 % faster: the first two need no scratch memory and one launch
-    const int result = tune_time((hipStream_t)stream, 4, iters, [&](int i) -> int { return conv2d_run(request, paths[i], (hipStream_t)stream); }, &best, &best_time, 0.03f);
+    // an earlier way stays unless a later one is more than 3 % faster: the first three need no scratch memory and one launch
+    const int result = tune_time((hipStream_t)stream, 5, iters, [&](int i) -> int { return conv2d_run(request, paths[i], (hipStream_t)stream); }, &best, &best_time, 0.03f);
     if (result != 0) return result;
     if (best < 0) return 0;  // (a stream under graph capture: nothing was timed)
     tune_record(kTuneConv2d, values, 11, paths[best]);
