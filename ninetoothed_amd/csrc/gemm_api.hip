@@ -498,6 +498,10 @@ hipError_t generic_launch(const GemmProblem &q, hipStream_t stream) {
     return f32out ? generic_launch_typed<bf16_t, float>(q, stream) : generic_launch_typed<bf16_t, bf16_t>(q, stream);
 }
 
+int heuristic_choice(const GemmProblem &q, int bm, int bn, int bk);
+template <bool kColumns> bool cut_accepts(const GemmProblem &q);
+template <bool kColumns> hipError_t cut_launch(const GemmProblem &q, hipStream_t stream);
+
 // BM, BN, BK, wave grid WM x WN, LDS stages, waves per SIMD the register budget allows
 #define NT_FAST_INSTANCE(BM, BN, BK, WM, WN, ST, OCC) \
     {#BM "x" #BN "x" #BK " waves " #WM "x" #WN " stages " #ST " lds-direct", BM, BN, BK, fast_accepts<BM, BN, BK, ST>, fast_launch<BM, BN, BK, WM, WN, ST, OCC>}
@@ -514,6 +518,7 @@ enum InstanceIndex {
     kAnyStride, k256x256x32, k256x256x64, k128x128x64, k64x64x64, k128x256x32,
     kTail256x256x32, kTail128x256x32, kTail128x128x64, kTail64x64x64, kSplit64x64x64, kSplit128x128x64,
     kSplit128x256x32, kSplit256x256x32, kSkinny16, kSkinny32, kDeep128x128x64, kDeep64x64x128, kDeep64x128x64,
+    kCutColumns, kCutRows,
 };
 
 const GemmInstance kInstances[] = {
@@ -538,6 +543,8 @@ const GemmInstance kInstances[] = {
     NT_TAIL_INSTANCE(128, 128, 64, 2, 4, 4, 2),
     NT_TAIL_INSTANCE(64, 64, 128, 2, 2, 4, 1),
     NT_TAIL_INSTANCE(64, 128, 64, 2, 4, 5, 2),
+    {"256x256x32 for whole rounds of the chip, the columns left on their own (smaller tiles or split-k)", 256, 256, 32, cut_accepts<true>, cut_launch<true>},
+    {"256x256x32 for whole rounds of the chip, the rows left on their own (smaller tiles or split-k)", 256, 256, 32, cut_accepts<false>, cut_launch<false>},
 #ifdef NT_GEMM_ABLATION
 #define NT_LOAD_INSTANCE(BM, BN, BK, WM, WN, ST, OCC, LD, AUX) \
     {#BM "x" #BN "x" #BK " waves " #WM "x" #WN " stages " #ST " load " #LD " aux " #AUX, BM, BN, BK, fast_accepts<BM, BN, BK, ST>, fast_launch<BM, BN, BK, WM, WN, ST, OCC, 0, LD, AUX>}
@@ -554,9 +561,10 @@ const GemmInstance kInstances[] = {
 #endif
 };
 constexpr int kNumInstances = sizeof(kInstances) / sizeof(kInstances[0]);
-static_assert(kNumInstances > kDeep64x128x64, "InstanceIndex names the first instances of the table");
+static_assert(kNumInstances > kCutRows, "InstanceIndex names the first instances of the table");
 
 inline bool is_split(int instance) { return instance >= kSplit64x64x64 && instance <= kSplit256x256x32; }
+inline bool is_cut(int instance) { return instance == kCutColumns || instance == kCutRows; }
 
 // choices read from a tuning file: an instance index counts only together with the block sizes saved next to it
 bool gemm_choice_known(int index, const int *extra, int extras) {
@@ -599,6 +607,70 @@ int skinny_choice(const GemmProblem &q) {
     if (q.k < (q.m <= 48 ? 1024 : 2048)) return -1;
     if (q.n <= 4096) return q.m <= 48 || !long_k || q.n <= 1024 ? (int)kSkinny16 : -1;
     return q.n <= 8192 && q.k > 2048 && !long_k ? (int)kSkinny32 : -1;
+}
+
+// ---- tiles over whole rounds of the chip ----
+// 336 tiles of 256 x 256 on 256 CUs take two rounds, the second with 80 CUs at work.  The columns (or rows) of tiles that fill whole
+// rounds run in one launch, what is left as a product of its own before it: K in parts where it has few tiles, else 128 x 128 tiles on a deep ring,
+// of which up to two rounds (128 tiles of 256 x 256 left) still take less time than another round of large ones.  Both launches read one operand whole: the
+// smaller one (rows cut off 1500 x 14336 x 4096 read its rhs of 117 MB twice: 168 us with inputs that come from memory, 144 with them in the caches).
+// One launch of 256 x 256 tiles / this, bf16, us, sustained with changing inputs: 1500 x 14336 x 4096 (84 tiles left) 169 / 156, 4608 x 4608 x 4096 (72) 153 /
+// 148, 1314 x 15104 x 13688 (102) 815 / 667, 1571 x 12672 x 1128 (98) 59.2 / 59.4; single products: 2079 x 9088 x 3264 (72) 132 / 104, 1153 x
+// 14208 x 12736 (25) 483 / 354, 4635 x 4736 x 12544 (114) 467 / 432, 2470 x 9536 x 1280 (130) 57.7 / 55.8; more left: 2311 x 11328 x 3136 (200) 130 / 139.
+// Of a short K, 2967 x 7872 x 512 (120) 31.9 / 28.9, but 2058 x 7680 x 512 (18) has 19.3 on 128 x 256 tiles against 22, which only the tuner knows.
+template <bool kColumns>
+int64_t cut_whole(const GemmProblem &q) {  // columns (rows) of 256 x 256 tiles that fill whole rounds
+    const int64_t along = ceil_div(kColumns ? q.n : q.m, 256), across = ceil_div(kColumns ? q.m : q.n, 256);
+    return along * across / 256 * 256 / across;
+}
+
+template <bool kColumns>
+int64_t cut_left(const GemmProblem &q) {  // 256 x 256 tiles that do not
+    return (ceil_div(kColumns ? q.n : q.m, 256) - cut_whole<kColumns>(q)) * ceil_div(kColumns ? q.m : q.n, 256);
+}
+
+template <bool kColumns>
+void cut_problem(const GemmProblem &q, GemmProblem &whole, GemmProblem &left) {
+    const int64_t size = 2, out_size = q.out_dtype == NINETOOTHED_FLOAT32 ? 4 : 2;
+    const int64_t at = cut_whole<kColumns>(q) * 256;
+    whole = left = q;
+    if (kColumns) {
+        whole.n = (int)at;
+        left.n = q.n - whole.n;
+        left.b = (const char *)q.b + at * q.sbn * size;
+        left.c = (char *)q.c + at * q.scn * out_size;
+        if (q.bias != nullptr) left.bias = (const char *)q.bias + at * q.sin * size;
+        if (q.column_bias != nullptr) left.column_bias = (const char *)q.column_bias + at * q.sin * (q.bias_float ? 4 : size);
+    } else {
+        whole.m = (int)at;
+        left.m = q.m - whole.m;
+        left.a = (const char *)q.a + at * q.sam * size;
+        left.c = (char *)q.c + at * q.scm * out_size;
+        if (q.bias != nullptr) left.bias = (const char *)q.bias + at * q.sim * size;
+    }
+}
+
+template <bool kColumns>
+bool cut_accepts(const GemmProblem &q) {
+    if ((q.dtype != NINETOOTHED_FLOAT16 && q.dtype != NINETOOTHED_BFLOAT16) || q.batch != 1 || q.hinted || q.fixed_scratch != nullptr || q.m <= 0 || q.n <= 0) return false;
+    const int64_t tiles = (int64_t)ceil_div(q.m, 256) * ceil_div(q.n, 256), whole = cut_whole<kColumns>(q);
+    if (kColumns != (q.m <= q.n) || tiles <= 256 || tiles % 256 == 0 || q.k < 512 || whole < 1 || cut_left<kColumns>(q) > 128) return false;
+    if (tiles > 4 * 256 + 128) return false;  // (what a round costs shrinks to the spread between runs)
+    GemmProblem top, left;
+    cut_problem<kColumns>(q, top, left);
+    return kInstances[kTail256x256x32].accepts(top) && kInstances[kDeep128x128x64].accepts(left);
+}
+
+template <bool kColumns>
+hipError_t cut_launch(const GemmProblem &q, hipStream_t stream) {
+    GemmProblem whole, left;
+    cut_problem<kColumns>(q, whole, left);
+    int rest = (int64_t)ceil_div(left.m, 128) * ceil_div(left.n, 128) <= 256 ? heuristic_choice(left, 0, 0, 0) : (int)kDeep128x128x64;
+    if (rest <= kAnyStride || !kInstances[rest].accepts(left)) rest = kDeep128x128x64;
+    hipError_t result = kInstances[rest].launch(left, stream);  // (first: a split-K instance may find no scratch memory)
+    if ((int)result == NINETOOTHED_NO_KERNEL && is_split(rest)) result = kInstances[kDeep128x128x64].launch(left, stream);
+    if (result != hipSuccess) return result;
+    return kInstances[kInstances[k256x256x32].accepts(whole) ? k256x256x32 : kTail256x256x32].launch(whole, stream);
 }
 
 // Untuned choice: the largest direct-to-LDS tile that still gives every CU a
@@ -653,6 +725,8 @@ int heuristic_choice(const GemmProblem &q, int bm, int bn, int bk) {
         if (q.k >= rule.min_k && tiles >= rule.min_tiles && inst.accepts(q)) return rule.instance;
         break;
     }
+    for (int cut : {(int)kCutColumns, (int)kCutRows})  // (the one of the longer dimension)
+        if (kInstances[cut].accepts(q)) return cut;
     // (an instance with tails accepts what its plain form accepts, so it comes right after it: a partial
     // last tile costs less than a smaller tile everywhere)
     const Rule rules[] = {{k256x256x32, 256}, {k256x256x64, 256}, {kTail256x256x32, 256}, {k128x256x32, 128}, {kTail128x256x32, 128},
@@ -841,8 +915,6 @@ hipError_t repack_operand(hipStream_t stream, const void *src, int64_t d0, int64
     repack_operand_kernel<<<dim3((unsigned)tiles, (unsigned)batch), dim3(256), 0, stream>>>((const uint16_t *)src, d0, d1, s0, s1, dst, pitch, src_batch);
     return hipGetLastError();
 }
-
-int heuristic_choice(const GemmProblem &q, int bm, int bn, int bk);
 
 // Writes the dense copies of q's operands into the stream's buffers (`lease` must stay alive until everything that
 // reads them is enqueued) and describes the product on them in `dense`.  0, an error, or NINETOOTHED_NO_KERNEL when
@@ -1210,7 +1282,7 @@ NineToothedResult nt_tune_gemm_for_caller(NineToothedStream stream_, NineToothed
         const int instance = instance_of(i);
         if (!kInstances[instance].accepts(q)) return NINETOOTHED_NO_KERNEL;
         return (int)kInstances[instance].launch(q, stream);
-    }, &best, &best_time, margin, [&](int i, float measured) { return std::max(measured, is_split(instance_of(i)) ? split_call_ms : call_ms); });
+    }, &best, &best_time, margin, [&](int i, float measured) { return std::max(measured, is_split(instance_of(i)) || is_cut(instance_of(i)) ? split_call_ms : call_ms); });
     if (best >= 0) best = instance_of(best);
     if (best_config) *best_config = best;
     if (best_ms) *best_ms = best_time;
@@ -1333,6 +1405,7 @@ int conv2d_pointwise(const Conv2dRequest &r, hipStream_t stream) {
     q.a_batch = 0;
     q.b_batch = r.xs[0];
     q.c_batch = r.ys[0];
+    q.hinted = true;  // (one launch, no scratch memory)
     const int choice = heuristic_choice(q, 0, 0, 0);
     if (choice <= kAnyStride || is_split(choice)) return NINETOOTHED_NO_KERNEL;
     note_launch(kLaunchConv2d, kConvPointwise, kInstances[choice].name);
