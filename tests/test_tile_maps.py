@@ -1165,3 +1165,21 @@ def test_grouped_elements_in_tile_mode_match_the_interpreter(dtype, monkeypatch)
                 results.append(out)
             assert torch.allclose(results[0].float(), results[1].float(), rtol=2 * ulp, atol=2 * ulp), (rows, cols, kernel.kernel_name)
             assert torch.allclose(results[1].float(), expected, rtol=2e-2, atol=2e-2), (rows, cols, kernel.kernel_name)
+
+
+@gpu
+@pytest.mark.parametrize("dtype", (torch.float32, torch.float16))
+@pytest.mark.parametrize("rows, cols", ((9, 33), (3, 513), (5, 2047), (2, 2049), (7, 7360), (3, 8191), (9, 8200), (2, 16383), (4, 16384)))
+def test_rows_of_no_whole_number_of_elements_per_thread(rows, cols, dtype):
+    """Rows whose last elements only some threads have, in a buffer that holds NaN around every row: an element read from
+    outside a row or counted twice would show.  (fp32: a dozen roundings of 2^-23 along a sum, values below 16; fp16: six of 2^-11.)"""
+    rtol, atol = (1e-5, 1e-5) if dtype == torch.float32 else (6 * 2.0**-11, 6 * 2.0**-11 * 4)
+    for kernel, inputs, expected in _normalisation_cases("cuda", dtype, rows, cols):
+        storage = torch.full((rows, cols + 5), float("nan"), dtype=dtype, device="cuda")
+        input = storage[:, 2 : 2 + cols]
+        input.copy_(inputs[0])
+        out = torch.full((rows, cols + 3), 7.0, dtype=dtype, device="cuda")
+        kernel(input, *inputs[1:], out[:, 1 : 1 + cols])
+        _served_by_map(kernel)
+        assert torch.allclose(out[:, 1 : 1 + cols].float(), expected, rtol=rtol, atol=atol), kernel.kernel_name
+        assert bool((out[:, :1] == 7).all()) and bool((out[:, 1 + cols :] == 7).all())
