@@ -66,3 +66,30 @@ def test_linear_with_bias_activation_and_residual(m, n, k, dtype):
         kernel(lhs, rhs, bias, residual, scale, output)
         assert "launch_nt_matmul" in kernel.last_plan and "launch_nt_map" in kernel.last_plan
         assert torch.allclose(output.float(), expected.float(), rtol=1e-2, atol=1e-2)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("form", ("whole", "odd pitch", "one row", "columns apart", "in place"))
+@pytest.mark.parametrize("m, n, k", ((5, 8, 64), (129, 136, 576), (257, 264, 64), (300, 1000, 128), (2049, 1288, 96), (300, 204, 128)))
+def test_addmm_inputs_at_the_edges_of_tiles(m, n, k, form):
+    """The input's values are asked for before the product is done, those of rows and columns behind the output's last ones from there: NaN
+    around the input would show in the output.  (The product rounds to fp16 before it is combined, the result once more: an ulp each of the largest value, and an ulp where
+    the product's own rounding falls the other way.)"""
+    mat1, mat2 = torch.randn(m, k, device="cuda").half(), (torch.randn(k, n, device="cuda") * k**-0.5).half()
+    values = torch.randn(1 if form == "one row" else m, n, device="cuda").half()
+    if form == "odd pitch":
+        input = torch.full((m, n + 3), float("nan"), dtype=torch.float16, device="cuda")[:, 1 : 1 + n]
+    elif form == "columns apart":
+        input = torch.full((n, m + 1), float("nan"), dtype=torch.float16, device="cuda")[:, :m].t()
+    else:
+        input = torch.empty_like(values)
+    input.copy_(values)
+    if form == "one row":
+        input = input.expand(m, n)
+    output = input if form == "in place" else torch.full((m, n), float("nan"), dtype=torch.float16, device="cuda")
+    kernel = ninetoothed.make(programs.addmm.arrangement, programs.addmm.application, programs.addmm.tensors())
+    kernel(input, mat1, mat2, 0.5, 2.0, output)
+    product = (mat1.double() @ mat2.double()).half().double()
+    expected = 0.5 * values.double() + 2.0 * product
+    ulp = 2.0**-10 * float(expected.abs().max())
+    assert torch.allclose(output.double(), expected, rtol=0, atol=3 * ulp)
