@@ -119,30 +119,49 @@ void fill_params(GemmParams &p, const GemmProblem &q, int bm, int bn) {
     p.bias_batch = q.bias_batch;
 }
 
-template <typename T, int BM, int BN, int BK, int WM, int WN, int kStages, int kOcc, int kAblate, int kLoad, int kAux, bool kTail>
-hipError_t fast_launch_typed(const GemmProblem &q, hipStream_t stream) {
+template <typename T, int BM, int BN, int BK, int WM, int WN, int kStages, int kOcc, int kAblate, int kLoad, int kAux, bool kTail, bool kLines>
+hipError_t fast_launch_form(const GemmProblem &q, hipStream_t stream) {
     GemmParams p;
     fill_params(p, q, BM, BN);
     const dim3 grid(p.tiles_m * p.tiles_n * q.batch), block(WM * WN * 64);
     const bool f32 = q.out_dtype == NINETOOTHED_FLOAT32, addmm = q.addmm();
     if (b_is_transposed(q)) {
-        if (f32) gemm_nn_fast_kernel<T, BM, BN, BK, WM, WN, kStages, kOcc, kPlain, kAblate, kLoad, kAux, true, true, kTail><<<grid, block, 0, stream>>>(p);
-        else if (addmm) gemm_nn_fast_kernel<T, BM, BN, BK, WM, WN, kStages, kOcc, kAddmm, kAblate, kLoad, kAux, false, true, kTail><<<grid, block, 0, stream>>>(p);
-        else if (q.linear) gemm_nn_fast_kernel<T, BM, BN, BK, WM, WN, kStages, kOcc, kLinear, kAblate, kLoad, kAux, false, true, kTail><<<grid, block, 0, stream>>>(p);
-        else gemm_nn_fast_kernel<T, BM, BN, BK, WM, WN, kStages, kOcc, kPlain, kAblate, kLoad, kAux, false, true, kTail><<<grid, block, 0, stream>>>(p);
+        if (f32) gemm_nn_fast_kernel<T, BM, BN, BK, WM, WN, kStages, kOcc, kPlain, kAblate, kLoad, kAux, true, true, kTail, false, kLines><<<grid, block, 0, stream>>>(p);
+        else if (addmm) gemm_nn_fast_kernel<T, BM, BN, BK, WM, WN, kStages, kOcc, kAddmm, kAblate, kLoad, kAux, false, true, kTail, false, kLines><<<grid, block, 0, stream>>>(p);
+        else if (q.linear) gemm_nn_fast_kernel<T, BM, BN, BK, WM, WN, kStages, kOcc, kLinear, kAblate, kLoad, kAux, false, true, kTail, false, kLines><<<grid, block, 0, stream>>>(p);
+        else gemm_nn_fast_kernel<T, BM, BN, BK, WM, WN, kStages, kOcc, kPlain, kAblate, kLoad, kAux, false, true, kTail, false, kLines><<<grid, block, 0, stream>>>(p);
     } else {
-        if (f32) gemm_nn_fast_kernel<T, BM, BN, BK, WM, WN, kStages, kOcc, kPlain, kAblate, kLoad, kAux, true, false, kTail><<<grid, block, 0, stream>>>(p);
-        else if (addmm) gemm_nn_fast_kernel<T, BM, BN, BK, WM, WN, kStages, kOcc, kAddmm, kAblate, kLoad, kAux, false, false, kTail><<<grid, block, 0, stream>>>(p);
-        else if (q.linear) gemm_nn_fast_kernel<T, BM, BN, BK, WM, WN, kStages, kOcc, kLinear, kAblate, kLoad, kAux, false, false, kTail><<<grid, block, 0, stream>>>(p);
-        else gemm_nn_fast_kernel<T, BM, BN, BK, WM, WN, kStages, kOcc, kPlain, kAblate, kLoad, kAux, false, false, kTail><<<grid, block, 0, stream>>>(p);
+        if (f32) gemm_nn_fast_kernel<T, BM, BN, BK, WM, WN, kStages, kOcc, kPlain, kAblate, kLoad, kAux, true, false, kTail, false, kLines><<<grid, block, 0, stream>>>(p);
+        else if (addmm) gemm_nn_fast_kernel<T, BM, BN, BK, WM, WN, kStages, kOcc, kAddmm, kAblate, kLoad, kAux, false, false, kTail, false, kLines><<<grid, block, 0, stream>>>(p);
+        else if (q.linear) gemm_nn_fast_kernel<T, BM, BN, BK, WM, WN, kStages, kOcc, kLinear, kAblate, kLoad, kAux, false, false, kTail, false, kLines><<<grid, block, 0, stream>>>(p);
+        else gemm_nn_fast_kernel<T, BM, BN, BK, WM, WN, kStages, kOcc, kPlain, kAblate, kLoad, kAux, false, false, kTail, false, kLines><<<grid, block, 0, stream>>>(p);
     }
     return hipGetLastError();
 }
 
-template <int BM, int BN, int BK, int WM, int WN, int kStages, int kOcc, int kAblate = 0, int kLoad = 1, int kAux = 0, bool kTail = false>
+// Whether rows of the k-contiguous operands are staged by whole cache lines, in a ring of five stages (kLines of the kernel): where some begin inside a
+// 128-byte line; of a product with a row-major rhs only from 65 rows on, since its lhs is all that gains (17 x 768 x 11104 12.1 us without, 12.9 with).
+// bf16, one k tile after another / by whole lines, us, rhs transposed and not: 128 x 128 tiles 4096 x 1024 x 4088 58.5 / 39.9, 47.1 / 39.5; 1394 x
+// 2176 x 3080 41.3 / 30.1, 34.4 / 29.8; 64 x 64 4096 x 1024 x 4088 95.4 / 63.5, 79.5 / 64.3; 300 x 4096 x 1000 10.2 / 8.8, 9.2 / 8.5; 64 x 128 77 x 832 x
+// 5576 36.9 / 26.6, 28.8 / 26.3.  Rows that begin with a line gain nothing and wait for a line more: 2048^3 on 64 x 128 23.7 / 27.0, on 64 x 64 27.8 /
+// 28.4, fp16 863 x 2368 x 704 on 128 x 128 7.7 / 8.1, 283 x 1016 x 12224 there in parts 24.6 / 25.7.
+bool rows_straddle_lines(const GemmProblem &q) {
+    const auto inside = [&](const void *data, int64_t pitch, int64_t batch) { return ((uintptr_t)data | (uintptr_t)(pitch * 2) | (uintptr_t)(q.batch > 1 ? batch * 2 : 0)) % 128 != 0; };
+    if (b_is_transposed(q)) return inside(q.a, q.sam, q.a_batch) || inside(q.b, q.sbn, q.b_batch);
+    return q.m > 64 && inside(q.a, q.sam, q.a_batch);
+}
+
+template <typename T, int BM, int BN, int BK, int WM, int WN, int kStages, int kOcc, int kAblate, int kLoad, int kAux, bool kTail, bool kLines>
+hipError_t fast_launch_typed(const GemmProblem &q, hipStream_t stream) {
+    if constexpr (kLines)
+        if (rows_straddle_lines(q)) return fast_launch_form<T, BM, BN, BK, WM, WN, 5, kOcc, kAblate, kLoad, kAux, kTail, true>(q, stream);
+    return fast_launch_form<T, BM, BN, BK, WM, WN, kStages, kOcc, kAblate, kLoad, kAux, kTail, false>(q, stream);
+}
+
+template <int BM, int BN, int BK, int WM, int WN, int kStages, int kOcc, int kAblate = 0, int kLoad = 1, int kAux = 0, bool kTail = false, bool kLines = false>
 hipError_t fast_launch(const GemmProblem &q, hipStream_t stream) {
-    if (q.dtype == NINETOOTHED_FLOAT16) return fast_launch_typed<half_t, BM, BN, BK, WM, WN, kStages, kOcc, kAblate, kLoad, kAux, kTail>(q, stream);
-    return fast_launch_typed<bf16_t, BM, BN, BK, WM, WN, kStages, kOcc, kAblate, kLoad, kAux, kTail>(q, stream);
+    if (q.dtype == NINETOOTHED_FLOAT16) return fast_launch_typed<half_t, BM, BN, BK, WM, WN, kStages, kOcc, kAblate, kLoad, kAux, kTail, kLines>(q, stream);
+    return fast_launch_typed<bf16_t, BM, BN, BK, WM, WN, kStages, kOcc, kAblate, kLoad, kAux, kTail, kLines>(q, stream);
 }
 
 // ---- split-K: problems with too few output tiles for 256 CUs (a few rows, or small M x N with a long K) ----
@@ -262,7 +281,7 @@ __global__ __launch_bounds__(256) void gemm_split_reduce_kernel(const float *par
     }
 }
 
-template <typename T, int BM, int BN, int BK, int WM, int WN, int kStages, int kOcc>
+template <typename T, int BM, int BN, int BK, int WM, int WN, int kStages, int kOcc, bool kLines>
 hipError_t split_launch_typed(const GemmProblem &q, hipStream_t stream) {
     static_assert(split_cost(BM, BN) != nullptr, "a cost for the tile");
     int kt_per_part = 0;
@@ -290,8 +309,14 @@ hipError_t split_launch_typed(const GemmProblem &q, hipStream_t stream) {
     p.bias = nullptr;
     p.kt_per_split = kt_per_part;
     const dim3 grid(p.tiles_m * p.tiles_n * parts), block(WM * WN * 64);
-    if (b_is_transposed(q)) gemm_nn_fast_kernel<T, BM, BN, BK, WM, WN, kStages, kOcc, kPlain, 0, 1, 0, true, true, true, true><<<grid, block, 0, stream>>>(p);
-    else gemm_nn_fast_kernel<T, BM, BN, BK, WM, WN, kStages, kOcc, kPlain, 0, 1, 0, true, false, true, true><<<grid, block, 0, stream>>>(p);
+    const auto launch = [&](auto stages_tag, auto lines_tag) {
+        constexpr int kRing = decltype(stages_tag)::value;
+        constexpr bool kByLines = decltype(lines_tag)::value;
+        if (b_is_transposed(q)) gemm_nn_fast_kernel<T, BM, BN, BK, WM, WN, kRing, kOcc, kPlain, 0, 1, 0, true, true, true, true, kByLines><<<grid, block, 0, stream>>>(p);
+        else gemm_nn_fast_kernel<T, BM, BN, BK, WM, WN, kRing, kOcc, kPlain, 0, 1, 0, true, false, true, true, kByLines><<<grid, block, 0, stream>>>(p);
+    };
+    if (kLines && rows_straddle_lines(q)) launch(std::integral_constant<int, kLines ? 5 : kStages>(), std::integral_constant<bool, kLines>());
+    else launch(std::integral_constant<int, kStages>(), std::false_type());
     hipError_t err = hipGetLastError();
     if (err != hipSuccess) return err;
     const int64_t values = (int64_t)q.m * (pitch / 4);
@@ -317,10 +342,10 @@ hipError_t split_launch_typed(const GemmProblem &q, hipStream_t stream) {
     return hipGetLastError();
 }
 
-template <int BM, int BN, int BK, int WM, int WN, int kStages, int kOcc>
+template <int BM, int BN, int BK, int WM, int WN, int kStages, int kOcc, bool kLines>
 hipError_t split_launch(const GemmProblem &q, hipStream_t stream) {
-    if (q.dtype == NINETOOTHED_FLOAT16) return split_launch_typed<half_t, BM, BN, BK, WM, WN, kStages, kOcc>(q, stream);
-    return split_launch_typed<bf16_t, BM, BN, BK, WM, WN, kStages, kOcc>(q, stream);
+    if (q.dtype == NINETOOTHED_FLOAT16) return split_launch_typed<half_t, BM, BN, BK, WM, WN, kStages, kOcc, kLines>(q, stream);
+    return split_launch_typed<bf16_t, BM, BN, BK, WM, WN, kStages, kOcc, kLines>(q, stream);
 }
 
 // ---- skinny products: at most 64 rows against a k-contiguous rhs, the k range over the waves of a workgroup ----
@@ -506,12 +531,12 @@ template <bool kColumns> hipError_t cut_launch(const GemmProblem &q, hipStream_t
 #define NT_FAST_INSTANCE(BM, BN, BK, WM, WN, ST, OCC) \
     {#BM "x" #BN "x" #BK " waves " #WM "x" #WN " stages " #ST " lds-direct", BM, BN, BK, fast_accepts<BM, BN, BK, ST>, fast_launch<BM, BN, BK, WM, WN, ST, OCC>}
 
-// the same kernels with partial last tiles along N and K (both multiples of 8)
-#define NT_TAIL_INSTANCE(BM, BN, BK, WM, WN, ST, OCC) \
-    {#BM "x" #BN "x" #BK " waves " #WM "x" #WN " stages " #ST " lds-direct tails", BM, BN, BK, fast_accepts<BM, BN, BK, ST, true>, fast_launch<BM, BN, BK, WM, WN, ST, OCC, 0, 1, 0, true>}
+// the same kernels with partial last tiles along N and K (both multiples of 8); LINES: with the form for rows that begin inside cache lines
+#define NT_TAIL_INSTANCE(BM, BN, BK, WM, WN, ST, OCC, LINES) \
+    {#BM "x" #BN "x" #BK " waves " #WM "x" #WN " stages " #ST " lds-direct tails", BM, BN, BK, fast_accepts<BM, BN, BK, ST, true>, fast_launch<BM, BN, BK, WM, WN, ST, OCC, 0, 1, 0, true, LINES>}
 
-#define NT_SPLIT_INSTANCE(BM, BN, BK, WM, WN, ST, OCC) \
-    {#BM "x" #BN "x" #BK " waves " #WM "x" #WN " stages " #ST " lds-direct tails split-k", BM, BN, BK, split_accepts<BM, BN, BK, ST>, split_launch<BM, BN, BK, WM, WN, ST, OCC>}
+#define NT_SPLIT_INSTANCE(BM, BN, BK, WM, WN, ST, OCC, LINES) \
+    {#BM "x" #BN "x" #BK " waves " #WM "x" #WN " stages " #ST " lds-direct tails split-k", BM, BN, BK, split_accepts<BM, BN, BK, ST>, split_launch<BM, BN, BK, WM, WN, ST, OCC, LINES>}
 
 // positions in kInstances (the tuning cache and the heuristics refer to instances by position)
 enum InstanceIndex {
@@ -528,21 +553,21 @@ const GemmInstance kInstances[] = {
     NT_FAST_INSTANCE(128, 128, 64, 2, 2, 2, 2),
     NT_FAST_INSTANCE(64, 64, 64, 2, 2, 4, 2),  // small problems: more, smaller tiles to occupy the CUs
     NT_FAST_INSTANCE(128, 256, 32, 1, 4, 3, 2),  // two workgroups per CU: mid-size problems
-    NT_TAIL_INSTANCE(256, 256, 32, 2, 4, 5, 2),
-    NT_TAIL_INSTANCE(128, 256, 32, 1, 4, 3, 2),
-    NT_TAIL_INSTANCE(128, 128, 64, 2, 2, 2, 2),
-    NT_TAIL_INSTANCE(64, 64, 64, 2, 2, 4, 2),
-    NT_SPLIT_INSTANCE(64, 64, 64, 2, 2, 4, 2),
-    NT_SPLIT_INSTANCE(128, 128, 64, 2, 4, 4, 2),  // (two stages, two workgroups per CU: 222 x 2752 x 15040 43.3 us, here 39.4; 283 x 1016 x 12224 26.8, 23.3; 256 x 8192 x 8192 59.9, 52.2)
-    NT_SPLIT_INSTANCE(128, 256, 32, 1, 4, 3, 2),  // a few hundred rows against a wide rhs: 64 to 160 large tiles
-    NT_SPLIT_INSTANCE(256, 256, 32, 2, 4, 5, 2),
+    NT_TAIL_INSTANCE(256, 256, 32, 2, 4, 5, 2, false),
+    NT_TAIL_INSTANCE(128, 256, 32, 1, 4, 3, 2, false),
+    NT_TAIL_INSTANCE(128, 128, 64, 2, 2, 2, 2, false),
+    NT_TAIL_INSTANCE(64, 64, 64, 2, 2, 4, 2, true),
+    NT_SPLIT_INSTANCE(64, 64, 64, 2, 2, 4, 2, true),
+    NT_SPLIT_INSTANCE(128, 128, 64, 2, 4, 4, 2, true),  // (two stages, two workgroups per CU: 222 x 2752 x 15040 43.3 us, here 39.4; 283 x 1016 x 12224 26.8, 23.3; 256 x 8192 x 8192 59.9, 52.2)
+    NT_SPLIT_INSTANCE(128, 256, 32, 1, 4, 3, 2, false),  // a few hundred rows against a wide rhs: 64 to 160 large tiles
+    NT_SPLIT_INSTANCE(256, 256, 32, 2, 4, 5, 2, false),
     {"64x16x64 skinny, split-k over the waves of a workgroup", 64, 16, 64, skinny_accepts, skinny_launch<1>},
     {"64x32x64 skinny, split-k over the waves of a workgroup", 64, 32, 64, skinny_accepts, skinny_launch<2>},
     // One workgroup per CU with most of its LDS: three or four fills of 16 to 32 KiB in flight instead of one, for products whose
     // tiles the chip holds all at once, so that nothing else covers the latency of a fill.
-    NT_TAIL_INSTANCE(128, 128, 64, 2, 4, 4, 2),
-    NT_TAIL_INSTANCE(64, 64, 128, 2, 2, 4, 1),
-    NT_TAIL_INSTANCE(64, 128, 64, 2, 4, 5, 2),
+    NT_TAIL_INSTANCE(128, 128, 64, 2, 4, 4, 2, true),
+    NT_TAIL_INSTANCE(64, 64, 128, 2, 2, 4, 1, false),
+    NT_TAIL_INSTANCE(64, 128, 64, 2, 4, 5, 2, true),
     {"256x256x32 for whole rounds of the chip, the columns left on their own (smaller tiles or split-k)", 256, 256, 32, cut_accepts<true>, cut_launch<true>},
     {"256x256x32 for whole rounds of the chip, the rows left on their own (smaller tiles or split-k)", 256, 256, 32, cut_accepts<false>, cut_launch<false>},
 #ifdef NT_GEMM_ABLATION

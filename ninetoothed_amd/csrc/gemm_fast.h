@@ -133,6 +133,13 @@ NT_DEVICE void lds_barrier_reads_in_flight() {
     __builtin_amdgcn_sched_barrier(0);
 }
 
+// A fill of 1 KiB of LDS from 64 lanes' 16 bytes that the compiler does not know for one: it makes no read of the same array wait for it.
+// (A wave's own waits and the barriers order them.)
+NT_DEVICE void fill_lds(__amdgpu_buffer_rsrc_t rsrc, NT_LDS unsigned char *to, unsigned offset, int uniform_offset) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+                 :: "s"((unsigned)(uintptr_t)to), "v"(offset), "s"(rsrc), "s"(uniform_offset) : "m0");
+}
+
 // What happens to the sums of products.  kAddmm: rounded to the element type, then beta * input + alpha * product in fp32.
 // kLinear: max(sum * alpha + bias[column], lower) in fp32, rounded once on the store -- on the accumulators, before they pass through
 // LDS as 16-bit values: a lane's columns stay the same over all rows, so their bias costs TN16 loads per tile.
@@ -168,7 +175,7 @@ NT_DEVICE float linear_bias(const GemmParams &p, int col) {
 // kAblate is a measurement aid (bit 0: no global loads inside the K loop,
 // bit 1: operand fragments read from LDS only once); 0 in every shipped instance.
 template <typename T, int BM, int BN, int BK, int WM, int WN, int kStages, int kWavesPerSimd, int kEpilogue, int kAblate = 0, int kLoad = 0, int kAux = 0,
-          bool kFloatOut = false, bool kBT = false, bool kTail = false, bool kSplit = false>
+          bool kFloatOut = false, bool kBT = false, bool kTail = false, bool kSplit = false, bool kLines = false>
 __global__ __launch_bounds__(WM *WN * 64, kWavesPerSimd) void gemm_nn_fast_kernel(GemmParams p) {
 #if defined(__HIP_DEVICE_COMPILE__)  // the body uses device-only builtins; the host pass only needs the stub
     typedef Elem<T> E;
@@ -213,23 +220,33 @@ __global__ __launch_bounds__(WM *WN * 64, kWavesPerSimd) void gemm_nn_fast_kerne
     static_assert(kStages >= 2 && kStages <= 5, "2..5 stages");
     static_assert((kStages - 2) * kLoadsPerTile < 64, "vmcnt range");
 
+    // kLines: rows of A (and of a transposed B) that begin anywhere in a cache line.  A k tile of 128 bytes of such a row straddles two lines,
+    // so that every fill asks for twice as many and the L1's rate bounds the step.  Instead stage t holds the row's t-th whole line, whatever part
+    // of a line lies before the row's beginning; a k tile then lies in stages t and t + 1, split at a chunk that depends on the row alone (period 16:
+    // the pitch is a multiple of 16 bytes), and a lane keeps for its row in which of the two its chunks are.  A chunk has the same
+    // place within its stage as in an aligned row, so the reads stay free of conflicts.  One stage more must have landed; a ring of five holds as
+    // many fills in flight as four do otherwise.  4096 x 1024 x 4088 bf16 in 128 x 128 tiles, rhs transposed: 58.5 -> 39.9 us (0.59 -> 0.86 PFLOP/s; a K of 4096 39.1).
+    static_assert(!kLines || (kTile16 && BK == 64 && kTail && kStages == 5 && kAux == 0), "rows of whole cache lines");
+
     // One array per stage and operand: distinct LDS objects let the compiler prove
     // that the asynchronous fill of one stage does not alias reads of another,
     // so it does not wait for the fill before the MFMA operand reads.
     // (kPairA uses a0 .. a2 and b0 .. b3; arrays that nothing refers to take no LDS)
-    __shared__ __attribute__((aligned(1024))) unsigned char lds_a0[kBytesA];
+    // (kLines picks a stage per lane: one array, and fills that the compiler does not see as such)
+    __shared__ __attribute__((aligned(1024))) unsigned char lds_a0[kLines ? kStages * kStageA : kBytesA];
     __shared__ __attribute__((aligned(1024))) unsigned char lds_a1[kBytesA];
     __shared__ __attribute__((aligned(1024))) unsigned char lds_a2[kStages > 2 ? kBytesA : 16];
     __shared__ __attribute__((aligned(1024))) unsigned char lds_a3[kStages > 3 ? kStageA : 16];
     __shared__ __attribute__((aligned(1024))) unsigned char lds_a4[kStages > 4 ? kStageA : 16];
-    __shared__ __attribute__((aligned(1024))) unsigned char lds_b0[kStageB];
+    __shared__ __attribute__((aligned(1024))) unsigned char lds_b0[kLines ? kStages * kStageB : kStageB];
     __shared__ __attribute__((aligned(1024))) unsigned char lds_b1[kStageB];
     __shared__ __attribute__((aligned(1024))) unsigned char lds_b2[kStages > 2 ? kStageB : 16];
     __shared__ __attribute__((aligned(1024))) unsigned char lds_b3[kStages > 3 ? kStageB : 16];
     __shared__ __attribute__((aligned(1024))) unsigned char lds_b4[kStages > 4 ? kStageB : 16];
     auto stage_a = [&](auto tag) -> NT_LDS unsigned char * {
         constexpr int i = decltype(tag)::value;
-        if constexpr (i == 0) return (NT_LDS unsigned char *)lds_a0;
+        if constexpr (kLines) return (NT_LDS unsigned char *)lds_a0 + i * kStageA;
+        else if constexpr (i == 0) return (NT_LDS unsigned char *)lds_a0;
         else if constexpr (i == 1) return (NT_LDS unsigned char *)lds_a1;
         else if constexpr (i == 2) return (NT_LDS unsigned char *)lds_a2;
         else if constexpr (i == 3) return (NT_LDS unsigned char *)lds_a3;
@@ -237,7 +254,8 @@ __global__ __launch_bounds__(WM *WN * 64, kWavesPerSimd) void gemm_nn_fast_kerne
     };
     auto stage_b = [&](auto tag) -> NT_LDS unsigned char * {
         constexpr int i = decltype(tag)::value;
-        if constexpr (i == 0) return (NT_LDS unsigned char *)lds_b0;
+        if constexpr (kLines) return (NT_LDS unsigned char *)lds_b0 + i * kStageB;
+        else if constexpr (i == 0) return (NT_LDS unsigned char *)lds_b0;
         else if constexpr (i == 1) return (NT_LDS unsigned char *)lds_b1;
         else if constexpr (i == 2) return (NT_LDS unsigned char *)lds_b2;
         else if constexpr (i == 3) return (NT_LDS unsigned char *)lds_b3;
@@ -320,12 +338,45 @@ __global__ __launch_bounds__(WM *WN * 64, kWavesPerSimd) void gemm_nn_fast_kerne
         }
         b_rsrc = __builtin_amdgcn_make_buffer_rsrc((void *)b_base, 0, b_bytes, 0x00020000);
     }
+    // kLines: descriptors from the beginning of the line that the tile's first row begins in; per lane the chunk of a row's
+    // k range that it fills (the same in every instruction, less 8 where it lies in the line before) and its offset
+    unsigned a_line_src[kLines ? kAInstr : 1], b_line_src[kLines && kBT ? kBInstr : 1];
+    int a_line_chunk = 0, b_line_chunk = 0;
+    if constexpr (kLines) {
+        static_assert(kWaves * kARowsPerInstr % 16 == 0, "where rows begin in a line repeats every 16 rows");
+        const int row = wave * 8 + lane / 8, chunk = a_phys_chunk16<BK>(row, lane % 8);
+        const auto lines = [&](const unsigned char *base, int64_t pitch, int64_t rows, __amdgpu_buffer_rsrc_t &rsrc, unsigned *src, int count, int &line_chunk) {
+            const int before = (int)((uintptr_t)base & 127);
+            const int shift = ((before + row * (int)pitch * 2) & 127) >> 4;  // 16-byte chunks of the row's first line that lie before it
+            line_chunk = chunk + shift >= 8 ? chunk - 8 : chunk;
+            for (int j = 0; j < count; ++j) src[j] = (unsigned)(before + (j * kWaves * 8 + row) * (int)pitch * 2 + line_chunk * 16);
+            rsrc = __builtin_amdgcn_make_buffer_rsrc((void *)(base - before), 0, (unsigned)(before + ((rows - 1) * pitch + p.k) * 2), 0x00020000);
+        };
+        lines(a_base, p.lda, min((int64_t)BM, (int64_t)p.m - m0), a_rsrc, a_line_src, kAInstr, a_line_chunk);
+        if constexpr (kBT) lines(b_base, p.ldb, min((int64_t)BN, (int64_t)p.n - n0), b_rsrc, b_line_src, kBInstr, b_line_chunk);
+    }
     const int all_k = kTail ? (p.k + BK - 1) / BK : p.k / BK;  // k tiles of the problem
     const int k_first = kSplit ? part * p.kt_per_split : 0;     // this workgroup's first
     const int num_k = kSplit ? min(p.kt_per_split, all_k - k_first) : all_k;
     const int last_k = num_k - 1;
     // 16-byte chunks of the problem's last k tile that lie inside K (all of them without a tail)
     const int tail_chunks = kTail ? (p.k - (all_k - 1) * BK) / 8 : kAChunksPerRow;
+    // kLines: fills [kFirst, kLast) of line kt of the rows (of k tile kt of a B that is not transposed) into a stage; chunks that lie outside
+    // the rows' k range are zeros
+    auto issue_lines = [&](auto stage_tag, int kt, auto first_tag, auto last_tag) {
+        constexpr int kFirst = decltype(first_tag)::value, kLast = decltype(last_tag)::value;
+        constexpr unsigned kBehind = 0x7fffffffu;
+        const unsigned chunks = (unsigned)p.k / 8;
+        kt += k_first;
+        const bool a_inside = (unsigned)(kt * 8 + a_line_chunk) < chunks, b_inside = (unsigned)(kt * 8 + b_line_chunk) < chunks;
+        const int b_kt = min(kt, all_k - 1);
+#pragma unroll
+        for (int j = kFirst; j < kLast; ++j) {
+            if (j < kAInstr) fill_lds(a_rsrc, stage_a(stage_tag) + (j * kWaves + wave) * 1024, a_inside ? a_line_src[kLines ? j : 0] : kBehind, kt * 128);
+            else if constexpr (kBT) fill_lds(b_rsrc, stage_b(stage_tag) + ((j - kAInstr) * kWaves + wave) * 1024, b_inside ? b_line_src[kLines ? j - kAInstr : 0] : kBehind, kt * 128);
+            else fill_lds(b_rsrc, stage_b(stage_tag) + ((j - kAInstr) * kWaves + wave) * 1024, b_src[j - kAInstr], b_kt * BK * (int)p.ldb * 2);
+        }
+    };
     auto issue_loads = [&](auto stage_tag, int kt) {
         NT_LDS unsigned char *sa = stage_a(stage_tag);
         NT_LDS unsigned char *sb = stage_b(stage_tag);
@@ -477,6 +528,7 @@ __global__ __launch_bounds__(WM *WN * 64, kWavesPerSimd) void gemm_nn_fast_kerne
     constexpr int TM16 = kWaveM / 16, TN16 = kWaveN / 16, KS16 = BK / 32;
     // ... with the fragment reads of the next k step under the MFMAs of this one, across the barrier
     constexpr bool kCross16 = kM16 && kStages >= 3 && (KS16 * TM16) % 4 == 0 && TM16 >= TN16;
+    static_assert(!kLines || kCross16, "the steps that wait for a line more");
     float4_t acc16[kM16 ? TM16 : 1][kM16 ? TN16 : 1];
 #pragma unroll
     for (int ti = 0; ti < (kM16 ? TM16 : 1); ++ti)
@@ -506,12 +558,37 @@ __global__ __launch_bounds__(WM *WN * 64, kWavesPerSimd) void gemm_nn_fast_kerne
             b16_hi[tj] = k_hi * (BN * 2) + b_phys_chunk16<BN>(k_hi, ncol >> 3) * 16 + (ncol & 7) * 2;
         }
     }
+    // kLines: a chunk's offset from stage t where t + 1 is the next place of the ring, and from the ring where t is the last
+    int a_line_off[kLines ? 2 : 1][KS16], b_line_off[kLines && kBT ? 2 : 1][KS16];
+    if constexpr (kLines) {
+        const int a_shift = (int)(((uintptr_t)a_base + (uintptr_t)((wave_m * kWaveM + i16) * (int)p.lda * 2)) & 127) >> 4;
+        const int b_shift = (int)(((uintptr_t)b_base + (uintptr_t)((wave_n * kWaveN + i16) * (int)p.ldb * 2)) & 127) >> 4;
+#pragma unroll
+        for (int ks = 0; ks < KS16; ++ks) {
+            const bool a_next = ks * 4 + kg + a_shift >= 8, b_next = ks * 4 + kg + b_shift >= 8;
+            a_line_off[0][ks] = a16_off[ks] + (a_next ? kStageA : 0);
+            a_line_off[kLines ? 1 : 0][ks] = a16_off[ks] + (a_next ? 0 : (kStages - 1) * kStageA);
+            if constexpr (kBT) {
+                b_line_off[0][ks] = bt16_off[ks] + (b_next ? kStageB : 0);
+                b_line_off[kLines && kBT ? 1 : 0][ks] = bt16_off[ks] + (b_next ? 0 : (kStages - 1) * kStageB);
+            }
+        }
+    }
     auto read_a16 = [&](auto stage_tag, int ks, int ti) -> vec8 {
+        if constexpr (kLines) {
+            constexpr int kS = decltype(stage_tag)::value;
+            if constexpr (kS == kStages - 1) return *(const NT_LDS vec8 *)((NT_LDS unsigned char *)lds_a0 + a_line_off[1][ks] + ti * 16 * (BK * 2));
+            else return *(const NT_LDS vec8 *)((NT_LDS unsigned char *)lds_a0 + a_line_off[0][ks] + (kS * kStageA + ti * 16 * (BK * 2)));
+        } else
         return *(const NT_LDS vec8 *)(stage_a(stage_tag) + a16_off[ks] + ti * 16 * (BK * 2));
     };
     auto read_b16 = [&](auto stage_tag, int ks, int tj) -> vec8 {
         const NT_LDS unsigned char *sb = stage_b(stage_tag);
-        if constexpr (kBT) {
+        if constexpr (kLines && kBT) {
+            constexpr int kS = decltype(stage_tag)::value;
+            if constexpr (kS == kStages - 1) return *(const NT_LDS vec8 *)((NT_LDS unsigned char *)lds_b0 + b_line_off[1][ks] + tj * 16 * (BK * 2));
+            else return *(const NT_LDS vec8 *)((NT_LDS unsigned char *)lds_b0 + b_line_off[0][ks] + (kS * kStageB + tj * 16 * (BK * 2)));
+        } else if constexpr (kBT) {
             return *(const NT_LDS vec8 *)(sb + bt16_off[ks] + tj * 16 * (BK * 2));
         } else {
             short4_t lo = lds_read_tr16_b64(sb + b16_lo[kBT ? 0 : tj] + ks * 32 * (BN * 2));
@@ -637,7 +714,8 @@ __global__ __launch_bounds__(WM *WN * 64, kWavesPerSimd) void gemm_nn_fast_kerne
             if (body_k + (int)decltype(i)::value < num_k) step(i, body_k);
         });
     }
-    if constexpr (!kPairA) static_for<0, kStages - 1>([&](auto s) { issue_loads(s, min((int)decltype(s)::value, last_k)); });
+    if constexpr (kLines) static_for<0, kStages - 1>([&](auto s) { issue_lines(s, (int)decltype(s)::value, std::integral_constant<int, 0>(), std::integral_constant<int, kLoadsPerTile>()); });
+    else if constexpr (!kPairA) static_for<0, kStages - 1>([&](auto s) { issue_loads(s, min((int)decltype(s)::value, last_k)); });
     if constexpr (kPairA) {
         // (done above)
     } else if constexpr (kCross16) {
@@ -646,7 +724,7 @@ __global__ __launch_bounds__(WM *WN * 64, kWavesPerSimd) void gemm_nn_fast_kerne
         constexpr int Q = KS16 * TM16;  // A fragments of a k tile, in the order they are used
         vec8 as[4];
         vec8 bs[2][TN16];
-        wait_vmcnt<(kStages - 2) * kLoadsPerTile>();
+        wait_vmcnt<(kStages - (kLines ? 3 : 2)) * kLoadsPerTile>();  // (kLines: the first two lines)
         lds_barrier();
 #pragma unroll
         for (int tj = 0; tj < TN16; ++tj) bs[0][tj] = read_b16(std::integral_constant<int, 0>(), 0, tj);
@@ -657,11 +735,14 @@ __global__ __launch_bounds__(WM *WN * 64, kWavesPerSimd) void gemm_nn_fast_kerne
             constexpr int kS = kI % kStages;
             typedef std::integral_constant<int, kS> Stage;
             typedef std::integral_constant<int, (kS + 1) % kStages> NextStage;
-            wait_vmcnt<(kStages - 3) * kLoadsPerTile>();
+            wait_vmcnt<(kStages - (kLines ? 4 : 3)) * kLoadsPerTile>();
             lds_barrier_reads_in_flight();
-            issue_loads(std::integral_constant<int, (kS + kStages - 1) % kStages>(), min(kt + kI + kStages - 1, last_k));
+            if constexpr (!kLines) issue_loads(std::integral_constant<int, (kS + kStages - 1) % kStages>(), min(kt + kI + kStages - 1, last_k));
             static_for<0, Q>([&](auto q_tag) {
                 constexpr int q = decltype(q_tag)::value;
+                if constexpr (kLines)
+                    issue_lines(std::integral_constant<int, (kS + kStages - 1) % kStages>(), kt + kI + kStages - 1, std::integral_constant<int, q * kLoadsPerTile / Q>(),
+                                std::integral_constant<int, (q + 1) * kLoadsPerTile / Q>());
                 constexpr int ks = q / TM16, ti = q % TM16;
                 constexpr int cur = (kI * KS16 + ks) & 1, nxt = cur ^ 1;
                 constexpr int kBReadsPerBlock = kBT ? 1 : 2;
@@ -688,7 +769,7 @@ __global__ __launch_bounds__(WM *WN * 64, kWavesPerSimd) void gemm_nn_fast_kerne
                     } else if constexpr (j == 0) {
                         __builtin_amdgcn_sched_group_barrier(0x100, kReads, 0);
                     }
-                    if constexpr (j == (TN16 > 1 ? 1 : 0) && kFills > 0) __builtin_amdgcn_sched_group_barrier(0x020, kFills, 0);
+                    if constexpr (j == (TN16 > 1 ? 1 : 0) && kFills > 0 && !kLines) __builtin_amdgcn_sched_group_barrier(0x020, kFills, 0);
                 });
 #endif
             });
@@ -854,10 +935,10 @@ __global__ __launch_bounds__(WM *WN * 64, kWavesPerSimd) void gemm_nn_fast_kerne
         } else if ((w -= kSlabsA) < kSlabsB) {
             slab = (NT_LDS unsigned char *)lds_b0;
         } else if ((w -= kSlabsB) < kSlabsA) {
-            slab = (NT_LDS unsigned char *)lds_a1;
+            slab = stage_a(std::integral_constant<int, 1>());
         } else {
             w -= kSlabsA;
-            slab = (NT_LDS unsigned char *)lds_b1;
+            slab = stage_b(std::integral_constant<int, 1>());
         }
         slab += w * kSlabBytes;
     }
