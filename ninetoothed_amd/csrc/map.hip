@@ -980,8 +980,8 @@ struct MapCodegen {
     // Tile mode with the elements in registers: every operand's values of the thread's elements (or groups), requested together
     // before the phases and converted once all are on their way.  What bounded rows of no whole number of elements per thread was a chain of trips to
     // memory: behind a branch around each load, its conversion or its use waited for it before the next was asked for.  So a thread whose last
-    // elements lie behind the tile asks for the tile's last one again (not where it has only one: a branch
-    // there costs nothing, and whole waves skip the load).  Operands that only the stored expression reads join while all take up to 48 registers.
+    // elements lie behind the tile asks for the tile's last one again (not where it has only one, or one group: one branch around all
+    // operands lets whole waves skip them, fp16 12995 x 1440 11.8 us, 12.5 with a test for each).  Operands that only the stored expression reads join while all take up to 48 registers.
     // Rms norm, us, before -> after: fp32 4541 x 3200 26.9 -> 21.0 (5.5 TB/s), 3350 x 1680 13.3 -> 10.2, 787 x 4160 9.6 -> 6.1, fp16 4702 x 7208
     // 28.4 -> 26.9; branches kept and only the conversions moved: 21.1, 10.9, 6.7, 27.8.
     void preload(long long tile_elements, int per_thread) {
@@ -999,6 +999,14 @@ struct MapCodegen {
             kept[slot] = true;
         }
         if (tile_width > 0) vector_typedefs(width, "        ");
+        if (tile_width > 0 && groups == 1) {
+            out << "        if (const nt_idx element = member * " << width << "; element < " << lit(tile_elements) << ") {\n";
+            indent = "            ";
+            decode_tile_variables();
+            for (int slot : slots) load_group(slot, width, "0");
+            out << "        }\n";
+            return;
+        }
         const auto grouped = [&](int slot) { return tile_width > 0 && group_step(p.operands[slot].segment, p.num_vars - 1, width) == 1; };
         for (int slot : slots)
             out << "        " << (grouped(slot) ? vector_type(p.operands[slot].dtype) : std::string(c_type(p.operands[slot].dtype))) << " raw" << slot << "[" << groups << "]; bool in" << slot << "["
