@@ -225,8 +225,8 @@ NineToothedResult launch_nt_attention(NineToothedStream stream,
  * dilation 1 (launch_nt_conv2d_strided takes others) and zero padding (padding_h, padding_w), computed as the implicit
  * GEMM [N*P*Q, C*R*S] x [C*R*S, K] the arrangement of
  * tests/test_conv2d.py:13-48 describes.
- * Ways to run it, tried in this order unless block_size_m names one (4, 3, 5, 2, 1)
- * or nt_tune_conv2d has recorded one for the problem:
+ * Ways to run it, tried in this order (4, 3, 5, 2, 1) unless block_size_m names one -- 1 to 4 by their numbers, way 5 by
+ * NINETOOTHED_CONV2D_WINDOWS, since a program's own block size of 5 names none -- or nt_tune_conv2d has recorded one for the problem:
  * 4 -- 1 x 1 filters without padding (P*Q and C multiples of 8): one batched
  *   launch of the GEMM kernels on the tensors as they lie, without scratch;
  * 3 -- one launch on the tensors as they lie, no scratch memory: the filter is
@@ -235,8 +235,8 @@ NineToothedResult launch_nt_attention(NineToothedStream stream,
  *   multiple of 8, padding_w <= 1, C*R*S a multiple of 32, R*S / gcd(32, R*S) <= 25, pixels of an input row
  *   contiguous, contiguous filter and output, K filling 256-wide tiles to 4/5;
  * 5 -- 3 x 3 filters, C >= 32 a multiple of 8, positions of a channel and each filter's values contiguous, input windows of 224 output
- *   positions that fit LDS: one launch, no scratch memory, a workgroup reads its input rows once for all taps.  Without
- *   block_size_m = 5 taken only where way 2 is expected to be slower;
+ *   positions that fit LDS: one launch, no scratch memory, a workgroup reads its input rows once for all taps.  Unless
+ *   it is named taken only where way 2 is expected to be slower; where it is named and does not take the problem, as if it were not named;
  * 2 -- fp16 / bf16 tensors of any strides (a contiguous NCHW output is stored in
  *   16-byte pieces of 8 positions, a channels-last one in pieces of 8 channels,
  *   any other element by element): the
@@ -250,6 +250,7 @@ NineToothedResult launch_nt_attention(NineToothedStream stream,
  *   scratch cannot be allocated (out of memory; a stream under graph capture that
  *   has no buffer yet).
  * FLOAT32 tensors run on way 1 with the fp32 MFMA. */
+#define NINETOOTHED_CONV2D_WINDOWS (-5)
 NineToothedResult launch_nt_conv2d(NineToothedStream stream,
                                    NineToothedTensor input,
                                    NineToothedTensor filter,
@@ -267,7 +268,7 @@ NineToothedResult launch_nt_conv2d(NineToothedStream stream,
  * (`floor_mode=True`: (H + 2 padding - dilation (R - 1) - 1) / stride + 1, rounded down) or one more that hangs over
  * the edge (`Tensor.tile`'s default rounds up; what hangs over reads as padding); other sizes are rejected.
  * Steps of 1 with the fitting output are launch_nt_conv2d.  Otherwise way 5, way 2 (repacking pass plus GEMM loop) --
- * same conditions and scratch buffers -- or way 1 (gather kernel) runs; block_size_m = 5, 2 or 1 names one. */
+ * same conditions and scratch buffers -- or way 1 (gather kernel) runs; block_size_m = NINETOOTHED_CONV2D_WINDOWS, 2 or 1 names one. */
 NineToothedResult launch_nt_conv2d_strided(NineToothedStream stream,
                                            NineToothedTensor input,
                                            NineToothedTensor filter,
@@ -395,8 +396,8 @@ NineToothedResult nt_tune_attention(NineToothedStream stream,
 
 /* As nt_tune_gemm for launch_nt_conv2d: times the ways to run the convolution -- 4 = a 1 x 1 filter as a batch of
  * plain products, 3 = one launch on the tensors as they lie, 5 = one launch with input windows in LDS, 2 = repacking pass plus GEMM loop, 1 = gather kernel; a
- * way that does not take the problem is skipped -- and records the fastest (the block_size_m value that selects
- * it) for later launches of the same problem with block_size_m = 0; a way that needs scratch memory or more
+ * way that does not take the problem is skipped -- and records the fastest (the way's
+ * number) for later launches of the same problem with block_size_m = 0; a way that needs scratch memory or more
  * launches replaces one before it in that order only when it is more than 3 % faster.  *best_path = -1 when
  * nothing was timed (graph capture). */
 NineToothedResult nt_tune_conv2d(NineToothedStream stream,

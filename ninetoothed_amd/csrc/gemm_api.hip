@@ -1485,8 +1485,8 @@ NineToothedResult launch_nt_conv2d(NineToothedStream stream, NineToothedTensor i
     const int status = conv2d_request(request, input, filter, output, dtype, padding_h, padding_w);
     if (status != 0) return status < 0 ? 0 : status;
     // block_size_m: 1 = the gather kernel, 2 = the repacking path, 3 = the one-launch path, 4 = a 1 x 1 filter as a
-    // batch of plain products, 5 = input windows in LDS; otherwise the tuned choice for this problem, else the library's order
-    int path = block_size_m >= kConvGather && block_size_m <= kConvWindow ? block_size_m : kConvAuto;
+    // batch of plain products, NINETOOTHED_CONV2D_WINDOWS = input windows in LDS; otherwise the tuned choice for this problem, else the library's order
+    int path = block_size_m >= kConvGather && block_size_m <= kConvPointwise ? block_size_m : block_size_m == NINETOOTHED_CONV2D_WINDOWS ? kConvWindow : kConvAuto;
     if (block_size_m == 0) {
         int values[11];
         conv2d_tune_values(request, values);
@@ -1494,8 +1494,8 @@ NineToothedResult launch_nt_conv2d(NineToothedStream stream, NineToothedTensor i
         if (tuned >= kConvGather && tuned <= kConvWindow) path = tuned;
     }
     int result = conv2d_run(request, path, (hipStream_t)stream);
-    // (a tuned path that needs scratch memory it cannot get, e.g. under graph capture: the library's order)
-    if (result == NINETOOTHED_NO_KERNEL && path != kConvAuto && block_size_m == 0) result = conv2d_run(request, kConvAuto, (hipStream_t)stream);
+    // (a tuned path that needs scratch memory it cannot get, e.g. under graph capture, or windows that do not take the problem: the library's order)
+    if (result == NINETOOTHED_NO_KERNEL && path != kConvAuto && (block_size_m == 0 || path == kConvWindow)) result = conv2d_run(request, kConvAuto, (hipStream_t)stream);
     return result;
 }
 
@@ -1515,10 +1515,11 @@ NineToothedResult launch_nt_conv2d_strided(NineToothedStream stream, NineToothed
     Conv2dRequest request;
     const int status = conv2d_request(request, input, filter, output, dtype, padding_h, padding_w, stride_h, stride_w, dilation_h, dilation_w);
     if (status != 0) return status < 0 ? 0 : status;
-    // the ways that take windows with steps: 5 = input windows in LDS, 2 = repacking pass plus GEMM loop, 1 = gather kernel (nothing is tuned here)
-    const int path = block_size_m == kConvGather || block_size_m == kConvRepack || block_size_m == kConvWindow ? block_size_m : kConvAuto;
+    // the ways that take windows with steps: input windows in LDS, 2 = repacking pass plus GEMM loop, 1 = gather kernel (nothing is tuned here)
+    const int path = block_size_m == kConvGather || block_size_m == kConvRepack ? block_size_m : block_size_m == NINETOOTHED_CONV2D_WINDOWS ? kConvWindow : kConvAuto;
     int result = conv2d_run(request, path, (hipStream_t)stream);
     if (result == NINETOOTHED_NO_KERNEL && path == kConvRepack) result = conv2d_run(request, kConvGather, (hipStream_t)stream);
+    if (result == NINETOOTHED_NO_KERNEL && path == kConvWindow) result = conv2d_run(request, kConvAuto, (hipStream_t)stream);
     return result;
 }
 

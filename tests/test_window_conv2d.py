@@ -7,7 +7,7 @@ import torch.nn.functional as F
 
 pytestmark = pytest.mark.gpu
 
-WINDOW = 5  # launch_nt_conv2d's block_size_m: input windows in LDS
+WINDOW = -5  # NINETOOTHED_CONV2D_WINDOWS, launch_nt_conv2d's block_size_m: input windows in LDS
 
 
 def _launch(x, weight, out, padding, stride, dilation, way):
@@ -37,7 +37,10 @@ def _output(shape, dtype, layout):
 def _check(x, weight, padding, stride, dilation, layout):
     expected = F.conv2d(x.cpu().double(), weight.cpu().double(), padding=padding, stride=stride, dilation=dilation)
     buffer, out = _output(expected.shape, x.dtype, layout)
+    from ninetoothed_amd import runtime
+
     assert _launch(x, weight, out, padding, stride, dilation, WINDOW) == 0
+    assert "conv2d_window_kernel" in runtime.last_launch()
     # one rounding of each result (half a unit in the last place) and fp32 sums of C * 9 products
     unit = 2.0**-11 if x.dtype == torch.float16 else 2.0**-8
     bound = unit * expected.abs() + 2.0**-24 * weight[0].numel() ** 0.5 * 4 + 2.0**-25
@@ -98,3 +101,38 @@ def test_the_choice_follows_the_size():
         assert "conv2d_window_kernel" in served(32, 64, 56, 128, 2)
         assert "conv2d_repack_kernel" in served(1, 128, 14, 64, 2)  # few workgroups: the contraction in parts
         assert "conv2d_repack_kernel" in served(32, 256, 56, 512, 2)  # several rounds of long blocks
+
+
+@pytest.mark.parametrize("stride", (1, 2))
+@pytest.mark.parametrize("channels, side, way", ((16, 9, 5), (128, 14, 5), (16, 9, WINDOW)))
+def test_a_block_size_of_five_and_windows_that_do_not_apply_are_left_to_the_library(channels, side, way, stride):
+    """Block sizes of a program arrive where ways are named: 5 of them name none.  (Input windows take no layer of 16 channels; of 128
+    channels and this few positions they are slower.)"""
+    from ninetoothed_amd import runtime
+
+    torch.manual_seed(channels)
+    x, weight = torch.randn(1, channels, side, side, device="cuda").half(), (torch.randn(64, channels, 3, 3, device="cuda") * (9 * channels) ** -0.5).half()
+    expected = F.conv2d(x.cpu().double(), weight.cpu().double(), padding=1, stride=stride)
+    out = torch.full(expected.shape, float("nan"), dtype=torch.float16, device="cuda")
+    assert _launch(x, weight, out, 1, stride, 1, way) == 0
+    served = runtime.last_launch()
+    assert "conv2d_window_kernel" not in served
+    assert bool(((out.cpu().double() - expected).abs() <= 2.0**-11 * expected.abs() + 2.0**-24 * weight[0].numel() ** 0.5 * 4 + 2.0**-25).all())
+    assert _launch(x, weight, out, 1, stride, 1, 0) == 0 and runtime.last_launch() == served
+
+
+@pytest.mark.parametrize("stride", (1, 2))
+def test_a_program_of_blocks_of_five_positions(stride):
+    import functools
+
+    import ninetoothed_amd as ninetoothed
+    from ninetoothed_amd import programs
+
+    torch.manual_seed(stride)
+    side = 16 * stride + 3 - stride
+    x, weight = torch.randn(2, 16, side, side, device="cuda").half(), (torch.randn(32, 16, 3, 3, device="cuda") / 12).half()
+    expected = F.conv2d(x.cpu().double(), weight.cpu().double(), stride=stride)
+    out = torch.full(expected.shape, float("nan"), dtype=torch.float16, device="cuda")
+    arrangement = functools.partial(programs.conv2d.arrangement, enable_padding=False, BLOCK_SIZE_M=5, BLOCK_SIZE_N=64, BLOCK_SIZE_K=64, stride=(stride, stride), floor_mode=True)
+    ninetoothed.make(arrangement, programs.conv2d.application, programs.conv2d.tensors())(x, weight, out)
+    assert bool(((out.cpu().double() - expected).abs() <= 2.0**-11 * expected.abs() + 2.0**-24 * weight[0].numel() ** 0.5 * 4 + 2.0**-25).all())
