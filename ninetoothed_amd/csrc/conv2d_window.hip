@@ -257,6 +257,31 @@ __global__ __launch_bounds__(kWindowThreads, 2) void conv2d_window_kernel(ConvWi
 #endif
 }
 
+// bytes from the first to the last element that the kernel reads
+int64_t x_extent(const Conv2dRequest &q) { return ((int64_t)(q.N - 1) * q.xs[0] + (int64_t)(q.C - 1) * q.xs[1] + (int64_t)q.H * q.W) * 2; }
+int64_t w_extent(const Conv2dRequest &q) { return ((int64_t)(q.K - 1) * q.ws[0] + (int64_t)q.C * q.R * q.S) * 2; }
+
+// The positions of the largest window, 0 when the kernel does not take the problem.
+int window_positions(const Conv2dRequest &q) {
+    if (q.R != 3 || q.S != 3 || q.C % 8 || q.C < 32) return 0;
+    if (q.xs[3] != 1 || q.xs[2] != q.W || q.W < 4 || q.xs[0] < 0 || q.xs[1] < 0) return 0;  // the pixels of a channel lie one after another
+    if (q.ws[3] != 1 || q.ws[2] != q.S || q.ws[1] != (int64_t)q.R * q.S || q.ws[0] < 0) return 0;
+    if (x_extent(q) >= (int64_t(1) << 31) || w_extent(q) >= (int64_t(1) << 31)) return 0;  // 32-bit buffer offsets
+    if ((int64_t)q.N * q.H * q.W > 0x3fffffffll || (int64_t)q.N * q.P * q.Q > 0x3fffffffll) return 0;
+    if (q.N > 1 << 20 || q.P > 1 << 20) return 0;  // (quick_quotient)
+    // Every output row looks at the image at its top or below it, and at its bottom or above it, so that the first and the last row of a
+    // window are those of its first and its last position, but for what lies in the padding.
+    if (q.pad_h > (q.R - 1) * q.dil_h || (int64_t)(q.P - 1) * q.stride_h - q.pad_h > q.H - 1) return 0;
+    const int PQ = q.P * q.Q;
+    // the most rows that a tile of positions looks at: output rows of an image are stride_h input rows apart, the first of an image and the
+    // last of the one before it H - P * stride_h more
+    const int64_t images = std::min<int64_t>(q.N, (kWindowBM - 2) / PQ + 2), out_rows = std::min<int64_t>((kWindowBM + q.Q - 2) / q.Q + 1, (int64_t)q.N * q.P);
+    const int64_t rows = std::min<int64_t>(images * q.H, (out_rows - 1) * q.stride_h + (images - 1) * std::max(0, q.H - q.P * q.stride_h) + (q.R - 1) * q.dil_h + 1);
+    const int64_t window = rows * q.W;
+    if (((window + 3 * images) / 4 + 1) * 4 > kWindowItems * kWindowThreads) return 0;
+    return (int)window;
+}
+
 // Whether this kernel is expected to be faster than the repacking path, in microseconds, by both models fitted to 320 convolutions (1 to
 // 32 images of 7 x 7 to 112 x 112, 32 to 256 channels, 16 to 512 filters, steps 1 and 2; 8 and 6 % off on average): it wins where its
 // workgroups fill the chip about once -- fewer leave CUs idle that the other path's parts of the contraction use, more pay the long block.  Of
@@ -272,25 +297,8 @@ bool window_pays(const Conv2dRequest &q) {
 }
 
 template <typename T>
-int run_window(const Conv2dRequest &q, hipStream_t stream) {
-    if (q.R != 3 || q.S != 3 || q.C % 8 || q.C < 32) return NINETOOTHED_NO_KERNEL;
-    if (q.xs[3] != 1 || q.xs[2] != q.W || q.W < 4 || q.xs[0] < 0 || q.xs[1] < 0) return NINETOOTHED_NO_KERNEL;  // the pixels of a channel lie one after another
-    if (q.ws[3] != 1 || q.ws[2] != q.S || q.ws[1] != (int64_t)q.R * q.S || q.ws[0] < 0) return NINETOOTHED_NO_KERNEL;
-    const int64_t x_bytes = ((int64_t)(q.N - 1) * q.xs[0] + (int64_t)(q.C - 1) * q.xs[1] + (int64_t)q.H * q.W) * 2;
-    const int64_t w_bytes = ((int64_t)(q.K - 1) * q.ws[0] + (int64_t)q.C * q.R * q.S) * 2;
-    if (x_bytes >= (int64_t(1) << 31) || w_bytes >= (int64_t(1) << 31)) return NINETOOTHED_NO_KERNEL;  // 32-bit buffer offsets
-    if ((int64_t)q.N * q.H * q.W > 0x3fffffffll || (int64_t)q.N * q.P * q.Q > 0x3fffffffll) return NINETOOTHED_NO_KERNEL;
-    if (q.N > 1 << 20 || q.P > 1 << 20) return NINETOOTHED_NO_KERNEL;  // (quick_quotient)
-    // Every output row looks at the image at its top or below it, and at its bottom or above it, so that the first and the last row of a
-    // window are those of its first and its last position, but for what lies in the padding.
-    if (q.pad_h > (q.R - 1) * q.dil_h || (int64_t)(q.P - 1) * q.stride_h - q.pad_h > q.H - 1) return NINETOOTHED_NO_KERNEL;
+int run_window(const Conv2dRequest &q, int window, hipStream_t stream) {
     const int M = q.N * q.P * q.Q, PQ = q.P * q.Q;
-    // the most rows that a tile of positions looks at: output rows of an image are stride_h input rows apart, the first of an image and the
-    // last of the one before it H - P * stride_h more
-    const int64_t images = std::min<int64_t>(q.N, (kWindowBM - 2) / PQ + 2), out_rows = std::min<int64_t>((kWindowBM + q.Q - 2) / q.Q + 1, (int64_t)q.N * q.P);
-    const int64_t rows = std::min<int64_t>(images * q.H, (out_rows - 1) * q.stride_h + (images - 1) * std::max(0, q.H - q.P * q.stride_h) + (q.R - 1) * q.dil_h + 1);
-    const int64_t window = rows * q.W;
-    if (((window + 3 * images) / 4 + 1) * 4 > kWindowItems * kWindowThreads) return NINETOOTHED_NO_KERNEL;
     ConvWindowParams p;
     p.x = q.x; p.w = q.w; p.y = q.y;
     p.N = q.N; p.C = q.C; p.H = q.H; p.W = q.W; p.K = q.K; p.P = q.P; p.Q = q.Q;
@@ -302,13 +310,15 @@ int run_window(const Conv2dRequest &q, hipStream_t stream) {
     p.one_by_pq = 1.0f / (float)PQ;
     p.one_by_q = 1.0f / (float)q.Q;
     p.one_by_runs = 1.0f / (float)((q.H * q.W + 3) / 4);
-    p.x_bytes = (unsigned)x_bytes;
-    p.w_bytes = (unsigned)w_bytes;
-    p.window = (int)window;
+    p.x_bytes = (unsigned)x_extent(q);
+    p.w_bytes = (unsigned)w_extent(q);
+    p.window = window;
     // the rows that a read of fragments serves together are four positions of one group and four of the next: a step of 1 fills 16-byte slots one
     // after another in both, a step of 2 every other slot, so that the next group is moved by one
-    p.plane = ((int)window * 16 + 255) / 256 * 256 + (q.stride_w % 2 == 0 ? 16 : 0);
-    // (at most 118 KiB; the sums that the groups exchange take the same place, 7 KiB a wave)
+    p.plane = (window * 16 + 255) / 256 * 256 + (q.stride_w % 2 == 0 ? 16 : 0);
+    // (the sums that the groups exchange take the same place, 7 KiB a wave)
+    constexpr int kMostBytes = kWindowZeros + 4 * (kWindowItems * kWindowThreads * 16 + 16) + 9 * 4 * kWindowBN * 16;
+    static_assert(kMostBytes <= 160 * 1024, "the largest window and its filters in LDS (132.3 KiB)");
     const size_t bytes = std::max(kWindowZeros + 4 * (size_t)p.plane + (size_t)q.R * q.S * 4 * kWindowBN * 16, (size_t)(kWindowThreads / 64) * (kWindowWaveM / 16) * 1024);
     const dim3 grid((unsigned)ceil_div(M, kWindowBM), (unsigned)ceil_div(q.K, kWindowBN));
     if (grid.y > 65535) return NINETOOTHED_NO_KERNEL;
@@ -321,8 +331,10 @@ int run_window(const Conv2dRequest &q, hipStream_t stream) {
 
 int conv2d_window(const Conv2dRequest &q, hipStream_t stream, bool if_it_pays) {
     if (q.dtype != NINETOOTHED_FLOAT16 && q.dtype != NINETOOTHED_BFLOAT16) return NINETOOTHED_NO_KERNEL;
-    if (if_it_pays && !window_pays(q)) return NINETOOTHED_NO_KERNEL;
-    return q.dtype == NINETOOTHED_FLOAT16 ? run_window<half_t>(q, stream) : run_window<bf16_t>(q, stream);
+    // (what the kernel takes comes first: the expected times go through all tiles and numbers of parts of the other path)
+    const int window = window_positions(q);
+    if (window == 0 || (if_it_pays && !window_pays(q))) return NINETOOTHED_NO_KERNEL;
+    return q.dtype == NINETOOTHED_FLOAT16 ? run_window<half_t>(q, window, stream) : run_window<bf16_t>(q, window, stream);
 }
 
 }  // namespace nt

@@ -69,6 +69,7 @@ def _check(x, weight, padding, stride, dilation, layout):
         (2, 48, 26, 19, 17, 2, 2, 2),
         (6, 32, 6, 22, 40, 1, 3, 1),
         (2, 32, 31, 17, 64, 0, 4, 1),  # steps longer than the window
+        (2, 40, 7, 109, 70, 0, 2, 1),  # a window of 1526 positions, of the most that fit (1532): 132 KiB of LDS
     ),
 )
 def test_against_64_bits(n, c, height, width, k, padding, stride, dilation, dtype, layout):
