@@ -981,23 +981,34 @@ struct MapCodegen {
     // before the phases and converted once all are on their way.  What bounded rows of no whole number of elements per thread was a chain of trips to
     // memory: behind a branch around each load, its conversion or its use waited for it before the next was asked for.  So a thread whose last
     // elements lie behind the tile asks for the tile's last one again (not where it has only one, or one group: one branch around all
-    // operands lets whole waves skip them, fp16 12995 x 1440 11.8 us, 12.5 with a test for each).  Operands that only the stored expression reads join while all take up to 48 registers.
+    // operands lets whole waves skip them, fp16 12995 x 1440 11.8 us, 12.5 with a test for each).  Operands that only the stored expression reads join while all take up to 48 registers; several of them
+    // on 1024 threads, 128 registers each, only where that is at most 45 (layer norm with a bias, fp32 1024 x 16384: joined 49.5 us with 36 bytes of scratch, not joined 34.8).
     // Rms norm, us, before -> after: fp32 4541 x 3200 26.9 -> 21.0 (5.5 TB/s), 3350 x 1680 13.3 -> 10.2, 787 x 4160 9.6 -> 6.1, fp16 4702 x 7208
     // 28.4 -> 26.9; branches kept and only the conversions moved: 21.1, 10.9, 6.7, 27.8.
     void preload(long long tile_elements, int per_thread) {
         const int width = tile_width > 0 ? tile_width : 1, groups = per_thread / width;
-        std::vector<int> slots;
+        const auto registers_of = [&](int slot) { return kept_as_float(slot) ? per_thread : 2 * per_thread; };
+        std::vector<int> slots, stored_only;
+        int registers = 0, all = 0;
         for (int pc = 0; pc < p.value_code_length; ++pc) {
-            if ((p.value_code[pc] & 0xff) == NT_MAP_V_SETVAR) return;  // (an index that is itself loaded)
             if ((p.value_code[pc] & 0xff) != NT_MAP_V_LOAD) continue;
             const int slot = p.value_code[pc] >> 8;
-            if (kept[slot]) continue;
-            int registers = kept_as_float(slot) ? per_thread : 2 * per_thread;
-            for (int other : slots) registers += kept_as_float(other) ? per_thread : 2 * per_thread;
-            if (tile_width == 0 && pc >= p.phase_end[p.num_phases - 1] && registers > 48) continue;
-            slots.push_back(slot);
-            kept[slot] = true;
+            if (std::find(slots.begin(), slots.end(), slot) != slots.end() || std::find(stored_only.begin(), stored_only.end(), slot) != stored_only.end()) continue;
+            all += registers_of(slot);
+            if (pc >= p.phase_end[p.num_phases - 1]) {
+                stored_only.push_back(slot);
+            } else {
+                registers += registers_of(slot);
+                slots.push_back(slot);
+            }
         }
+        const bool too_many = threads == 1024 && stored_only.size() > 1 && all > 45;
+        for (int slot : stored_only) {
+            if (tile_width == 0 && (too_many || registers + registers_of(slot) > 48)) continue;
+            registers += registers_of(slot);
+            slots.push_back(slot);
+        }
+        for (int slot : slots) kept[slot] = true;
         if (tile_width > 0) vector_typedefs(width, "        ");
         if (tile_width > 0 && groups == 1) {
             out << "        if (const nt_idx element = member * " << width << "; element < " << lit(tile_elements) << ") {\n";
@@ -1141,6 +1152,11 @@ struct MapCodegen {
             tile_width = 0;
             return out.str();
         }
+        // The elements' places are worked out again here: kept from the loads on, they took a register per element and tensor, which at 1024 threads
+        // cost a second workgroup per CU (more than 64) or went to scratch (more than 128).  Us, with the places kept -> here: layer norm with a bias fp32
+        // 900 x 14336 46.3 -> 26.4, fp64 1024 x 12288 84.1 -> 47.3, softmax of a sum of two rows fp32 1000 x 12288 35.8 -> 28.7, but 1024 x 16384 41.7 -> 42.4.
+        if (keep_loads)
+            out << "        nt_idx again = member;\n        asm volatile(\"\" : \"+v\"(again));\n        __builtin_assume(again >= 0 && again < " << group << ");\n        {\n        const nt_idx member = again;\n";
         open_element_loop(tile_elements, per_thread, "        ");
         indent = "            ";
         decode_tile_variables();
@@ -1149,7 +1165,7 @@ struct MapCodegen {
         const std::string offset = index_segment(target.segment, "store_ok");
         out << indent << "if (store_ok) " << store_stmt("a.data[" + std::to_string(p.output) + "]", target.dtype, offset, result) << "\n";
         close_element_loop("        ");
-        out << "    }\n}\n";
+        out << (keep_loads ? "        }\n" : "") << "    }\n}\n";
         keep_loads = false;
         return out.str();
     }

@@ -1085,6 +1085,74 @@ def test_generated_source_groups_elements_of_16_bit_tensors():
     assert "nt_vec_f16" in _generated_source(layer_norm, (half(64, 16384), half(16384), half(64, 16384)))
 
 
+def _row_bias_arrangement(input, weight, bias, output):
+    return _rows(input), weight.tile((-1,)).expand((input.shape[0],)), bias.tile((-1,)).expand((input.shape[0],)), _rows(output)
+
+
+def _layer_norm_bias_application(input, weight, bias, output):
+    mean = ntl.sum(input) / input.shape[-1]
+    centred = input - mean
+    variance = ntl.sum(centred * centred) / input.shape[-1]
+    output = centred * ntl.rsqrt(variance + 1e-5) * weight + bias  # noqa: F841
+
+
+def _two_rows_arrangement(input, other, output):
+    return _rows(input), _rows(other), _rows(output)
+
+
+def _masked_softmax_application(input, other, output):
+    scores = input * 0.125 + other
+    numerator = ntl.exp(scores - ntl.max(scores))
+    output = numerator / ntl.sum(numerator)  # noqa: F841
+
+
+def _layer_norm_bias():
+    return ninetoothed.make(_row_bias_arrangement, _layer_norm_bias_application, (Tensor(2), Tensor(1), Tensor(1), Tensor(2)))
+
+
+def _masked_softmax():
+    return ninetoothed.make(_two_rows_arrangement, _masked_softmax_application, (Tensor(2), Tensor(2), Tensor(2)))
+
+
+@pytest.mark.parametrize("dtype, cols, rows, most", (("fp32", 14336, 900, 128), ("fp32", 16384, 1024, 128), ("fp16", 14336, 900, 128), ("fp32", 12288, 1000, 64), ("fp16", 12288, 1000, 64)))
+def test_rows_of_1024_threads_keep_to_their_registers(dtype, cols, rows, most, tmp_path):
+    """A lane of 1024 threads has 128 registers, 64 where a CU shall hold two workgroups: row programs of three tensors and two
+    reductions keep to them and use no scratch memory."""
+    import re
+    import subprocess
+
+    from ninetoothed_amd import build_library
+
+    element = torch.float32 if dtype == "fp32" else torch.float16
+    row, column = (torch.empty(shape, dtype=element) for shape in ((rows, cols), (cols,)))
+    source = _generated_source(_layer_norm_bias(), (row, column, column, row)) if most == 128 else _generated_source(_masked_softmax(), (row, row, row))
+    path = tmp_path / "map.hip"
+    path.write_text("#include <hip/hip_runtime.h>\n" + source)
+    flags = ["--offload-arch=gfx950", "-O3", "-ffp-contract=off", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", "--offload-device-only", "-S"]
+    subprocess.run([build_library._hipcc(), *flags, str(path), "-o", str(tmp_path / "map.s")], check=True, capture_output=True)
+    assembly = (tmp_path / "map.s").read_text()
+    assert int(re.search(r"\.vgpr_count:\s*(\d+)", assembly).group(1)) <= most
+    assert int(re.search(r"\.private_segment_fixed_size:\s*(\d+)", assembly).group(1)) == 0
+
+
+@gpu
+@pytest.mark.parametrize("rows, cols", ((3, 8193), (2, 12288), (5, 14336), (2, 15001), (3, 16384)))
+def test_rows_of_three_tensors_on_1024_threads(rows, cols):
+    """(fp32: a dozen roundings of 2^-23 along a sum, values below 16.)"""
+    torch.manual_seed(cols)
+    x, other = torch.randn(rows, cols, device="cuda"), torch.randn(rows, cols, device="cuda")
+    weight, bias = torch.randn(cols, device="cuda"), torch.randn(cols, device="cuda")
+    out = torch.full((rows, cols), float("nan"), device="cuda")
+    kernel = _layer_norm_bias()
+    kernel(x, weight, bias, out)
+    _served_by_map(kernel)
+    assert torch.allclose(out.double(), F.layer_norm(x.double(), (cols,), weight.double(), bias.double(), 1e-5), rtol=1e-5, atol=1e-5)
+    kernel = _masked_softmax()
+    kernel(x, other, out)
+    _served_by_map(kernel)
+    assert torch.allclose(out.double(), torch.softmax(x.double() * 0.125 + other.double(), -1), rtol=1e-5, atol=1e-9)
+
+
 @gpu
 @pytest.mark.parametrize("dtype", (torch.float16, torch.bfloat16))
 def test_grouped_elements_of_16_bit_tensors(dtype):
