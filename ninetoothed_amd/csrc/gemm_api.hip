@@ -87,6 +87,14 @@ bool fast_accepts(const GemmProblem &q) {
     return true;
 }
 
+// Whether a product's tiles are dealt to the XCDs one by one (bit 8 of GemmParams::order) instead of in contiguous ranges: a tall product -- at least 9 rows
+// of tiles and twice as many as columns -- whose number of tiles is no multiple of 8.  One by one, a strip of 8 tile rows gives every XCD a row
+// of its own, whose panel of the lhs it reads once for all the few columns; ranges read it into two or three L2s.  Us, ranges / one by one: 128 x 128
+// tiles with K in parts 19 x 3 of them, K 12800 40.7 / 32.8, 17 x 3, 6400 24.2 / 20.5, 23 x 2, 6400 22.4 / 20.2, 12 x 7, 12800 44.4 / 41.9; 64 x 64 in parts 41 x 2,
+// 12800 27.2 / 23.9; 128 x 256 39 x 7, 2368 53.1 / 47.8; 128 x 128 on a deep ring 17 x 3, 4672 29.0 / 27.6.  Less tall ones gain by ranges (11 x 7 of 128 x 128 in parts
+// 0.9 of the time), and so do 256 x 256 tiles (44 x 9, K 4672 0.92).
+bool tiles_one_by_one(const GemmParams &p, int bm) { return bm <= 128 && p.tiles_m * (int64_t)p.tiles_n % 8 != 0 && p.tiles_n > 1 && p.tiles_m >= 9 && p.tiles_m / 2 >= p.tiles_n; }
+
 void fill_params(GemmParams &p, const GemmProblem &q, int bm, int bn) {
     p.a = q.a;
     p.b = q.b;
@@ -107,7 +115,7 @@ void fill_params(GemmParams &p, const GemmProblem &q, int bm, int bn) {
     p.beta = q.beta;
     p.tiles_m = (q.m + bm - 1) / bm;
     p.tiles_n = (q.n + bn - 1) / bn;
-    p.order = g_tile_order;
+    p.order = g_tile_order | (tiles_one_by_one(p, bm) ? 0x100 : 0);
     p.bias_vector = q.bias != nullptr && q.sin == 1 && q.sim % 8 == 0 && ((uintptr_t)q.bias & 15) == 0 && q.n % 8 == 0 && (q.batch == 1 || q.bias_batch % 8 == 0);
     p.c_vector = ((uintptr_t)q.c & 15) == 0 && q.scm % 8 == 0 && q.n % 8 == 0 && (q.batch == 1 || q.c_batch % 8 == 0);
     p.kt_per_split = 0;

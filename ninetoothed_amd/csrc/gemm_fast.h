@@ -34,7 +34,7 @@ struct GemmParams {
     float lower;     // ... and its results are at least this
     int tiles_m, tiles_n;
     int bias_vector;  // addmm input readable with aligned 16-byte loads along N
-    int order;  // tile order: 0 = XCD-aware strips of 8 tile rows; other values are measurement aids
+    int order;  // tile order: 0 = XCD-aware strips of 8 tile rows, 0x100 = the strips' tiles dealt to the XCDs one by one; other values are measurement aids
     int kt_per_split;  // split-K instances: k tiles per part (the grid holds tiles * parts workgroups)
     int out_float;     // skinny kernel: C holds fp32 (the tile kernels have it as a template parameter)
     int c_vector;      // rows of C take aligned 16-byte stores (else, in the instances with tails: element stores)
@@ -86,7 +86,7 @@ NT_HOST_DEVICE constexpr int b_phys_chunk16(int krow, int chunk) {
 // tile-rows so that concurrently running tiles reuse A and B panels in L2.  Also where the
 // number of tiles is no multiple of 8: dealt out one by one such tiles fetch their panels into
 // all eight L2s (bf16, us, before / with ranges: 348 x 9536 x 1152 14.5 / 11.5, 371 x 9280 x 6848
-// 62.1 / 50.0, 728 x 4736 x 3904 36.9 / 29.4, 7497 x 14080 x 2112 371 / 347).
+// 62.1 / 50.0, 728 x 4736 x 3904 36.9 / 29.4, 7497 x 14080 x 2112 371 / 347); the callers except tall products (bit 8 of `order`).
 NT_DEVICE void map_tile(int tiles_m, int tiles_n, int order, int &tile_m, int &tile_n, int bid = blockIdx.x, int nblocks = gridDim.x) {
     // order: low 8 bits = tile rows per strip (0 -> 8), bit 8 = skip the XCD remap
     const int group_m = (order & 0xff) ? (order & 0xff) : 8;
