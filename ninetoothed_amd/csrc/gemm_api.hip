@@ -159,10 +159,23 @@ bool rows_straddle_lines(const GemmProblem &q) {
     return q.m > 64 && inside(q.a, q.sam, q.a_batch);
 }
 
+// ... and whether that pays: another line has to land before the first step, which short contractions do not make up for.  In one piece from a K of
+// 256 on with a transposed rhs and of 768 without, and 5e8 products (bf16, us, k tiles / lines: 64 x 64 tiles 4096 x 4096 x 72 18.5 / 21.1, 2048 x 1024 x
+// 136 4.7 / 5.0, 1024 x 512 x 520 4.2 / 4.5, 4096 x 1024 x 264 8.8 / 8.4; not transposed 4096 x 1024 x 264 7.9 / 8.3, x 776 15.7 / 14.6; 128 x 128 tiles 4096 x 4096 x 24
+// 13.3 / 15.0, 2048 x 1024 x 392 6.7 / 6.4).  In parts, of a few k tiles each, on 128 x 128 tiles only with a transposed rhs and 32 tiles or more (256 x
+// 512 x 16392 19.3 / 20.9, 1024 x 1024 x 8200 34.3 / 32.6; not transposed 270 x 232 x 16392 16.5 / 19.3, 1024 x 512 x 8200 22.4 / 23.8), on 64 x 64 from 16 tiles on
+// and 64 without (128 x 128 x 8200 9.4 / 10.1, 1024 x 1024 x 8200 38.3 / 34.4).
+bool lines_pay(const GemmProblem &q, int bm, int bn, bool in_parts) {
+    const bool transposed = b_is_transposed(q);
+    if (!in_parts) return q.k >= (transposed ? 256 : 768) && (double)q.batch * q.m * q.n * q.k >= 5e8;
+    const int64_t tiles = (int64_t)ceil_div(q.m, bm) * ceil_div(q.n, bn);
+    return bm == 128 ? transposed && tiles >= 32 : tiles >= (transposed ? 16 : 64);
+}
+
 template <typename T, int BM, int BN, int BK, int WM, int WN, int kStages, int kOcc, int kAblate, int kLoad, int kAux, bool kTail, bool kLines>
 hipError_t fast_launch_typed(const GemmProblem &q, hipStream_t stream) {
     if constexpr (kLines)
-        if (rows_straddle_lines(q)) return fast_launch_form<T, BM, BN, BK, WM, WN, 5, kOcc, kAblate, kLoad, kAux, kTail, true>(q, stream);
+        if (rows_straddle_lines(q) && lines_pay(q, BM, BN, false)) return fast_launch_form<T, BM, BN, BK, WM, WN, 5, kOcc, kAblate, kLoad, kAux, kTail, true>(q, stream);
     return fast_launch_form<T, BM, BN, BK, WM, WN, kStages, kOcc, kAblate, kLoad, kAux, kTail, false>(q, stream);
 }
 
@@ -323,7 +336,7 @@ hipError_t split_launch_typed(const GemmProblem &q, hipStream_t stream) {
         if (b_is_transposed(q)) gemm_nn_fast_kernel<T, BM, BN, BK, WM, WN, kRing, kOcc, kPlain, 0, 1, 0, true, true, true, true, kByLines><<<grid, block, 0, stream>>>(p);
         else gemm_nn_fast_kernel<T, BM, BN, BK, WM, WN, kRing, kOcc, kPlain, 0, 1, 0, true, false, true, true, kByLines><<<grid, block, 0, stream>>>(p);
     };
-    if (kLines && rows_straddle_lines(q)) launch(std::integral_constant<int, kLines ? 5 : kStages>(), std::integral_constant<bool, kLines>());
+    if (kLines && rows_straddle_lines(q) && lines_pay(q, BM, BN, true)) launch(std::integral_constant<int, kLines ? 5 : kStages>(), std::integral_constant<bool, kLines>());
     else launch(std::integral_constant<int, kStages>(), std::false_type());
     hipError_t err = hipGetLastError();
     if (err != hipSuccess) return err;
