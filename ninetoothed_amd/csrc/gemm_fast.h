@@ -903,28 +903,27 @@ __global__ __launch_bounds__(WM *WN * 64, kWavesPerSimd) void gemm_nn_fast_kerne
     static_assert(kWaves <= 2 * (kSlabsA + kSlabsB), "epilogue slabs do not fit two stages");
     typedef vec8 unaligned_vec8 __attribute__((aligned(2)));  // (global accesses need no more than the element's alignment)
     const T *bias = (const T *)p.bias + batch * p.bias_batch;
-    // addmm: the input's values of the first blocks of rows (64 registers, which the fragments leave) are asked for before the last fills
-    // have landed, those of later blocks a round of blocks ahead.  Asked for where they are used, behind the branch for rows that are not there, they were a chain
+    // addmm: the input's values of the wave's whole tile (64 registers at most, which the fragments leave) are asked for before the last fills
+    // have landed.  Asked for where they are used, behind the branch for rows that are not there, they were a chain
     // of trips to memory, 16 in a wave's 128 x 64 tile: 4918 x 16160 x 576 bf16 155 -> 130 us, 6606 x 2208 x 448 30.3 -> 24.9, 8192^3 fp16 786 -> 775.
     // Not where a row's last chunk is partial or columns lie apart.
-    constexpr int kInputChunks = kEpilogue == kAddmm ? kCChunks / 2 : 1, kInputBlocks = kEpilogue == kAddmm ? (TM * kInputChunks <= 16 ? TM : 16 / kInputChunks) : 1;
-    static_assert(kInputChunks <= 16 && kInputBlocks >= 1, "registers for a block of the input");
+    constexpr int kInputChunks = kEpilogue == kAddmm ? kCChunks / 2 : 1, kInputBlocks = kEpilogue == kAddmm ? TM : 1;
+    static_assert(kInputChunks * kInputBlocks <= 16, "registers for the input");
     const bool input_ahead = kEpilogue == kAddmm && p.bias_stride_n == 1 && p.n % 8 == 0;
     unaligned_vec8 input[kInputBlocks][kInputChunks];
-    const auto request_input = [&](auto ti_tag) {
-        constexpr int ti = decltype(ti_tag)::value;
-        if constexpr (kEpilogue == kAddmm) {
-            if (!input_ahead) return;
+    if constexpr (kEpilogue == kAddmm) {
+        if (input_ahead) {
 #pragma unroll
-            for (int it = 0; it < kInputChunks; ++it) {
-                const int row = (it * 64 + lane) / kCChunks, phys = (it * 64 + lane) % kCChunks;
-                const int chunk = phys ^ ((row >> kCShift) & (kCChunks - 1));
-                const int grow = min(m0 + wave_m * kWaveM + ti * 32 + row, p.m - 1), gcol = min(n0 + wave_n * kWaveN + chunk * 8, p.n - 8);  // (rows and columns that are not there: the last ones)
-                input[ti % kInputBlocks][it] = *(const unaligned_vec8 *)(bias + (int64_t)grow * p.bias_stride_m + gcol);
-            }
+            for (int ti = 0; ti < TM; ++ti)
+#pragma unroll
+                for (int it = 0; it < kInputChunks; ++it) {
+                    const int row = (it * 64 + lane) / kCChunks, phys = (it * 64 + lane) % kCChunks;
+                    const int chunk = phys ^ ((row >> kCShift) & (kCChunks - 1));
+                    const int grow = min(m0 + wave_m * kWaveM + ti * 32 + row, p.m - 1), gcol = min(n0 + wave_n * kWaveN + chunk * 8, p.n - 8);  // (rows and columns that are not there: the last ones)
+                    input[ti][it] = *(const unaligned_vec8 *)(bias + (int64_t)grow * p.bias_stride_m + gcol);
+                }
         }
-    };
-    static_for<0, kInputBlocks>(request_input);
+    }
     wait_vmcnt<0>();
     lds_barrier();
     NT_LDS unsigned char *slab;
@@ -956,8 +955,9 @@ __global__ __launch_bounds__(WM *WN * 64, kWavesPerSimd) void gemm_nn_fast_kerne
                 column_bias[tj][e] = !kTail || col < p.n ? linear_bias<T>(p, col) : 0.0f;
             }
     }
-    static_for<0, TM>([&](auto ti_tag) {
-        constexpr int ti = decltype(ti_tag)::value;
+    // (a loop, no chain of calls: with one the kernel's parameters were loaded again for every store, 0.4 us of a workgroup's 5)
+#pragma unroll
+    for (int ti = 0; ti < TM; ++ti) {
         if constexpr (kM16) {
             // 16x16 blocks: lane (i16, kg) holds columns 4 kg .. + 3 of row i16; two blocks of rows fill a slab
 #pragma unroll
@@ -1017,7 +1017,7 @@ __global__ __launch_bounds__(WM *WN * 64, kWavesPerSimd) void gemm_nn_fast_kerne
                 const T *src = bias + (int64_t)grow * p.bias_stride_m + (int64_t)gcol * p.bias_stride_n;
                 vec8 in;
                 if (input_ahead) {
-                    in = input[ti % kInputBlocks][kEpilogue == kAddmm ? it : 0];
+                    in = input[kEpilogue == kAddmm ? ti : 0][kEpilogue == kAddmm ? it : 0];
                 } else if (p.bias_vector) {
                     in = *(const vec8 *)src;
                 } else if (p.bias_stride_n == 1 && (!kTail || gcol + 8 <= p.n)) {
@@ -1045,8 +1045,7 @@ __global__ __launch_bounds__(WM *WN * 64, kWavesPerSimd) void gemm_nn_fast_kerne
             // (4096^3 addmm +3 %, 8192^3 +0.3 %)
             __builtin_nontemporal_store(v, (vec_out *)(C + (int64_t)grow * p.ldc + gcol));
         }
-        if constexpr (ti + kInputBlocks < TM) request_input(std::integral_constant<int, ti + kInputBlocks>());
-    });
+    }
 #endif
 }
 
