@@ -658,7 +658,7 @@ int skinny_choice(const GemmProblem &q) {
 // ---- tiles over whole rounds of the chip ----
 // 336 tiles of 256 x 256 on 256 CUs take two rounds, the second with 80 CUs at work.  The columns (or rows) of tiles that fill whole
 // rounds run in one launch, what is left as a product of its own before it: K in parts where it has few tiles, else 128 x 128 tiles on a deep ring,
-// of which up to two rounds (128 tiles of 256 x 256 left) still take less time than another round of large ones.  Both launches read one operand whole: the
+// of which up to two rounds (half a round of 256 x 256 tiles left, 128) still take less time than another round of large ones.  Both launches read one operand whole: the
 // smaller one (rows cut off 1500 x 14336 x 4096 read its rhs of 117 MB twice: 168 us with inputs that come from memory, 144 with them in the caches).
 // One launch of 256 x 256 tiles / this, bf16, us, sustained with changing inputs: 1500 x 14336 x 4096 (84 tiles left) 169 / 156, 4608 x 4608 x 4096 (72) 153 /
 // 148, 1314 x 15104 x 13688 (102) 815 / 667, 1571 x 12672 x 1128 (98) 59.2 / 59.4; single products: 2079 x 9088 x 3264 (72) 132 / 104, 1153 x
@@ -666,8 +666,8 @@ int skinny_choice(const GemmProblem &q) {
 // Of a short K, 2967 x 7872 x 512 (120) 31.9 / 28.9, but 2058 x 7680 x 512 (18) has 19.3 on 128 x 256 tiles against 22, which only the tuner knows.
 template <bool kColumns>
 int64_t cut_whole(const GemmProblem &q) {  // columns (rows) of 256 x 256 tiles that fill whole rounds
-    const int64_t along = ceil_div(kColumns ? q.n : q.m, 256), across = ceil_div(kColumns ? q.m : q.n, 256);
-    return along * across / 256 * 256 / across;
+    const int64_t along = ceil_div(kColumns ? q.n : q.m, 256), across = ceil_div(kColumns ? q.m : q.n, 256), units = std::max(1, compute_units());
+    return along * across / units * units / across;
 }
 
 template <bool kColumns>
@@ -699,9 +699,9 @@ void cut_problem(const GemmProblem &q, GemmProblem &whole, GemmProblem &left) {
 template <bool kColumns>
 bool cut_accepts(const GemmProblem &q) {
     if ((q.dtype != NINETOOTHED_FLOAT16 && q.dtype != NINETOOTHED_BFLOAT16) || q.batch != 1 || q.hinted || q.fixed_scratch != nullptr || q.m <= 0 || q.n <= 0) return false;
-    const int64_t tiles = (int64_t)ceil_div(q.m, 256) * ceil_div(q.n, 256), whole = cut_whole<kColumns>(q);
-    if (kColumns != (q.m <= q.n) || tiles <= 256 || tiles % 256 == 0 || q.k < 512 || whole < 1 || cut_left<kColumns>(q) > 128) return false;
-    if (tiles > 4 * 256 + 128) return false;  // (what a round costs shrinks to the spread between runs)
+    const int64_t tiles = (int64_t)ceil_div(q.m, 256) * ceil_div(q.n, 256), whole = cut_whole<kColumns>(q), units = compute_units();
+    if (units <= 0 || kColumns != (q.m <= q.n) || tiles <= units || tiles % units == 0 || q.k < 512 || whole < 1 || 2 * cut_left<kColumns>(q) > units) return false;
+    if (tiles > 4 * units + units / 2) return false;  // (what a round costs shrinks to the spread between runs)
     GemmProblem top, left;
     cut_problem<kColumns>(q, top, left);
     return kInstances[kTail256x256x32].accepts(top) && kInstances[kDeep128x128x64].accepts(left);
@@ -711,7 +711,7 @@ template <bool kColumns>
 hipError_t cut_launch(const GemmProblem &q, hipStream_t stream) {
     GemmProblem whole, left;
     cut_problem<kColumns>(q, whole, left);
-    int rest = (int64_t)ceil_div(left.m, 128) * ceil_div(left.n, 128) <= 256 ? heuristic_choice(left, 0, 0, 0) : (int)kDeep128x128x64;
+    int rest = (int64_t)ceil_div(left.m, 128) * ceil_div(left.n, 128) <= compute_units() ? heuristic_choice(left, 0, 0, 0) : (int)kDeep128x128x64;
     if (rest <= kAnyStride || !kInstances[rest].accepts(left)) rest = kDeep128x128x64;
     hipError_t result = kInstances[rest].launch(left, stream);  // (first: a split-K instance may find no scratch memory)
     if ((int)result == NINETOOTHED_NO_KERNEL && is_split(rest)) result = kInstances[kDeep128x128x64].launch(left, stream);
