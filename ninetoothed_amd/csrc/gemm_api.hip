@@ -159,6 +159,8 @@ bool rows_straddle_lines(const GemmProblem &q) {
     return q.m > 64 && inside(q.a, q.sam, q.a_batch);
 }
 
+constexpr const char *kLinesNote = "rows by whole lines";  // (of a launch)
+
 // ... and whether that pays: another line has to land before the first step, which short contractions do not make up for.  In one piece from a K of
 // 256 on with a transposed rhs and of 768 without, and 5e8 products (bf16, us, k tiles / lines: 64 x 64 tiles 4096 x 4096 x 72 18.5 / 21.1, 2048 x 1024 x
 // 136 4.7 / 5.0, 1024 x 512 x 520 4.2 / 4.5, 4096 x 1024 x 264 8.8 / 8.4; not transposed 4096 x 1024 x 264 7.9 / 8.3, x 776 15.7 / 14.6; 128 x 128 tiles 4096 x 4096 x 24
@@ -175,7 +177,10 @@ bool lines_pay(const GemmProblem &q, int bm, int bn, bool in_parts) {
 template <typename T, int BM, int BN, int BK, int WM, int WN, int kStages, int kOcc, int kAblate, int kLoad, int kAux, bool kTail, bool kLines>
 hipError_t fast_launch_typed(const GemmProblem &q, hipStream_t stream) {
     if constexpr (kLines)
-        if (rows_straddle_lines(q) && lines_pay(q, BM, BN, false)) return fast_launch_form<T, BM, BN, BK, WM, WN, 5, kOcc, kAblate, kLoad, kAux, kTail, true>(q, stream);
+        if (rows_straddle_lines(q) && lines_pay(q, BM, BN, false)) {
+            note_launch_detail(kLinesNote);
+            return fast_launch_form<T, BM, BN, BK, WM, WN, 5, kOcc, kAblate, kLoad, kAux, kTail, true>(q, stream);
+        }
     return fast_launch_form<T, BM, BN, BK, WM, WN, kStages, kOcc, kAblate, kLoad, kAux, kTail, false>(q, stream);
 }
 
@@ -336,7 +341,9 @@ hipError_t split_launch_typed(const GemmProblem &q, hipStream_t stream) {
         if (b_is_transposed(q)) gemm_nn_fast_kernel<T, BM, BN, BK, WM, WN, kRing, kOcc, kPlain, 0, 1, 0, true, true, true, true, kByLines><<<grid, block, 0, stream>>>(p);
         else gemm_nn_fast_kernel<T, BM, BN, BK, WM, WN, kRing, kOcc, kPlain, 0, 1, 0, true, false, true, true, kByLines><<<grid, block, 0, stream>>>(p);
     };
-    if (kLines && rows_straddle_lines(q) && lines_pay(q, BM, BN, true)) launch(std::integral_constant<int, kLines ? 5 : kStages>(), std::integral_constant<bool, kLines>());
+    const bool by_lines = kLines && rows_straddle_lines(q) && lines_pay(q, BM, BN, true);
+    if (by_lines) note_launch_detail(kLinesNote);
+    if (by_lines) launch(std::integral_constant<int, kLines ? 5 : kStages>(), std::integral_constant<bool, kLines>());
     else launch(std::integral_constant<int, kStages>(), std::false_type());
     hipError_t err = hipGetLastError();
     if (err != hipSuccess) return err;
@@ -714,8 +721,12 @@ hipError_t cut_launch(const GemmProblem &q, hipStream_t stream) {
     int rest = (int64_t)ceil_div(left.m, 128) * ceil_div(left.n, 128) <= compute_units() ? heuristic_choice(left, 0, 0, 0) : (int)kDeep128x128x64;
     if (rest <= kAnyStride || !kInstances[rest].accepts(left)) rest = kDeep128x128x64;
     hipError_t result = kInstances[rest].launch(left, stream);  // (first: a split-K instance may find no scratch memory)
-    if ((int)result == NINETOOTHED_NO_KERNEL && is_split(rest)) result = kInstances[kDeep128x128x64].launch(left, stream);
+    if ((int)result == NINETOOTHED_NO_KERNEL && is_split(rest)) {
+        rest = kDeep128x128x64;
+        result = kInstances[rest].launch(left, stream);
+    }
     if (result != hipSuccess) return result;
+    note_launch_detail(kInstances[rest].name);
     return kInstances[kInstances[k256x256x32].accepts(whole) ? k256x256x32 : kTail256x256x32].launch(whole, stream);
 }
 
@@ -1276,6 +1287,7 @@ NineToothedResult launch_nt_gemm_config(NineToothedStream stream, int config, Ni
     if (int err = build_problem(q, &input, mat1, mat2, &beta, &alpha, output, dtype, output_dtype)) return err;
     if (q.m == 0 || q.n == 0) return 0;
     if (!kInstances[config].accepts(q)) return NINETOOTHED_NO_KERNEL;
+    note_launch(kLaunchGemm, config, kInstances[config].name);
     return (int)kInstances[config].launch(q, (hipStream_t)stream);
 }
 

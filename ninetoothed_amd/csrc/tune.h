@@ -32,10 +32,11 @@ bool tune_register_check(int kind, TuneChoiceCheck check);
 constexpr int kTuneFileFormat = 6;
 
 // Which kernel served the latest launch_nt_* call of the calling host thread: the launch functions leave a note
-// (four thread-local stores), nt_last_launch formats it.  `name` must point to a string that lives as long as
+// (five thread-local stores), nt_last_launch formats it.  `name` must point to a string that lives as long as
 // the library (a literal or an instance table entry); `parts` of more than 1 follow it.
 enum LaunchProgram { kLaunchNone = 0, kLaunchGemm, kLaunchAttention, kLaunchConv2d, kLaunchSoftmax, kLaunchMap };
 void note_launch(int program, int choice, const char *name, int parts = 1);
+void note_launch_detail(const char *detail);  // follows the note of the launch under way; a string that lives as long
 
 // Times candidates 0 .. candidates - 1 on `stream` with device events and reports the fastest.  `launch(i)` returns 0,
 // NINETOOTHED_NO_KERNEL (the candidate does not take the problem: skipped) or an error (returned).

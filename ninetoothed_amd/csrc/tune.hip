@@ -82,6 +82,7 @@ thread_local int t_launch_program = kLaunchNone;
 thread_local int t_launch_choice = -1;
 thread_local const char *t_launch_name = nullptr;
 thread_local int t_launch_parts = 1;
+thread_local const char *t_launch_detail = nullptr;
 }  // namespace
 
 void note_launch(int program, int choice, const char *name, int parts) {
@@ -89,7 +90,10 @@ void note_launch(int program, int choice, const char *name, int parts) {
     t_launch_choice = choice;
     t_launch_name = name;
     t_launch_parts = parts;
+    t_launch_detail = nullptr;
 }
+
+void note_launch_detail(const char *detail) { t_launch_detail = detail; }
 
 }  // namespace nt
 
@@ -106,7 +110,7 @@ NineToothedResult nt_last_launch(char *buffer, int size) {
     const char *name = t_launch_name ? t_launch_name : "";
     if (program == kLaunchNone) snprintf(buffer, (size_t)size, "none");
     else if (t_launch_parts > 1) snprintf(buffer, (size_t)size, "%s %d: %s, %d parts", programs[program], t_launch_choice, name, t_launch_parts);
-    else snprintf(buffer, (size_t)size, "%s %d: %s", programs[program], t_launch_choice, name);
+    else snprintf(buffer, (size_t)size, "%s %d: %s%s%s", programs[program], t_launch_choice, name, t_launch_detail ? ", " : "", t_launch_detail ? t_launch_detail : "");
     return 0;
 }
 

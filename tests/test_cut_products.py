@@ -34,6 +34,7 @@ def _check(out, expected, unit, magnitude, k, extra=0.0):
         (33000, 304, 512, False, "rows"),
         (8500, 1800, 2048, True, "rows"),  # 272 tiles, 16 left with K in parts
         (1030, 16640, 2304, False, "columns"),  # five rows of tiles, 70 left
+        (24988, 2040, 2304, True, "rows"),  # 784 tiles, 16 left with K in parts: more rounds than launch_nt_linear's own rule for last rows takes
     ),
 )
 def test_both_parts_with_every_epilogue(m, n, k, transposed, kind, dtype):
@@ -53,9 +54,11 @@ def test_both_parts_with_every_epilogue(m, n, k, transposed, kind, dtype):
     def untouched(buffer):
         return bool((buffer[m] == 7.0).all()) and bool((buffer[:, n:] == 7.0).all())
 
+    in_parts = (m, n) in ((8500, 1800), (24988, 2040))
     for element, tag in ((dtype, name), (torch.float32, "fp32")):
         buffer, out = output(element)
         assert library.launch_nt_gemm_config(stream, index, null, like(lhs), like(rhs), null, null, like(out), TAGS[name], TAGS[tag]) == 0
+        assert ("lds-direct tails split-k" in runtime.last_launch()) == in_parts
         _check(out, product, unit if element == dtype else 2.0**-24, magnitude, k)
         assert untouched(buffer)
     bias = torch.randn(m, n, device="cuda").to(dtype)
@@ -68,6 +71,7 @@ def test_both_parts_with_every_epilogue(m, n, k, transposed, kind, dtype):
     column = torch.randn(n, device="cuda")
     buffer, out = output(dtype)
     runtime.check(library.launch_nt_linear(stream, like(lhs), like(rhs), like(column), TAGS["fp32"], 0.5, 0.0, like(out), TAGS[name], 0, 0, 0))
+    assert "whole rounds" in runtime.last_launch() if m != 8500 else "the last rows with the k range in parts" in runtime.last_launch()
     _check(out, (0.5 * product + column.double()).clamp_min(0.0), unit, magnitude + column.double().abs(), k, 2.0**-23)
     assert untouched(buffer)
 

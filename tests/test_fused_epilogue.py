@@ -75,6 +75,13 @@ def test_addmm_inputs_at_the_edges_of_tiles(m, n, k, form):
     """The input's values are asked for before the product is done, those of rows and columns behind the output's last ones from there: NaN
     around the input would show in the output.  (The product rounds to fp16 before it is combined, the result once more: an ulp each of the largest value, and an ulp where
     the product's own rounding falls the other way.)"""
+    mat1, mat2, input, output, expected, atol = _addmm_case(m, n, k, form)
+    kernel = ninetoothed.make(programs.addmm.arrangement, programs.addmm.application, programs.addmm.tensors())
+    kernel(input, mat1, mat2, 0.5, 2.0, output)
+    assert torch.allclose(output.double(), expected, rtol=0, atol=atol)
+
+
+def _addmm_case(m, n, k, form):
     mat1, mat2 = torch.randn(m, k, device="cuda").half(), (torch.randn(k, n, device="cuda") * k**-0.5).half()
     values = torch.randn(1 if form == "one row" else m, n, device="cuda").half()
     if form == "odd pitch":
@@ -87,9 +94,24 @@ def test_addmm_inputs_at_the_edges_of_tiles(m, n, k, form):
     if form == "one row":
         input = input.expand(m, n)
     output = input if form == "in place" else torch.full((m, n), float("nan"), dtype=torch.float16, device="cuda")
-    kernel = ninetoothed.make(programs.addmm.arrangement, programs.addmm.application, programs.addmm.tensors())
-    kernel(input, mat1, mat2, 0.5, 2.0, output)
     product = (mat1.double() @ mat2.double()).half().double()
     expected = 0.5 * values.double() + 2.0 * product
     ulp = 2.0**-10 * float(expected.abs().max())
-    assert torch.allclose(output.double(), expected, rtol=0, atol=3 * ulp)
+    return mat1, mat2, input, output, expected, 3 * ulp
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("form", ("whole", "odd pitch", "one row", "columns apart", "in place"))
+@pytest.mark.parametrize("tile", ("256x256x32", "128x256x32", "128x128x64 waves 2x2", "128x128x64 waves 2x4", "64x64x64", "64x64x128", "64x128x64"))
+def test_addmm_inputs_on_every_tile(tile, form):
+    """As above, on each instance by its index: a lane holds 2 to 16 chunks of the input, and the last rows and columns of tiles are not there."""
+    from ninetoothed_amd import runtime
+
+    (index,) = (i for i, name in enumerate(runtime.gemm_config_names()) if name.startswith(tile) and name.endswith("lds-direct tails"))
+    like, tag = runtime.ArgumentTensor.from_torch_tensor, runtime.DATA_TYPE_INDEX["fp16"]
+    beta, alpha = (runtime.ArgumentTensor.from_scalar(value) for value in (0.5, 2.0))
+    for m, n, k in ((517, 776, 136), (250, 8, 64), (258, 264, 328)):
+        mat1, mat2, input, output, expected, atol = _addmm_case(m, n, k, form)
+        arguments = like(input), like(mat1), like(mat2), beta, alpha, like(output)
+        runtime.check(runtime.library().launch_nt_gemm_config(runtime.current_stream(), index, *arguments, tag, tag))
+        assert torch.allclose(output.double(), expected, rtol=0, atol=atol)
