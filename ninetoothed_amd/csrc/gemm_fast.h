@@ -906,11 +906,10 @@ __global__ __launch_bounds__(WM *WN * 64, kWavesPerSimd) void gemm_nn_fast_kerne
     // addmm: the input's values of the wave's whole tile (64 registers at most, which the fragments leave) are asked for before the last fills
     // have landed.  Asked for where they are used, behind the branch for rows that are not there, they were a chain
     // of trips to memory, 16 in a wave's 128 x 64 tile: 4918 x 16160 x 576 bf16 155 -> 130 us, 6606 x 2208 x 448 30.3 -> 24.9, 8192^3 fp16 786 -> 775.
-    // Not where a row's last chunk is partial or columns lie apart, nor where all rows are one, which the first load brings near: 7341 x 7208 x 16 59.6 us
-    // ahead, 45.2 where used, fp16 1519 x 4232 x 64 10.0 and 9.1.
+    // Not where a row's last chunk is partial or columns lie apart.
     constexpr int kInputChunks = kEpilogue == kAddmm ? kCChunks / 2 : 1, kInputBlocks = kEpilogue == kAddmm ? TM : 1;
     static_assert(kInputChunks * kInputBlocks <= 16, "registers for the input");
-    const bool input_ahead = kEpilogue == kAddmm && p.bias_stride_n == 1 && p.bias_stride_m != 0 && p.n % 8 == 0;
+    const bool input_ahead = kEpilogue == kAddmm && p.bias_stride_n == 1 && p.n % 8 == 0;
     unaligned_vec8 input[kInputBlocks][kInputChunks];
     if constexpr (kEpilogue == kAddmm) {
         if (input_ahead) {
