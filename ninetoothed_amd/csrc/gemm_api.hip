@@ -1116,21 +1116,16 @@ int run_gemm(hipStream_t stream, const GemmProblem &q, int bm, int bn, int bk, b
     int choice = -1;
     if ((bm <= 0 || bn <= 0) && q.batch == 1) choice = lookup_tuned(q);  // (tuned choices are recorded for single products)
     // (choices are timed and recorded for the plain product, which the any-stride kernel may win; it has no linear epilogue)
-    if (choice < 0 || !kInstances[choice].accepts(q) || (choice == kAnyStride && q.linear)) choice = heuristic_choice(q, bm, bn, bk);
+    GemmProblem asked = q;
+    asked.hinted = bm > 0 || bn > 0 || bk > 0;
+    if (choice < 0 || !kInstances[choice].accepts(asked) || (choice == kAnyStride && q.linear)) choice = heuristic_choice(asked, bm, bn, bk);
     if (choice < 0 || (choice == kAnyStride && q.linear)) return NINETOOTHED_NO_KERNEL;
     if (choice == kAnyStride && may_copy) {
         const int copied = run_gemm_on_repacked_copies(stream, q, bm, bn, bk);
         if (copied != NINETOOTHED_NO_KERNEL) return copied;
     }
     note_launch(kLaunchGemm, choice, kInstances[choice].name);
-    int result;
-    if (bm > 0 || bn > 0 || bk > 0) {
-        GemmProblem hinted = q;
-        hinted.hinted = true;
-        result = (int)kInstances[choice].launch(hinted, stream);
-    } else {
-        result = (int)kInstances[choice].launch(q, stream);
-    }
+    int result = (int)kInstances[choice].launch(asked, stream);
     if (result == NINETOOTHED_NO_KERNEL && is_split(choice)) {  // a split-K instance without scratch memory
         for (int fallback : {(int)kTail64x64x64, (int)kTail128x128x64, (int)kTail256x256x32, (int)kAnyStride})
             if (kInstances[fallback].accepts(q) && !(fallback == kAnyStride && q.linear)) {

@@ -88,3 +88,4 @@ def test_which_products_are_cut():
     assert not served(256, 65536, 512)  # one whole round
     assert not served(520, 32512, 448)  # a short contraction
     assert not served(520, 32512, 512, (256, 256, 32))  # block sizes: one launch, no scratch memory
+    assert not served(520, 32512, 512, (256, 0, 0)) and not served(520, 32512, 512, (0, 0, 32))  # ... also some of them
