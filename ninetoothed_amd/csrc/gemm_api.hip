@@ -88,14 +88,16 @@ bool fast_accepts(const GemmProblem &q) {
 }
 
 // Whether a product's tiles are dealt to the XCDs one by one (bit 8 of GemmParams::order) instead of in contiguous ranges: a tall product -- at least 9 rows
-// of tiles and twice as many as columns -- whose number of tiles is no multiple of 8.  One by one, a strip of 8 tile rows gives every XCD a row
+// of tiles and three times as many as columns, with K in parts twice as many -- whose number of tiles is no multiple of 8.  One by one, a strip of 8 tile rows gives every XCD a row
 // of its own, whose panel of the lhs it reads once for all the few columns; ranges read it into two or three L2s.  Us, ranges / one by one: 128 x 128
 // tiles with K in parts 19 x 3 of them, K 12800 40.7 / 32.8, 17 x 3, 6400 24.2 / 20.5, 23 x 2, 6400 22.4 / 20.2, 12 x 7, 12800 44.4 / 41.9; 64 x 64 in parts 41 x 2,
 // 12800 27.2 / 23.9; 128 x 256 39 x 7, 2368 53.1 / 47.8; 128 x 128 on a deep ring 17 x 3, 4672 29.0 / 27.6.  Less tall ones gain by ranges (11 x 7 of 128 x 128 in parts
-// 0.9 of the time), and so do 256 x 256 tiles (44 x 9, K 4672 0.92).
-bool tiles_one_by_one(const GemmParams &p, int bm) { return bm <= 128 && p.tiles_m * (int64_t)p.tiles_n % 8 != 0 && p.tiles_n > 1 && p.tiles_m >= 9 && p.tiles_m / 2 >= p.tiles_n; }
+// 0.9 of the time, 46 x 19 in one piece 0.91), and so do 256 x 256 tiles (44 x 9, K 4672 0.92).
+bool tiles_one_by_one(const GemmParams &p, int bm, bool in_parts) {
+    return bm <= 128 && p.tiles_m * (int64_t)p.tiles_n % 8 != 0 && p.tiles_n > 1 && p.tiles_m >= 9 && p.tiles_m / (in_parts ? 2 : 3) >= p.tiles_n;
+}
 
-void fill_params(GemmParams &p, const GemmProblem &q, int bm, int bn) {
+void fill_params(GemmParams &p, const GemmProblem &q, int bm, int bn, bool in_parts = false) {
     p.a = q.a;
     p.b = q.b;
     p.c = q.c;
@@ -115,7 +117,7 @@ void fill_params(GemmParams &p, const GemmProblem &q, int bm, int bn) {
     p.beta = q.beta;
     p.tiles_m = (q.m + bm - 1) / bm;
     p.tiles_n = (q.n + bn - 1) / bn;
-    p.order = g_tile_order | (tiles_one_by_one(p, bm) ? 0x100 : 0);
+    p.order = g_tile_order | (tiles_one_by_one(p, bm, in_parts) ? 0x100 : 0);
     p.bias_vector = q.bias != nullptr && q.sin == 1 && q.sim % 8 == 0 && ((uintptr_t)q.bias & 15) == 0 && q.n % 8 == 0 && (q.batch == 1 || q.bias_batch % 8 == 0);
     p.c_vector = ((uintptr_t)q.c & 15) == 0 && q.scm % 8 == 0 && q.n % 8 == 0 && (q.batch == 1 || q.c_batch % 8 == 0);
     p.kt_per_split = 0;
@@ -162,16 +164,17 @@ bool rows_straddle_lines(const GemmProblem &q) {
 constexpr const char *kLinesNote = "rows by whole lines";  // (of a launch)
 
 // ... and whether that pays: another line has to land before the first step, which short contractions do not make up for.  In one piece from a K of
-// 256 on with a transposed rhs and of 768 without, and 5e8 products (bf16, us, k tiles / lines: 64 x 64 tiles 4096 x 4096 x 72 18.5 / 21.1, 2048 x 1024 x
-// 136 4.7 / 5.0, 1024 x 512 x 520 4.2 / 4.5, 4096 x 1024 x 264 8.8 / 8.4; not transposed 4096 x 1024 x 264 7.9 / 8.3, x 776 15.7 / 14.6; 128 x 128 tiles 4096 x 4096 x 24
-// 13.3 / 15.0, 2048 x 1024 x 392 6.7 / 6.4).  In parts, of a few k tiles each, on 128 x 128 tiles only with a transposed rhs and 32 tiles or more (256 x
-// 512 x 16392 19.3 / 20.9, 1024 x 1024 x 8200 34.3 / 32.6; not transposed 270 x 232 x 16392 16.5 / 19.3, 1024 x 512 x 8200 22.4 / 23.8), on 64 x 64 from 16 tiles on
+// 256 on with a transposed rhs and of 768 without, and 5e8 products, of batches, whose matrices begin anywhere in a line too, 1e8 (bf16, us, k tiles / lines:
+// 64 x 64 tiles 4096 x 4096 x 72 18.5 / 21.1, 2048 x 1024 x 136 4.7 / 5.0, 1024 x 512 x 520 4.2 / 4.5, 4096 x 1024 x 264 8.8 / 8.4, 11 of 66 x 288 x 760 6.7 / 6.1; not transposed
+// 4096 x 1024 x 264 7.9 / 8.3, x 776 15.7 / 14.6; 128 x 128 tiles 4096 x 4096 x 24 13.3 / 15.0, 2048 x 1024 x 392 6.7 / 6.4).  In parts, of a few k tiles each, on 128 x 128 tiles only
+// with a transposed rhs, from 8 tiles on where K is at most 9000, from 32 on otherwise (416 x 832 x 3800 16.3 / 15.0, 1024 x 1024 x 16392 55.1 / 50.9, but 256 x
+// 512 x 16392 19.3 / 20.9, 166 x 120 x 3488 9.6 / 10.5; not transposed 270 x 232 x 16392 16.5 / 19.3, 1024 x 512 x 8200 22.4 / 23.8), on 64 x 64 from 16 tiles on
 // and 64 without (128 x 128 x 8200 9.4 / 10.1, 1024 x 1024 x 8200 38.3 / 34.4).
 bool lines_pay(const GemmProblem &q, int bm, int bn, bool in_parts) {
     const bool transposed = b_is_transposed(q);
-    if (!in_parts) return q.k >= (transposed ? 256 : 768) && (double)q.batch * q.m * q.n * q.k >= 5e8;
+    if (!in_parts) return q.k >= (transposed ? 256 : 768) && (double)q.batch * q.m * q.n * q.k >= (q.batch > 1 ? 1e8 : 5e8);
     const int64_t tiles = (int64_t)ceil_div(q.m, bm) * ceil_div(q.n, bn);
-    return bm == 128 ? transposed && tiles >= 32 : tiles >= (transposed ? 16 : 64);
+    return bm == 128 ? transposed && tiles >= (q.k <= 9000 ? 8 : 32) : tiles >= (transposed ? 16 : 64);
 }
 
 template <typename T, int BM, int BN, int BK, int WM, int WN, int kStages, int kOcc, int kAblate, int kLoad, int kAux, bool kTail, bool kLines>
@@ -327,7 +330,7 @@ hipError_t split_launch_typed(const GemmProblem &q, hipStream_t stream) {
         if (scratch == nullptr) return (hipError_t)NINETOOTHED_NO_KERNEL;  // no scratch (graph capture, out of memory): the caller takes a one-pass instance
     }
     GemmParams result;  // (the summing kernel's)
-    fill_params(result, q, BM, BN);
+    fill_params(result, q, BM, BN, true);
     GemmParams p = result;
     p.c = scratch;
     p.ldc = pitch;
