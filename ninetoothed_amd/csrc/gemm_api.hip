@@ -92,9 +92,13 @@ bool fast_accepts(const GemmProblem &q) {
 // of its own, whose panel of the lhs it reads once for all the few columns; ranges read it into two or three L2s.  Us, ranges / one by one: 128 x 128
 // tiles with K in parts 19 x 3 of them, K 12800 40.7 / 32.8, 17 x 3, 6400 24.2 / 20.5, 23 x 2, 6400 22.4 / 20.2, 12 x 7, 12800 44.4 / 41.9; 64 x 64 in parts 41 x 2,
 // 12800 27.2 / 23.9; 128 x 256 39 x 7, 2368 53.1 / 47.8; 128 x 128 on a deep ring 17 x 3, 4672 29.0 / 27.6.  Less tall ones gain by ranges (11 x 7 of 128 x 128 in parts
-// 0.9 of the time, 46 x 19 in one piece 0.91), and so do 256 x 256 tiles (44 x 9, K 4672 0.92).
-bool tiles_one_by_one(const GemmParams &p, int bm, bool in_parts) {
-    return bm <= 128 && p.tiles_m * (int64_t)p.tiles_n % 8 != 0 && p.tiles_n > 1 && p.tiles_m >= 9 && p.tiles_m / (in_parts ? 2 : 3) >= p.tiles_n;
+// 0.9 of the time, 46 x 19 in one piece 0.91), and so do 256 x 256 tiles (44 x 9, K 4672 0.92) -- but for products with
+// next to no contraction whose output's rows are no whole lines: one by one an XCD writes neighbouring tiles of a row at the same time, whose shared lines meet
+// in its L2 (bf16, ranges / one by one: 7388 x 9416 x 88 73.4 / 61.3, 7341 x 7208 x 16 57.6 / 45.3, 6692 x 5960 x 88 52.2 / 45.5; a K of 192 no difference).
+bool tiles_one_by_one(const GemmParams &p, int bm, bool in_parts, int64_t out_row_bytes) {
+    if (p.tiles_m * (int64_t)p.tiles_n % 8 == 0) return false;
+    if (bm > 128) return p.k <= 128 && out_row_bytes % 128 != 0;
+    return p.tiles_n > 1 && p.tiles_m >= 9 && p.tiles_m / (in_parts ? 2 : 3) >= p.tiles_n;
 }
 
 void fill_params(GemmParams &p, const GemmProblem &q, int bm, int bn, bool in_parts = false) {
@@ -117,7 +121,7 @@ void fill_params(GemmParams &p, const GemmProblem &q, int bm, int bn, bool in_pa
     p.beta = q.beta;
     p.tiles_m = (q.m + bm - 1) / bm;
     p.tiles_n = (q.n + bn - 1) / bn;
-    p.order = g_tile_order | (tiles_one_by_one(p, bm, in_parts) ? 0x100 : 0);
+    p.order = g_tile_order | (tiles_one_by_one(p, bm, in_parts, q.scm * (q.out_dtype == NINETOOTHED_FLOAT32 ? 4 : 2)) ? 0x100 : 0);
     p.bias_vector = q.bias != nullptr && q.sin == 1 && q.sim % 8 == 0 && ((uintptr_t)q.bias & 15) == 0 && q.n % 8 == 0 && (q.batch == 1 || q.bias_batch % 8 == 0);
     p.c_vector = ((uintptr_t)q.c & 15) == 0 && q.scm % 8 == 0 && q.n % 8 == 0 && (q.batch == 1 || q.c_batch % 8 == 0);
     p.kt_per_split = 0;
