@@ -285,14 +285,19 @@ int window_positions(const Conv2dRequest &q) {
 // Whether this kernel is expected to be faster than the repacking path, in microseconds, by both models fitted to 320 convolutions (1 to
 // 32 images of 7 x 7 to 112 x 112, 32 to 256 channels, 16 to 512 filters, steps 1 and 2; 8 and 6 % off on average): it wins where its
 // workgroups fill the chip about once -- fewer leave CUs idle that the other path's parts of the contraction use, more pay the long block.  Of
-// the 320 the 44 it is taken for run in 0.84 of the other paths' time on average, 1.03 at worst.
+// the 320 the 44 it is taken for run in 0.84 of the other paths' time on average, 1.03 at worst.  With steps of 2 and more a block takes longer the fuller the chip is, and
+// the data hardly counts beside it (379 others of up to 512 channels, steps 1 to 3): without the second estimate the longer contractions of such layers were taken too (us, repacked /
+// here: 14 images of 240 x 112 x 115, 264 filters 139 / 168; 9 of 328 x 56 x 59, 352 44 / 53).  With it the 93 of 260 drawn ones that are taken run in 0.83 of the
+// other path's time, three of them in more than 1.04 (480 channels of 112 x 115, 208 filters, step 2 65.3 / 75.5), two of 103 that were taken before in more than 1.02.
 bool window_pays(const Conv2dRequest &q) {
     const int units = std::max(1, compute_units());
-    const int64_t positions = (int64_t)q.N * q.P * q.Q;
-    const float rounds = (float)(((positions + kWindowBM - 1) / kWindowBM * ceil_div(q.K, kWindowBN) + units - 1) / units);
+    const int64_t positions = (int64_t)q.N * q.P * q.Q, workgroups = (positions + kWindowBM - 1) / kWindowBM * ceil_div(q.K, kWindowBN);
+    const float rounds = (float)((workgroups + units - 1) / units), blocks = (float)ceil_div(q.C, 32);
     const float megabytes = ((float)q.N * q.C * q.H * q.W + (float)positions * q.K + (float)q.K * q.C * q.R * q.S) * 2e-6f;
     const bool scattered = conv2d_dense_output(q) == 0 || (conv2d_dense_output(q) == 1 && q.P * q.Q % 8 != 0);
-    const float time = 2.8f + rounds * (2.2f + 2.85f * (float)ceil_div(q.C, 32) + (scattered ? 5.3f : 0.0f)) + 0.153f * megabytes;
+    float time = 2.8f + rounds * (2.2f + 2.85f * blocks + (scattered ? 5.3f : 0.0f)) + 0.153f * megabytes;
+    if (q.stride_h > 1 || q.stride_w > 1)
+        time = std::max(time, 2.7f + rounds * (2.1f + 3.39f * blocks + (scattered ? 3.9f : 0.0f)) + 0.47f * blocks * (float)workgroups / (float)units + 0.063f * megabytes);
     return time < 0.95f * conv2d_repacked_time(q);
 }
 
