@@ -679,20 +679,15 @@ int skinny_choice(const GemmProblem &q) {
 // 14208 x 12736 (25) 483 / 354, 4635 x 4736 x 12544 (114) 467 / 432, 2470 x 9536 x 1280 (130) 57.7 / 55.8; more left: 2311 x 11328 x 3136 (200) 130 / 139.
 // Of a short K, 2967 x 7872 x 512 (120) 31.9 / 28.9, but 2058 x 7680 x 512 (18) has 19.3 on 128 x 256 tiles against 22, which only the tuner knows.
 template <bool kColumns>
-int64_t cut_whole(const GemmProblem &q) {  // columns (rows) of 256 x 256 tiles that fill whole rounds
-    const int64_t along = ceil_div(kColumns ? q.n : q.m, 256), across = ceil_div(kColumns ? q.m : q.n, 256), units = std::max(1, compute_units());
+int64_t cut_whole(const GemmProblem &q, int64_t units) {  // columns (rows) of 256 x 256 tiles that fill whole rounds
+    const int64_t along = ceil_div(kColumns ? q.n : q.m, 256), across = ceil_div(kColumns ? q.m : q.n, 256);
     return along * across / units * units / across;
 }
 
 template <bool kColumns>
-int64_t cut_left(const GemmProblem &q) {  // 256 x 256 tiles that do not
-    return (ceil_div(kColumns ? q.n : q.m, 256) - cut_whole<kColumns>(q)) * ceil_div(kColumns ? q.m : q.n, 256);
-}
-
-template <bool kColumns>
-void cut_problem(const GemmProblem &q, GemmProblem &whole, GemmProblem &left) {
+void cut_problem(const GemmProblem &q, int64_t whole_tiles, GemmProblem &whole, GemmProblem &left) {
     const int64_t size = 2, out_size = q.out_dtype == NINETOOTHED_FLOAT32 ? 4 : 2;
-    const int64_t at = cut_whole<kColumns>(q) * 256;
+    const int64_t at = whole_tiles * 256;
     whole = left = q;
     if (kColumns) {
         whole.n = (int)at;
@@ -713,19 +708,24 @@ void cut_problem(const GemmProblem &q, GemmProblem &whole, GemmProblem &left) {
 template <bool kColumns>
 bool cut_accepts(const GemmProblem &q) {
     if ((q.dtype != NINETOOTHED_FLOAT16 && q.dtype != NINETOOTHED_BFLOAT16) || q.batch != 1 || q.hinted || q.fixed_scratch != nullptr || q.m <= 0 || q.n <= 0) return false;
-    const int64_t tiles = (int64_t)ceil_div(q.m, 256) * ceil_div(q.n, 256), whole = cut_whole<kColumns>(q), units = compute_units();
-    if (units <= 0 || kColumns != (q.m <= q.n) || tiles <= units || tiles % units == 0 || q.k < 512 || whole < 1 || 2 * cut_left<kColumns>(q) > units) return false;
-    if (tiles > 4 * units + units / 2) return false;  // (what a round costs shrinks to the spread between runs)
+    const int64_t along = ceil_div(kColumns ? q.n : q.m, 256), across = ceil_div(kColumns ? q.m : q.n, 256), tiles = along * across;
+    // (asking for the number of compute units takes longer than the rest of a small product's choice: no part has as few as 16)
+    if (kColumns != (q.m <= q.n) || q.k < 512 || tiles <= 16) return false;
+    const int64_t units = compute_units();
+    if (units <= 0 || tiles <= units || tiles % units == 0 || tiles > 4 * units + units / 2) return false;  // (what a round costs shrinks to the spread between runs)
+    const int64_t whole = cut_whole<kColumns>(q, units);
+    if (whole < 1 || 2 * (along - whole) * across > units) return false;
     GemmProblem top, left;
-    cut_problem<kColumns>(q, top, left);
+    cut_problem<kColumns>(q, whole, top, left);
     return kInstances[kTail256x256x32].accepts(top) && kInstances[kDeep128x128x64].accepts(left);
 }
 
 template <bool kColumns>
 hipError_t cut_launch(const GemmProblem &q, hipStream_t stream) {
+    const int64_t units = std::max(1, compute_units());
     GemmProblem whole, left;
-    cut_problem<kColumns>(q, whole, left);
-    int rest = (int64_t)ceil_div(left.m, 128) * ceil_div(left.n, 128) <= compute_units() ? heuristic_choice(left, 0, 0, 0) : (int)kDeep128x128x64;
+    cut_problem<kColumns>(q, cut_whole<kColumns>(q, units), whole, left);
+    int rest = (int64_t)ceil_div(left.m, 128) * ceil_div(left.n, 128) <= units ? heuristic_choice(left, 0, 0, 0) : (int)kDeep128x128x64;
     if (rest <= kAnyStride || !kInstances[rest].accepts(left)) rest = kDeep128x128x64;
     hipError_t result = kInstances[rest].launch(left, stream);  // (first: a split-K instance may find no scratch memory)
     if ((int)result == NINETOOTHED_NO_KERNEL && is_split(rest)) {
