@@ -41,11 +41,11 @@ struct ConvWindowParams {
 
 // Tiles of 224 positions x 64 filters on eight waves of 112 x 32: two groups of four waves take turns with the taps and add up at the end.
 // What bounds it where the chip holds all tiles at once: a chain per block of channels -- the loads' way from memory, the filters' twice
-// through LDS, nine taps -- of which MFMAs are a fifth (3 us a block of 32 channels, and 6 for the launch, the first loads and the output).  So: large tiles,
+// through LDS, nine taps -- in which MFMAs are busy 15 % of the time, vector instructions 43 %, LDS 33 % (3 us a block of 32 channels, and 6 for the launch, the first loads and the output).  So: large tiles,
 // that few workgroups load the same filters (112 positions 15 us where these take 13), 64 filters rather than 128, whose values would take twice as long
 // through LDS (14), loads dealt out between the taps (all at once they held up the first tap by 1.2 us), quotients by reciprocals before the first loads
 // (0.8 us).  Exchanging the filters' pieces inside quads of lanes instead of LDS costs more vector instructions than it saves (18 us).
-// 32 images of 64 x 56 x 56, 128 filters, step 2: 20.2 -> 13.2 us; 64 filters, step 1: 28.5 -> 21; 32 of 128 x 28 x 28, 128 filters: 22.8 -> 17.7;
+// 32 images of 64 x 56 x 56, 128 filters, step 2, alone: 20.2 -> 13.2 us (among others 19.2 -> 12.1); 64 filters, step 1: 28.5 -> 21; 32 of 128 x 28 x 28, 128 filters: 22.8 -> 17.7;
 // 8 of 64 x 112 x 112, 128 filters, step 2: 18.5 -> 12.6.
 template <typename T, int R, int S>
 __global__ __launch_bounds__(kWindowThreads, 2) void conv2d_window_kernel(ConvWindowParams p) {
