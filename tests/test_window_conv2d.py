@@ -102,6 +102,7 @@ def test_the_choice_follows_the_size():
         assert "conv2d_window_kernel" in served(32, 64, 56, 128, 2)
         assert "conv2d_repack_kernel" in served(1, 128, 14, 64, 2)  # few workgroups: the contraction in parts
         assert "conv2d_repack_kernel" in served(32, 256, 56, 512, 2)  # several rounds of long blocks
+        assert "conv2d_repack_kernel" in served(9, 328, 56, 352, 2)  # ... and one of them, with steps of 2
 
 
 @pytest.mark.parametrize("stride", (1, 2))
